@@ -32,15 +32,19 @@ sys.path.insert(0, str(ROOT))
 
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 PEAK_F32_TFLOPS = 157.3  # MI355X dense fp32 MFMA
+PEAK_SPLIT_TFLOPS = PEAK_BF16_TFLOPS / 3  # fp32 products as three f16 MFMAs (f16 runs at the bf16 rate)
 PEAK_HBM_GBS = 8000.0  # MI355X HBM3E
 
 
 def _peak(bound: str) -> tuple[float, str, float]:
-    """(published peak, unit, divisor of work/s) for a kernel's bound: bf16 MFMA, fp32 MFMA or HBM."""
+    """(published peak, unit, divisor of work/s) for a kernel's bound: bf16 MFMA, fp32 MFMA, split f16
+    MFMA or HBM."""
     if bound == "mfma":
         return PEAK_BF16_TFLOPS, "TFLOP/s", 1e12
     if bound == "mfma_f32":
         return PEAK_F32_TFLOPS, "TFLOP/s", 1e12
+    if bound == "mfma_split":
+        return PEAK_SPLIT_TFLOPS, "TFLOP/s", 1e12
     return PEAK_HBM_GBS, "GB/s", 1e9
 
 

@@ -6,8 +6,14 @@
 // token transitions (transition.py:52-91) compute in fp32 on fp32 inputs.  These
 // entry points do the same: fp32 operands and fp32 accumulation throughout.
 //
-//   gemm_f32      out = epi(A W^T) on v_mfma_f32_32x32x2_f32 (qkvg_f32: the four
-//                 token projections of an attention in one launch).  A wave owns a
+// The projections of the attentions, the transitions and the pairwise
+// conditioning run on split f16 operands (split.h, split_gemm.hip,
+// split_transition.hip, split_pair.hip): as accurate, and 2 to 5 times as fast.
+// Here:
+//
+//   gemm_f32      out = epi(A W^T) on v_mfma_f32_32x32x2_f32, for the products not
+//                 moved to split operands (the distogram, whose raw inputs may be
+//                 infinite, the trunk glue and the MSA-module ops).  A wave owns a
 //                 32 x 32 output block: weight rows (output channels) are the
 //                 MFMA A operand in perm32 order (pairtile.h), token rows the B
 //                 operand, so a lane ends with 16 consecutive channels of one
@@ -16,8 +22,8 @@
 //                 supplies k0 + 4h + e to MFMA e, the same k permutation on both
 //                 operands, so every k is summed once.
 //   rows_ln_f32   LayerNorm per row (biased variance, eps 1e-5), one wave per row.
-//   pair_proj_f32 pair bias: LN(z) W^T per pair row, one thread per row, written
-//                 head-major ([outer][head][inner]).
+//   pair_proj_f32 pair bias of 16- and 32-channel pair rows: LN(z) W^T, one thread
+//                 per row, written head-major ([outer][head][inner]).
 //   attn_f32      softmax(q k^T / sqrt(d) + bias; masked keys -> -1e6) v, gated by
 //                 g: flash attention on the same fp32 MFMA, a wave per 32
 //                 queries, 32-key blocks, online softmax in registers.
@@ -28,16 +34,15 @@
 #include "common.h"
 #include "internal.h"
 #include "pairtile.h"
+#include "split_gemm.h"
+#include "split_rows.h"
 
 namespace bioemu {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kGemmEpiStore = 0, kGemmEpiSigmoid = 1, kGemmEpiSwiGLU = 2, kGemmEpiResidual = 3;
-// kGemmEpiStoreT writes the transpose per sequence: row m = s * T + t, channel
-// c -> out[(s * N + c) * ldT + t] (keys contiguous, for the P.V operand).
-constexpr int kGemmEpiStoreT = 4;
+constexpr int kGemmEpiStore = 0, kGemmEpiSigmoid = 1, kGemmEpiResidual = 2;
 
 __device__ __forceinline__ f32x16 mfma_f32(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
@@ -51,9 +56,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 template <int kEpi>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                                                       const float* __restrict__ W2, const float* __restrict__ bias,
-                                                       const float* res, float* out, long long M, int K, int N,
-                                                       int T, int ldT) {
+                                                       const float* __restrict__ bias, const float* res, float* out,
+                                                       long long M, int K, int N) {
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int n = lane & 31, h = lane >> 5;
   const int nbc = N / 32;
@@ -65,20 +69,13 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
   const long long m = mb * 32 + n;
   const bool mvalid = m < M;
   const float* arow = A + (size_t)(mvalid ? m : 0) * K + 4 * h;
-  const size_t wr = (size_t)(cb * 32 + perm32(n)) * K + 4 * h;
-  const float* wrow = W + wr;
-  const float* w2row = kEpi == kGemmEpiSwiGLU ? W2 + wr : nullptr;
-  f32x16 acc = zero16(), acc2 = zero16();
+  const float* wrow = W + (size_t)(cb * 32 + perm32(n)) * K + 4 * h;
+  f32x16 acc = zero16();
   for (int k0 = 0; k0 < K; k0 += 8) {
     const f32x4 a4 = *reinterpret_cast<const f32x4*>(arow + k0);
     const f32x4 w4 = *reinterpret_cast<const f32x4*>(wrow + k0);
-    f32x4 v4;
-    if (kEpi == kGemmEpiSwiGLU) v4 = *reinterpret_cast<const f32x4*>(w2row + k0);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      acc = mfma_f32(w4[e], a4[e], acc);
-      if (kEpi == kGemmEpiSwiGLU) acc2 = mfma_f32(v4[e], a4[e], acc2);
-    }
+    for (int e = 0; e < 4; ++e) acc = mfma_f32(w4[e], a4[e], acc);
   }
   if (!mvalid) return;
   // D lane (n, h): token row m, register u <-> output channel cb*32 + 16h + u
@@ -89,15 +86,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
     float x = acc[u];
     if (bias) x += bias[c0 + u];
     if (kEpi == kGemmEpiSigmoid) x = 1.0f / (1.0f + __expf(-x));
-    if (kEpi == kGemmEpiSwiGLU) x = x / (1.0f + __expf(-x)) * acc2[u];
     v[u] = x;
-  }
-  if (kEpi == kGemmEpiStoreT) {
-    const long long sq = m / T, t = m % T;
-    float* col = out + ((size_t)sq * N + c0) * ldT + t;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) col[(size_t)u * ldT] = v[u];
-    return;
   }
   float* dst = out + (size_t)m * N + c0;
   if (kEpi == kGemmEpiResidual) {
@@ -115,65 +104,6 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 #pragma unroll
     for (int e = 0; e < 4; ++e) o4[e] = v[4 * q + e];
     *reinterpret_cast<f32x4*>(dst + 4 * q) = o4;
-  }
-}
-
-// The four token projections of an attention in one launch: column blocks
-// [0, c_s) -> q (+ q bias), [c_s, 2c_s) -> k, [2c_s, 3c_s) -> v stored
-// transposed per sequence (as kGemmEpiStoreT), [3c_s, 4c_s) -> sigmoid(g).
-// Same wave tiling as gemm_f32_kernel; the column block picks weight rows and
-// epilogue (wave-uniform).
-__global__ __launch_bounds__(256) void qkvg_f32_kernel(const float* __restrict__ A, const float* __restrict__ w_qkv,
-                                                       const float* __restrict__ w_g, const float* __restrict__ q_bias,
-                                                       float* __restrict__ q, float* __restrict__ k,
-                                                       float* __restrict__ vt, float* __restrict__ g, long long M,
-                                                       int c_s, int T, int ldT) {
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int n = lane & 31, h = lane >> 5;
-  const int nbc = c_s / 32;
-  const long long blk = (long long)blockIdx.x * 4 + wave;
-  const long long mblocks = (M + 31) / 32;
-  if (blk >= mblocks * 4 * nbc) return;   // no barriers in this kernel
-  const long long mb = blk / (4 * nbc);
-  const int cbt = (int)(blk % (4 * nbc));
-  const int part = cbt / nbc, cb = cbt % nbc;
-  const long long m = mb * 32 + n;
-  const bool mvalid = m < M;
-  const int K = c_s;
-  const float* arow = A + (size_t)(mvalid ? m : 0) * K + 4 * h;
-  const float* wbase = part < 3 ? w_qkv + (size_t)part * c_s * c_s : w_g;
-  const float* wrow = wbase + (size_t)(cb * 32 + perm32(n)) * K + 4 * h;
-  f32x16 acc = zero16();
-  for (int k0 = 0; k0 < K; k0 += 8) {
-    const f32x4 a4 = *reinterpret_cast<const f32x4*>(arow + k0);
-    const f32x4 w4 = *reinterpret_cast<const f32x4*>(wrow + k0);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc = mfma_f32(w4[e], a4[e], acc);
-  }
-  if (!mvalid) return;
-  const int c0 = cb * 32 + 16 * h;
-  if (part == 2) {
-    const long long sq = m / T, t = m % T;
-    float* col = vt + ((size_t)sq * c_s + c0) * ldT + t;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) col[(size_t)u * ldT] = acc[u];
-    return;
-  }
-  float v[16];
-#pragma unroll
-  for (int u = 0; u < 16; ++u) {
-    float x = acc[u];
-    if (part == 0 && q_bias) x += q_bias[c0 + u];
-    if (part == 3) x = 1.0f / (1.0f + __expf(-x));
-    v[u] = x;
-  }
-  float* dst = (part == 0 ? q : part == 1 ? k : g) + (size_t)m * c_s + c0;
-#pragma unroll
-  for (int qd = 0; qd < 4; ++qd) {
-    f32x4 o4;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o4[e] = v[4 * qd + e];
-    *reinterpret_cast<f32x4*>(dst + 4 * qd) = o4;
   }
 }
 
@@ -604,22 +534,19 @@ __global__ __launch_bounds__(256) void fill_zero_f32_kernel(float* __restrict__ 
   if (i < count) p[i] = 0.f;
 }
 
-int gemm_f32(int epi, const float* A, const float* W, const float* W2, const float* bias, const float* res, float* out,
-             long long M, int K, int N, hipStream_t stream, const char* name, int T = 1, int ldT = 1) {
+int gemm_f32(int epi, const float* A, const float* W, const float* bias, const float* res, float* out, long long M,
+             int K, int N, hipStream_t stream, const char* name) {
   if (K % 8 || N % 32 || M <= 0)
     return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: fp32 GEMM needs K %% 8 == 0 and N %% 32 == 0 (K=%d N=%d)", name, K,
                      N);
   const long long blocks = (M + 31) / 32 * (N / 32);
   const unsigned grid = (unsigned)((blocks + 3) / 4);
   KernelTimerScope timed(name, stream);
-#define BIOEMU_GEMM_F32(E)                                                                                      \
-  hipLaunchKernelGGL(gemm_f32_kernel<E>, dim3(grid), dim3(256), 0, stream, A, W, W2, bias, res, out, M, K, N, T, \
-                     ldT)
+#define BIOEMU_GEMM_F32(E) \
+  hipLaunchKernelGGL(gemm_f32_kernel<E>, dim3(grid), dim3(256), 0, stream, A, W, bias, res, out, M, K, N)
   switch (epi) {
     case kGemmEpiStore: BIOEMU_GEMM_F32(kGemmEpiStore); break;
     case kGemmEpiSigmoid: BIOEMU_GEMM_F32(kGemmEpiSigmoid); break;
-    case kGemmEpiSwiGLU: BIOEMU_GEMM_F32(kGemmEpiSwiGLU); break;
-    case kGemmEpiStoreT: BIOEMU_GEMM_F32(kGemmEpiStoreT); break;
     default: BIOEMU_GEMM_F32(kGemmEpiResidual); break;
   }
 #undef BIOEMU_GEMM_F32
@@ -653,47 +580,129 @@ int pair_proj_f32(const float* z, const float* g, const float* b, const float* w
   return check_launch(name);
 }
 
-// Token-side projections shared by both attentions: optional LN, then q (+ q bias), k, v, sigmoid(g).
+// Buffers of one split-operand product: activation fragments, weight fragments and their scales.
+struct SplitBuffers {
+  f16 *a, *w;
+  float *ainv, *winv;
+};
+
+// Carves `elems` floats (or the fragments of rows x K) out of a workspace; base may be null to count bytes.
+struct Carve {
+  char* base;
+  size_t off = 0;
+  template <class T>
+  T* bytes(size_t n) {
+    T* p = reinterpret_cast<T*>(base + off);
+    off += (size_t)round_up((int64_t)n, 256);
+    return p;
+  }
+  float* floats(size_t n) { return bytes<float>(n * 4); }
+  f16* frags(int64_t rows, int64_t K) { return bytes<f16>(split_frag_bytes(rows, K)); }
+};
+
+// Token-side buffers shared by both attentions.
 struct AttnF32Buffers {
-  float *sn, *q, *k, *v, *g, *go, *bias;
+  SplitBuffers sp;   // a: the rows of s, later of g * o; w: [Wq; Wk; Wv; Wg; Wo]
+  float *q, *k, *v, *g, *go, *bias;
+  f16* wz;       // pair-bias weights
+  float *wzinv, *wzbias;
+  float* wbias;  // projections of LayerNormed rows of 128 channels: W beta
 };
 
 // v is stored transposed per sequence ([sequence][c_s][ldv], keys contiguous): v_elems = sequences * c_s * ldv.
-size_t attn_f32_layout(long long rows, int c_s, long long v_elems, long long bias_elems, bool norm,
+size_t attn_f32_layout(long long rows, int c_s, int heads, long long v_elems, long long bias_elems,
                        AttnF32Buffers* buf, char* base) {
-  size_t off = 0;
-  auto take = [&](float** p, size_t elems) {
-    if (buf) *p = reinterpret_cast<float*>(base + off);
-    off += (size_t)round_up((int64_t)(elems * 4), 256);
-  };
+  Carve c{base};
   AttnF32Buffers dummy;
   AttnF32Buffers* b = buf ? buf : &dummy;
-  take(&b->sn, norm ? (size_t)rows * c_s : 0);
-  take(&b->q, (size_t)rows * c_s);
-  take(&b->k, (size_t)rows * c_s);
-  take(&b->v, (size_t)v_elems);
-  take(&b->g, (size_t)rows * c_s);
-  take(&b->go, (size_t)rows * c_s);
-  take(&b->bias, (size_t)bias_elems);
-  return off;
+  b->sp.a = c.frags(rows, c_s);
+  b->sp.ainv = c.floats((size_t)rows);
+  b->sp.w = c.frags(5 * (int64_t)c_s, c_s);
+  b->sp.winv = c.floats((size_t)5 * c_s / 32 + 1);
+  b->q = c.floats((size_t)rows * c_s);
+  b->k = c.floats((size_t)rows * c_s);
+  b->v = c.floats((size_t)v_elems);
+  b->g = c.floats((size_t)rows * c_s);
+  b->go = c.floats((size_t)rows * c_s);
+  b->bias = c.floats((size_t)bias_elems);
+  b->wz = c.frags(heads, 128);
+  b->wzinv = c.floats((size_t)heads / 32 + 1);
+  b->wzbias = c.floats((size_t)heads);
+  b->wbias = c.floats((size_t)4 * c_s);
+  return c.off;
 }
 
+// The pair rows of an attention's bias: P rows = outer x nrows x ncols of c_z channels -> bias[outer][head][row][col]
+// (row stride ld), LayerNormed with g, b.
+struct PairBiasF32 {
+  const float *z, *g, *b, *w;
+  long long P;
+  int nrows, ncols, ld, H, c_z;
+  const char* name;
+};
+
+// Fragments of the attention's weights, then the pair bias and q (+ q bias), k, v^T, sigmoid(g) of the optionally
+// normalised rows.
 int attn_f32_projections(const float* s, const float* norm_s_w, const float* norm_s_b, const float* w_qkv,
-                         const float* q_bias, const float* w_g, AttnF32Buffers& buf, long long rows, int c_s,
-                         int seq_len, int ldv, hipStream_t stream) {
-  const float* src = s;
-  int rc = 0;
-  if (norm_s_w) {
-    rc = rows_ln_f32(s, norm_s_w, norm_s_b, buf.sn, rows, c_s, stream, "f32_layernorm");
-    src = buf.sn;
+                         const float* q_bias, const float* w_g, const float* w_o, const PairBiasF32& pb,
+                         AttnF32Buffers& buf, long long rows, int c_s, int seq_len, int ldv, hipStream_t stream) {
+  const int nb = c_s / 32;
+  const size_t per = (size_t)nb * split_ksteps(c_s) * kFrag;   // f16 elements of one c_s x c_s weight
+  const bool bias_split = pb.c_z == 128 && pb.H <= 64 && pb.P < (1LL << 31) && aligned16(pb.w);
+  SplitMats mats{};
+  mats.m[0] = split_gemm_weight(w_qkv, buf.sp.w, buf.sp.winv, nullptr, 3 * (int64_t)c_s, c_s);
+  mats.m[1] = split_gemm_weight(w_g, buf.sp.w + 3 * per, buf.sp.winv + 3 * nb, nullptr, c_s, c_s);
+  mats.m[2] = split_gemm_weight(w_o, buf.sp.w + 4 * per, buf.sp.winv + 4 * nb, nullptr, c_s, c_s);
+  if (bias_split)
+    mats.m[3] = with_fold(split_gemm_weight(pb.w, buf.wz, buf.wzinv, nullptr, pb.H, 128), pb.g, pb.b, buf.wzbias);
+  const bool r128 = c_s == 128;
+  if (r128 && norm_s_w) {
+    mats.m[0] = with_fold(mats.m[0], norm_s_w, norm_s_b, buf.wbias);
+    mats.m[1] = with_fold(mats.m[1], norm_s_w, norm_s_b, buf.wbias + 3 * c_s);
   }
+  int rc = split_weights(mats, bias_split ? 4 : 3, stream);
   if (rc) return rc;
-  if (c_s % 32) return set_error(BIOEMU_ERR_UNSUPPORTED, "f32 attention: c_s %d is not a multiple of 32", c_s);
-  const long long blocks = (rows + 31) / 32 * (4 * (c_s / 32));
-  KernelTimerScope timed("f32_proj_qkvg", stream);
-  hipLaunchKernelGGL(qkvg_f32_kernel, dim3((unsigned)((blocks + 3) / 4)), dim3(256), 0, stream, src, w_qkv, w_g, q_bias,
-                     buf.q, buf.k, buf.v, buf.g, rows, c_s, seq_len, ldv);
-  return check_launch("f32_proj_qkvg");
+  if (bias_split)
+    rc = split_pair_bias(pb.z, buf.wz, buf.wzinv, buf.wzbias, buf.bias, pb.P, pb.nrows, pb.ncols, pb.ld, pb.H, stream,
+                         pb.name);
+  else
+    rc = pair_proj_f32(pb.z, pb.g, pb.b, pb.w, buf.bias, pb.P, pb.nrows, pb.ncols, pb.ld, pb.H, pb.c_z, stream, pb.name);
+  if (rc) return rc;
+  SplitGemmEpi e;
+  e.out = buf.q;
+  e.bias = q_bias;
+  e.ldo = c_s;
+  e.k = buf.k;
+  e.vt = buf.v;
+  e.g = buf.g;
+  e.T = seq_len;
+  e.ldT = ldv;
+  if (r128)
+    return split_gemm_r128(kSplitQkvg, s, buf.sp.w, buf.sp.winv, norm_s_w ? buf.wbias : nullptr, e, rows, 4 * c_s,
+                           stream, "f32_proj_qkvg");
+  rc = split_rows(s, c_s, nullptr, 0, norm_s_w, norm_s_b, buf.sp.a, buf.sp.ainv, nullptr, rows, stream,
+                  "f32_split_rows");
+  if (rc) return rc;
+  return split_gemm(kSplitQkvg, buf.sp.a, buf.sp.ainv, buf.sp.w, buf.sp.winv, e, rows, c_s, 4 * c_s, stream,
+                    "f32_proj_qkvg");
+}
+
+// out = go Wo^T (+ res)
+int attn_f32_out(const float* go, const float* res, float* out, AttnF32Buffers& buf, long long rows, int c_s,
+                 hipStream_t stream, const char* name) {
+  const int nb = c_s / 32;
+  const f16* w = buf.sp.w + (size_t)4 * nb * split_ksteps(c_s) * kFrag;
+  const float* winv = buf.sp.winv + 4 * nb;
+  SplitGemmEpi e;
+  e.out = out;
+  e.res = res;
+  e.ldo = c_s;
+  if (c_s == 128)
+    return split_gemm_r128(kSplitStore, go, w, winv, nullptr, e, rows, c_s, stream, name);
+  const int rc = split_rows(go, c_s, nullptr, 0, nullptr, nullptr, buf.sp.a, buf.sp.ainv, nullptr, rows, stream,
+                            "f32_split_rows");
+  if (rc) return rc;
+  return split_gemm(kSplitStore, buf.sp.a, buf.sp.ainv, w, winv, e, rows, c_s, c_s, stream, name);
 }
 
 }  // namespace
@@ -704,7 +713,7 @@ using namespace bioemu;
 extern "C" size_t bioemu_apb_f32_workspace_bytes(int64_t B, int64_t mult, int64_t N, int64_t c_s, int64_t H) {
   if (B <= 0 || mult <= 0 || N <= 0 || c_s <= 0 || H <= 0) return 0;
   const int64_t ld = round_up(N, 32);
-  return attn_f32_layout(B * mult * N, (int)c_s, B * mult * c_s * ld, B * H * N * ld, true, nullptr, nullptr);
+  return attn_f32_layout(B * mult * N, (int)c_s, (int)H, B * mult * c_s * ld, B * H * N * ld, nullptr, nullptr);
 }
 
 extern "C" int bioemu_apb_fwd_f32(const float* s, const float* z, const uint8_t* mask, const float* norm_s_w,
@@ -732,11 +741,10 @@ extern "C" int bioemu_apb_fwd_f32(const float* s, const float* z, const uint8_t*
   const long long rows = B * mult * N;
   AttnF32Buffers buf;
   const int ldb = (int)round_up(N, 32);
-  attn_f32_layout(rows, (int)c_s, B * mult * c_s * ldb, B * H * N * ldb, true, &buf, static_cast<char*>(workspace));
-  int rc = attn_f32_projections(s, norm_s_w, norm_s_b, w_qkv, q_bias, w_g, buf, rows, (int)c_s, (int)N, ldb, stream);
-  if (rc) return rc;
-  rc = pair_proj_f32(z, norm_z_w, norm_z_b, w_z, buf.bias, B * N * N, (int)N, (int)N, ldb, (int)H, (int)c_z, stream,
-                     "f32_pair_bias");
+  attn_f32_layout(rows, (int)c_s, (int)H, B * mult * c_s * ldb, B * H * N * ldb, &buf, static_cast<char*>(workspace));
+  const PairBiasF32 pb{z, norm_z_w, norm_z_b, w_z, B * N * N, (int)N, (int)N, ldb, (int)H, (int)c_z, "f32_pair_bias"};
+  int rc = attn_f32_projections(s, norm_s_w, norm_s_b, w_qkv, q_bias, w_g, w_o, pb, buf, rows, (int)c_s, (int)N, ldb,
+                                stream);
   if (rc) return rc;
   {
     KernelTimerScope timed("f32_attention", stream);
@@ -752,15 +760,13 @@ extern "C" int bioemu_apb_fwd_f32(const float* s, const float* z, const uint8_t*
   }
   rc = check_launch("f32_attention");
   if (rc) return rc;
-  return gemm_f32(residual ? kGemmEpiResidual : kGemmEpiStore, buf.go, w_o, nullptr, nullptr, s, out, rows, (int)c_s,
-                  (int)c_s, stream, "f32_proj_o");
+  return attn_f32_out(buf.go, residual ? s : nullptr, out, buf, rows, (int)c_s, stream, "f32_proj_o");
 }
 
 extern "C" size_t bioemu_swa_f32_workspace_bytes(int64_t B, int64_t mult, int64_t NW, int64_t W, int64_t H,
                                                  int64_t c_s, int64_t heads) {
   if (B <= 0 || mult <= 0 || NW <= 0 || W != 32 || H <= 0 || c_s <= 0 || heads <= 0) return 0;
-  return attn_f32_layout(B * mult * NW * W, (int)c_s, B * mult * NW * W * c_s, B * NW * heads * W * H, true, nullptr,
-                         nullptr);
+  return attn_f32_layout(B * mult * NW * W, (int)c_s, (int)heads, B * mult * NW * W * c_s, B * NW * heads * W * H, nullptr, nullptr);
 }
 
 extern "C" int bioemu_swa_fwd_f32(const float* s, const float* z, const uint8_t* mask, const float* norm_s_w,
@@ -792,12 +798,11 @@ extern "C" int bioemu_swa_fwd_f32(const float* s, const float* z, const uint8_t*
     return set_error(BIOEMU_ERR_WORKSPACE, "swa_f32: workspace too small");
   const long long rows = B * mult * NW * W;
   AttnF32Buffers buf;
-  attn_f32_layout(rows, (int)c_s, rows * c_s, B * NW * heads * W * H, true, &buf, static_cast<char*>(workspace));
-  int rc = attn_f32_projections(s, norm_s_w, norm_s_b, w_qkv, q_bias, w_g, buf, rows, (int)c_s, (int)(NW * W),
-                                (int)(NW * W), stream);
-  if (rc) return rc;
-  rc = pair_proj_f32(z, norm_z_w, norm_z_b, w_z, buf.bias, B * NW * W * H, (int)W, (int)H, (int)H, (int)heads,
-                     (int)c_z, stream, "f32_swa_pair_bias");
+  attn_f32_layout(rows, (int)c_s, (int)heads, rows * c_s, B * NW * heads * W * H, &buf, static_cast<char*>(workspace));
+  const PairBiasF32 pb{z, norm_z_w, norm_z_b, w_z, B * NW * W * H, (int)W, (int)H, (int)H, (int)heads, (int)c_z,
+                       "f32_swa_pair_bias"};
+  int rc = attn_f32_projections(s, norm_s_w, norm_s_b, w_qkv, q_bias, w_g, w_o, pb, buf, rows, (int)c_s,
+                                (int)(NW * W), (int)(NW * W), stream);
   if (rc) return rc;
   {
     KernelTimerScope timed("f32_swa_attention", stream);
@@ -807,35 +812,89 @@ extern "C" int bioemu_swa_fwd_f32(const float* s, const float* z, const uint8_t*
   }
   rc = check_launch("f32_swa_attention");
   if (rc) return rc;
-  return gemm_f32(residual ? kGemmEpiResidual : kGemmEpiStore, buf.go, w_o, nullptr, nullptr, s, out, rows, (int)c_s,
-                  (int)c_s, stream, "f32_proj_o");
+  return attn_f32_out(buf.go, residual ? s : nullptr, out, buf, rows, (int)c_s, stream, "f32_proj_o");
 }
 
 // out = (res +) Transition(x) over M rows; res may differ from x (the trunk's unconditional branch adds the
-// transition of LN(z_init) to z_init).  workspace: the LN rows [M][Dc], then the hidden rows [M][hidden].
+// transition of LN(z_init) to z_init).
+struct TransitionF32Buffers {
+  f16 *x, *w12, *h, *w3;
+  float *xinv, *xnorm, *w12inv, *w12norm, *hinv, *w3inv;
+  float* scales;   // the fused kernel's
+};
+
+// fc3 weights are laid out (and multiplied) at most this many output channels at a time: the workspace size does
+// not depend on the output width.
+constexpr int64_t kTransitionOutRows = 1024;
+
+static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, TransitionF32Buffers* buf, char* base) {
+  Carve c{base};
+  TransitionF32Buffers dummy;
+  TransitionF32Buffers* b = buf ? buf : &dummy;
+  b->x = c.frags(M, Dc);
+  b->xinv = c.floats((size_t)M);
+  b->xnorm = c.floats((size_t)M);
+  b->w12 = c.frags(3 * hidden, Dc);   // fc1 and fc2; with fc3 in the fused kernel's chunks
+  b->w12inv = c.floats((size_t)hidden / 16);
+  b->w12norm = c.floats((size_t)hidden / 16);
+  b->h = c.frags(M, hidden);
+  b->hinv = c.floats((size_t)M);
+  b->w3 = c.frags(kTransitionOutRows, hidden);
+  b->w3inv = c.floats((size_t)kTransitionOutRows / 32);
+  b->scales = c.floats(split_transition_scales(Dc, hidden));
+  return c.off;
+}
+
 static int transition_f32_res(const float* x, const float* res, const float* norm_w, const float* norm_b,
                               const float* fc1_w, const float* fc2_w, const float* fc3_w, float* out, void* workspace,
                               int64_t M, int64_t Dc, int64_t hidden, int64_t out_dim, int use_norm, int residual,
                               hipStream_t stream) {
-  float* xn = static_cast<float*>(workspace);
-  float* hbuf = reinterpret_cast<float*>(static_cast<char*>(workspace) + round_up(M * Dc * 4, 256));
-  const float* src = x;
-  int rc = 0;
-  if (use_norm) {
-    rc = rows_ln_f32(x, norm_w, norm_b, xn, M, (int)Dc, stream, "f32_layernorm");
-    src = xn;
-  }
-  if (!rc)
-    rc = gemm_f32(kGemmEpiSwiGLU, src, fc1_w, fc2_w, nullptr, nullptr, hbuf, M, (int)Dc, (int)hidden, stream,
+  TransitionF32Buffers buf;
+  transition_f32_layout(M, Dc, hidden, &buf, static_cast<char*>(workspace));
+  // Rows of 64 or 128 channels: one kernel at every row count (590k rows 128 -> 256: 0.46 ms against 2.1 ms for the
+  // three fp32-MFMA kernels it replaced; 200 rows: one launch and 8 chunks of weights instead of three products).
+  if ((Dc == 128 || Dc == 64) && out_dim == Dc && hidden <= kTransitionMaxHidden)
+    return split_transition_rows(x, residual ? res : nullptr, use_norm ? norm_w : nullptr, norm_b, fc1_w, fc2_w, fc3_w,
+                                 buf.w12, buf.scales, out, M, (int)Dc, (int)hidden, stream, "f32_transition_rows");
+  const int64_t out0 = out_dim < kTransitionOutRows ? out_dim : kTransitionOutRows;
+  SplitMats mats{};
+  mats.m[0] = split_gemm_weight(fc1_w, buf.w12, buf.w12inv, buf.w12norm, hidden, Dc, 2, 0);
+  mats.m[1] = split_gemm_weight(fc2_w, buf.w12, buf.w12inv, buf.w12norm, hidden, Dc, 2, 1);
+  mats.m[2] = split_gemm_weight(fc3_w, buf.w3, buf.w3inv, nullptr, out0, hidden);
+  int rc = split_weights(mats, 3, stream);
+  if (rc) return rc;
+  rc = split_rows(x, (int)Dc, nullptr, 0, use_norm ? norm_w : nullptr, norm_b, buf.x, buf.xinv, buf.xnorm, M, stream,
+                  "f32_split_rows");
+  if (rc) return rc;
+  SplitGemmEpi e1;
+  e1.hfrag = buf.h;
+  e1.hinv = buf.hinv;
+  e1.hsteps = split_ksteps(hidden);
+  e1.rnorm = buf.xnorm;
+  e1.wnorm = buf.w12norm;
+  rc = split_gemm(kSplitSwiGLU, buf.x, buf.xinv, buf.w12, buf.w12inv, e1, M, (int)Dc, (int)(2 * hidden), stream,
                   "f32_transition_swiglu");
   if (rc) return rc;
-  return gemm_f32(residual ? kGemmEpiResidual : kGemmEpiStore, hbuf, fc3_w, nullptr, nullptr, res, out, M,
-                  (int)hidden, (int)out_dim, stream, "f32_transition_out");
+  for (int64_t c0 = 0; c0 < out_dim; c0 += kTransitionOutRows) {
+    const int64_t nc = out_dim - c0 < kTransitionOutRows ? out_dim - c0 : kTransitionOutRows;
+    if (c0) {
+      mats.m[0] = split_gemm_weight(fc3_w + c0 * hidden, buf.w3, buf.w3inv, nullptr, nc, hidden);
+      if ((rc = split_weights(mats, 1, stream))) return rc;
+    }
+    SplitGemmEpi e2;
+    e2.out = out + c0;
+    e2.res = residual ? res + c0 : nullptr;
+    e2.ldo = (int)out_dim;
+    rc = split_gemm(kSplitStore, buf.h, buf.hinv, buf.w3, buf.w3inv, e2, M, (int)hidden, (int)nc, stream,
+                    "f32_transition_out");
+    if (rc) return rc;
+  }
+  return 0;
 }
 
 extern "C" size_t bioemu_transition_f32_workspace_bytes(int64_t M, int64_t Dc, int64_t hidden) {
   if (M <= 0 || Dc <= 0 || hidden <= 0) return 0;
-  return (size_t)round_up(M * Dc * 4, 256) + (size_t)round_up(M * hidden * 4, 256);
+  return transition_f32_layout(M, Dc, hidden, nullptr, nullptr);
 }
 
 extern "C" int bioemu_transition_fwd_f32(const float* x, const float* norm_w, const float* norm_b, const float* fc1_w,
@@ -863,7 +922,9 @@ extern "C" int bioemu_transition_fwd_f32(const float* x, const float* norm_w, co
 
 extern "C" size_t bioemu_pair_cond_f32_workspace_bytes(int64_t P, int64_t token_z, int64_t c_rel) {
   if (P <= 0 || token_z <= 0 || c_rel < 0) return 0;
-  return (size_t)round_up(P * (token_z + c_rel) * 4, 256);
+  // the normalised rows, or the projection's weight fragments
+  const size_t rows = (size_t)round_up(P * (token_z + c_rel) * 4, 256);
+  return rows > (size_t)(192 << 10) ? rows : (size_t)(192 << 10);
 }
 
 extern "C" int bioemu_pair_cond_proj_fwd_f32(const float* z_trunk, const float* rel, const float* ln_w,
@@ -881,10 +942,21 @@ extern "C" int bioemu_pair_cond_proj_fwd_f32(const float* z_trunk, const float* 
     return set_error(BIOEMU_ERR_INVALID_ARG, "pair_cond_f32: tensors must be 16-byte aligned");
   if (workspace_bytes < bioemu_pair_cond_f32_workspace_bytes(P, token_z, c_rel))
     return set_error(BIOEMU_ERR_WORKSPACE, "pair_cond_f32: workspace too small");
+  if (token_z == 128 && c_rel == 128 && a_z == 128 && aligned16(z_trunk) && aligned16(rel)) {
+    // the denoiser's widths: one pass over both inputs
+    Carve c{static_cast<char*>(workspace)};
+    f16* wf = c.frags(128, 256);
+    float *winv = c.floats(4), *wbias = c.floats(128);
+    SplitMats mats{};
+    mats.m[0] = with_fold(split_gemm_weight(w, wf, winv, nullptr, 128, 256), ln_w, ln_b, wbias);
+    const int rs = split_weights(mats, 1, stream);
+    if (rs) return rs;
+    return split_cat_proj(z_trunk, rel, wf, winv, wbias, out, P, stream, "f32_pair_cond_proj");
+  }
   float* xn = static_cast<float*>(workspace);
   int rc = rows_ln_f32(z_trunk, ln_w, ln_b, xn, P, (int)token_z, stream, "f32_pair_cond_layernorm", rel, (int)c_rel);
   if (rc) return rc;
-  return gemm_f32(kGemmEpiStore, xn, w, nullptr, nullptr, nullptr, out, P, (int)(token_z + c_rel), (int)a_z, stream,
+  return gemm_f32(kGemmEpiStore, xn, w, nullptr, nullptr, out, P, (int)(token_z + c_rel), (int)a_z, stream,
                   "f32_pair_cond_proj");
 }
 
@@ -949,7 +1021,7 @@ extern "C" int bioemu_trimul_fwd_f32(const float* x, const uint8_t* mask, const 
                        g_in_w, mask, planes, (int)N, (int)Np, D, P, outgoing);
   }
   if ((rc = check_launch("f32_trimul_proj"))) return rc;
-  rc = gemm_f32(kGemmEpiSigmoid, xn, g_out_w, nullptr, nullptr, nullptr, gate, P, D, D, stream, "f32_trimul_gate");
+  rc = gemm_f32(kGemmEpiSigmoid, xn, g_out_w, nullptr, nullptr, gate, P, D, D, stream, "f32_trimul_gate");
   if (rc) return rc;
   {
     const long long nb = Np / 32;
@@ -1144,7 +1216,7 @@ extern "C" int bioemu_opm_fwd_f32(const float* m, const uint8_t* mask, int mean_
                        aT, bT, inv, Y, (int)N, Sp);
   }
   if ((rc = check_launch("f32_opm_contract"))) return rc;
-  return gemm_f32(z_res ? kGemmEpiResidual : kGemmEpiStore, Y, w_o, nullptr, b_o, z_res, out, B * N * N,
+  return gemm_f32(z_res ? kGemmEpiResidual : kGemmEpiStore, Y, w_o, b_o, z_res, out, B * N * N,
                   kOpmCH * kOpmCH, (int)c_out, stream, "f32_opm_out");
 }
 
@@ -1323,7 +1395,7 @@ extern "C" int bioemu_pwa_fwd_f32(const float* m, const float* z, const uint8_t*
                        (int)S, (int)N, Np8, (int)c_m, (int)H, M);
   }
   if ((rc = check_launch("f32_pwa_v"))) return rc;
-  rc = gemm_f32(kGemmEpiSigmoid, mn, w_g, nullptr, nullptr, nullptr, g, M, (int)c_m, hc, stream, "f32_pwa_gate");
+  rc = gemm_f32(kGemmEpiSigmoid, mn, w_g, nullptr, nullptr, g, M, (int)c_m, hc, stream, "f32_pwa_gate");
   if (rc) return rc;
   rc = pair_proj_f32(z, norm_z_w, norm_z_b, w_z, lg, B * N * N, (int)N, (int)N, Np8, (int)H, (int)c_z, stream,
                      "f32_pwa_logits");
@@ -1342,7 +1414,7 @@ extern "C" int bioemu_pwa_fwd_f32(const float* m, const float* z, const uint8_t*
                        lg, vT, g, go, (int)S, (int)N, Np8, (int)H);
   }
   if ((rc = check_launch("f32_pwa_average"))) return rc;
-  return gemm_f32(residual ? kGemmEpiResidual : kGemmEpiStore, go, w_o, nullptr, nullptr, m, out, M, hc, (int)c_m,
+  return gemm_f32(residual ? kGemmEpiResidual : kGemmEpiStore, go, w_o, nullptr, m, out, M, hc, (int)c_m,
                   stream, "f32_pwa_out");
 }
 
@@ -1395,7 +1467,7 @@ extern "C" int bioemu_ln_linear_fwd_f32(const float* x, const float* norm_w, con
   float* xn = static_cast<float*>(workspace);
   const int rc = rows_ln_f32(x, norm_w, norm_b, xn, M, (int)K, stream, "f32_ln_linear_layernorm");
   if (rc) return rc;
-  return gemm_f32(base ? kGemmEpiResidual : kGemmEpiStore, xn, w, nullptr, nullptr, base, out, M, (int)K, (int)N,
+  return gemm_f32(base ? kGemmEpiResidual : kGemmEpiStore, xn, w, nullptr, base, out, M, (int)K, (int)N,
                   stream, "f32_ln_linear");
 }
 
@@ -1454,7 +1526,7 @@ extern "C" int bioemu_distogram_fwd_f32(const float* z, const float* w, const fl
   }
   const int rc = check_launch("f32_symmetrize");
   if (rc) return rc;
-  return gemm_f32(kGemmEpiStore, sym, w, nullptr, b, nullptr, out, B * N * N, (int)c_z, (int)num_bins, stream,
+  return gemm_f32(kGemmEpiStore, sym, w, b, nullptr, out, B * N * N, (int)c_z, (int)num_bins, stream,
                   "f32_distogram");
 }
 
@@ -1514,7 +1586,7 @@ extern "C" size_t bioemu_triatt_f32_workspace_bytes(int64_t B, int64_t N, int64_
   if (B <= 0 || N <= 0 || D <= 0 || H <= 0) return 0;
   const int64_t P = B * N * N, ld = round_up(N, 32);
   return (size_t)round_up(P * D * 4, 256) + (size_t)round_up(P, 256) +
-         attn_f32_layout(P, (int)D, B * N * D * ld, B * H * N * ld, true, nullptr, nullptr);
+         attn_f32_layout(P, (int)D, (int)H, B * N * D * ld, B * H * N * ld, nullptr, nullptr);
 }
 
 extern "C" int bioemu_triatt_fwd_f32(const float* z, const uint8_t* mask, const float* norm_w, const float* norm_b,
@@ -1544,7 +1616,7 @@ extern "C" int bioemu_triatt_fwd_f32(const float* z, const uint8_t* mask, const 
   uint8_t* mt = reinterpret_cast<uint8_t*>(p);
   p += round_up(P, 256);
   AttnF32Buffers buf;
-  attn_f32_layout(P, c, B * N * D * ld, B * H * N * ld, true, &buf, p);
+  attn_f32_layout(P, c, (int)H, B * N * D * ld, B * H * N * ld, &buf, p);
   const float* src = z;
   const uint8_t* msk = mask;
   int rc = 0;
@@ -1560,10 +1632,9 @@ extern "C" int bioemu_triatt_fwd_f32(const float* z, const uint8_t* mask, const 
     msk = mt;
   }
   // w_proj rows: [Wq; Wk; Wv] (3c), Wg (c), Wb (H)
-  rc = attn_f32_projections(src, norm_w, norm_b, w_proj, nullptr, w_proj + 3 * D * D, buf, P, c, (int)N, ld, stream);
-  if (rc) return rc;
-  rc = pair_proj_f32(src, norm_w, norm_b, w_proj + 4 * D * D, buf.bias, P, (int)N, (int)N, ld, (int)H, c, stream,
-                     "f32_triatt_bias");
+  const PairBiasF32 pb{src, norm_w, norm_b, w_proj + 4 * D * D, P, (int)N, (int)N, ld, (int)H, c, "f32_triatt_bias"};
+  rc = attn_f32_projections(src, norm_w, norm_b, w_proj, nullptr, w_proj + 3 * D * D, w_o, pb, buf, P, c, (int)N, ld,
+                            stream);
   if (rc) return rc;
   {
     KernelTimerScope timed("f32_triatt_attention", stream);
@@ -1577,6 +1648,5 @@ extern "C" int bioemu_triatt_fwd_f32(const float* z, const uint8_t* mask, const 
     if ((rc = transpose_pairs_f32(buf.go, zt, B, (int)N, c, stream, "f32_triatt_transpose_out"))) return rc;
     go = zt;
   }
-  return gemm_f32(residual ? kGemmEpiResidual : kGemmEpiStore, go, w_o, nullptr, nullptr, z, out, P, c, c, stream,
-                  "f32_triatt_proj_o");
+  return attn_f32_out(go, residual ? z : nullptr, out, buf, P, c, stream, "f32_triatt_proj_o");
 }

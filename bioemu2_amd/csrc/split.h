@@ -1,0 +1,136 @@
+// fp32 products on the f16 matrix cores, for gfx950.
+//
+// An fp32 value x, scaled by a power of two, is carried as two f16 values
+//   hi = f16(x),  lo = f16(x - hi)          (22-24 significant bits together)
+// and a product of two such operands as three f16 MFMAs with fp32
+// accumulation: lo*hi + hi*lo + hi*hi (lo*lo is below half an ulp of x*y).
+// v_mfma_f32_32x32x16_f16 does 16 k in 32 cycles against 8 x 64 cycles of
+// v_mfma_f32_32x32x2_f32, so the three cost 96 cycles where the fp32 MFMA
+// takes 512.  Against float64 the result is at least as close as the fp32
+// MFMA's for K >= 64, because it rounds its accumulator K / 16 * 3 times
+// instead of K / 2 (relative error of a 32 x 32 block of normal data, measured:
+// K = 64 1.15e-7 vs 1.49e-7, K = 128 1.47e-7 vs 1.89e-7, K = 384 2.3e-7 vs
+// 3.5e-7, K = 1024 3.8e-7 vs 5.8e-7; K = 32 is a tie, so shorter products stay
+// off this path).
+//
+// Range: the scale brings the largest magnitude of a scaling group (one
+// activation row, one block of 32 weight rows) into [2^14, 2^15).  hi + lo is
+// then exact to 2^-23 relative for elements down to 2^-16 of that maximum and
+// to 2^-39 of the maximum below it (the f16 MFMA multiplies subnormals).  A
+// scale depends on its own row (or on the weights) alone, so a row's result
+// never depends on another row.
+//
+// Operand fragments: 32 rows x 16 k are 1 KB of hi followed by 1 KB of lo,
+// lane (n, h) = 8 consecutive values, row n, k = 8 h .. 8 h + 7.  Weight rows
+// are stored in perm32 order (pairtile.h), so an accumulator lane ends with 16
+// consecutive output channels of one activation row.
+#pragma once
+
+#include "common.h"
+#include "internal.h"
+#include "pairtile.h"
+
+namespace bioemu {
+
+typedef _Float16 f16;
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kFragHalf = 512;         // f16 elements of one 32 x 16 plane (hi or lo): 1 KB
+constexpr int kFrag = 2 * kFragHalf;   // hi | lo
+
+struct SplitFrag {
+  f16x8 hi, lo;
+};
+
+__device__ __forceinline__ f32x16 mfma_f16(f16x8 a, f16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ void mfma_split(const SplitFrag& a, const SplitFrag& b, f32x16& acc) {
+  acc = mfma_f16(a.lo, b.hi, acc);
+  acc = mfma_f16(a.hi, b.lo, acc);
+  acc = mfma_f16(a.hi, b.hi, acc);
+}
+
+// 2^(14 - floor(log2 amax)), limited to 2^100 (amax = 0 or below 2^-86).
+__device__ __forceinline__ float split_scale(float amax) {
+  const int f = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xffu);
+  return __builtin_bit_cast(float, (uint32_t)min(268 - f, 227) << 23);
+}
+// 1 / s of a power of two s from split_scale (exact).
+__device__ __forceinline__ float split_inv(float s) {
+  return __builtin_bit_cast(float, (uint32_t)(254 - (int)(__builtin_bit_cast(uint32_t, s) >> 23)) << 23);
+}
+
+// x * s as hi + lo.  s is a power of two: the compiler may round the product to f16 in one step for hi and in two
+// steps (through f32) for the hi that lo is taken from, and only an exact product makes both the same value.
+__device__ __forceinline__ void split_value(float x, float s, f16& hi, f16& lo) {
+  hi = (f16)(x * s);
+  lo = (f16)__builtin_fmaf(x, s, -(float)hi);
+}
+
+__device__ __forceinline__ SplitFrag load_frag(const f16* p, int lane) {
+  SplitFrag f;
+  f.hi = *reinterpret_cast<const f16x8*>(p + lane * 8);
+  f.lo = *reinterpret_cast<const f16x8*>(p + kFragHalf + lane * 8);
+  return f;
+}
+
+__device__ __forceinline__ void copy1k_to_lds(__amdgpu_buffer_rsrc_t r, const f16* lds, unsigned voff, unsigned soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, 0);
+}
+
+// ---------------------------------------------------------------------------
+// Host side (split_gemm.hip).
+// ---------------------------------------------------------------------------
+// One weight matrix [rows][K] fp32 (K % 8 == 0; rows past the last are zeros) to fragments.  The block of
+// rows 32 rb .. and the k-step ks (16 columns, zero past K) go to
+//   dst + rb * rb_stride + (ks / kgrp) * kgrp_stride + (ks % kgrp) * kFrag
+// for ks < ksteps; inv[rb * inv_stride] = 1 / scale of the block and, unless null,
+// norm[rb * inv_stride] bounds |row . x| / |x| of its rows (their largest 2-norm).
+//
+// With gamma, a preceding LayerNorm's affine is folded in, so that rows are only
+// centred and divided by their deviation: the fragments hold W diag(gamma),
+// bias[row] = W beta (fp32; zero when beta is null) and norm bounds |W LN(x)|.
+struct SplitMat {
+  const float* w;
+  f16* dst;
+  float* inv;
+  float* norm;
+  int rows, K, ksteps, kgrp;
+  long long rb_stride, kgrp_stride;
+  int inv_stride;
+  const float *gamma, *beta;
+  float* bias;
+};
+constexpr int kSplitMats = 4;
+struct SplitMats {
+  SplitMat m[kSplitMats];
+};
+int split_weights(const SplitMats& mats, int count, hipStream_t stream);
+
+// k-steps of a GEMM operand of K columns: whole pairs of 16 (the tile loop stages two at a time).
+inline int split_ksteps(int64_t K) { return (int)(round_up(K, 32) / 16); }
+// Bytes of the fragments of `rows` x K (rows rounded up to 32).
+inline size_t split_frag_bytes(int64_t rows, int64_t K) {
+  return (size_t)(round_up(rows, 32) / 32) * split_ksteps(K) * kFrag * sizeof(f16);
+}
+
+// A plain GEMM weight: row blocks in order (stride 1) or interleaved with a
+// second matrix's (SwiGLU: fc1 blocks at even positions, fc2 at odd).
+inline SplitMat split_gemm_weight(const float* w, f16* dst, float* inv, float* norm, int64_t rows, int64_t K,
+                                  int interleave = 1, int first = 0) {
+  const int ks = split_ksteps(K);
+  return SplitMat{w, dst + (size_t)first * ks * kFrag, inv + first, norm ? norm + first : nullptr, (int)rows, (int)K,
+                  ks, ks, (long long)interleave * ks * kFrag, 0, interleave, nullptr, nullptr, nullptr};
+}
+// With a LayerNorm's affine folded in.
+inline SplitMat with_fold(SplitMat m, const float* gamma, const float* beta, float* bias) {
+  m.gamma = gamma;
+  m.beta = beta;
+  m.bias = bias;
+  return m;
+}
+
+}  // namespace bioemu

@@ -1,0 +1,43 @@
+// Host interface of the split-operand GEMMs (split_gemm.hip).
+#pragma once
+
+#include "split.h"
+
+namespace bioemu {
+
+constexpr int kSplitStore = 0;     // out = v (+ bias) (+ res)
+constexpr int kSplitSigmoid = 1;   // out = sigmoid(v)
+constexpr int kSplitSwiGLU = 2;    // fc1 / fc2 column blocks interleaved; silu(a) b as operand fragments
+constexpr int kSplitQkvg = 3;      // the four token projections of an attention
+
+struct SplitGemmEpi {
+  float* out = nullptr;          // kSplitQkvg: q
+  const float* bias = nullptr;   // kSplitQkvg: q bias
+  const float* res = nullptr;
+  int ldo = 0;                   // row length of out (kSplitQkvg: c_s)
+  float *k = nullptr, *vt = nullptr, *g = nullptr;   // kSplitQkvg
+  int T = 1, ldT = 1;                                // kSplitQkvg: rows per sequence, stride of vt's channels
+  f16* hfrag = nullptr;          // kSplitSwiGLU
+  float* hinv = nullptr;
+  const float *rnorm = nullptr, *wnorm = nullptr;
+  int hsteps = 0;
+};
+
+// Widest row split_rows holds in registers (12 k-steps in each of 4 waves); longer rows are read once per pass.
+constexpr int kSplitMaxK = 12 * 4 * 16;
+// Fewest 128 x 128 tiles worth the tiled kernel.
+constexpr int kSplitTiledMin = 128;
+
+// Rows [x1 | x2] (K1, K2 multiples of 8, 16-byte aligned; K2 = 0 past kSplitMaxK), LayerNormed when g, to fragments.
+int split_rows(const float* x1, int K1, const float* x2, int K2, const float* g, const float* b, f16* dst, float* inv,
+               float* norm, long long M, hipStream_t stream, const char* name);
+// M rows x N columns (N % 32 == 0; kSplitSwiGLU: both matrices' columns), K columns of A and W fragments.
+int split_gemm(int epi, const f16* A, const float* ainv, const f16* W, const float* winv, const SplitGemmEpi& e,
+               long long M, int K, int N, hipStream_t stream, const char* name);
+
+// The same straight from M fp32 rows of 128 channels; kSplitStore and kSplitQkvg.  With wbias (kSplitQkvg) the rows
+// are LayerNormed, the affine folded into W and wbias (SplitMat).
+int split_gemm_r128(int epi, const float* x, const f16* W, const float* winv, const float* wbias,
+                    const SplitGemmEpi& e, long long M, int N, hipStream_t stream, const char* name);
+
+}  // namespace bioemu

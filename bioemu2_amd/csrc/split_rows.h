@@ -1,0 +1,123 @@
+// Rows of fp32 activations held in registers as split operands (split.h): the
+// two lanes (n, 0) and (n, 1) of row slot n hold alternate 8-channel chunks, lane
+// half h channels 16 s + 8 h .. + 7 of every k-step s, i.e. the MFMA operand layout.
+#pragma once
+
+#include "split.h"
+
+namespace bioemu {
+
+// This lane's C / 2 channels of a row (16-byte aligned).
+template <int C>
+__device__ __forceinline__ void load_row_half(const float* row, int h, float (&v)[C / 2]) {
+#pragma unroll
+  for (int s = 0; s < C / 16; ++s)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const f32x4 t = *reinterpret_cast<const f32x4*>(row + 16 * s + 8 * h + 4 * q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[8 * s + 4 * q + e] = t[e];
+    }
+}
+
+// Squared 2-norm of the row.
+template <int C>
+__device__ __forceinline__ float row_norm2(const float (&v)[C / 2]) {
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < C / 2; ++i) ss += v[i] * v[i];
+  return ss + __shfl_xor(ss, 32);
+}
+
+// Largest magnitude of the row.
+template <int C>
+__device__ __forceinline__ float row_absmax(const float (&v)[C / 2]) {
+  float amax = 0.f;
+#pragma unroll
+  for (int i = 0; i < C / 2; ++i) amax = fmaxf(amax, fabsf(v[i]));
+  return fmaxf(amax, __shfl_xor(amax, 32));
+}
+
+// Fragments of v * s, s a power of two.
+template <int C>
+__device__ __forceinline__ void split_half(const float (&v)[C / 2], float s, SplitFrag* f) {
+#pragma unroll
+  for (int i = 0; i < C / 2; ++i) {
+    f16 hi, lo;
+    split_value(v[i], s, hi, lo);
+    f[i >> 3].hi[i & 7] = hi;
+    f[i >> 3].lo[i & 7] = lo;
+    if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);   // a k-step's fp32 values die before the next one's fragments
+  }
+}
+
+// The row's fragments under its own scale; returns 1 / scale.
+template <int C>
+__device__ __forceinline__ float split_row_half(const float (&v)[C / 2], SplitFrag (&f)[C / 16]) {
+  const float s = split_scale(row_absmax<C>(v));
+  split_half<C>(v, s, f);
+  return split_inv(s);
+}
+
+// A normalised row of up to 256 channels is below 16 in magnitude: it takes this scale, which brings it below 2^14,
+// whatever its values.
+constexpr float kNormScale = 1024.f;
+
+// Centres the row (v -= mean) and returns 1 / sqrt(biased variance + 1e-5): the affine-free LayerNorm in fp32, two
+// passes, over the C channels of lanes l and l ^ 32.
+template <int C>
+__device__ __forceinline__ float center_row_half(float (&v)[C / 2]) {
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < C / 2; ++i) s += v[i];
+  s += __shfl_xor(s, 32);
+  const float mean = s * (1.0f / C);
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < C / 2; ++i) {
+    v[i] -= mean;
+    ss += v[i] * v[i];
+  }
+  ss += __shfl_xor(ss, 32);
+  return 1.0f / sqrtf(ss * (1.0f / C) + 1e-5f);
+}
+
+// Fragments of kNormScale * v * rstd.  v * rstd is rounded to fp32 by itself (see split_value).
+template <int C>
+__device__ __forceinline__ void split_normalized(float (&v)[C / 2], float rstd, SplitFrag* f) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int i = 0; i < C / 2; ++i) v[i] = v[i] * rstd;
+  split_half<C>(v, kNormScale, f);
+}
+
+// Fragments of the normalised row; returns 1 / scale.
+template <int C>
+__device__ __forceinline__ float normalized_row_half(float (&v)[C / 2], SplitFrag (&f)[C / 16]) {
+  split_normalized<C>(v, center_row_half<C>(v), f);
+  return 1.0f / kNormScale;
+}
+
+// ---------------------------------------------------------------------------
+// Host side.
+// ---------------------------------------------------------------------------
+// Fused transition over rows of C = 64 or 128 channels (split_transition.hip): hidden % 32 == 0, at most
+// kTransitionMaxHidden.  `W` holds split_transition_weight_elems f16, `scales` split_transition_scales floats.
+constexpr int kTransitionMaxHidden = 2048;
+inline size_t split_transition_scales(int64_t C, int64_t hidden) { return (size_t)(hidden / 8 + C / 32 + 2 * hidden); }
+size_t split_transition_weight_elems(int64_t C, int64_t hidden);
+int split_transition_rows(const float* x, const float* res, const float* norm_w, const float* norm_b,
+                          const float* fc1, const float* fc2, const float* fc3, f16* W, float* scales, float* out,
+                          long long M, int C, int hidden, hipStream_t stream, const char* name);
+
+// out [P][128] = LN([x1 | x2]) W^T of P rows of 128 + 128 channels (split_pair.hip); W, winv, wbias: 128 x 256
+// weights with the LayerNorm folded in (SplitMat).
+int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* winv, const float* wbias, float* out,
+                   long long P, hipStream_t stream, const char* name);
+
+// Pair bias LN(z) W^T of P < 2^31 rows of 128 channels, head-major: row p = (outer, r, c) -> out[outer][head][r][c],
+// rows ld apart (split_pair.hip); W, winv, wbias: H x 128 weights with the LayerNorm folded in, H <= 64.
+int split_pair_bias(const float* z, const f16* W, const float* winv, const float* wbias, float* out, long long P,
+                    int nrows, int ncols, int ld, int H, hipStream_t stream, const char* name);
+
+}  // namespace bioemu

@@ -813,10 +813,12 @@ class SwaWorkload(Workload):
     def kernel_work(self, kernel: str) -> tuple[str, float]:
         rows = self.mult * self.na
         if self.fp32:
-            if kernel == "f32_proj_qkvg":
-                return ("mfma_f32", 4 * 2.0 * rows * 128 * 128)
+            if kernel == "f32_split_weights":   # reads the five weights, writes them as operand fragments
+                return ("hbm", float(2 * 5 * 128 * 128 * 4))
+            if kernel == "f32_proj_qkvg":   # reads s, writes q, k, v^T, g
+                return ("hbm", float(5 * rows * 128 * 4))
             if kernel == "f32_proj_o":
-                return ("mfma_f32", 2.0 * rows * 128 * 128)
+                return ("hbm", float(2 * rows * 128 * 4))
             if kernel == "f32_swa_pair_bias":   # reads z, writes the 4-head bias
                 return ("hbm", float(self.nw * 32 * 128 * (16 + 4) * 4))
             if kernel == "f32_swa_attention":   # QK^T and PV over the 128-key window, every copy and head
@@ -890,12 +892,14 @@ class ApbWorkload(Workload):
         n, B, M = self.n, self.B, self.mult
         if self.fp32:
             rows = B * M * n
-            if kernel == "f32_proj_qkvg":
-                return ("mfma_f32", 4 * 2.0 * rows * 384 * 384)
-            if kernel == "f32_proj_o":
-                return ("mfma_f32", 2.0 * rows * 384 * 384)
-            if kernel == "f32_layernorm":
+            if kernel == "f32_split_weights":   # reads the weights, writes them as operand fragments
+                return ("hbm", float(2 * (5 * 384 * 384 + 32 * 128) * 4))
+            if kernel == "f32_split_rows":   # reads rows, writes them as operand fragments
                 return ("hbm", float(2 * rows * 384 * 4))
+            if kernel == "f32_proj_qkvg":
+                return ("mfma_split", 4 * 2.0 * rows * 384 * 384)
+            if kernel == "f32_proj_o":
+                return ("mfma_split", 2.0 * rows * 384 * 384)
             if kernel == "f32_pair_bias":   # reads z, writes the 16-head bias
                 return ("hbm", float(B * n * n * (128 + 16) * 4))
             if kernel == "f32_attention":   # QK^T and PV: 4 N^2 c_s per copy
@@ -987,16 +991,12 @@ class PairCondWorkload(Workload):
     def kernel_work(self, kernel: str) -> tuple[str, float]:
         P = self.n * self.n
         if self.fp32:
-            if kernel == "f32_pair_cond_layernorm":   # reads both inputs, writes the normalised concatenation
-                return ("hbm", float(P * 256 * 4 * 2))
-            if kernel == "f32_layernorm":
-                return ("hbm", float(P * 128 * 4 * 2))
-            if kernel == "f32_pair_cond_proj":
-                return ("mfma_f32", 2.0 * P * 256 * 128)
-            if kernel == "f32_transition_swiglu":   # fc1 and fc2, 128 -> 256 each
-                return ("mfma_f32", 2.0 * 2 * P * 128 * 256)
-            if kernel == "f32_transition_out":
-                return ("mfma_f32", 2.0 * P * 256 * 128)
+            if kernel == "f32_split_weights":   # the projection's weights and both transitions', once each
+                return ("hbm", float(2 * (128 * 256 + 2 * 3 * 128 * 256) * 4) / 3)
+            if kernel == "f32_pair_cond_proj":   # reads both inputs, writes the stream
+                return ("hbm", float(P * (256 + 128) * 4))
+            if kernel == "f32_transition_rows":   # fc1 and fc2 (128 -> 256 each), fc3
+                return ("mfma_split", 2.0 * 3 * P * 128 * 256)
             raise KeyError(kernel)
         if kernel == "pair_cond_proj":
             return ("hbm", float(P * (256 + 128) * 2))

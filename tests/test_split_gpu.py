@@ -1,0 +1,146 @@
+"""fp32 products on split f16 operands (csrc/split.h): tile edges, row counts and value ranges.
+
+The reference is float64 on the CPU.  Bound: an operand is exact to 2^-23 and a sum of K products rounds its fp32
+accumulator 3 K / 16 times, each by at most 2^-24 of a partial sum that is about the result's size, so the relative
+2-norm error stays below (sqrt(3 K / 16) + 2) * 2^-23 per product; two products in a row and the activation between
+them (2^-21) add up to TOL for every width below.
+"""
+
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from bioemu2_amd import _ops
+from bioemu2_amd.attention_pair_bias import AttentionPairBias, AttentionPairBiasSlidingWindow
+from bioemu2_amd.glue import PairwiseConditioning
+from bioemu2_amd.transition import Transition
+from tests._helpers import randomize_params, rel_l2
+
+pytestmark = pytest.mark.gpu
+TOL = 4e-6
+
+
+def _params(module):
+    return {k: v.detach().double().cpu() for k, v in module.state_dict().items()}
+
+
+def _ln(x, p, name):
+    return F.layer_norm(x, (x.shape[-1],), p[name + ".weight"], p.get(name + ".bias"), 1e-5)
+
+
+def _transition(x, p, use_norm=True):
+    x = _ln(x, p, "norm") if use_norm else x
+    return (F.silu(x @ p["fc1.weight"].T) * (x @ p["fc2.weight"].T)) @ p["fc3.weight"].T
+
+
+@pytest.mark.parametrize(
+    "dim,hidden,out_dim,use_norm,rows",
+    [
+        (128, 32, None, True, 1),        # fused kernel: one hidden chunk, one row
+        (128, 256, None, True, 255),     # a workgroup's rows less one
+        (128, 512, None, False, 257),
+        (128, 2048, None, True, 300),    # its widest hidden dimension
+        (128, 2080, None, True, 70),     # one past it: the separate products
+        (64, 256, None, True, 513),
+        (64, 128, None, False, 31),
+        (384, 768, None, True, 33),      # 32 x 64 tiles, k-steps split over the waves
+        (384, 768, None, True, 2100),    # 128 x 128 tiles
+        (40, 96, 32, False, 65),         # columns that end inside a k-step; an odd count of column blocks
+        (1032, 64, 1056, True, 40),      # rows longer than the registers hold, more than 1024 output channels
+    ],
+)
+def test_transition_split_edges(gpu_device, dim, hidden, out_dim, use_norm, rows):
+    torch.manual_seed(0)
+    m = randomize_params(Transition(dim, hidden, out_dim=out_dim, use_norm=use_norm), 3)
+    x = torch.randn(rows, dim)
+    want = _transition(x.double(), _params(m), use_norm)
+    m = m.to(gpu_device)
+    with torch.no_grad():
+        assert rel_l2(m(x.to(gpu_device)).cpu(), want) <= TOL
+
+
+@pytest.mark.parametrize("dim,rows", [(128, 300), (384, 300), (384, 4200)])
+def test_transition_split_ranges(gpu_device, dim, rows):
+    """Row magnitudes from 1e-12 to 1e12 in one call, checked row by row: each row has its own scale."""
+    torch.manual_seed(1)
+    m = randomize_params(Transition(dim, 256, use_norm=False), 3)
+    x = torch.randn(rows, dim) * torch.logspace(-12, 12, rows)[:, None]
+    x[5] = 0.0
+    want = _transition(x.double(), _params(m), False)
+    m = m.to(gpu_device)
+    with torch.no_grad():
+        got = m(x.to(gpu_device)).cpu()
+    err = (got.double() - want).norm(dim=1) / want.norm(dim=1).clamp_min(1e-300)
+    assert torch.equal(got[5], torch.zeros(dim))
+    err[5] = 0.0
+    assert float(err.max()) <= TOL
+
+
+@pytest.mark.parametrize("kind", ["128", "384"])
+def test_split_rows_are_independent(gpu_device, kind):
+    """A row's result does not change with what the other rows hold."""
+    dim = int(kind)
+    torch.manual_seed(2)
+    m = randomize_params(Transition(dim, 256), 3).to(gpu_device)
+    x = torch.randn(600, dim, device=gpu_device)
+    y = x.clone()
+    y[300:] = 1e6 * torch.randn(300, dim, device=gpu_device)
+    with torch.no_grad():
+        assert torch.equal(m(x)[:300], m(y)[:300])
+
+
+def _apb64(s, z, mask, p, heads, mult, norm):
+    n, cs = s.shape[1:]
+    d = cs // heads
+    s = _ln(s, p, "norm_s") if norm else s
+    q, k, v = (s @ p["proj_qkv.weight"].T).chunk(3, -1)
+    q = q + p["proj_q_bias"]
+    q, k, v = (t.view(-1, n, heads, d).transpose(1, 2) for t in (q, k, v))
+    bias = (_ln(z, p, "norm_z") @ p["proj_z.weight"].T).permute(0, 3, 1, 2).repeat_interleave(mult, 0)
+    lg = (q @ k.transpose(2, 3)) / math.sqrt(d) + bias
+    keep = mask.repeat_interleave(mult, 0)[:, None, None, :]
+    o = lg.masked_fill(~keep, -1e6).softmax(-1) @ v
+    return (torch.sigmoid(s @ p["proj_g.weight"].T) * o.transpose(1, 2).reshape(s.shape)) @ p["proj_o.weight"].T
+
+
+@pytest.mark.parametrize(
+    "c_s,heads,n,mult,norm,lnb",
+    [
+        (384, 16, 300, 8, False, False),   # 128 x 128 tiles with ragged rows and sequences
+        (384, 16, 31, 1, True, True),      # a bias in the pair LayerNorm
+        (1152, 48, 20, 1, False, False),   # more than 32 heads in the pair bias
+        (128, 4, 97, 3, True, False),      # rows of 128 channels, LayerNorm folded
+    ],
+)
+def test_apb_split_projections(gpu_device, c_s, heads, n, mult, norm, lnb):
+    torch.manual_seed(3)
+    m = AttentionPairBias(c_s, 128, heads, initial_norm=norm, use_bias_in_layer_norm=lnb)
+    m = randomize_params(m, 7)
+    s, z = torch.randn(mult, n, c_s), torch.randn(1, n, n, 128)
+    mask = torch.ones(1, n, dtype=torch.bool)
+    mask[:, n - n // 10:] = False
+    want = _apb64(s.double(), z.double(), mask, _params(m), heads, mult, norm)
+    m = m.to(gpu_device)
+    with torch.no_grad():
+        got = m(s.to(gpu_device), z.to(gpu_device), mask.to(gpu_device), multiplicity=mult).cpu()
+    assert rel_l2(got, want) <= TOL
+
+
+def test_pair_cond_split_and_general(gpu_device):
+    """The one-pass projection (128 + 128 -> 128) against float64, and the general kernels behind a rel tensor that
+    is not 16-byte aligned (same values)."""
+    torch.manual_seed(4)
+    m = randomize_params(PairwiseConditioning(128, 128), 5)
+    p = _params(m)
+    z, rel = torch.randn(1, 37, 37, 128), torch.randn(1, 37, 37, 128)
+    x = _ln(torch.cat([z, rel], -1).double(), p, "dim_pairwise_init_proj.0") @ p["dim_pairwise_init_proj.1.weight"].T
+    for i in range(2):
+        x = x + _transition(x, {k[len(f"transitions.{i}."):]: v for k, v in p.items() if k.startswith(f"transitions.{i}.")})
+    m = m.to(gpu_device)
+    zd, rd = z.to(gpu_device), rel.to(gpu_device)
+    shifted = torch.empty(rd.numel() + 1, device=gpu_device)[1:].view(rd.shape).copy_(rd)
+    with torch.no_grad():
+        assert rel_l2(m(zd, rd).cpu(), x) <= TOL
+        assert rel_l2(m(zd, shifted).cpu(), x) <= TOL
