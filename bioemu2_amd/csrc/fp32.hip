@@ -967,6 +967,7 @@ static int64_t trimul_f32_np(int64_t N) { return round_up(N, 32); }
 
 extern "C" size_t bioemu_trimul_f32_workspace_bytes(int64_t B, int64_t N, int64_t Dc) {
   if (B <= 0 || N <= 0 || Dc <= 0 || Dc % 32) return 0;
+  if (Dc == 128) return split_trimul_workspace_bytes(B, N);
   const size_t P = (size_t)B * N * N, Np = (size_t)trimul_f32_np(N);
   // xn (then LN_out(o)), the output gate, o: [P][D] each; the planes [B][2D][Np][Np]
   return (size_t)round_up(P * Dc * 4, 256) * 3 + (size_t)round_up(B * 2 * Dc * Np * Np * 4, 256);
@@ -993,6 +994,9 @@ extern "C" int bioemu_trimul_fwd_f32(const float* x, const uint8_t* mask, const 
     return set_error(BIOEMU_ERR_INVALID_ARG, "trimul_f32: out may alias x only with residual=1");
   if (workspace_bytes < bioemu_trimul_f32_workspace_bytes(B, N, Dc))
     return set_error(BIOEMU_ERR_WORKSPACE, "trimul_f32: workspace too small");
+  if (Dc == 128)
+    return split_trimul(x, mask, norm_in_w, norm_in_b, p_in_w, g_in_w, norm_out_w, norm_out_b, p_out_w, g_out_w, out,
+                        workspace, B, N, outgoing, residual, stream);
   const long long P = B * N * N;
   const int64_t Np = trimul_f32_np(N);
   const int D = (int)Dc;

@@ -17,14 +17,6 @@ constexpr int kCatWaves = 8;
 constexpr int kCatWeights = 4 * 16 * kFrag;               // f16: [4 column blocks][16 k-steps]
 constexpr int kCatSmem = kCatWeights * (int)sizeof(f16);  // 128 KB
 
-// Copies `kb` KB of fragments into LDS, split over the workgroup's waves.
-__device__ __forceinline__ void stage_fragments(const f16* W, f16* smem, int kb, int waves, int wave, int lane) {
-  const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, (unsigned)kb * 1024);
-  for (int c = wave; c < kb; c += waves) copy1k_to_lds(rw, smem + c * kFragHalf, lane * 16, (unsigned)c * 1024);
-  __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
-  __syncthreads();
-}
-
 __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
     const float* __restrict__ x1, const float* __restrict__ x2, const f16* __restrict__ W,
     const float* __restrict__ winv, const float* __restrict__ wbias, float* __restrict__ out, long long P, int tiles) {

@@ -98,6 +98,14 @@ __device__ __forceinline__ float normalized_row_half(float (&v)[C / 2], SplitFra
   return 1.0f / kNormScale;
 }
 
+// Copies `kb` KB of fragments into LDS, split over the workgroup's waves.
+__device__ __forceinline__ void stage_fragments(const f16* W, f16* smem, int kb, int waves, int wave, int lane) {
+  const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, (unsigned)kb * 1024);
+  for (int c = wave; c < kb; c += waves) copy1k_to_lds(rw, smem + c * kFragHalf, lane * 16, (unsigned)c * 1024);
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+  __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
@@ -119,5 +127,12 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
 // rows ld apart (split_pair.hip); W, winv, wbias: H x 128 weights with the LayerNorm folded in, H <= 64.
 int split_pair_bias(const float* z, const f16* W, const float* winv, const float* wbias, float* out, long long P,
                     int nrows, int ncols, int ld, int H, hipStream_t stream, const char* name);
+
+// Triangle multiplication of 128 channels (split_trimul.hip): the arguments of bioemu_trimul_fwd_f32.
+size_t split_trimul_workspace_bytes(int64_t B, int64_t N);
+int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, const float* norm_in_b,
+                 const float* p_in_w, const float* g_in_w, const float* norm_out_w, const float* norm_out_b,
+                 const float* p_out_w, const float* g_out_w, float* out, void* workspace, int64_t B, int64_t N,
+                 int outgoing, int residual, hipStream_t stream);
 
 }  // namespace bioemu

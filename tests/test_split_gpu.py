@@ -16,6 +16,7 @@ from bioemu2_amd import _ops
 from bioemu2_amd.attention_pair_bias import AttentionPairBias, AttentionPairBiasSlidingWindow
 from bioemu2_amd.glue import PairwiseConditioning
 from bioemu2_amd.transition import Transition
+from bioemu2_amd.triangle_multiplication import TriangleMultiplicationHip
 from tests._helpers import randomize_params, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -144,3 +145,23 @@ def test_pair_cond_split_and_general(gpu_device):
     with torch.no_grad():
         assert rel_l2(m(zd, rd).cpu(), x) <= TOL
         assert rel_l2(m(zd, shifted).cpu(), x) <= TOL
+
+
+@pytest.mark.parametrize("mode", ["outgoing", "incoming"])
+@pytest.mark.parametrize("n,b", [(1, 1), (31, 2), (33, 1), (127, 1), (129, 2)])
+def test_trimul_split_edges(gpu_device, mode, n, b):
+    """Lines that end inside a 32-pair tile, planes that end inside a 128 x 128 contraction tile, two batches."""
+    torch.manual_seed(5)
+    m = randomize_params(TriangleMultiplicationHip(128, mode), 6)
+    p = _params(m)
+    x = torch.randn(b, n, n, 128)
+    mask = torch.rand(b, n, n) < 0.8
+    xn = _ln(x.double(), p, "norm_in")
+    proj = (xn @ p["p_in.weight"].T) * torch.sigmoid(xn @ p["g_in.weight"].T) * mask[..., None]
+    a, c = proj.permute(0, 3, 1, 2).chunk(2, 1)
+    o = (a @ c.transpose(2, 3) if mode == "outgoing" else a.transpose(2, 3) @ c).permute(0, 2, 3, 1)
+    want = (_ln(o, p, "norm_out") @ p["p_out.weight"].T) * torch.sigmoid(xn @ p["g_out.weight"].T)
+    m = m.to(gpu_device)
+    with torch.no_grad():
+        got = m(x.to(gpu_device), mask.to(gpu_device)).cpu()
+    assert rel_l2(got, want) <= TOL
