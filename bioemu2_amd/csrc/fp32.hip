@@ -138,7 +138,7 @@ template <int CZ>
 __global__ __launch_bounds__(256) void pair_proj_f32_kernel(const float* __restrict__ z, const float* __restrict__ g,
                                                             const float* __restrict__ b, const float* __restrict__ w,
                                                             float* __restrict__ out, long long P, int nrows, int ncols,
-                                                            int ld, int H) {
+                                                            int ld, int H, float scale) {
   const long long p = (long long)blockIdx.x * 256 + threadIdx.x;
   if (p >= P) return;
   float v[CZ];
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void pair_proj_f32_kernel(const float* __restr
     float acc = 0.f;
 #pragma unroll
     for (int c = 0; c < CZ; ++c) acc += w[hh * CZ + c] * v[c];
-    out[(((size_t)outer * H + hh) * nrows + r) * ld + col] = acc;
+    out[(((size_t)outer * H + hh) * nrows + r) * ld + col] = acc * scale;
   }
 }
 
@@ -267,101 +267,6 @@ __device__ __forceinline__ void load_q_f32(const float* qr, float (&qv)[D / 2]) 
 #pragma unroll
     for (int e = 0; e < 4; ++e) qv[4 * j + e] = t[e];
   }
-}
-
-// Full attention: grid (ceil(N / 128), H, B * mult), 4 waves of 32 queries
-// sharing each 32-key block of K, V^T and the mask through LDS (staged once
-// per workgroup, double-buffered).  bias [B][H][N][ld], V^T [B*mult][c_s][ld]
-// (ld = N rounded up to 32; columns >= N unused).  Key mask: one row of N
-// bytes per batch ([B][N], mask_per_copy = 0) or per copy ([B*mult][N],
-// mask_per_copy = 1: triangle attention's per-sequence mask).
-template <int D>
-__global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                       const float* __restrict__ vt, const float* __restrict__ g,
-                                                       const float* __restrict__ bias,
-                                                       const uint8_t* __restrict__ mask, float* __restrict__ go,
-                                                       int N, int ld, int H, int c_s, int mult, float rsq,
-                                                       int mask_per_copy) {
-  constexpr int KS = D + 4, VS = 36, KQ = D / 4;
-  __shared__ __attribute__((aligned(16))) float ks[2][32][KS];
-  __shared__ __attribute__((aligned(16))) float vs[2][D][VS];
-  __shared__ __attribute__((aligned(16))) uint8_t ms[2][32];
-  const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, h = lane >> 5;
-  const int hd = blockIdx.y, bm = blockIdx.z, b = bm / mult;
-  const int q0 = (blockIdx.x * 4 + wave_id()) * 32;
-  // waves past N run on a clamped row and store nothing: they stage their
-  // share of every block and meet every barrier
-  const int qi = min(q0 + n, N - 1);
-  float qv[D / 2];
-  load_q_f32<D>(q + ((size_t)bm * N + qi) * c_s + hd * D + h * (D / 2), qv);
-  const float* brow = bias + (((size_t)b * H + hd) * N + qi) * ld;
-  const float* kbase = k + (size_t)bm * N * c_s + hd * D;
-  const float* vtb = vt + ((size_t)bm * c_s + hd * D) * ld;
-  const uint8_t* mrow = mask + (size_t)(mask_per_copy ? bm : b) * N;
-  // staging: thread tid moves K float4 (key tid / KQ, chunk tid % KQ) and
-  // V^T float4 (channel tid / 8, keys 4 (tid % 8) ..), thread tid < 32 a mask byte
-  const int sk_key = tid / KQ, sk_chunk = tid % KQ;
-  const int sv_row = tid >> 3, sv_chunk = tid & 7;
-  f32x4 rk, rv;
-  uint8_t rm = 0;
-  auto gload = [&](int k0) {
-    if (tid < 32 * KQ) rk = *reinterpret_cast<const f32x4*>(kbase + (size_t)min(k0 + sk_key, N - 1) * c_s + 4 * sk_chunk);
-    if (tid < D * 8) {
-      rv = *reinterpret_cast<const f32x4*>(vtb + (size_t)sv_row * ld + k0 + 4 * sv_chunk);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (k0 + 4 * sv_chunk + e >= N) rv[e] = 0.f;   // unwritten columns past N
-    }
-    if (tid < 32) rm = k0 + tid < N ? mrow[k0 + tid] : 0;
-  };
-  auto lstore = [&](int st) {
-    if (tid < 32 * KQ) *reinterpret_cast<f32x4*>(&ks[st][sk_key][4 * sk_chunk]) = rk;
-    if (tid < D * 8) *reinterpret_cast<f32x4*>(&vs[st][sv_row][4 * sv_chunk]) = rv;
-    if (tid < 32) ms[st][tid] = rm;
-  };
-  auto bload = [&](int k0, f32x4 (&bb)[4]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) bb[j] = *reinterpret_cast<const f32x4*>(brow + k0 + 8 * j + 4 * h);
-  };
-  f32x16 o = zero16();
-  float m = -INFINITY, l = 0.f;
-  F32KeyBlock<D> kb;
-  f32x4 bnext[4];
-  gload(0);
-  bload(0, kb.bias);
-  lstore(0);
-  __syncthreads();
-  int st = 0;
-#pragma unroll 1
-  for (int k0 = 0; k0 < N; k0 += 32) {
-    const bool more = k0 + 32 < N;
-    if (more) {
-      gload(k0 + 32);
-      bload(k0 + 32, bnext);
-    }
-#pragma unroll
-    for (int j = 0; j < D / 8; ++j) kb.k[j] = *reinterpret_cast<const f32x4*>(&ks[st][n][h * (D / 2) + 4 * j]);
-    unsigned w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      kb.v[j] = n < D ? *reinterpret_cast<const f32x4*>(&vs[st][n < D ? n : 0][8 * j + 4 * h]) : f32x4{0.f, 0.f, 0.f, 0.f};
-      w[j] = *reinterpret_cast<const unsigned*>(&ms[st][8 * j + 4 * h]);
-    }
-    kb.keep = keep_bits(w);
-    kb.live = 0u;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) kb.live |= (unsigned)(k0 + 8 * (u >> 2) + 4 * h + (u & 3) < N) << u;
-    f32_attend_block<D>(kb, qv, rsq, o, m, l);
-    if (more) {
-      lstore(st ^ 1);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) kb.bias[j] = bnext[j];
-    }
-    __syncthreads();
-    st ^= 1;
-  }
-  const size_t off = ((size_t)bm * N + qi) * c_s + hd * D;
-  f32_attend_store<D>(o, l, g + off, go + off, q0 + n < N);
 }
 
 // Sliding-window attention: grid (NW, ceil(heads / 4), B * mult); wave = head,
@@ -563,18 +468,18 @@ int rows_ln_f32(const float* x, const float* g, const float* b, float* y, long l
 
 // Bias rows: P pair rows = outer x nrows x ncols -> out[outer][head][row][col] with row stride ld.
 int pair_proj_f32(const float* z, const float* g, const float* b, const float* w, float* out, long long P,
-                  int nrows, int ncols, int ld, int H, int c_z, hipStream_t stream, const char* name) {
+                  int nrows, int ncols, int ld, int H, int c_z, float scale, hipStream_t stream, const char* name) {
   const unsigned grid = (unsigned)((P + 255) / 256);
   KernelTimerScope timed(name, stream);
   if (c_z == 128)
     hipLaunchKernelGGL(pair_proj_f32_kernel<128>, dim3(grid), dim3(256), 0, stream, z, g, b, w, out, P, nrows, ncols,
-                       ld, H);
+                       ld, H, scale);
   else if (c_z == 32)
     hipLaunchKernelGGL(pair_proj_f32_kernel<32>, dim3(grid), dim3(256), 0, stream, z, g, b, w, out, P, nrows, ncols,
-                       ld, H);
+                       ld, H, scale);
   else if (c_z == 16)
     hipLaunchKernelGGL(pair_proj_f32_kernel<16>, dim3(grid), dim3(256), 0, stream, z, g, b, w, out, P, nrows, ncols,
-                       ld, H);
+                       ld, H, scale);
   else
     return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: c_z %d unsupported (16, 32 or 128)", name, c_z);
   return check_launch(name);
@@ -604,14 +509,18 @@ struct Carve {
 struct AttnF32Buffers {
   SplitBuffers sp;   // a: the rows of s, later of g * o; w: [Wq; Wk; Wv; Wg; Wo]
   float *q, *k, *v, *g, *go, *bias;
+  f16* kv;       // full attention: split_attn's scratch
+  float* kvinv;
+  uint32_t* words;
   f16* wz;       // pair-bias weights
   float *wzinv, *wzbias;
   float* wbias;  // projections of LayerNormed rows of 128 channels: W beta
 };
 
-// v is stored transposed per sequence ([sequence][c_s][ldv], keys contiguous): v_elems = sequences * c_s * ldv.
-size_t attn_f32_layout(long long rows, int c_s, int heads, long long v_elems, long long bias_elems,
-                       AttnF32Buffers* buf, char* base) {
+// seq_len: rows per sequence of full attention, 0 for the sliding window (whose v is stored transposed per sequence,
+// [sequence][c_s][rows], keys contiguous).
+size_t attn_f32_layout(long long rows, int c_s, int heads, int64_t seq_len, long long bias_elems, AttnF32Buffers* buf,
+                       char* base) {
   Carve c{base};
   AttnF32Buffers dummy;
   AttnF32Buffers* b = buf ? buf : &dummy;
@@ -621,10 +530,17 @@ size_t attn_f32_layout(long long rows, int c_s, int heads, long long v_elems, lo
   b->sp.winv = c.floats((size_t)5 * c_s / 32 + 1);
   b->q = c.floats((size_t)rows * c_s);
   b->k = c.floats((size_t)rows * c_s);
-  b->v = c.floats((size_t)v_elems);
+  b->v = c.floats((size_t)rows * c_s);
   b->g = c.floats((size_t)rows * c_s);
   b->go = c.floats((size_t)rows * c_s);
   b->bias = c.floats((size_t)bias_elems);
+  if (seq_len) {
+    const int64_t seqs = rows / seq_len;
+    b->kv = c.bytes<f16>(split_attn_kv_elems(seqs, heads, seq_len) * sizeof(f16));
+    const size_t blocks = (size_t)seqs * heads * ((seq_len + 31) / 32);
+    b->kvinv = c.floats(2 * blocks);
+    b->words = c.bytes<uint32_t>(blocks * 4);
+  }
   b->wz = c.frags(heads, 128);
   b->wzinv = c.floats((size_t)heads / 32 + 1);
   b->wzbias = c.floats((size_t)heads);
@@ -638,14 +554,15 @@ struct PairBiasF32 {
   const float *z, *g, *b, *w;
   long long P;
   int nrows, ncols, ld, H, c_z;
+  float scale;
   const char* name;
 };
 
-// Fragments of the attention's weights, then the pair bias and q (+ q bias), k, v^T, sigmoid(g) of the optionally
-// normalised rows.
+// Fragments of the attention's weights, then the pair bias and q (+ q bias), k, v, sigmoid(g) of the optionally
+// normalised rows; v_transposed_len: v transposed per sequence of that many rows (0: row-major).
 int attn_f32_projections(const float* s, const float* norm_s_w, const float* norm_s_b, const float* w_qkv,
                          const float* q_bias, const float* w_g, const float* w_o, const PairBiasF32& pb,
-                         AttnF32Buffers& buf, long long rows, int c_s, int seq_len, int ldv, hipStream_t stream) {
+                         AttnF32Buffers& buf, long long rows, int c_s, int v_transposed_len, hipStream_t stream) {
   const int nb = c_s / 32;
   const size_t per = (size_t)nb * split_ksteps(c_s) * kFrag;   // f16 elements of one c_s x c_s weight
   const bool bias_split = pb.c_z == 128 && pb.H <= 64 && pb.P < (1LL << 31) && aligned16(pb.w);
@@ -663,20 +580,20 @@ int attn_f32_projections(const float* s, const float* norm_s_w, const float* nor
   int rc = split_weights(mats, bias_split ? 4 : 3, stream);
   if (rc) return rc;
   if (bias_split)
-    rc = split_pair_bias(pb.z, buf.wz, buf.wzinv, buf.wzbias, buf.bias, pb.P, pb.nrows, pb.ncols, pb.ld, pb.H, stream,
-                         pb.name);
+    rc = split_pair_bias(pb.z, buf.wz, buf.wzinv, buf.wzbias, buf.bias, pb.P, pb.nrows, pb.ncols, pb.ld, pb.H,
+                         pb.scale, stream, pb.name);
   else
-    rc = pair_proj_f32(pb.z, pb.g, pb.b, pb.w, buf.bias, pb.P, pb.nrows, pb.ncols, pb.ld, pb.H, pb.c_z, stream, pb.name);
+    rc = pair_proj_f32(pb.z, pb.g, pb.b, pb.w, buf.bias, pb.P, pb.nrows, pb.ncols, pb.ld, pb.H, pb.c_z, pb.scale, stream,
+                       pb.name);
   if (rc) return rc;
   SplitGemmEpi e;
   e.out = buf.q;
   e.bias = q_bias;
   e.ldo = c_s;
   e.k = buf.k;
-  e.vt = buf.v;
+  e.v = buf.v;
   e.g = buf.g;
-  e.T = seq_len;
-  e.ldT = ldv;
+  e.T = v_transposed_len;
   if (r128)
     return split_gemm_r128(kSplitQkvg, s, buf.sp.w, buf.sp.winv, norm_s_w ? buf.wbias : nullptr, e, rows, 4 * c_s,
                            stream, "f32_proj_qkvg");
@@ -713,7 +630,7 @@ using namespace bioemu;
 extern "C" size_t bioemu_apb_f32_workspace_bytes(int64_t B, int64_t mult, int64_t N, int64_t c_s, int64_t H) {
   if (B <= 0 || mult <= 0 || N <= 0 || c_s <= 0 || H <= 0) return 0;
   const int64_t ld = round_up(N, 32);
-  return attn_f32_layout(B * mult * N, (int)c_s, (int)H, B * mult * c_s * ld, B * H * N * ld, nullptr, nullptr);
+  return attn_f32_layout(B * mult * N, (int)c_s, (int)H, N, B * H * N * ld, nullptr, nullptr);
 }
 
 extern "C" int bioemu_apb_fwd_f32(const float* s, const float* z, const uint8_t* mask, const float* norm_s_w,
@@ -741,24 +658,14 @@ extern "C" int bioemu_apb_fwd_f32(const float* s, const float* z, const uint8_t*
   const long long rows = B * mult * N;
   AttnF32Buffers buf;
   const int ldb = (int)round_up(N, 32);
-  attn_f32_layout(rows, (int)c_s, (int)H, B * mult * c_s * ldb, B * H * N * ldb, &buf, static_cast<char*>(workspace));
-  const PairBiasF32 pb{z, norm_z_w, norm_z_b, w_z, B * N * N, (int)N, (int)N, ldb, (int)H, (int)c_z, "f32_pair_bias"};
-  int rc = attn_f32_projections(s, norm_s_w, norm_s_b, w_qkv, q_bias, w_g, w_o, pb, buf, rows, (int)c_s, (int)N, ldb,
-                                stream);
+  attn_f32_layout(rows, (int)c_s, (int)H, N, B * H * N * ldb, &buf, static_cast<char*>(workspace));
+  const PairBiasF32 pb{z, norm_z_w, norm_z_b, w_z, B * N * N, (int)N, (int)N, ldb, (int)H, (int)c_z, kLog2e,
+                       "f32_pair_bias"};
+  int rc = attn_f32_projections(s, norm_s_w, norm_s_b, w_qkv, q_bias, w_g, w_o, pb, buf, rows, (int)c_s, 0, stream);
   if (rc) return rc;
-  {
-    KernelTimerScope timed("f32_attention", stream);
-    const dim3 grid((unsigned)((N + 127) / 128), (unsigned)H, (unsigned)(B * mult));
-    const int d = (int)(c_s / H);
-    const float rsq = 1.0f / std::sqrt((float)d);
-    if (d == 24)
-      hipLaunchKernelGGL(attn_f32_kernel<24>, grid, dim3(256), 0, stream, buf.q, buf.k, buf.v, buf.g, buf.bias, mask,
-                         buf.go, (int)N, ldb, (int)H, (int)c_s, (int)mult, rsq, 0);
-    else
-      hipLaunchKernelGGL(attn_f32_kernel<32>, grid, dim3(256), 0, stream, buf.q, buf.k, buf.v, buf.g, buf.bias, mask,
-                         buf.go, (int)N, ldb, (int)H, (int)c_s, (int)mult, rsq, 0);
-  }
-  rc = check_launch("f32_attention");
+  const SplitAttn at{buf.q, buf.k, buf.v, buf.g, buf.bias, mask, buf.go, buf.kv, buf.kvinv, buf.words,
+                     (int)(B * mult), (int)mult, (int)N, ldb, (int)H, (int)c_s, 0};
+  rc = split_attn(at, stream, "f32_attention");
   if (rc) return rc;
   return attn_f32_out(buf.go, residual ? s : nullptr, out, buf, rows, (int)c_s, stream, "f32_proj_o");
 }
@@ -766,7 +673,7 @@ extern "C" int bioemu_apb_fwd_f32(const float* s, const float* z, const uint8_t*
 extern "C" size_t bioemu_swa_f32_workspace_bytes(int64_t B, int64_t mult, int64_t NW, int64_t W, int64_t H,
                                                  int64_t c_s, int64_t heads) {
   if (B <= 0 || mult <= 0 || NW <= 0 || W != 32 || H <= 0 || c_s <= 0 || heads <= 0) return 0;
-  return attn_f32_layout(B * mult * NW * W, (int)c_s, (int)heads, B * mult * NW * W * c_s, B * NW * heads * W * H, nullptr, nullptr);
+  return attn_f32_layout(B * mult * NW * W, (int)c_s, (int)heads, 0, B * NW * heads * W * H, nullptr, nullptr);
 }
 
 extern "C" int bioemu_swa_fwd_f32(const float* s, const float* z, const uint8_t* mask, const float* norm_s_w,
@@ -798,11 +705,11 @@ extern "C" int bioemu_swa_fwd_f32(const float* s, const float* z, const uint8_t*
     return set_error(BIOEMU_ERR_WORKSPACE, "swa_f32: workspace too small");
   const long long rows = B * mult * NW * W;
   AttnF32Buffers buf;
-  attn_f32_layout(rows, (int)c_s, (int)heads, rows * c_s, B * NW * heads * W * H, &buf, static_cast<char*>(workspace));
+  attn_f32_layout(rows, (int)c_s, (int)heads, 0, B * NW * heads * W * H, &buf, static_cast<char*>(workspace));
   const PairBiasF32 pb{z, norm_z_w, norm_z_b, w_z, B * NW * W * H, (int)W, (int)H, (int)H, (int)heads, (int)c_z,
-                       "f32_swa_pair_bias"};
+                       1.0f, "f32_swa_pair_bias"};
   int rc = attn_f32_projections(s, norm_s_w, norm_s_b, w_qkv, q_bias, w_g, w_o, pb, buf, rows, (int)c_s,
-                                (int)(NW * W), (int)(NW * W), stream);
+                                (int)(NW * W), stream);
   if (rc) return rc;
   {
     KernelTimerScope timed("f32_swa_attention", stream);
@@ -1401,7 +1308,7 @@ extern "C" int bioemu_pwa_fwd_f32(const float* m, const float* z, const uint8_t*
   if ((rc = check_launch("f32_pwa_v"))) return rc;
   rc = gemm_f32(kGemmEpiSigmoid, mn, w_g, nullptr, nullptr, g, M, (int)c_m, hc, stream, "f32_pwa_gate");
   if (rc) return rc;
-  rc = pair_proj_f32(z, norm_z_w, norm_z_b, w_z, lg, B * N * N, (int)N, (int)N, Np8, (int)H, (int)c_z, stream,
+  rc = pair_proj_f32(z, norm_z_w, norm_z_b, w_z, lg, B * N * N, (int)N, (int)N, Np8, (int)H, (int)c_z, 1.0f, stream,
                      "f32_pwa_logits");
   if (rc) return rc;
   {
@@ -1590,7 +1497,7 @@ extern "C" size_t bioemu_triatt_f32_workspace_bytes(int64_t B, int64_t N, int64_
   if (B <= 0 || N <= 0 || D <= 0 || H <= 0) return 0;
   const int64_t P = B * N * N, ld = round_up(N, 32);
   return (size_t)round_up(P * D * 4, 256) + (size_t)round_up(P, 256) +
-         attn_f32_layout(P, (int)D, (int)H, B * N * D * ld, B * H * N * ld, nullptr, nullptr);
+         attn_f32_layout(P, (int)D, (int)H, N, B * H * N * ld, nullptr, nullptr);
 }
 
 extern "C" int bioemu_triatt_fwd_f32(const float* z, const uint8_t* mask, const float* norm_w, const float* norm_b,
@@ -1620,7 +1527,7 @@ extern "C" int bioemu_triatt_fwd_f32(const float* z, const uint8_t* mask, const 
   uint8_t* mt = reinterpret_cast<uint8_t*>(p);
   p += round_up(P, 256);
   AttnF32Buffers buf;
-  attn_f32_layout(P, c, (int)H, B * N * D * ld, B * H * N * ld, &buf, p);
+  attn_f32_layout(P, c, (int)H, N, B * H * N * ld, &buf, p);
   const float* src = z;
   const uint8_t* msk = mask;
   int rc = 0;
@@ -1636,17 +1543,13 @@ extern "C" int bioemu_triatt_fwd_f32(const float* z, const uint8_t* mask, const 
     msk = mt;
   }
   // w_proj rows: [Wq; Wk; Wv] (3c), Wg (c), Wb (H)
-  const PairBiasF32 pb{src, norm_w, norm_b, w_proj + 4 * D * D, P, (int)N, (int)N, ld, (int)H, c, "f32_triatt_bias"};
-  rc = attn_f32_projections(src, norm_w, norm_b, w_proj, nullptr, w_proj + 3 * D * D, w_o, pb, buf, P, c, (int)N, ld,
-                            stream);
+  const PairBiasF32 pb{src, norm_w, norm_b, w_proj + 4 * D * D, P, (int)N, (int)N, ld, (int)H, c, kLog2e,
+                       "f32_triatt_bias"};
+  rc = attn_f32_projections(src, norm_w, norm_b, w_proj, nullptr, w_proj + 3 * D * D, w_o, pb, buf, P, c, 0, stream);
   if (rc) return rc;
-  {
-    KernelTimerScope timed("f32_triatt_attention", stream);
-    const dim3 grid((unsigned)((N + 127) / 128), (unsigned)H, (unsigned)(B * N));
-    hipLaunchKernelGGL(attn_f32_kernel<32>, grid, dim3(256), 0, stream, buf.q, buf.k, buf.v, buf.g, buf.bias, msk,
-                       buf.go, (int)N, ld, (int)H, c, (int)N, 1.0f / std::sqrt(32.0f), 1);
-  }
-  if ((rc = check_launch("f32_triatt_attention"))) return rc;
+  const SplitAttn at{buf.q, buf.k, buf.v, buf.g, buf.bias, msk, buf.go, buf.kv, buf.kvinv, buf.words,
+                     (int)(B * N), (int)N, (int)N, ld, (int)H, c, 1};
+  if ((rc = split_attn(at, stream, "f32_triatt_attention"))) return rc;
   const float* go = buf.go;
   if (!starting) {
     if ((rc = transpose_pairs_f32(buf.go, zt, B, (int)N, c, stream, "f32_triatt_transpose_out"))) return rc;

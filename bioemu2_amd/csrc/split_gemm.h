@@ -15,8 +15,8 @@ struct SplitGemmEpi {
   const float* bias = nullptr;   // kSplitQkvg: q bias
   const float* res = nullptr;
   int ldo = 0;                   // row length of out (kSplitQkvg: c_s)
-  float *k = nullptr, *vt = nullptr, *g = nullptr;   // kSplitQkvg
-  int T = 1, ldT = 1;                                // kSplitQkvg: rows per sequence, stride of vt's channels
+  float *k = nullptr, *v = nullptr, *g = nullptr;   // kSplitQkvg
+  int T = 0;                                        // kSplitQkvg: v transposed per sequence of T rows (0: row-major)
   f16* hfrag = nullptr;          // kSplitSwiGLU
   float* hinv = nullptr;
   const float *rnorm = nullptr, *wnorm = nullptr;

@@ -329,11 +329,11 @@ __device__ __forceinline__ void epi_quad(const SplitGemmEpi& e, long long m, int
   } else if (kEpi == kSplitQkvg) {
     // columns [q | k | v | g], c_s each; a quad lies in one part
     const int cs = e.ldo, part = c / cs, cc = c - part * cs;
-    if (part == 2) {   // v transposed per sequence of T rows, keys contiguous
+    if (part == 2 && e.T) {   // v transposed per sequence of T rows, keys contiguous
       const long long sq = m / e.T, t = m - sq * e.T;
-      float* col = e.vt + ((size_t)sq * cs + cc) * e.ldT + t;
+      float* col = e.v + ((size_t)sq * cs + cc) * e.T + t;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) col[(size_t)u * e.ldT] = v[u];
+      for (int u = 0; u < 4; ++u) col[(size_t)u * e.T] = v[u];
       return;
     }
     if (part == 0 && e.bias) {
@@ -344,7 +344,7 @@ __device__ __forceinline__ void epi_quad(const SplitGemmEpi& e, long long m, int
 #pragma unroll
       for (int t = 0; t < 4; ++t) v[t] = sigmoid_f32(v[t]);
     }
-    float* d = (part == 0 ? e.out : part == 1 ? e.k : e.g) + (size_t)m * cs + cc;
+    float* d = (part == 0 ? e.out : part == 1 ? e.k : part == 2 ? e.v : e.g) + (size_t)m * cs + cc;
     *reinterpret_cast<f32x4*>(d) = v;
   }
 }

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(256, 3) void pair_bias_split_kernel(const float* __
                                                                  const float* __restrict__ winv,
                                                                  const float* __restrict__ wbias,
                                                                  float* __restrict__ out, unsigned P, unsigned nrows,
-                                                                 unsigned ncols, int ld, int H, int tiles) {
+                                                                 unsigned ncols, int ld, int H, float scale, int tiles) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f16* smem = reinterpret_cast<f16*>(smem_raw);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256, 3) void pair_bias_split_kernel(const float* __
         float* d = out + (((size_t)outer * H + h0) * nrows + r) * ld + col;
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
-          if (h0 + u < H) *d = acc[u] * sc + wbias[h0 + u];
+          if (h0 + u < H) *d = (acc[u] * sc + wbias[h0 + u]) * scale;
           d += (size_t)nrows * ld;
         }
       }
@@ -130,12 +130,12 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
 }
 
 int split_pair_bias(const float* z, const f16* W, const float* winv, const float* wbias, float* out, long long P,
-                    int nrows, int ncols, int ld, int H, hipStream_t stream, const char* name) {
+                    int nrows, int ncols, int ld, int H, float scale, hipStream_t stream, const char* name) {
   const int tiles = (int)((P + 31) / 32), smem = (H + 31) / 32 * 8 * kFrag * (int)sizeof(f16);
   const int grid = std::min((tiles + 3) / 4, 1024);   // four workgroups per CU
   KernelTimerScope timed(name, stream);
   hipLaunchKernelGGL(pair_bias_split_kernel, dim3((unsigned)grid), dim3(256), (unsigned)smem, stream, z, W, winv, wbias,
-                     out, (unsigned)P, (unsigned)nrows, (unsigned)ncols, ld, H, tiles);
+                     out, (unsigned)P, (unsigned)nrows, (unsigned)ncols, ld, H, scale, tiles);
   return check_launch(name);
 }
 

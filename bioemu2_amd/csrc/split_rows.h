@@ -124,9 +124,24 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
                    long long P, hipStream_t stream, const char* name);
 
 // Pair bias LN(z) W^T of P < 2^31 rows of 128 channels, head-major: row p = (outer, r, c) -> out[outer][head][r][c],
-// rows ld apart (split_pair.hip); W, winv, wbias: H x 128 weights with the LayerNorm folded in, H <= 64.
+// rows ld apart, times `scale` (split_pair.hip); W, winv, wbias: H x 128 weights with the LayerNorm folded in, H <= 64.
 int split_pair_bias(const float* z, const f16* W, const float* winv, const float* wbias, float* out, long long P,
-                    int nrows, int ncols, int ld, int H, hipStream_t stream, const char* name);
+                    int nrows, int ncols, int ld, int H, float scale, hipStream_t stream, const char* name);
+
+// Attention of BM = B * mult sequences of N tokens, heads of 24 or 32 channels (split_attn.hip): q, k, v, g, go
+// [BM][N][c_s], bias [B][H][N][ld] times log2(e), mask [B][N] or, mask_per_copy, [BM][N].  Scratch: kv
+// split_attn_kv_elems, kvinv 2 floats and words one 32-bit word per 32 keys of every (sequence, head).
+struct SplitAttn {
+  const float *q, *k, *v, *g, *bias;
+  const uint8_t* mask;
+  float* go;
+  f16* kv;
+  float* kvinv;
+  uint32_t* words;
+  int BM, mult, N, ld, H, c_s, mask_per_copy;
+};
+size_t split_attn_kv_elems(int64_t BM, int64_t H, int64_t N);
+int split_attn(const SplitAttn& a, hipStream_t stream, const char* name);
 
 // Triangle multiplication of 128 channels (split_trimul.hip): the arguments of bioemu_trimul_fwd_f32.
 size_t split_trimul_workspace_bytes(int64_t B, int64_t N);

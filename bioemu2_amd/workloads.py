@@ -902,8 +902,10 @@ class ApbWorkload(Workload):
                 return ("mfma_split", 2.0 * rows * 384 * 384)
             if kernel == "f32_pair_bias":   # reads z, writes the 16-head bias
                 return ("hbm", float(B * n * n * (128 + 16) * 4))
+            if kernel == "f32_kv_fragments":   # reads k and v, writes them as fragments (head dim padded to 32)
+                return ("hbm", float(2 * rows * 384 * 4 * (1 + 32 / 24)))
             if kernel == "f32_attention":   # QK^T and PV: 4 N^2 c_s per copy
-                return ("mfma_f32", 4.0 * B * M * n * n * 384)
+                return ("mfma_split", 4.0 * B * M * n * n * 384)
             raise KeyError(kernel)
         np_ = -(-n // 32) * 32
         tok = B * M * np_ * 384 * 2

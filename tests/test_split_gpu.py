@@ -165,3 +165,36 @@ def test_trimul_split_edges(gpu_device, mode, n, b):
     with torch.no_grad():
         got = m(x.to(gpu_device), mask.to(gpu_device)).cpu()
     assert rel_l2(got, want) <= TOL
+
+
+@pytest.mark.parametrize("n,pad", [(1, 0), (31, 3), (33, 0), (97, 96), (129, 40)])
+def test_attention_split_edges(gpu_device, n, pad):
+    """Key counts around a 32-key block and a 128-query workgroup; whole blocks masked; values of masked tokens,
+    however large, never reach the others' results (bit for bit)."""
+    torch.manual_seed(6)
+    m = randomize_params(AttentionPairBias(384, 128, 16, initial_norm=False), 8)
+    s, z = torch.randn(2, n, 384), torch.randn(1, n, n, 128)
+    mask = torch.ones(1, n, dtype=torch.bool)
+    mask[:, n - pad:] = False
+    want = _apb64(s.double(), z.double(), mask, _params(m), 16, 2, False)
+    m = m.to(gpu_device)
+    big = s.clone()
+    big[:, n - pad:] *= 1e8
+    with torch.no_grad():
+        got = m(s.to(gpu_device), z.to(gpu_device), mask.to(gpu_device), multiplicity=2).cpu()
+        got_big = m(big.to(gpu_device), z.to(gpu_device), mask.to(gpu_device), multiplicity=2).cpu()
+    assert rel_l2(got, want) <= TOL
+    assert torch.equal(got[:, : n - pad], got_big[:, : n - pad])
+
+
+def test_attention_split_all_masked(gpu_device):
+    """A sequence without a valid key averages its values (equal logits), next to one that has some."""
+    torch.manual_seed(7)
+    m = randomize_params(AttentionPairBias(384, 128, 16, initial_norm=False), 9)
+    s, z = torch.randn(2, 70, 384), torch.randn(2, 70, 70, 128)
+    mask = torch.ones(2, 70, dtype=torch.bool)
+    mask[1] = False
+    want = _apb64(s.double(), z.double(), mask, _params(m), 16, 1, False)
+    m = m.to(gpu_device)
+    with torch.no_grad():
+        assert rel_l2(m(s.to(gpu_device), z.to(gpu_device), mask.to(gpu_device)).cpu(), want) <= TOL
