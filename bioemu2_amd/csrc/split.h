@@ -89,6 +89,49 @@ __device__ __forceinline__ SplitFrag load_frag(const f16* p, int lane) {
   return f;
 }
 
+// acc += the product of a 32 x 16 KS weight block (fragments in LDS at w) with xf; kWeightRows: the weights are the
+// MFMA rows.  Two k-steps' fragments are in flight ahead of the one multiplied.
+template <int KS, bool kWeightRows = true>
+__device__ __forceinline__ void mfma_block(const f16* w, const SplitFrag* xf, int lane, f32x16& acc) {
+  SplitFrag f[3];
+  f[0] = load_frag(w, lane);
+  f[1] = load_frag(w + kFrag, lane);
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    if (s + 2 < KS) f[(s + 2) % 3] = load_frag(w + (s + 2) * kFrag, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kWeightRows)
+      mfma_split(f[s % 3], xf[s], acc);
+    else
+      mfma_split(xf[s], f[s % 3], acc);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+// Two weight blocks and two accumulators, a k-step of each at a time.
+template <int KS, bool kWeightRows = true>
+__device__ __forceinline__ void mfma_block2(const f16* w1, const f16* w2, const SplitFrag* x1, const SplitFrag* x2,
+                                            int lane, f32x16& acc1, f32x16& acc2) {
+  SplitFrag f1[2], f2[2];
+  f1[0] = load_frag(w1, lane);
+  f2[0] = load_frag(w2, lane);
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    if (s + 1 < KS) {
+      f1[(s + 1) & 1] = load_frag(w1 + (s + 1) * kFrag, lane);
+      f2[(s + 1) & 1] = load_frag(w2 + (s + 1) * kFrag, lane);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (kWeightRows) {
+      mfma_split(f1[s & 1], x1[s], acc1);
+      mfma_split(f2[s & 1], x2[s], acc2);
+    } else {
+      mfma_split(x1[s], f1[s & 1], acc1);
+      mfma_split(x2[s], f2[s & 1], acc2);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 __device__ __forceinline__ void copy1k_to_lds(__amdgpu_buffer_rsrc_t r, const f16* lds, unsigned voff, unsigned soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(lds), 16, voff, soff, 0, 0);
 }

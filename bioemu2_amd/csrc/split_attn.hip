@@ -17,7 +17,7 @@
 // Blocks without an unmasked key are left out unless the sequence has none at all (then every
 // weight is the same, as in softmax over equal logits).
 //
-// 16 heads of 24, 768 tokens, 8 copies sharing one bias: 0.056 ms and 0.011 ms for the fragments, against 0.129 ms
+// 16 heads of 24, 768 tokens, 8 copies sharing one bias: 0.054 ms and 0.011 ms for the fragments, against 0.129 ms
 // for the same flash form on fp32 MFMAs with per-key mask tests (28 MFMAs of 64 cycles and about 290 VALU
 // instructions per block and wave; now 12 of 32 and about 130).  Bound by the VALU work of the softmax and the split
 // of the weights.
@@ -204,19 +204,24 @@ __global__ __launch_bounds__(256, 3) void attn_split_kernel(const float* __restr
     const int kcur = kb;
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies (and bias loads) of the block landed
     __syncthreads();                       // ... and everyone's; the other stage is free again
+    const f16* f = smem[st];
+    SplitFrag kf[2], vf[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) kf[ks] = load_frag(f + ks * kFrag, lane);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) vf[ks] = load_frag(f + (2 + ks) * kFrag, lane);
+    const int nk = a + 1 < na ? __builtin_amdgcn_readfirstlane(active[a + 1]) : kb;
+    // every LDS read of the block precedes the next block's copies: the compiler makes a later one wait for them
+    __builtin_amdgcn_sched_barrier(0);
     f32x4 bn[4];
     if (a + 1 < na) {
-      kb = __builtin_amdgcn_readfirstlane(active[a + 1]);
+      kb = nk;
       stage(kb, st ^ 1);
       load_bias(kb, bn);
     }
-    const f16* f = smem[st];
     f32x16 s = zero16();
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) mfma_split(load_frag(f + ks * kFrag, lane), qf[ks], s);
-    SplitFrag vf[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) vf[ks] = load_frag(f + (2 + ks) * kFrag, lane);
+    for (int ks = 0; ks < 2; ++ks) mfma_split(kf[ks], qf[ks], s);
     float x[16];
 #pragma unroll
     for (int u = 0; u < 16; ++u) x[u] = s[u] * sk + bb[u >> 2][u & 3];

@@ -5,10 +5,9 @@
 
 namespace bioemu {
 
-constexpr int kSplitStore = 0;     // out = v (+ bias) (+ res)
-constexpr int kSplitSigmoid = 1;   // out = sigmoid(v)
-constexpr int kSplitSwiGLU = 2;    // fc1 / fc2 column blocks interleaved; silu(a) b as operand fragments
-constexpr int kSplitQkvg = 3;      // the four token projections of an attention
+constexpr int kSplitStore = 0;     // out = v (+ res)
+constexpr int kSplitSwiGLU = 1;    // fc1 / fc2 column blocks interleaved; silu(a) b as operand fragments
+constexpr int kSplitQkvg = 2;      // the four token projections of an attention
 
 struct SplitGemmEpi {
   float* out = nullptr;          // kSplitQkvg: q

@@ -309,23 +309,28 @@ __global__ __launch_bounds__(256) void split_long_rows_kernel(const float* __res
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
+// What is added to channels c0 .. c0 + 15 of row m: the residual (kSplitStore), the q bias (kSplitQkvg).
 template <int kEpi>
-__device__ __forceinline__ void epi_quad(const SplitGemmEpi& e, long long m, int c, f32x4 v) {
+__device__ __forceinline__ void load_addend(const SplitGemmEpi& e, long long m, int c0, f32x4 (&r)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (kEpi == kSplitStore && e.res)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = *reinterpret_cast<const f32x4*>(e.res + (size_t)m * e.ldo + c0 + 4 * q);
+  if (kEpi == kSplitQkvg && e.bias && c0 < e.ldo)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) r[q][t] = e.bias[c0 + 4 * q + t];
+}
+
+template <int kEpi>
+__device__ __forceinline__ void epi_quad(const SplitGemmEpi& e, long long m, int c, f32x4 v, f32x4 r) {
   if (kEpi == kSplitStore) {
-    if (e.bias)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) v[t] += e.bias[c + t];
     float* d = e.out + (size_t)m * e.ldo + c;
-    if (e.res) {
-      const f32x4 r = *reinterpret_cast<const f32x4*>(e.res + (size_t)m * e.ldo + c);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) v[t] += r[t];
-    }
+    for (int t = 0; t < 4; ++t) v[t] += r[t];
     *reinterpret_cast<f32x4*>(d) = v;
-  } else if (kEpi == kSplitSigmoid) {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) v[t] = sigmoid_f32(v[t]);
-    *reinterpret_cast<f32x4*>(e.out + (size_t)m * e.ldo + c) = v;
   } else if (kEpi == kSplitQkvg) {
     // columns [q | k | v | g], c_s each; a quad lies in one part
     const int cs = e.ldo, part = c / cs, cc = c - part * cs;
@@ -338,7 +343,7 @@ __device__ __forceinline__ void epi_quad(const SplitGemmEpi& e, long long m, int
     }
     if (part == 0 && e.bias) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) v[t] += e.bias[cc + t];
+      for (int t = 0; t < 4; ++t) v[t] += r[t];
     }
     if (part == 3) {
 #pragma unroll
@@ -475,12 +480,15 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         if (cb0 + j >= nblocks) break;
+        const int c0 = (cb0 + j) * 32 + 16 * h;
+        f32x4 res[4];   // read ahead of the stores (out may be res)
+        load_addend<kEpi>(e, m, c0, res);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           f32x4 v;
 #pragma unroll
           for (int t = 0; t < 4; ++t) v[t] = acc[j][i][4 * q + t] * s * (j ? w1 : w0);
-          epi_quad<kEpi>(e, m, (cb0 + j) * 32 + 16 * h + 4 * q, v);
+          epi_quad<kEpi>(e, m, c0 + 4 * q, v, res[q]);
         }
       }
     }
@@ -561,8 +569,22 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
     if (cb0 == 0 && h == 0 && wave == 0) e.hinv[m] = split_inv(hs);
     epi_swiglu_quad(e, m, cb0 * 16 + c, sum[0], sum[1], hs);
   } else {
-    epi_quad<kEpi>(e, m, cb0 * 32 + c, sum[0]);
-    if (two) epi_quad<kEpi>(e, m, (cb0 + 1) * 32 + c, sum[1]);
+    f32x4 r0 = {0.f, 0.f, 0.f, 0.f}, r1 = r0;
+    const int c0 = cb0 * 32 + c;
+    if (kEpi == kSplitStore && e.res) {
+      const float* r = e.res + (size_t)m * e.ldo + c0;
+      r0 = *reinterpret_cast<const f32x4*>(r);
+      if (two) r1 = *reinterpret_cast<const f32x4*>(r + 32);
+    }
+    if (kEpi == kSplitQkvg && e.bias) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (c0 < e.ldo) r0[t] = e.bias[c0 + t];
+        if (two && c0 + 32 < e.ldo) r1[t] = e.bias[c0 + 32 + t];
+      }
+    }
+    epi_quad<kEpi>(e, m, cb0 * 32 + c, sum[0], r0);
+    if (two) epi_quad<kEpi>(e, m, (cb0 + 1) * 32 + c, sum[1], r1);
   }
 }
 
@@ -571,6 +593,7 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
 // through double-buffered LDS.  For K = 128 this replaces the separate fragment pass and the short k-loop of the
 // tiled kernel.
 constexpr int kR128Block = 8 * kFrag;   // f16 elements of one 32-channel block
+constexpr int kR128MaxN = 512;          // output channels with a bias
 
 template <int kEpi, bool kLn>
 __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __restrict__ x, const f16* __restrict__ W,
@@ -578,6 +601,7 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
                                                                  const float* __restrict__ wbias, SplitGemmEpi e,
                                                                  long long M, int nblocks) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][kR128Block];
+  __shared__ __attribute__((aligned(16))) float sbias[kLn ? kR128MaxN : 4];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, (unsigned)nblocks * kR128Block * 2);
   auto stage = [&](int cb) {
@@ -588,6 +612,7 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
     }
   };
   stage(0);
+  if (kLn) stage_floats(sbias, wbias, nblocks * 32, nblocks * 32);
   const long long m = ((long long)blockIdx.x * 4 + wave) * 32 + n;
   const bool valid = m < M;
   SplitFrag xf[8];
@@ -603,18 +628,19 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
     __syncthreads();                       // ... and everyone's; the other stage is free again
     if (cb + 1 < nblocks) stage(cb + 1);
     f32x16 acc = zero16();
-#pragma unroll
-    for (int s = 0; s < 8; ++s) mfma_split(load_frag(&smem[cb & 1][s * kFrag], lane), xf[s], acc);
+    mfma_block<8>(smem[cb & 1], xf, lane, acc);
     const float sc = xinv * winv[cb];
     if (valid) {
+      const int c0 = cb * 32 + 16 * h;
+      f32x4 res[4];
+      load_addend<kEpi>(e, m, c0, res);
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int c = cb * 32 + 16 * h + 4 * q;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
-        if (kLn) v = *reinterpret_cast<const f32x4*>(wbias + c);
+        if (kLn) v = *reinterpret_cast<const f32x4*>(&sbias[c0 + 4 * q]);
 #pragma unroll
         for (int t = 0; t < 4; ++t) v[t] += acc[4 * q + t] * sc;
-        epi_quad<kEpi>(e, m, c, v);
+        epi_quad<kEpi>(e, m, c0 + 4 * q, v, res[q]);
       }
     }
   }
@@ -625,6 +651,7 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
 int split_gemm_r128(int epi, const float* x, const f16* W, const float* winv, const float* wbias,
                     const SplitGemmEpi& e, long long M, int N, hipStream_t stream, const char* name) {
   const dim3 grid((unsigned)((M + 127) / 128));
+  if (wbias && N > kR128MaxN) return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: %d output channels", name, N);
   KernelTimerScope timed(name, stream);
 #define BIOEMU_R128(E, L) \
   hipLaunchKernelGGL((split_gemm_r128_kernel<E, L>), grid, dim3(256), 0, stream, x, W, winv, wbias, e, M, N / 32)
@@ -703,7 +730,6 @@ int split_gemm(int epi, const f16* A, const float* ainv, const f16* W, const flo
   } while (0)
   switch (epi) {
     case kSplitStore: BIOEMU_SPLIT_GEMM(kSplitStore); break;
-    case kSplitSigmoid: BIOEMU_SPLIT_GEMM(kSplitSigmoid); break;
     case kSplitSwiGLU: BIOEMU_SPLIT_GEMM(kSplitSwiGLU); break;
     default: BIOEMU_SPLIT_GEMM(kSplitQkvg); break;
   }

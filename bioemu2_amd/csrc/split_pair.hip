@@ -2,9 +2,11 @@
 // the rows each: a wave normalises 32 rows in registers and multiplies them with
 // weights that stay in LDS for the whole launch (grid of resident workgroups,
 // waves walking row tiles).  Both are bound by reading the rows: the conditioning
-// projection (590k rows of 256, 906 MB) takes 0.221 ms, 4.1 TB/s, against 1.17 ms for
+// projection (590k rows of 256, 906 MB) takes 0.217 ms, 4.2 TB/s, against 1.17 ms for
 // a LayerNorm pass and an fp32-MFMA product; the 16-head pair bias (590k rows of 128,
-// 340 MB) 0.097 ms, 3.5 TB/s, against 0.109 ms for one thread per row on the VALU.
+// 340 MB) 0.076 ms, 4.5 TB/s (a copy on this card: 4.9), against 0.109 ms for one
+// thread per row on the VALU.  Rows requested a tile ahead and biases read from LDS
+// (a global load in the epilogue waits for the stores before it) took it from 0.097.
 #include <algorithm>
 
 #include "split.h"
@@ -15,7 +17,7 @@ namespace {
 
 constexpr int kCatWaves = 8;
 constexpr int kCatWeights = 4 * 16 * kFrag;               // f16: [4 column blocks][16 k-steps]
-constexpr int kCatSmem = kCatWeights * (int)sizeof(f16);  // 128 KB
+constexpr int kCatSmem = kCatWeights * (int)sizeof(f16) + 128 * 4;  // 128 KB and the biases
 
 __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
     const float* __restrict__ x1, const float* __restrict__ x2, const f16* __restrict__ W,
@@ -23,16 +25,22 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f16* smem = reinterpret_cast<f16*>(smem_raw);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
-  stage_fragments(W, smem, kCatSmem / 1024, kCatWaves, wave, lane);
+  float* sbias = reinterpret_cast<float*>(smem + kCatWeights);
+  stage_floats(sbias, wbias, 128, 128);
+  stage_fragments(W, smem, kCatWeights / kFragHalf, kCatWaves, wave, lane);
+  // half of the next tile's rows is requested as soon as this tile's are fragments, ahead of its products and stores
+  float a[64];
+  auto row_of = [&](int tile) { return (size_t)std::min((long long)tile * 32 + n, P - 1) * 128; };
+  const int first = blockIdx.x * kCatWaves + wave, step = gridDim.x * kCatWaves;
+  if (first < tiles) load_row_half<128>(x1 + row_of(first), h, a);
 #pragma unroll 1
-  for (int tile = blockIdx.x * kCatWaves + wave; tile < tiles; tile += gridDim.x * kCatWaves) {
+  for (int tile = first; tile < tiles; tile += step) {
     const long long m = (long long)tile * 32 + n;
     const bool valid = m < P;
     SplitFrag xf[16];
     {
-      float a[64], c[64];
-      load_row_half<128>(x1 + (size_t)(valid ? m : 0) * 128, h, a);
-      load_row_half<128>(x2 + (size_t)(valid ? m : 0) * 128, h, c);
+      float c[64];
+      load_row_half<128>(x2 + row_of(tile), h, c);
       float s = 0.f;   // LayerNorm statistics over the concatenation
 #pragma unroll
       for (int i = 0; i < 64; ++i) s += a[i] + c[i];
@@ -50,19 +58,20 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
       split_normalized<128>(a, rstd, xf);
       split_normalized<128>(c, rstd, xf + 8);
     }
+    if (tile + step < tiles) load_row_half<128>(x1 + row_of(tile + step), h, a);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
     for (int cb = 0; cb < 4; ++cb) {
       const f16* w = smem + cb * 16 * kFrag;
       f32x16 acc = zero16();
-#pragma unroll
-      for (int s = 0; s < 16; ++s) mfma_split(load_frag(w + s * kFrag, lane), xf[s], acc);
+      mfma_block<16>(w, xf, lane, acc);
       const float sc = winv[cb] * (1.0f / kNormScale);
       if (valid) {
         const int c0 = cb * 32 + 16 * h;
         float* d = out + (size_t)m * 128 + c0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          f32x4 v = *reinterpret_cast<const f32x4*>(wbias + c0 + 4 * q);
+          f32x4 v = *reinterpret_cast<const f32x4*>(sbias + c0 + 4 * q);
 #pragma unroll
           for (int t = 0; t < 4; ++t) v[t] += acc[4 * q + t] * sc;
           *reinterpret_cast<f32x4*>(d + 4 * q) = v;
@@ -74,7 +83,7 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
 
 // Heads are the MFMA rows, pair rows its columns: register u of lane (n, h) is
 // head 32 hb + 16 h + u of pair n, so a store writes 32 consecutive columns.
-__global__ __launch_bounds__(256, 3) void pair_bias_split_kernel(const float* __restrict__ z, const f16* __restrict__ W,
+__global__ __launch_bounds__(256, 2) void pair_bias_split_kernel(const float* __restrict__ z, const f16* __restrict__ W,
                                                                  const float* __restrict__ winv,
                                                                  const float* __restrict__ wbias,
                                                                  float* __restrict__ out, unsigned P, unsigned nrows,
@@ -83,30 +92,33 @@ __global__ __launch_bounds__(256, 3) void pair_bias_split_kernel(const float* __
   f16* smem = reinterpret_cast<f16*>(smem_raw);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const int nhb = (H + 31) / 32;
+  float* sbias = reinterpret_cast<float*>(smem + nhb * 8 * kFrag);
+  stage_floats(sbias, wbias, H, nhb * 32);
   stage_fragments(W, smem, nhb * 16, 4, wave, lane);
+  float v[64];
+  auto load_rows = [&](int tile) { load_row_half<128>(z + (size_t)min((unsigned)tile * 32 + n, P - 1) * 128, h, v); };
+  const int first = blockIdx.x * 4 + wave, step = gridDim.x * 4;
+  if (first < tiles) load_rows(first);
 #pragma unroll 1
-  for (int tile = blockIdx.x * 4 + wave; tile < tiles; tile += gridDim.x * 4) {
+  for (int tile = first; tile < tiles; tile += step) {
     const unsigned p = (unsigned)tile * 32 + n;
     const bool valid = p < P;
     SplitFrag xf[8];
-    {
-      float v[64];
-      load_row_half<128>(z + (size_t)(valid ? p : 0) * 128, h, v);
-      normalized_row_half<128>(v, xf);
-    }
+    normalized_row_half<128>(v, xf);
+    if (tile + step < tiles) load_rows(tile + step);
+    __builtin_amdgcn_sched_barrier(0);
     const unsigned rr = p / ncols, col = p - rr * ncols, outer = rr / nrows, r = rr - outer * nrows;
 #pragma unroll 1
     for (int hb = 0; hb < nhb; ++hb) {
       f32x16 acc = zero16();
-#pragma unroll
-      for (int s = 0; s < 8; ++s) mfma_split(load_frag(smem + (hb * 8 + s) * kFrag, lane), xf[s], acc);
+      mfma_block<8>(smem + hb * 8 * kFrag, xf, lane, acc);
       const float sc = winv[hb] * (1.0f / kNormScale);
       const int h0 = hb * 32 + 16 * h;
       if (valid) {
         float* d = out + (((size_t)outer * H + h0) * nrows + r) * ld + col;
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
-          if (h0 + u < H) *d = (acc[u] * sc + wbias[h0 + u]) * scale;
+          if (h0 + u < H) *d = (acc[u] * sc + sbias[h0 + u]) * scale;
           d += (size_t)nrows * ld;
         }
       }
@@ -131,7 +143,7 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
 
 int split_pair_bias(const float* z, const f16* W, const float* winv, const float* wbias, float* out, long long P,
                     int nrows, int ncols, int ld, int H, float scale, hipStream_t stream, const char* name) {
-  const int tiles = (int)((P + 31) / 32), smem = (H + 31) / 32 * 8 * kFrag * (int)sizeof(f16);
+  const int tiles = (int)((P + 31) / 32), smem = (H + 31) / 32 * (8 * kFrag * (int)sizeof(f16) + 32 * 4);
   const int grid = std::min((tiles + 3) / 4, 1024);   // four workgroups per CU
   KernelTimerScope timed(name, stream);
   hipLaunchKernelGGL(pair_bias_split_kernel, dim3((unsigned)grid), dim3(256), (unsigned)smem, stream, z, W, winv, wbias,

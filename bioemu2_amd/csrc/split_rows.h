@@ -106,6 +106,12 @@ __device__ __forceinline__ void stage_fragments(const f16* W, f16* smem, int kb,
   __syncthreads();
 }
 
+// Copies `count` floats into LDS (whole workgroup; no barrier).  Epilogues read their biases from LDS: a global load
+// there would wait for every store before it (vmcnt counts both, in order).
+__device__ __forceinline__ void stage_floats(float* dst, const float* __restrict__ src, int count, int padded) {
+  for (int i = threadIdx.x; i < padded; i += blockDim.x) dst[i] = i < count ? src[i] : 0.f;
+}
+
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------

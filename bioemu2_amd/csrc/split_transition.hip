@@ -95,21 +95,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
     const f16* st = smem + (hc & 1) * G::Chunk;
     const float s1 = xinv * inv12[2 * hc], s2 = xinv * inv12[2 * hc + 1];
     f32x16 a = zero16(), gt = zero16();
-    // each k-step's fragments are requested during the previous one's products
-    SplitFrag f1[2], f2[2];
-    f1[0] = load_frag(st, lane);
-    f2[0] = load_frag(st + G::KS * kFrag, lane);
-#pragma unroll
-    for (int s = 0; s < G::KS; ++s) {
-      if (s + 1 < G::KS) {
-        f1[(s + 1) & 1] = load_frag(st + (s + 1) * kFrag, lane);
-        f2[(s + 1) & 1] = load_frag(st + (G::KS + s + 1) * kFrag, lane);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      mfma_split(f1[s & 1], xf[s], a);
-      mfma_split(f2[s & 1], xf[s], gt);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    mfma_block2<G::KS>(st, st + G::KS * kFrag, xf, xf, lane, a, gt);
     SplitFrag hf[2];
     const float* sb = sbias + hc * 64 + 16 * h;
 #pragma unroll

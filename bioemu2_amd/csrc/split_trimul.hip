@@ -15,7 +15,7 @@
 // N = 333, against the fp32-MFMA kernels these replace (operands from L2, the contraction stored 4 bytes at a time
 // pair-major, LayerNorms and the gate through memory): projection 0.079 ms (was 0.283, with 0.030 of zero fill and
 // 0.042 of LayerNorm), contraction 0.057 (0.376; 166 TFLOP/s of fp32 products on the padded 384 x 384 x 352, bound by
-// LDS like split_gemm_kernel), output 0.070 (0.226, with 0.042 of LayerNorm and 0.067 of gate).  The sigmoids
+// LDS like split_gemm_kernel), output 0.057 (0.226, with 0.042 of LayerNorm and 0.067 of gate).  The sigmoids
 // keep an ulp's accuracy: with the plain hardware exp2 and reciprocal the result was 1.4 times as far from float64.
 #include <algorithm>
 
@@ -40,6 +40,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
                                                                f16* __restrict__ lo, int N, int outgoing,
                                                                unsigned tiles) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][2 * kWBlock];   // p | g block, double-buffered: 64 KB
+  __shared__ float sbias[4 * D];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, 8 * 2 * kWBlock * 2);
   auto stage = [&](int cb) {
@@ -50,6 +51,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
     }
   };
   stage(0);
+  stage_floats(sbias, wbias, 4 * D, 4 * D);
   // tile (b, i, kb): 32 pairs k = 32 kb .. of line i; a wave past the last tile works on tile 0 and stores nothing
   const unsigned tile = blockIdx.x * 4 + wave;
   const bool live = tile < tiles;
@@ -76,14 +78,10 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
     // consecutive pairs 16 h + u of channel perm32(n)
     const f16* st = smem[cb & 1];
     f32x16 p = zero16(), g = zero16();
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      mfma_split(xf[s], load_frag(st + s * kFrag, lane), p);
-      mfma_split(xf[s], load_frag(st + (8 + s) * kFrag, lane), g);
-    }
+    mfma_block2<8, false>(st, st + kWBlock, xf, xf, lane, p, g);
     const int c = cb * 32 + perm32(n);
     const float sp = winv[2 * cb] * (1.0f / kNormScale), sg = winv[2 * cb + 1] * (1.0f / kNormScale);
-    const float bp = wbias[c], bg = wbias[2 * D + c], s = split_scale(wnorm[2 * cb] * 1.01f);
+    const float bp = sbias[c], bg = sbias[2 * D + c], s = split_scale(wnorm[2 * cb] * 1.01f);
     f16x8 vh[2], vl[2];
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
@@ -210,7 +208,8 @@ __device__ __forceinline__ float gated(float p, float g) {
 #pragma clang fp contract(off)
   return p * sigmoid_ulp(g);
 }
-constexpr int kOutSmem = 2 * 4 * kWBlock * (int)sizeof(f16);   // p_out | g_out: 128 KB
+constexpr int kOutWeights = 2 * 4 * kWBlock;                                  // f16: p_out | g_out
+constexpr int kOutSmem = kOutWeights * (int)sizeof(f16) + 2 * D * 4;          // 128 KB and the biases
 
 __global__ __launch_bounds__(64 * kOutWaves, 2) void trimul_out_kernel(const float* x, const float* __restrict__ o,
                                                                        const f16* __restrict__ W,
@@ -220,7 +219,9 @@ __global__ __launch_bounds__(64 * kOutWaves, 2) void trimul_out_kernel(const flo
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f16* smem = reinterpret_cast<f16*>(smem_raw);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
-  stage_fragments(W, smem, kOutSmem / 1024, kOutWaves, wave, lane);
+  float* sbias = reinterpret_cast<float*>(smem + kOutWeights);
+  stage_floats(sbias, wbias, 2 * D, 2 * D);
+  stage_fragments(W, smem, kOutWeights / kFragHalf, kOutWaves, wave, lane);
   const int ld = plane_ld(N);
   const size_t plane = (size_t)N * ld;
 #pragma unroll 1
@@ -248,26 +249,25 @@ __global__ __launch_bounds__(64 * kOutWaves, 2) void trimul_out_kernel(const flo
     for (int cb = 0; cb < 4; ++cb) {
       const f16* w = smem + cb * kWBlock;
       f32x16 p = zero16(), g = zero16();
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        mfma_split(load_frag(w + s * kFrag, lane), of[s], p);
-        mfma_split(load_frag(w + 4 * kWBlock + s * kFrag, lane), xf[s], g);
-      }
+      mfma_block2<8>(w, w + 4 * kWBlock, of, xf, lane, p, g);
       const float sp = winv[cb] * (1.0f / kNormScale), sg = winv[4 + cb] * (1.0f / kNormScale);
       const int c = cb * 32 + 16 * h;
       if (valid) {
+        f32x4 xr[4];   // read ahead of the stores (out may be x)
+        if (residual)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) xr[q] = *reinterpret_cast<const f32x4*>(x + m * D + c + 4 * q);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const f32x4 bp = *reinterpret_cast<const f32x4*>(wbias + c + 4 * q);
-          const f32x4 bg = *reinterpret_cast<const f32x4*>(wbias + D + c + 4 * q);
+          const f32x4 bp = *reinterpret_cast<const f32x4*>(sbias + c + 4 * q);
+          const f32x4 bg = *reinterpret_cast<const f32x4*>(sbias + D + c + 4 * q);
           f32x4 r;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
             r[e] = gated(p[4 * q + e] * sp + bp[e], g[4 * q + e] * sg + bg[e]);
           if (residual) {
-            const f32x4 xr = *reinterpret_cast<const f32x4*>(x + m * D + c + 4 * q);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r[e] += xr[e];
+            for (int e = 0; e < 4; ++e) r[e] += xr[q][e];
           }
           *reinterpret_cast<f32x4*>(out + m * D + c + 4 * q) = r;
         }
