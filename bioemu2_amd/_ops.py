@@ -30,7 +30,7 @@ def _ptr(t: Tensor | None) -> int | None:
 
 
 def _stream(t: Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_gpu(t: Tensor, what: str) -> None:
@@ -44,7 +44,7 @@ def require_gpu(t: Tensor, what: str) -> None:
 def _check_tensor(t: Tensor, what: str, dtype: torch.dtype, shape: tuple[int, ...], device) -> None:
     if t.dtype != dtype:
         raise ValueError(f"{what}: expected dtype {dtype}, got {t.dtype}")
-    if tuple(t.shape) != tuple(shape):
+    if t.shape != shape:
         raise ValueError(f"{what}: expected shape {tuple(shape)}, got {tuple(t.shape)}")
     if not t.is_contiguous():
         raise ValueError(f"{what}: tensor must be contiguous")
@@ -53,10 +53,43 @@ def _check_tensor(t: Tensor, what: str, dtype: torch.dtype, shape: tuple[int, ..
 
 
 def mask_u8(mask: Tensor) -> Tensor:
-    """Reference masks are bool or 0/1 numbers; nonzero = valid (``mask.bool()``)."""
+    """Reference masks are bool or 0/1 numbers; nonzero = valid (``mask.bool()``), and so it is for every kernel,
+    which makes a uint8 mask its own answer."""
+    if mask.dtype == torch.uint8:
+        return mask.contiguous()
     if mask.dtype == torch.bool:
         return mask.contiguous().view(torch.uint8)
     return mask.ne(0).contiguous().view(torch.uint8)
+
+
+def _plain_call(args: tuple) -> bool:
+    """True where the dispatcher has nothing to do for an op but to run its body: no gradients, no compiler, tracer,
+    functorch transform, forward-mode level or mode looking on, and plain tensors only."""
+    if torch.compiler.is_compiling() or torch.is_grad_enabled():
+        return False
+    for a in args:
+        if isinstance(a, Tensor) and (type(a) is not Tensor or not a.is_cuda):
+            return False
+    c = torch._C
+    return (c._len_torch_dispatch_stack() == 0 and c._len_torch_function_stack() == 0 and not c._is_tracing()
+            and c._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0)
+
+
+class _Op:
+    """A ``torch.library`` custom op (``torch.ops.bioemu_mi355x.<name>``, HIP only) whose body an inference program's
+    calls reach directly: the dispatcher's Python layers cost as much host time as the op's own launches."""
+
+    def __init__(self, name: str, body):
+        self.body = body
+        self.op = torch.library.custom_op(f"bioemu_mi355x::{name}", body, mutates_args=(), device_types="cuda")
+        self.register_fake = self.op.register_fake
+
+    def __call__(self, *args):
+        return self.body(*args) if _plain_call(args) else self.op(*args)
+
+
+def _op(name: str):
+    return lambda body: _Op(name, body)
 
 
 def workspace(nbytes: int, device) -> Tensor:
@@ -158,7 +191,7 @@ def launch_trimul(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::trimul", mutates_args=(), device_types="cuda")
+@_op("trimul")
 def trimul(
     x: Tensor,
     mask: Tensor,
@@ -237,7 +270,7 @@ def launch_trimul_f32(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::trimul_f32", mutates_args=(), device_types="cuda")
+@_op("trimul_f32")
 def trimul_f32(
     x: Tensor,
     mask: Tensor,
@@ -310,7 +343,7 @@ def launch_triatt(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::triangle_attention", mutates_args=(), device_types="cuda")
+@_op("triangle_attention")
 def triangle_attention(
     z: Tensor,
     mask: Tensor,
@@ -378,7 +411,7 @@ def launch_triatt_f32(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::triangle_attention_f32", mutates_args=(), device_types="cuda")
+@_op("triangle_attention_f32")
 def triangle_attention_f32(
     z: Tensor,
     mask: Tensor,
@@ -497,7 +530,7 @@ def _is_row_transition(x: Tensor, hidden: int) -> bool:
     return x.shape[-1] in (64, 128) and hidden in (2 * x.shape[-1], 4 * x.shape[-1])
 
 
-@torch.library.custom_op("bioemu_mi355x::transition", mutates_args=(), device_types="cuda")
+@_op("transition")
 def transition(
     x: Tensor, norm_w: Tensor | None, norm_b: Tensor | None, fc1_w: Tensor, fc2_w: Tensor, fc3_w: Tensor
 ) -> Tensor:
@@ -584,7 +617,7 @@ def launch_apb(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::attention_pair_bias", mutates_args=(), device_types="cuda")
+@_op("attention_pair_bias")
 def attention_pair_bias(
     s: Tensor,
     z: Tensor,
@@ -685,7 +718,7 @@ def launch_swa(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::attention_pair_bias_sliding_window", mutates_args=(), device_types="cuda")
+@_op("attention_pair_bias_sliding_window")
 def attention_pair_bias_sliding_window(
     s: Tensor,
     z: Tensor,
@@ -712,8 +745,11 @@ def attention_pair_bias_sliding_window(
     def h(t):
         return t.to(BF16).contiguous()
 
+    m = mask_u8(mask)
+    if m.data_ptr() % 16:   # the library takes a 16-byte aligned mask
+        m = m.clone()
     launch_swa(
-        sb, h(z), mask_u8(mask), f(norm_s_w), f(norm_s_b), h(w_qkv), f(q_bias), h(w_g), f(norm_z_w), f(norm_z_b),
+        sb, h(z), m, f(norm_s_w), f(norm_s_b), h(w_qkv), f(q_bias), h(w_g), f(norm_z_w), f(norm_z_b),
         h(w_z), h(w_o), out, num_heads, multiplicity,
     )
     return out.to(s.dtype)
@@ -807,7 +843,7 @@ def _f32c(t: Tensor | None) -> Tensor | None:
     return None if t is None else t.to(F32).contiguous()
 
 
-@torch.library.custom_op("bioemu_mi355x::attention_pair_bias_f32", mutates_args=(), device_types="cuda")
+@_op("attention_pair_bias_f32")
 def attention_pair_bias_f32(
     s: Tensor,
     z: Tensor,
@@ -891,9 +927,7 @@ def launch_swa_f32(
     return out
 
 
-@torch.library.custom_op(
-    "bioemu_mi355x::attention_pair_bias_sliding_window_f32", mutates_args=(), device_types="cuda"
-)
+@_op("attention_pair_bias_sliding_window_f32")
 def attention_pair_bias_sliding_window_f32(
     s: Tensor,
     z: Tensor,
@@ -966,7 +1000,7 @@ def launch_transition_f32(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::transition_f32", mutates_args=(), device_types="cuda")
+@_op("transition_f32")
 def transition_f32(
     x: Tensor, norm_w: Tensor | None, norm_b: Tensor | None, fc1_w: Tensor, fc2_w: Tensor, fc3_w: Tensor
 ) -> Tensor:
@@ -1197,7 +1231,7 @@ def launch_pwa(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::pair_weighted_averaging", mutates_args=(), device_types="cuda")
+@_op("pair_weighted_averaging")
 def pair_weighted_averaging(
     m: Tensor,
     z: Tensor,
@@ -1229,7 +1263,7 @@ def _(m, z, mask, norm_m_w, norm_m_b, w_m, w_g, norm_z_w, norm_z_b, w_z, w_o, nu
     return torch.empty_like(m)
 
 
-@torch.library.custom_op("bioemu_mi355x::outer_product_mean", mutates_args=(), device_types="cuda")
+@_op("outer_product_mean")
 def outer_product_mean(
     m: Tensor, mask: Tensor, norm_w: Tensor, norm_b: Tensor, w_ab: Tensor, w_o: Tensor, b_o: Tensor
 ) -> Tensor:
@@ -1299,7 +1333,7 @@ def launch_opm_f32(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::outer_product_mean_f32", mutates_args=(), device_types="cuda")
+@_op("outer_product_mean_f32")
 def outer_product_mean_f32(
     m: Tensor, mask: Tensor, norm_w: Tensor, norm_b: Tensor, w_ab: Tensor, w_o: Tensor, b_o: Tensor
 ) -> Tensor:
@@ -1376,7 +1410,7 @@ def launch_pwa_f32(
     return out
 
 
-@torch.library.custom_op("bioemu_mi355x::pair_weighted_averaging_f32", mutates_args=(), device_types="cuda")
+@_op("pair_weighted_averaging_f32")
 def pair_weighted_averaging_f32(
     m: Tensor,
     z: Tensor,

@@ -7,6 +7,20 @@ import torch.nn as nn
 from torch import Tensor
 
 
+def _find(module: nn.Module, path: tuple[str, ...]) -> nn.Parameter:
+    """``module.get_parameter``, through the modules' own tables (a few lookups instead of attribute protocols)."""
+    owner = module
+    for name in path[:-1]:
+        owner = owner._modules.get(name)
+        if owner is None:
+            break
+    else:
+        p = owner._parameters.get(path[-1])
+        if p is not None:
+            return p
+    return module.get_parameter(".".join(path))   # anything unusual: its answer, or its error
+
+
 class PreparedParams:
     """Caches ``(param.detach().to(dtype).contiguous(), ...)`` for a module.
 
@@ -17,11 +31,12 @@ class PreparedParams:
 
     def __init__(self, spec: list[tuple[str, torch.dtype]]):
         self.spec = spec
+        self._paths = [tuple(name.split(".")) for name, _ in spec]
         self._key: tuple | None = None
         self._val: tuple[Tensor, ...] | None = None
 
     def get(self, module: nn.Module) -> tuple[Tensor, ...]:
-        params = [module.get_parameter(name) for name, _ in self.spec]
+        params = [_find(module, path) for path in self._paths]
         key = tuple((p.data_ptr(), p._version, p.device, p.dtype) for p in params)
         if key != self._key or self._val is None:
             self._val = tuple(

@@ -109,10 +109,10 @@ class AttentionPairBias(nn.Module):
         if self.inf != 1e6:
             raise ValueError("AttentionPairBias (HIP): only inf=1e6, the reference default, is supported")
         if _ops.fp32_mode(s):
-            return torch.ops.bioemu_mi355x.attention_pair_bias_f32(
+            return _ops.attention_pair_bias_f32(
                 s, z, _ops.mask_u8(mask), *self.prepared_params_f32(), self.num_heads, multiplicity
             )
-        return torch.ops.bioemu_mi355x.attention_pair_bias(
+        return _ops.attention_pair_bias(
             s, z, _ops.mask_u8(mask), *self.prepared_params(), self.num_heads, multiplicity
         )
 
@@ -144,9 +144,9 @@ class AttentionPairBiasSlidingWindow(AttentionPairBias):
         if self.inf != 1e6:
             raise ValueError("AttentionPairBiasSlidingWindow (HIP): only inf=1e6, the reference default, is supported")
         if _ops.fp32_mode(s):
-            return torch.ops.bioemu_mi355x.attention_pair_bias_sliding_window_f32(
+            return _ops.attention_pair_bias_sliding_window_f32(
                 s, z, _ops.mask_u8(mask), *self.prepared_params_f32(), self.num_heads, multiplicity
             )
-        return torch.ops.bioemu_mi355x.attention_pair_bias_sliding_window(
+        return _ops.attention_pair_bias_sliding_window(
             s, z, _ops.mask_u8(mask), *self.prepared_params(), self.num_heads, multiplicity
         )

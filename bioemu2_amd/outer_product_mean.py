@@ -71,8 +71,8 @@ class OuterProductMeanHip(nn.Module):
     def forward(self, m: Tensor, mask: Tensor) -> Tensor:
         _ops.require_gpu(m, type(self).__name__)
         if _ops.fp32_mode(m):
-            return torch.ops.bioemu_mi355x.outer_product_mean_f32(m, mask, *self.prepared_params_f32())
-        return torch.ops.bioemu_mi355x.outer_product_mean(m, mask, *self.prepared_params())
+            return _ops.outer_product_mean_f32(m, mask, *self.prepared_params_f32())
+        return _ops.outer_product_mean(m, mask, *self.prepared_params())
 
 
 REGISTRY: dict[OPMVariant, tuple[str, str]] = {

@@ -73,8 +73,8 @@ class PairWeightedAveraging(nn.Module):
     def forward(self, m: Tensor, z: Tensor, mask: Tensor, chunk_heads: bool = False) -> Tensor:
         _ops.require_gpu(m, type(self).__name__)
         if _ops.fp32_mode(m):
-            return torch.ops.bioemu_mi355x.pair_weighted_averaging_f32(
+            return _ops.pair_weighted_averaging_f32(
                 m, z, mask, *self.prepared_params_f32(), self.num_heads, float(self.inf))
         if self.inf != 1e6:
             raise ValueError(f"PairWeightedAveraging: only inf=1e6 is supported (got {self.inf})")
-        return torch.ops.bioemu_mi355x.pair_weighted_averaging(m, z, mask, *self.prepared_params(), self.num_heads)
+        return _ops.pair_weighted_averaging(m, z, mask, *self.prepared_params(), self.num_heads)

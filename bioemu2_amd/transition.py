@@ -63,5 +63,5 @@ class Transition(nn.Module):
     def forward(self, x: Tensor) -> Tensor:
         _ops.require_gpu(x, type(self).__name__)
         if _ops.fp32_mode(x):
-            return torch.ops.bioemu_mi355x.transition_f32(x, *self.prepared_params_f32())
-        return torch.ops.bioemu_mi355x.transition(x, *self.prepared_params())
+            return _ops.transition_f32(x, *self.prepared_params_f32())
+        return _ops.transition(x, *self.prepared_params())

@@ -101,10 +101,10 @@ class TriangleAttentionHip(nn.Module):
         if self.inf != 1e6:
             raise ValueError("TriangleAttentionHip: only inf=1e6 (the reference masking value) is supported")
         if _ops.fp32_mode(z):
-            return torch.ops.bioemu_mi355x.triangle_attention_f32(
+            return _ops.triangle_attention_f32(
                 z, _ops.mask_u8(mask), *self.prepared_params_f32(), self.starting, self.num_heads
             )
-        return torch.ops.bioemu_mi355x.triangle_attention(
+        return _ops.triangle_attention(
             z, _ops.mask_u8(mask), *self.prepared_params(), self.starting, self.num_heads
         )
 

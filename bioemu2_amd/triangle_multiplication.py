@@ -110,10 +110,10 @@ class TriangleMultiplicationHip(_TriMulBase):
     def forward(self, x: Tensor, mask: Tensor) -> Tensor:
         _ops.require_gpu(x, type(self).__name__)
         if _ops.fp32_mode(x):
-            return torch.ops.bioemu_mi355x.trimul_f32(
+            return _ops.trimul_f32(
                 x, _ops.mask_u8(mask), *self.prepared_params_f32(), self.mode == "outgoing"
             )
-        return torch.ops.bioemu_mi355x.trimul(
+        return _ops.trimul(
             x, _ops.mask_u8(mask), *self.prepared_params(), self.mode == "outgoing"
         )
 

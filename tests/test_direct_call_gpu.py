@@ -1,0 +1,103 @@
+"""Which calls reach an op's body directly and which go through the dispatcher, and that both give the same result."""
+
+import pytest
+import torch
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from bioemu2_amd import _ops
+from bioemu2_amd.attention_pair_bias import AttentionPairBiasSlidingWindow
+from bioemu2_amd.transition import Transition
+from bioemu2_amd.triangle_multiplication import TriangleMultiplicationHip
+from tests._helpers import randomize_params
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def counted(monkeypatch):
+    """Counts dispatcher calls of the trimul op."""
+    calls = []
+    op = _ops.trimul.op
+    monkeypatch.setattr(_ops.trimul, "op", lambda *a: (calls.append(1), op(*a))[1])
+    return calls
+
+
+def _case(device):
+    torch.manual_seed(0)
+    m = randomize_params(TriangleMultiplicationHip(128), 1).to(device).eval()
+    x = torch.randn(1, 20, 20, 128, device=device).to(torch.bfloat16)
+    return m, x, torch.rand(1, 20, 20, device=device) < 0.8
+
+
+def test_inference_calls_skip_the_dispatcher(gpu_device, counted):
+    m, x, mask = _case(gpu_device)
+    with torch.no_grad():
+        direct = m(x, mask)
+    with torch.inference_mode():
+        m(x, mask)
+    assert not counted
+    assert torch.equal(direct, m(x, mask).detach())   # gradients enabled: through the op
+    assert len(counted) == 1
+
+
+class _Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def test_onlookers_see_the_op(gpu_device, counted):
+    m, x, mask = _case(gpu_device)
+    with torch.no_grad():
+        want = m(x, mask)
+        with _Seen() as mode:
+            got = m(x, mask)
+        assert any("bioemu_mi355x.trimul" in n for n in mode.names) and torch.equal(got, want)
+
+        class Sub(torch.Tensor):
+            pass
+
+        m(x.as_subclass(Sub), mask)
+        with torch.autograd.forward_ad.dual_level():
+            m(x, mask)
+    assert len(counted) == 3
+
+
+def test_uint8_masks_mean_nonzero(gpu_device):
+    m, x, mask = _case(gpu_device)
+    with torch.no_grad():
+        want = m(x, mask)
+        assert torch.equal(m(x, mask.to(torch.uint8) * 255), want)
+        assert torch.equal(m(x, mask.to(torch.uint8).transpose(1, 2).contiguous().transpose(1, 2)), want)
+        assert torch.equal(m(x, mask.float()), want)
+
+
+def test_sliding_window_mask_of_any_alignment(gpu_device):
+    torch.manual_seed(1)
+    m = randomize_params(AttentionPairBiasSlidingWindow(128, 16, 4, initial_norm=False), 2).to(gpu_device).eval()
+    nw = 3
+    s = torch.randn(nw, 32, 128, device=gpu_device)
+    z = torch.randn(1, nw, 32, 128, 16, device=gpu_device)
+    mask = torch.rand(nw, 32, device=gpu_device) < 0.9
+    shifted = torch.zeros(nw * 32 + 3, dtype=torch.bool, device=gpu_device)[3:].view(nw, 32).copy_(mask)
+    with torch.no_grad():
+        for dt in (torch.bfloat16, torch.float32):
+            assert torch.equal(m(s.to(dt), z.to(dt), mask), m(s.to(dt), z.to(dt), shifted))
+
+
+def test_replaced_parameters_are_seen(gpu_device):
+    m = randomize_params(Transition(128, 256), 3).to(gpu_device).eval()
+    x = torch.randn(1, 40, 128, device=gpu_device)
+    with torch.no_grad():
+        before = m(x)
+        m.fc3.weight = torch.nn.Parameter(2.0 * m.fc3.weight)
+        assert torch.equal(m(x), 2.0 * before)
+        m.norm = torch.nn.LayerNorm(128).to(gpu_device)
+        assert not torch.equal(m(x), 2.0 * before)
+        del m.fc3.weight
+        with pytest.raises(AttributeError):
+            m(x)
