@@ -42,51 +42,54 @@ constexpr int COUT = 128;
 constexpr int CH2 = CH * CH;  // 1024
 
 // ---------------------------------------------------------------------------
-// Row compaction.  One workgroup per batch.
+// Row compaction, in two launches: every row's flag (any valid entry) by a wave of its own, then the flags of a batch
+// compacted by one workgroup (in place: idx first holds the flags).  One workgroup that both scanned its batch's rows
+// and added the counts up on one thread took 24 us at S = 1024, N = 512 (4 rows in flight per thread, 256 dependent
+// LDS reads); this takes 5, and the flags' launch also carries the weight copy below.
 // ---------------------------------------------------------------------------
 constexpr int kRowsThreads = 256;
 
-__global__ __launch_bounds__(kRowsThreads) void opm_rows_kernel(const uint8_t* __restrict__ mask, int* __restrict__ idx,
-                                                                int* __restrict__ count, int S, int N) {
-  __shared__ int part[kRowsThreads];
-  const int b = blockIdx.x;
-  const int per = (S + kRowsThreads - 1) / kRowsThreads;
-  const int s0 = min(S, (int)threadIdx.x * per), s1 = min(S, s0 + per);
-  const uint8_t* mb = mask + (size_t)b * S * N;
+// Flags of row r = b S + s of the mask, one wave per row.
+__device__ __forceinline__ void opm_row_flag(const uint8_t* __restrict__ mask, int* __restrict__ flags, long long r,
+                                             int N) {
+  const int lane = threadIdx.x & 63;
+  const uint8_t* row = mask + (size_t)r * N;
   const bool vec = (N % 16 == 0) && ((reinterpret_cast<uintptr_t>(mask) & 15) == 0);
-  uint64_t bits = 0;  // per <= 64 rows per thread (S <= 16384)
-  int cnt = 0;
-  for (int s = s0; s < s1; ++s) {
-    const uint8_t* row = mb + (size_t)s * N;
-    bool any = false;
-    if (vec) {
-      for (int t = 0; t < N && !any; t += 16) {
-        const uint4 v = *reinterpret_cast<const uint4*>(row + t);
-        any = (v.x | v.y | v.z | v.w) != 0;
-      }
-    } else {
-      for (int t = 0; t < N && !any; ++t) any = row[t] != 0;
+  uint32_t any = 0;
+  if (vec) {
+    for (int t = lane * 16; t < N; t += 1024) {
+      const uint4 v = *reinterpret_cast<const uint4*>(row + t);
+      any |= v.x | v.y | v.z | v.w;
     }
-    if (any) {
-      bits |= 1ull << (s - s0);
-      ++cnt;
-    }
+  } else {
+    for (int t = lane; t < N; t += 64) any |= row[t];
   }
-  part[threadIdx.x] = cnt;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int t = 0; t < kRowsThreads; ++t) {
-      const int c = part[t];
-      part[t] = run;
-      run += c;
-    }
-    count[b] = run;
+  const bool some = __any(any != 0);
+  if (lane == 0) flags[r] = some;
+}
+
+__global__ __launch_bounds__(kRowsThreads) void opm_rows_kernel(int* idx, int* __restrict__ count, int S) {
+  __shared__ int wave_sum[kRowsThreads / 64];
+  const int b = blockIdx.x, lane = threadIdx.x & 63, wave = wave_id();
+  const int per = (S + kRowsThreads - 1) / kRowsThreads;   // <= 64 (S <= 16384)
+  const int s0 = min(S, (int)threadIdx.x * per), s1 = min(S, s0 + per);
+  int* ib = idx + (size_t)b * S;
+  uint64_t bits = 0;
+  for (int s = s0; s < s1; ++s) bits |= (uint64_t)(ib[s] != 0) << (s - s0);
+  const int cnt = __popcll(bits);
+  int incl = cnt;   // inclusive scan over the wave
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(incl, off);
+    if (lane >= off) incl += v;
   }
-  __syncthreads();
-  int out = part[threadIdx.x];
+  if (lane == 63) wave_sum[wave] = incl;
+  __syncthreads();   // ... and every flag is read before an index overwrites it
+  int out = incl - cnt;
+  for (int w = 0; w < wave; ++w) out += wave_sum[w];
+  if (threadIdx.x == kRowsThreads - 1) count[b] = out + cnt;
   for (int s = s0; s < s1; ++s)
-    if (bits >> (s - s0) & 1ull) idx[(size_t)b * S + out++] = s;
+    if (bits >> (s - s0) & 1ull) ib[out++] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -172,7 +175,17 @@ __global__ __launch_bounds__(kProjThreads) void opm_proj_kernel(
 // ---------------------------------------------------------------------------
 constexpr int kWoFrags = (COUT / 32) * (CH2 / 16) * 64;   // 16-byte slots
 
-__global__ __launch_bounds__(256) void opm_wo_tiles_kernel(const bf16* __restrict__ w_o, bf16* __restrict__ wt) {
+constexpr int kWoBlocks = (kWoFrags + 255) / 256;
+
+// The weight copy (workgroups [0, kWoBlocks)) and the rows' flags (the rest, four rows each): independent of each other.
+__global__ __launch_bounds__(256) void opm_wo_tiles_kernel(const bf16* __restrict__ w_o, bf16* __restrict__ wt,
+                                                           const uint8_t* __restrict__ mask, int* __restrict__ flags,
+                                                           int N, long long rows) {
+  if (blockIdx.x >= kWoBlocks) {
+    const long long r = (long long)(blockIdx.x - kWoBlocks) * 4 + wave_id();
+    if (r < rows) opm_row_flag(mask, flags, r, N);
+    return;
+  }
   const int f = blockIdx.x * 256 + threadIdx.x;
   if (f >= kWoFrags) return;
   const int lane = f & 63, ks = (f >> 6) % (CH2 / 16), eb = f / (64 * (CH2 / 16));
@@ -341,11 +354,18 @@ extern "C" int bioemu_opm_fwd(const void* m, const uint8_t* mask, int mean_rows,
   if (B * Nt * (Sp / 32) >= kMaxTiles) return set_error(BIOEMU_ERR_INVALID_ARG, "opm: too many row tiles");
 
   {
-    KernelTimerScope timed("opm_rows", stream);
-    hipLaunchKernelGGL(opm_rows_kernel, dim3((unsigned)B), dim3(kRowsThreads), 0, stream, mask, L.idx, L.count,
-                       (int)S, (int)N);
+    const long long rows = B * S;
+    KernelTimerScope timed("opm_wo_tiles", stream);
+    hipLaunchKernelGGL(opm_wo_tiles_kernel, dim3((unsigned)(kWoBlocks + (rows + 3) / 4)), dim3(256), 0, stream,
+                       static_cast<const bf16*>(w_o), L.wt, mask, L.idx, (int)N, rows);
   }
-  int rc = check_launch("opm_rows");
+  int rc = check_launch("opm_wo_tiles");
+  if (rc) return rc;
+  {
+    KernelTimerScope timed("opm_rows", stream);
+    hipLaunchKernelGGL(opm_rows_kernel, dim3((unsigned)B), dim3(kRowsThreads), 0, stream, L.idx, L.count, (int)S);
+  }
+  rc = check_launch("opm_rows");
   if (rc) return rc;
 
   int dev = 0, cus = 0;
@@ -362,13 +382,6 @@ extern "C" int bioemu_opm_fwd(const void* m, const uint8_t* mask, int mean_rows,
   rc = check_launch("opm_proj");
   if (rc) return rc;
 
-  {
-    KernelTimerScope timed("opm_wo_tiles", stream);
-    hipLaunchKernelGGL(opm_wo_tiles_kernel, dim3((kWoFrags + 255) / 256), dim3(256), 0, stream,
-                       static_cast<const bf16*>(w_o), L.wt);
-  }
-  rc = check_launch("opm_wo_tiles");
-  if (rc) return rc;
   if (hipFuncSetAttribute(reinterpret_cast<const void*>(opm_fused_kernel),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kFusedSmem) != hipSuccess)
     return set_error(BIOEMU_ERR_LAUNCH, "opm_fused: cannot set dynamic LDS size");
