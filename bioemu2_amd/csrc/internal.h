@@ -59,8 +59,9 @@ inline int pick_waves_per_wg(int64_t tiles, int cus, const int* waves, const dou
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Batched bf16 "NT" GEMM: C[z][i][j] = sum_k A[z][i][k] * B[z][j][k] for
-// z < batch, with M = N = K = n (a multiple of kGemmTile) and bf16 output.
+// z < batch over planes of n rows with stride bgemm_ld(n) (zero-filled past n), bf16 output.
 constexpr int kGemmTile = 256;
+inline int64_t bgemm_ld(int64_t n) { return round_up(n, 64); }
 int launch_bgemm_nt(const void* A, const void* B, void* C, int64_t batch, int64_t n,
                     hipStream_t stream);
 

@@ -19,9 +19,12 @@
 //   pwa_fused    : per head the averaging GEMM on MFMA, then the gate and
 //                  the output projection from the accumulator registers;
 //                  writes (g * o) Wo^T (+ m) once, after the last head.
-// Padding: tokens are padded to Np = N rounded up to 256 (GEMM tiles), MSA rows
+// Padding: keys are padded to Np = N rounded up to 64 (the GEMM's k-tile), MSA rows
 // to S8 = S rounded up to 8; padded keys have weight exactly 0 and padded v
-// rows are exactly 0, so padding never changes a valid output bit.
+// rows are exactly 0, so padding never changes a valid output bit.  Query tiles read
+// rows past N as zeros through the buffer bounds.  (Tokens padded to whole 256-tiles,
+// S = 511, N = 333: weights 25 -> 17 us, projections 63 -> 48, contraction 126 -> 80
+// without the padding.)
 #include <algorithm>
 
 #include "common.h"
@@ -40,7 +43,7 @@ constexpr int HC = NH * CH;   // 256
 constexpr int kLdw64 = CM + 8;
 
 // ---------------------------------------------------------------------------
-// Weights: grid = B * Np rows, 256 threads.  LDS: folded Wz rows (8, padded to
+// Weights: grid = B * N rows, 256 threads.  LDS: folded Wz rows (8, padded to
 // a 32-row MFMA block), their bias pairs, then the logits [8][Np] (fp32).
 // ---------------------------------------------------------------------------
 constexpr int kWThreads = 256;
@@ -55,13 +58,8 @@ __global__ __launch_bounds__(kWThreads) void pwa_weights_kernel(const bf16* __re
   bf16* wl = reinterpret_cast<bf16*>(smem);
   bf16* cl = wl + 32 * kLdw;
   float* lg = reinterpret_cast<float*>(smem + kWFixedSmem);
-  const int b = blockIdx.x / Np, i = blockIdx.x % Np;
-  const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
-  if (i >= N) {   // padded query rows: zero weights (their outputs are dropped)
-    for (int q = tid; q < NH * Np; q += kWThreads)
-      w[((size_t)(b * NH + q / Np) * Np + i) * Np + q % Np] = f2bf(0.f);
-    return;
-  }
+  const int b = blockIdx.x / N, i = blockIdx.x % N;
+  const int lane = threadIdx.x & 63, wave = wave_id();
   stage_weights(wl, wzf, NH, 32);
   stage_bias(cl, czf, NH, 32);
   __syncthreads();
@@ -101,7 +99,7 @@ __global__ __launch_bounds__(kWThreads) void pwa_weights_kernel(const bf16* __re
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off);
     const float inv = 1.0f / sum;
-    bf16* wo = w + ((size_t)(b * NH + hd) * Np + i) * Np;
+    bf16* wo = w + ((size_t)(b * NH + hd) * N + i) * Np;
     for (int j = lane; j < Np; j += 64) wo[j] = f2bf(fast_exp2((r[j] - mx) * kLog2e) * inv);
   }
 }
@@ -272,7 +270,7 @@ __global__ __launch_bounds__(kFuThreads) void pwa_fused_kernel(const bf16* __res
   const int per_xcd = gridDim.x / kNtXcds;
   const int item = (blockIdx.x % kNtXcds) * per_xcd + blockIdx.x / kNtXcds;
   if (item >= nitems) return;   // before any barrier: the whole workgroup leaves
-  const int nit = Np / kFuI, nst = S8 / kFuS;
+  const int nit = (N + kFuI - 1) / kFuI, nst = S8 / kFuS;
   const int it = item % nit, st = (item / nit) % nst, b = item / (nit * nst);
   const int i0 = it * kFuI, s0 = st * kFuS;
 
@@ -296,7 +294,7 @@ __global__ __launch_bounds__(kFuThreads) void pwa_fused_kernel(const bf16* __res
     voff[q] = (unsigned)(r * Np + c * 8) * 2;
   }
   auto rsrcs = [&](int h, __amdgpu_buffer_rsrc_t& rw, __amdgpu_buffer_rsrc_t& rv) {
-    rw = buffer_rsrc(w + ((size_t)(b * NH + h) * Np + i0) * Np, (unsigned)kFuI * Np * 2);
+    rw = buffer_rsrc(w + ((size_t)(b * NH + h) * N + i0) * Np, (unsigned)min(N - i0, kFuI) * Np * 2);
     rv = buffer_rsrc(vt + (((size_t)(b * NH + h) * S8 + s0) * CH) * Np, (unsigned)(kFuS * CH) * Np * 2);
   };
   auto stage = [&](__amdgpu_buffer_rsrc_t rw, __amdgpu_buffer_rsrc_t rv, int kt, int buf) {
@@ -309,6 +307,7 @@ __global__ __launch_bounds__(kFuThreads) void pwa_fused_kernel(const bf16* __res
   };
 
   const int nk = Np / kFuBK;
+  const bool live = i0 + wi * 64 < N;   // a wave whose 64 queries are all padding copies its share and no more
   int jrow[2], offi[2];
 #pragma unroll
   for (int si = 0; si < 2; ++si) jrow[si] = (2 * ws + si) * 32 + perm32(ln);
@@ -344,6 +343,7 @@ __global__ __launch_bounds__(kFuThreads) void pwa_fused_kernel(const bf16* __res
         rsrcs(h + 1, rw, rv);
         stage(rw, rv, 0, (gk + 1) & 1);
       }
+      if (!live) continue;
       const bf16* sa = smem + (gk & 1) * kFuStage;
       const bf16* sb = sa + kFuWTile;
       // fragments of k-step ks + 1 are read while k-step ks is multiplied
@@ -369,13 +369,14 @@ __global__ __launch_bounds__(kFuThreads) void pwa_fused_kernel(const bf16* __res
           for (int ib = 0; ib < 2; ++ib) acc[si][ib] = mfma32(fj[c][si], fi[c][ib], acc[si][ib]);
       }
     }
+    if (!live) continue;
     // acc[si][ib] lane (ln, lh) register u <-> O_h[i = i0 + wi*64 + ib*32 + ln][(s0 + 2 ws + si, d = 16 lh + u)]
 #pragma unroll
     for (int si = 0; si < 2; ++si) {
       const int s = s0 + 2 * ws + si;
 #pragma unroll
       for (int ib = 0; ib < 2; ++ib) {
-        const int i = i0 + offi[ib];
+        const int i = min(i0 + offi[ib], N - 1);   // rows past N are not stored
         const bf16* gp = g + (((size_t)b * S8 + s) * Np + i) * HC + h * CH + 16 * lh;
         const bf16x8 g0 = load8(gp), g1 = load8(gp + 8);
         bf16x8 go0, go1;
@@ -437,11 +438,11 @@ struct PwaLayout {
 
 PwaLayout pwa_layout(int64_t B, int64_t S, int64_t N) {
   PwaLayout L;
-  L.Np = round_up(N, kNtTile);
+  L.Np = round_up(N, kFuBK);
   L.S8 = round_up(S, 8);
   size_t p = 0;
   L.w = p;
-  p += round_up((size_t)B * NH * L.Np * L.Np * 2, 256);
+  p += round_up((size_t)B * NH * N * L.Np * 2, 256);
   L.vt = p;
   p += round_up((size_t)B * NH * L.S8 * CH * L.Np * 2, 256);
   L.g = p;
@@ -520,7 +521,7 @@ extern "C" int bioemu_pwa_fwd(const void* m, const void* z, const uint8_t* mask,
     return set_error(BIOEMU_ERR_LAUNCH, "pwa: cannot set dynamic LDS size");
   {
     KernelTimerScope timed("pwa_weights", stream);
-    hipLaunchKernelGGL(pwa_weights_kernel, dim3((unsigned)(B * Np)), dim3(kWThreads), wsmem, stream,
+    hipLaunchKernelGGL(pwa_weights_kernel, dim3((unsigned)(B * N)), dim3(kWThreads), wsmem, stream,
                        static_cast<const bf16*>(z), mask, wzf, czf, wbuf, (int)N, Np);
   }
   rc = check_launch("pwa_weights");
@@ -535,7 +536,7 @@ extern "C" int bioemu_pwa_fwd(const void* m, const void* z, const uint8_t* mask,
   rc = check_launch("pwa_proj");
   if (rc) return rc;
   {
-    const long long items = B * (S8 / kFuS) * (Np / kFuI);
+    const long long items = B * (S8 / kFuS) * ((N + kFuI - 1) / kFuI);
     const long long grid = (items + kNtXcds - 1) / kNtXcds * kNtXcds;
     if (grid > 0x7fffffffLL) return set_error(BIOEMU_ERR_INVALID_ARG, "pwa: too many work items");
     KernelTimerScope timed("pwa_fused", stream);

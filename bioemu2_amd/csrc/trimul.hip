@@ -9,9 +9,9 @@
 //                       (the incoming direction writes the transposed frame).
 //   2. bgemm_nt       : o[d][i][j] = sum_k a[d][i][k] * b[d][j][k]   (MFMA, fp32 acc)
 //   3. trimul_out     : LN_out(o) -> p_out, LN_in(x) -> g_out, out = p*sigmoid(g) (+x)
-// Padded planes (Np = N rounded up to the 256 contraction tile) are zero in every padded row and
-// column, so the contraction needs no edge handling and padding never changes
-// a valid output bit.
+// Planes are N rows of Np = N rounded up to 64 (the contraction's k-tile), zero in the padded columns, so
+// padding never changes a valid output bit.  (Planes of whole 256-tiles, N = 773: projection 238 -> 142 us,
+// contraction 289 -> 212 us, output 143 -> 124 us without the padding; N = 333: 51 -> 33, 39 -> 24 us.)
 #include <algorithm>
 
 #include "common.h"
@@ -31,9 +31,10 @@ constexpr int D = 128;               // pair channels (c_z)
 // as MFMA operands (pairtile.h); p_in and g_in (512 x 128) sit in LDS for the
 // whole persistent workgroup.  A masked pair's LayerNorm row is zeroed before
 // the bias-free projections, so its p is exactly 0 and so is p * sigmoid(g):
-// the masked_fill of the reference (triangle_multiplication.py:93).  Rows and
-// columns in [N, Np) come out zero, which the padded contraction relies on.
-// Output: a and b as channel-major planes [B][D][Np][Np] (k contiguous).
+// the masked_fill of the reference (triangle_multiplication.py:93).  Columns
+// in [N, Np) come out zero, which the contraction's whole k-tiles rely on.
+// Output: a and b as channel-major planes [B][D][N][Np] (k contiguous), Np = N
+// rounded up to 64.
 // ---------------------------------------------------------------------------
 // Workgroup size: kWaves = 8 or 12 waves, chosen per launch (in_waves_per_wg);
 // the staged weights (140 KB of LDS) allow one workgroup per CU, so kWaves
@@ -74,8 +75,8 @@ __global__ __launch_bounds__(64 * kWaves) void trimul_proj_in_kernel(
   const int rho = lane & 31, h = lane >> 5;
   constexpr int waves = kWaves;
   const unsigned tiles_per_row = Np / 32;
-  const unsigned ntiles = (unsigned)B * Np * tiles_per_row;
-  const size_t plane = (size_t)Np * Np;
+  const unsigned ntiles = (unsigned)B * N * tiles_per_row;
+  const size_t plane = (size_t)N * Np;
 
   // Software pipeline over this wave's tiles: tile t + stride's inputs (this
   // lane's half of its pair's x row and the pair's mask byte) are loaded
@@ -90,9 +91,9 @@ __global__ __launch_bounds__(64 * kWaves) void trimul_proj_in_kernel(
   uint8_t mraw = 0;
   bool inb_next = false;
   auto fetch = [&](unsigned tt) {
-    const TileIdx ti = split_tile(tt, tiles_per_row, Np);
+    const TileIdx ti = split_tile(tt, tiles_per_row, N);
     const int i = ti.row, b = ti.b, kk = ti.col * 32 + perm32(rho);
-    inb_next = i < N && kk < N;
+    inb_next = kk < N;
     const size_t pair = !inb_next ? 0 : kOutgoing ? ((size_t)b * N + i) * N + kk : ((size_t)b * N + kk) * N + i;
     mraw = mask[pair];
     const bf16* row = x + pair * D + 8 * h;
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(64 * kWaves) void trimul_proj_in_kernel(
   for (; t < ntiles; t += stride) {
     const unsigned tn = t + stride;
     if (tn < ntiles) fetch(tn);
-    const TileIdx ti = split_tile(t, tiles_per_row, Np);
+    const TileIdx ti = split_tile(t, tiles_per_row, N);
     const int kt = ti.col, i = ti.row, b = ti.b;
     const int k0 = kt * 32;
 #pragma unroll 1
@@ -280,7 +281,7 @@ __global__ __launch_bounds__(kOutThreads) void trimul_out_kernel(
   const unsigned tiles_per_row = (N + 31) / 32;
   const unsigned ntiles = (unsigned)B * N * tiles_per_row;
   const unsigned stride = gridDim.x * kOutWaves;
-  const size_t plane = (size_t)Np * Np;
+  const size_t plane = (size_t)N * Np;
   bf16* ob = obuf + wave * kOutTile;
 
   // Next tile's raw inputs.  o channel 32 (q & 3) + 8 (q >> 2) + 16 (s >> 3) +
@@ -296,7 +297,7 @@ __global__ __launch_bounds__(kOutThreads) void trimul_out_kernel(
   // Copy instruction q reads channels c_q + 16 (slot >> 3) + (slot & 7),
   // c_q = 32 (q & 3) + 8 (q >> 2), through a buffer resource based at its own
   // first plane: 24 planes from that base, so 32-bit offsets hold for
-  // 23 Np^2 + 32 elements (N <= 9472), the whole 128-plane span need not.
+  // 23 N Np + 32 elements (N <= 9472), the whole 128-plane span need not.
   const unsigned o_extent = (unsigned)((kOutPlaneSpan * plane + 32) * 2);
   auto fetch = [&](unsigned tt) {
     const TileIdx ti = split_tile(tt, tiles_per_row, N);
@@ -446,9 +447,9 @@ static int launch_proj_in(bool outgoing, int waves, unsigned grid, const bf16* x
 
 extern "C" size_t bioemu_trimul_workspace_bytes(int64_t B, int64_t N, int64_t Dc) {
   if (B <= 0 || N <= 0 || Dc <= 0) return 0;
-  const int64_t Np = round_up(N, kGemmTile);
+  const int64_t Np = bgemm_ld(N);
   // a, b, o planes + the folded output weights and biases
-  return (size_t)(3 * B * Dc * Np * Np) * sizeof(bf16) + (size_t)(2 * Dc * Dc) * sizeof(bf16) +
+  return (size_t)(3 * B * Dc * N * Np) * sizeof(bf16) + (size_t)(2 * Dc * Dc) * sizeof(bf16) +
          (size_t)(2 * Dc) * sizeof(float);
 }
 
@@ -480,8 +481,8 @@ extern "C" int bioemu_trimul_fwd(const void* x, const uint8_t* mask, const float
   if (workspace_bytes < need)
     return set_error(BIOEMU_ERR_WORKSPACE, "trimul: workspace %zu < required %zu", workspace_bytes, need);
 
-  const int64_t Np = round_up(N, kGemmTile);
-  const size_t plane_elems = (size_t)(B * D * Np * Np);
+  const int64_t Np = bgemm_ld(N);
+  const size_t plane_elems = (size_t)(B * D * N * Np);
   bf16* ab = static_cast<bf16*>(workspace);
   bf16* ob = ab + 2 * plane_elems;
   bf16* wfold = ob + plane_elems;                                  // [2][D][D]
@@ -494,7 +495,7 @@ extern "C" int bioemu_trimul_fwd(const void* x, const uint8_t* mask, const float
                               : reinterpret_cast<const void*>(trimul_out_kernel<false>);
   if (hipFuncSetAttribute(kout, hipFuncAttributeMaxDynamicSharedMemorySize, kOutSmem) != hipSuccess)
     return set_error(BIOEMU_ERR_LAUNCH, "trimul: cannot set dynamic LDS size");
-  const long long waves_in = (long long)B * Np * (Np / 32);
+  const long long waves_in = (long long)B * N * (Np / 32);
   if (waves_in >= kMaxTiles) return set_error(BIOEMU_ERR_INVALID_ARG, "trimul: too many pair tiles");
   const int in_waves = in_waves_per_wg(waves_in, cus);
   const unsigned grid1 = (unsigned)std::min<long long>(cus, (waves_in + in_waves - 1) / in_waves);
@@ -503,7 +504,7 @@ extern "C" int bioemu_trimul_fwd(const void* x, const uint8_t* mask, const float
   if (rc) return rc;
   rc = check_launch("trimul_proj_in");
   if (rc) return rc;
-  rc = launch_bgemm_nt(ab, ab + plane_elems, ob, B * D, Np, stream);
+  rc = launch_bgemm_nt(ab, ab + plane_elems, ob, B * D, N, stream);
   if (rc) return rc;
   {
     KernelTimerScope timed("trimul_fold", stream);

@@ -418,9 +418,9 @@ class OpmWorkload(Workload):
         if kernel == "opm_proj":
             return ("hbm", float(self.s_valid * n * 64 * 2 + 2 * S * n * 32 * 2))
         if kernel == "opm_rows":
-            return ("hbm", float(S * n))
-        if kernel == "opm_wo_tiles":  # proj_o weight [128][1024] read and written in fragment order
-            return ("hbm", float(2 * 128 * 1024 * 2))
+            return ("hbm", float(2 * S * 4))
+        if kernel == "opm_wo_tiles":  # proj_o weight [128][1024] read and written in fragment order; the mask read
+            return ("hbm", float(2 * 128 * 1024 * 2 + S * n))
         raise KeyError(kernel)
 
 
@@ -469,7 +469,7 @@ class PwaWorkload(Workload):
 
     def kernel_work(self, kernel: str) -> tuple[str, float]:
         n, S = self.n, self.S
-        npad = -(-n // 256) * 256
+        npad = -(-n // 64) * 64
         if kernel == "pwa_fused":
             # sum_j w[h,i,j] v[s,j,h,:] over the valid keys (every head and MSA row) and the
             # output projection (g * o) Wo^T
@@ -624,9 +624,9 @@ class PairMixerMsaWorkload(Workload):
         if kernel == "opm_proj":
             return ("hbm", float(self.s_valid * n * 64 * 2 + 2 * S * n * 32 * 2))
         if kernel == "opm_rows":
-            return ("hbm", float(S * n))
+            return ("hbm", float(2 * S * 4))
         if kernel == "opm_wo_tiles":
-            return ("hbm", float(2 * 128 * 1024 * 2))
+            return ("hbm", float(2 * 128 * 1024 * 2 + S * n))
         if kernel in ("pwa_weights", "pwa_proj", "pwa_fused"):
             return PwaWorkload.kernel_work(self, kernel)
         if kernel == "transition_msa":
