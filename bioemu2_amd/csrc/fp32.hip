@@ -577,7 +577,8 @@ int attn_f32_projections(const float* s, const float* norm_s_w, const float* nor
     mats.m[0] = with_fold(mats.m[0], norm_s_w, norm_s_b, buf.wbias);
     mats.m[1] = with_fold(mats.m[1], norm_s_w, norm_s_b, buf.wbias + 3 * c_s);
   }
-  int rc = split_weights(mats, bias_split ? 4 : 3, stream);
+  const SplitRows rs{s, norm_s_w, norm_s_b, buf.sp.a, buf.sp.ainv, nullptr, rows, c_s, 0};
+  int rc = r128 ? split_weights(mats, bias_split ? 4 : 3, stream) : split_prep(mats, bias_split ? 4 : 3, rs, stream);
   if (rc) return rc;
   if (bias_split)
     rc = split_pair_bias(pb.z, buf.wz, buf.wzinv, buf.wzbias, buf.bias, pb.P, pb.nrows, pb.ncols, pb.ld, pb.H,
@@ -597,9 +598,6 @@ int attn_f32_projections(const float* s, const float* norm_s_w, const float* nor
   if (r128)
     return split_gemm_r128(kSplitQkvg, s, buf.sp.w, buf.sp.winv, norm_s_w ? buf.wbias : nullptr, e, rows, 4 * c_s,
                            stream, "f32_proj_qkvg");
-  rc = split_rows(s, c_s, nullptr, 0, norm_s_w, norm_s_b, buf.sp.a, buf.sp.ainv, nullptr, rows, stream,
-                  "f32_split_rows");
-  if (rc) return rc;
   return split_gemm(kSplitQkvg, buf.sp.a, buf.sp.ainv, buf.sp.w, buf.sp.winv, e, rows, c_s, 4 * c_s, stream,
                     "f32_proj_qkvg");
 }
@@ -616,8 +614,8 @@ int attn_f32_out(const float* go, const float* res, float* out, AttnF32Buffers& 
   e.ldo = c_s;
   if (c_s == 128)
     return split_gemm_r128(kSplitStore, go, w, winv, nullptr, e, rows, c_s, stream, name);
-  const int rc = split_rows(go, c_s, nullptr, 0, nullptr, nullptr, buf.sp.a, buf.sp.ainv, nullptr, rows, stream,
-                            "f32_split_rows");
+  const SplitRows rs{go, nullptr, nullptr, buf.sp.a, buf.sp.ainv, nullptr, rows, c_s, 0};
+  const int rc = split_prep(SplitMats{}, 0, rs, stream);
   if (rc) return rc;
   return split_gemm(kSplitStore, buf.sp.a, buf.sp.ainv, w, winv, e, rows, c_s, c_s, stream, name);
 }
@@ -768,10 +766,8 @@ static int transition_f32_res(const float* x, const float* res, const float* nor
   mats.m[0] = split_gemm_weight(fc1_w, buf.w12, buf.w12inv, buf.w12norm, hidden, Dc, 2, 0);
   mats.m[1] = split_gemm_weight(fc2_w, buf.w12, buf.w12inv, buf.w12norm, hidden, Dc, 2, 1);
   mats.m[2] = split_gemm_weight(fc3_w, buf.w3, buf.w3inv, nullptr, out0, hidden);
-  int rc = split_weights(mats, 3, stream);
-  if (rc) return rc;
-  rc = split_rows(x, (int)Dc, nullptr, 0, use_norm ? norm_w : nullptr, norm_b, buf.x, buf.xinv, buf.xnorm, M, stream,
-                  "f32_split_rows");
+  const SplitRows rows{x, use_norm ? norm_w : nullptr, norm_b, buf.x, buf.xinv, buf.xnorm, M, (int)Dc, 0};
+  int rc = split_prep(mats, 3, rows, stream);
   if (rc) return rc;
   SplitGemmEpi e1;
   e1.hfrag = buf.h;

@@ -162,8 +162,21 @@ struct SplitMat {
 constexpr int kSplitMats = 4;
 struct SplitMats {
   SplitMat m[kSplitMats];
+  int block_end[kSplitMats];   // set by split_prep
+};
+// M rows x [M][K] fp32 (K % 8 == 0, 16-byte aligned), LayerNormed (biased variance, eps 1e-5) when g, to fragments;
+// inv[row] = 1 / scale, norm[row] (unless null) = the row's 2-norm after the LayerNorm.
+struct SplitRows {
+  const float* x;
+  const float *g, *b;
+  f16* dst;
+  float *inv, *norm;
+  long long M;
+  int K, ksteps;   // ksteps set by split_prep
 };
 int split_weights(const SplitMats& mats, int count, hipStream_t stream);
+// count weights (0: none) and rows.
+int split_prep(SplitMats mats, int count, SplitRows rows, hipStream_t stream);
 
 // k-steps of a GEMM operand of K columns: whole pairs of 16 (the tile loop stages two at a time).
 inline int split_ksteps(int64_t K) { return (int)(round_up(K, 32) / 16); }

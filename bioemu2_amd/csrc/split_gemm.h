@@ -22,14 +22,11 @@ struct SplitGemmEpi {
   int hsteps = 0;
 };
 
-// Widest row split_rows holds in registers (12 k-steps in each of 4 waves); longer rows are read once per pass.
+// Widest row split_prep holds in registers (12 k-steps in each of 4 waves); longer rows are read once per pass.
 constexpr int kSplitMaxK = 12 * 4 * 16;
 // Fewest 128 x 128 tiles worth the tiled kernel.
 constexpr int kSplitTiledMin = 128;
 
-// Rows [x1 | x2] (K1, K2 multiples of 8, 16-byte aligned; K2 = 0 past kSplitMaxK), LayerNormed when g, to fragments.
-int split_rows(const float* x1, int K1, const float* x2, int K2, const float* g, const float* b, f16* dst, float* inv,
-               float* norm, long long M, hipStream_t stream, const char* name);
 // M rows x N columns (N % 32 == 0; kSplitSwiGLU: both matrices' columns), K columns of A and W fragments.
 int split_gemm(int epi, const f16* A, const float* ainv, const f16* W, const float* winv, const SplitGemmEpi& e,
                long long M, int K, int N, hipStream_t stream, const char* name);

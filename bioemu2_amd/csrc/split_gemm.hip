@@ -2,9 +2,10 @@
 //
 //   split_weights_kernel  weights -> fragments, once per call (a workgroup per
 //                         block of 32 rows).
-//   split_rows_kernel     activation rows -> fragments, with the LayerNorm that
-//                         precedes the product: a workgroup per 32 rows, its four
-//                         waves sharing the k-steps, statistics through LDS.
+//   split_prep_kernel     the same and activation rows -> fragments, with the
+//                         LayerNorm that precedes the product: a workgroup per 32
+//                         rows of either, its four waves sharing the k-steps,
+//                         statistics through LDS.
 //   split_gemm_kernel     128 x 128 output tiles, 4 waves of 64 x 64; both operands
 //                         staged through LDS two k-steps at a time by copies that
 //                         write LDS directly (fragments are contiguous: no swizzle,
@@ -29,8 +30,8 @@
 namespace bioemu {
 namespace {
 
-// A workgroup per block of 32 rows; its 16 waves share the k-steps, so that a weight of up to 1024 columns is read
-// once, with every load in flight (longer ones are read again for the second pass).
+// A workgroup per block of 32 rows; its waves share the k-steps.  What fits in kWaves x kSteps k-steps is read once,
+// with every load in flight; longer weights are read again for the second pass.
 constexpr int kSwWaves = 16, kSwSteps = 4;
 
 // Columns k .. k + 7 of a row, times gamma; dot += the columns' product with beta.
@@ -55,19 +56,17 @@ __device__ __forceinline__ void weight_chunk(const SplitMat& m, const float* row
   }
 }
 
-__global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats mats) {
-  __shared__ float red[kSwWaves];
-  __shared__ float rown[kSwWaves][32], rowd[kSwWaves][32];
-  const SplitMat& m = mats.m[blockIdx.y];
-  const int rb = blockIdx.x;
-  if (rb * 32 >= m.rows) return;   // uniform over the workgroup
+template <int kWaves, int kSteps>
+__device__ __forceinline__ void split_weight_block(const SplitMat& m, int rb) {
+  __shared__ float red[kWaves];
+  __shared__ float rown[kWaves][32], rowd[kWaves][32];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const int r = rb * 32 + perm32(n), K = r < m.rows ? m.K : 0;   // rows past the matrix read as zeros
   const float* row = m.w + (size_t)r * m.K;
-  float v[kSwSteps][8];
+  float v[kSteps][8];
   float amax = 0.f, ss = 0.f, dot = 0.f, unused = 0.f;
 #pragma unroll
-  for (int i = 0; i < kSwSteps; ++i) weight_chunk(m, row, (wave + kSwWaves * i) * 16 + 8 * h, K, v[i], dot);
+  for (int i = 0; i < kSteps; ++i) weight_chunk(m, row, (wave + kWaves * i) * 16 + 8 * h, K, v[i], dot);
   auto scan = [&](const float (&c)[8]) {
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -76,8 +75,8 @@ __global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats 
     }
   };
 #pragma unroll
-  for (int i = 0; i < kSwSteps; ++i) scan(v[i]);
-  for (int ks = wave + kSwWaves * kSwSteps; ks < m.ksteps; ks += kSwWaves) {
+  for (int i = 0; i < kSteps; ++i) scan(v[i]);
+  for (int ks = wave + kWaves * kSteps; ks < m.ksteps; ks += kWaves) {
     float c[8];
     weight_chunk(m, row, ks * 16 + 8 * h, K, c, dot);
     scan(c);
@@ -93,13 +92,13 @@ __global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats 
   }
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kSwWaves; ++w) amax = fmaxf(amax, red[w]);
+  for (int w = 0; w < kWaves; ++w) amax = fmaxf(amax, red[w]);
   const float s = split_scale(amax);
   if (threadIdx.x == 0) m.inv[(size_t)rb * m.inv_stride] = split_inv(s);
   if (wave == 0 && (m.norm || m.bias)) {
     float q = 0.f, d = 0.f;
 #pragma unroll
-    for (int w = 0; w < kSwWaves; ++w) {
+    for (int w = 0; w < kWaves; ++w) {
       q += rown[w][n];
       d += rowd[w][n];
     }
@@ -124,13 +123,19 @@ __global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats 
     *reinterpret_cast<f16x8*>(d + kFragHalf + lane * 8) = lo;
   };
 #pragma unroll
-  for (int i = 0; i < kSwSteps; ++i)
-    if (wave + kSwWaves * i < m.ksteps) put(wave + kSwWaves * i, v[i]);
-  for (int ks = wave + kSwWaves * kSwSteps; ks < m.ksteps; ks += kSwWaves) {
+  for (int i = 0; i < kSteps; ++i)
+    if (wave + kWaves * i < m.ksteps) put(wave + kWaves * i, v[i]);
+  for (int ks = wave + kWaves * kSteps; ks < m.ksteps; ks += kWaves) {
     float c[8];
     weight_chunk(m, row, ks * 16 + 8 * h, K, c, unused);
     put(ks, c);
   }
+}
+
+__global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats mats) {
+  const SplitMat& m = mats.m[blockIdx.y];
+  if ((int)blockIdx.x * 32 >= m.rows) return;   // uniform over the workgroup
+  split_weight_block<kSwWaves, kSwSteps>(m, blockIdx.x);
 }
 
 // Sum over the row's two lanes and the workgroup's four waves (one value per row).
@@ -149,29 +154,27 @@ __device__ __forceinline__ float rows_max(float v, float (&buf)[4][32], int wave
   return fmaxf(fmaxf(buf[0][n], buf[1][n]), fmaxf(buf[2][n], buf[3][n]));
 }
 
-// Rows [x1 (K1 values) | x2 (K2 values)] (K1, K2 multiples of 8), optionally
-// LayerNormed (biased variance, eps 1e-5, fp32, two passes), to fragments.  A
-// lane holds KPW k-steps x 8 values in registers; wave w takes the k-steps w, w +
-// 4, ...  inv[row] = 1 / scale, norm[row] (unless null) = the row's 2-norm after
-// the LayerNorm.
+// Rows of K values (a multiple of 8), optionally LayerNormed (biased variance, eps
+// 1e-5, fp32, two passes), to fragments.  A lane holds KPW k-steps x 8 values in
+// registers; wave w takes the k-steps w, w + 4, ...  inv[row] = 1 / scale,
+// norm[row] (unless null) = the row's 2-norm after the LayerNorm.
 template <int KPW, bool kLn>
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x1, int K1,
-                                                         const float* __restrict__ x2, int K2,
-                                                         const float* __restrict__ g, const float* __restrict__ b,
-                                                         f16* __restrict__ dst, float* __restrict__ inv,
-                                                         float* __restrict__ norm, long long M, int ksteps) {
+__device__ __forceinline__ void split_row_block(const SplitRows& r, long long rb) {
   __shared__ float buf[4][4][32];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
-  const long long rb = blockIdx.x, m = rb * 32 + n;
+  const long long m = rb * 32 + n, M = r.M;
   const bool valid = m < M;
-  const int K = K1 + K2;
+  const int K = r.K, ksteps = r.ksteps;
+  const float *g = r.g, *b = r.b;
+  f16* dst = r.dst;
+  float *inv = r.inv, *norm = r.norm;
   float v[KPW][8];
 #pragma unroll
   for (int i = 0; i < KPW; ++i) {
     const int k = (wave + 4 * i) * 16 + 8 * h;
     f32x4 a = {0.f, 0.f, 0.f, 0.f}, c = a;
     if (valid && k < K) {
-      const float* p = k < K1 ? x1 + (size_t)m * K1 + k : x2 + (size_t)m * K2 + (k - K1);
+      const float* p = r.x + (size_t)m * K + k;
       a = *reinterpret_cast<const f32x4*>(p);
       c = *reinterpret_cast<const f32x4*>(p + 4);
     }
@@ -240,6 +243,25 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
       *reinterpret_cast<f16x8*>(d + kFragHalf + lane * 8) = lo;
     }
   }
+}
+
+// Weight blocks (mats.m[i] holding block_end[i - 1] .. block_end[i]) and row blocks in one launch: neither depends on
+// the other, and each alone is a chain of dependent memory round trips rather than bandwidth.  Two launches -> one at
+// K = 384 and 768: 200 rows 14.3 -> 9.4 us, 6144 rows 17.4 -> 10.7 us.
+template <int KPW, bool kLn>
+__global__ __launch_bounds__(256) void split_prep_kernel(SplitMats mats, SplitRows rows) {
+  const int blk = blockIdx.x;
+  if (blk < mats.block_end[kSplitMats - 1]) {   // uniform over the workgroup
+    int i = 0;
+    while (blk >= mats.block_end[i]) ++i;
+    const int rb = blk - (i ? mats.block_end[i - 1] : 0);
+    if (mats.m[i].ksteps <= 4 * 6)
+      split_weight_block<4, 6>(mats.m[i], rb);
+    else
+      split_weight_block<4, 12>(mats.m[i], rb);
+    return;
+  }
+  split_row_block<KPW, kLn>(rows, blk - mats.block_end[kSplitMats - 1]);
 }
 
 // The same for rows too long for registers: every pass reads them again.
@@ -671,42 +693,51 @@ int split_weights(const SplitMats& mats, int count, hipStream_t stream) {
   int blocks = 0;
   for (int i = 0; i < count; ++i) blocks = std::max(blocks, (mats.m[i].rows + 31) / 32);
   KernelTimerScope timed("f32_split_weights", stream);
-  hipLaunchKernelGGL(split_weights_kernel, dim3((unsigned)blocks, (unsigned)count), dim3(64 * kSwWaves), 0, stream, mats);
+  hipLaunchKernelGGL(split_weights_kernel, dim3(blocks, count), dim3(64 * kSwWaves), 0, stream, mats);
   return check_launch("f32_split_weights");
 }
 
-int split_rows(const float* x1, int K1, const float* x2, int K2, const float* g, const float* b, f16* dst, float* inv,
-               float* norm, long long M, hipStream_t stream, const char* name) {
-  const int ks = split_ksteps(K1 + K2), kpw = (ks + 3) / 4;
-  const dim3 grid((unsigned)((M + 31) / 32));
-  KernelTimerScope timed(name, stream);
-  if (K1 + K2 > kSplitMaxK) {
-    if (K2) return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: %d + %d columns", name, K1, K2);
-    if (g)
-      hipLaunchKernelGGL(split_long_rows_kernel<true>, grid, dim3(256), 0, stream, x1, K1, g, b, dst, inv, norm, M, ks);
-    else
-      hipLaunchKernelGGL(split_long_rows_kernel<false>, grid, dim3(256), 0, stream, x1, K1, g, b, dst, inv, norm, M, ks);
-    return check_launch(name);
+int split_prep(SplitMats mats, int count, SplitRows r, hipStream_t stream) {
+  const long long rblocks = (r.M + 31) / 32;
+  r.ksteps = split_ksteps(r.K);
+  const bool is_long = r.K > kSplitMaxK;
+  if (count && is_long) {
+    const int rc = split_weights(mats, count, stream);
+    if (rc) return rc;
+    count = 0;
   }
-#define BIOEMU_SPLIT_ROWS(KPW)                                                                                       \
-  do {                                                                                                               \
-    if (g)                                                                                                           \
-      hipLaunchKernelGGL((split_rows_kernel<KPW, true>), grid, dim3(256), 0, stream, x1, K1, x2, K2, g, b, dst, inv, \
-                         norm, M, ks);                                                                               \
-    else                                                                                                             \
-      hipLaunchKernelGGL((split_rows_kernel<KPW, false>), grid, dim3(256), 0, stream, x1, K1, x2, K2, g, b, dst,     \
-                         inv, norm, M, ks);                                                                          \
+  int wblocks = 0;
+  for (int i = 0; i < kSplitMats; ++i) {
+    if (i < count) wblocks += (mats.m[i].rows + 31) / 32;
+    mats.block_end[i] = wblocks;
+  }
+  const int kpw = (r.ksteps + 3) / 4;
+  const dim3 grid((unsigned)(wblocks + rblocks)), block(256);
+  KernelTimerScope timed("f32_split_rows", stream);
+  if (is_long) {
+    if (r.g)
+      hipLaunchKernelGGL(split_long_rows_kernel<true>, grid, block, 0, stream, r.x, r.K, r.g, r.b, r.dst, r.inv,
+                         r.norm, r.M, r.ksteps);
+    else
+      hipLaunchKernelGGL(split_long_rows_kernel<false>, grid, block, 0, stream, r.x, r.K, r.g, r.b, r.dst, r.inv,
+                         r.norm, r.M, r.ksteps);
+    return check_launch("f32_split_rows");
+  }
+#define BIOEMU_SPLIT_PREP(KPW)                                                                  \
+  do {                                                                                          \
+    if (r.g)                                                                                    \
+      hipLaunchKernelGGL((split_prep_kernel<KPW, true>), grid, block, 0, stream, mats, r);      \
+    else                                                                                        \
+      hipLaunchKernelGGL((split_prep_kernel<KPW, false>), grid, block, 0, stream, mats, r);     \
   } while (0)
   if (kpw <= 2)
-    BIOEMU_SPLIT_ROWS(2);
-  else if (kpw <= 4)
-    BIOEMU_SPLIT_ROWS(4);
+    BIOEMU_SPLIT_PREP(2);
   else if (kpw <= 6)
-    BIOEMU_SPLIT_ROWS(6);
+    BIOEMU_SPLIT_PREP(6);
   else
-    BIOEMU_SPLIT_ROWS(12);
-#undef BIOEMU_SPLIT_ROWS
-  return check_launch(name);
+    BIOEMU_SPLIT_PREP(12);
+#undef BIOEMU_SPLIT_PREP
+  return check_launch("f32_split_rows");
 }
 
 int split_gemm(int epi, const f16* A, const float* ainv, const f16* W, const float* winv, const SplitGemmEpi& e,
