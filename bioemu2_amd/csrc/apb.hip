@@ -27,16 +27,21 @@ constexpr int CZ = 128;
 constexpr int kBiasThreads = 256;
 
 // bias[b][h][i][j] = log2(e) * LN(z[b][i][j]) . Wz[h] for i, j < Np (zero pair rows outside
-// [0, N)), with the LayerNorm folded into Wz (wf, cf from launch_fold_ln).  The
+// [0, N)), with the LayerNorm folded into Wz (beta may be null).  The
 // attention's softmax runs in base 2, so the bias is stored in log2 units.
-__global__ __launch_bounds__(kBiasThreads) void pair_bias_kernel(const bf16* __restrict__ z,
-                                                                 const bf16* __restrict__ wf,
-                                                                 const bf16* __restrict__ cf, bf16* __restrict__ bias,
+// Two waves per SIMD: the 4 workgroups per CU then run as two full rounds (three at a time left the second round a
+// third full: 125 -> 139 us at B = 8, N = 512).
+__global__ __launch_bounds__(kBiasThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void pair_bias_kernel(const bf16* __restrict__ z,
+                                                                 const bf16* __restrict__ w_z,
+                                                                 const float* __restrict__ gamma,
+                                                                 const float* __restrict__ beta,
+                                                                 bf16* __restrict__ bias,
                                                                  int B, int N, int Np, int H) {
   __shared__ __attribute__((aligned(16))) bf16 wl[32 * kLdw];
   __shared__ bf16 cl[64];
-  stage_weights(wl, wf, H, 32);
-  stage_bias(cl, cf, H, 32);
+  stage_rows_ln<kBiasThreads, 32, CZ, kLdw>(
+      wl, gamma, beta, [&](int r) { return r < H ? w_z + (size_t)r * CZ : nullptr; },
+      [&](int r, float c) { put_bias(cl, r, c); });
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int rho = lane & 31, h = lane >> 5;
@@ -258,7 +263,7 @@ __global__ __launch_bounds__(256) void apb_flash_kernel(const bf16* __restrict__
 }
 
 struct ApbBuffers {
-  bf16 *sn, *q, *k, *vt, *g, *go, *bias, *wf, *cf;
+  bf16 *sn, *q, *k, *vt, *g, *go, *bias;
 };
 
 size_t apb_layout(int64_t B, int64_t BM, int64_t N, int64_t CS, int64_t H, ApbBuffers* buf, char* base) {
@@ -280,11 +285,8 @@ size_t apb_layout(int64_t B, int64_t BM, int64_t N, int64_t CS, int64_t H, ApbBu
     buf->go = reinterpret_cast<bf16*>(p);
     p += tok;
     buf->bias = reinterpret_cast<bf16*>(p);
-    p += bias_bytes;
-    buf->wf = reinterpret_cast<bf16*>(p);
-    buf->cf = reinterpret_cast<bf16*>(p + round_up((size_t)32 * 128 * 2, 256));
   }
-  return 6 * tok + bias_bytes + fold_bytes(32);
+  return 6 * tok + bias_bytes;
 }
 
 }  // namespace
@@ -342,12 +344,10 @@ extern "C" int bioemu_apb_fwd(const void* s, const void* z, const uint8_t* mask,
   const long long ntiles = B * Np * (Np / 32);
   if (ntiles >= kMaxTiles) return set_error(BIOEMU_ERR_INVALID_ARG, "apb: too many pair tiles");
   const unsigned grid1 = (unsigned)std::min<long long>(4LL * cus, (ntiles + 3) / 4);
-  rc = launch_fold_ln(w_z, norm_z_w, norm_z_b, buf.wf, buf.cf, H, stream);
-  if (rc) return rc;
   {
     KernelTimerScope timed("apb_pair_bias", stream);
     hipLaunchKernelGGL(pair_bias_kernel, dim3(grid1), dim3(kBiasThreads), 0, stream, static_cast<const bf16*>(z),
-                       buf.wf, buf.cf, buf.bias, (int)B, (int)N, (int)Np, (int)H);
+                       static_cast<const bf16*>(w_z), norm_z_w, norm_z_b, buf.bias, (int)B, (int)N, (int)Np, (int)H);
   }
   rc = check_launch("apb_pair_bias");
   if (rc) return rc;

@@ -218,4 +218,81 @@ __device__ __forceinline__ void stage_weights(bf16* wl, const bf16* __restrict__
   }
 }
 
+// Stages kRows weight rows of kC channels into LDS (row stride kLd), every load of a
+// thread issued before its first store, for persistent workgroups: where the call has
+// few tiles, staging is a large part of it.  (Workgroups that stage little and live
+// short use stage_weights: the registers held here cost pwa_weights an eighth of its
+// occupancy.)  src(r) is the row's address, null for a zero row.  Whole workgroup of
+// kThreads; no barrier.
+template <int kThreads, int kRows, int kC, int kLd, typename Src>
+__device__ __forceinline__ void stage_rows(bf16* wl, Src src) {
+  constexpr int kParts = kC / 8, kChunks = kRows * kParts, kPer = (kChunks + kThreads - 1) / kThreads;
+  bf16x8 v[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int q = threadIdx.x + i * kThreads;
+    const bf16* row = q < kChunks ? src(q / kParts) : nullptr;
+    v[i] = bf16x8{};
+    if (row) v[i] = load8(row + q % kParts * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int q = threadIdx.x + i * kThreads;
+    if (q < kChunks) store8(wl + q / kParts * kLd + q % kParts * 8, v[i]);
+  }
+}
+
+// The same with the LayerNorm affine that precedes the product folded in: LDS row r
+// = W[r] * gamma rounded to bf16, and put(r, W[r] . beta) once per row (beta null:
+// zero).  A fold in a launch of its own takes 4.3 us and the gap before the next one;
+// here it takes 2 us of triatt_proj (288 rows) and 1.3 of apb's pair bias (32).  (In
+// trimul_out, 256 rows of two LayerNorms, it took 7: that fold runs beside an earlier
+// kernel instead.)
+template <int kThreads, int kRows, int kC, int kLd, typename Src, typename Put>
+__device__ __forceinline__ void stage_rows_ln(bf16* wl, const float* __restrict__ gamma,
+                                              const float* __restrict__ beta, Src src, Put put) {
+  constexpr int kParts = kC / 8, kChunks = kRows * kParts, kPer = (kChunks + kThreads - 1) / kThreads;
+  static_assert(kThreads % kParts == 0 && 64 % kParts == 0, "a thread keeps its channels, a row one wave");
+  const int part = threadIdx.x % kParts;
+  bf16x8 v[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int q = threadIdx.x + i * kThreads;
+    const bf16* row = q < kChunks ? src(q / kParts) : nullptr;
+    v[i] = bf16x8{};
+    if (row) v[i] = load8(row + part * 8);
+  }
+  float ga[8], be[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+    ga[t] = gamma[part * 8 + t];
+    be[t] = beta ? beta[part * 8 + t] : 0.f;
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int q = threadIdx.x + i * kThreads;
+    float dot = 0.f;
+    bf16x8 o;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const float w = bf2f(v[i][t]);
+      o[t] = f2bf(w * ga[t]);
+      dot += w * be[t];
+    }
+#pragma unroll
+    for (int off = kParts / 2; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
+    if (q < kChunks) {
+      store8(wl + q / kParts * kLd + part * 8, o);
+      if (part == 0) put(q / kParts, dot);
+    }
+  }
+}
+
+// A folded bias as the pair (hi, lo) of bias_step_w.
+__device__ __forceinline__ void put_bias(bf16* cl, int row, float c) {
+  const bf16 hi = f2bf(c);
+  cl[2 * row] = hi;
+  cl[2 * row + 1] = f2bf(c - bf2f(hi));
+}
+
 }  // namespace bioemu

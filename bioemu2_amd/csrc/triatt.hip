@@ -73,20 +73,74 @@ __device__ __forceinline__ size_t bias_tile_index(int h, int q, int k, int Np) {
 }
 
 // ---------------------------------------------------------------------------
+// Weights of the attention kernel's own projections in MFMA A-operand
+// fragment order: fragment f of 32 weight rows x 16 inputs is 1 KB contiguous
+// (lane l at bytes 16 l), so each fragment load reads whole cache lines.
+//   f = 0 .. 31   q rows, LayerNorm gamma folded in: block hd = f / 8, k-step
+//                 s = f % 8, lane (n, hh) holds W'q[hd*32 + perm32(n)][16 s + 8 hh + 0..7]
+//   f = 32 .. 63  g rows, folded: W'g[hd*32 + perm32(n)][32 (s >> 1) + 16 hh + 8 (s & 1) + 0..7]
+//   f = 64 .. 95  Wo: Wo[cb*32 + perm32(n)][32 (s >> 1) + 16 hh + 8 (s & 1) + 0..7]
+// The folded values are W * gamma rounded to bf16, bit for bit the fold of the
+// projection rows.
+// ---------------------------------------------------------------------------
+constexpr int kFragCount = 96;
+constexpr int kFragElems = kFragCount * 64 * 8;
+
+// cf[row] = W[row] . beta as a (hi, lo) pair, for the q and g rows.
+// The first kPrepBlocks workgroups of the projection kernel write both, beside the
+// others' work: as launches of their own (the fold of all rows, then the fragments)
+// they took 8.6 us of a call, at N = 64 a tenth of it.
+constexpr int kPrepFragBlocks = kFragCount * 64 / kProjThreads;
+constexpr int kPrepBlocks = kPrepFragBlocks + 2 * C * (C / 8) / kProjThreads;
+
+__device__ __forceinline__ void triatt_prep(int block, const bf16* __restrict__ w_proj, const float* __restrict__ gamma,
+                                            const float* __restrict__ beta, const bf16* __restrict__ w_o,
+                                            bf16* __restrict__ wt, bf16* __restrict__ cf) {
+  if (block >= kPrepFragBlocks) {   // 16 lanes per row
+    const int q = (block - kPrepFragBlocks) * kProjThreads + threadIdx.x, part = q & 15, r = q >> 4;
+    const int row = r < C ? kRowQ + r : kRowG + r - C;
+    const bf16x8 w = load8(w_proj + (size_t)row * C + part * 8);
+    float dot = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dot += bf2f(w[e]) * beta[part * 8 + e];
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
+    if (part == 0) put_bias(cf, row, dot);
+    return;
+  }
+  const int slot = block * kProjThreads + threadIdx.x;   // 16-byte slot
+  const int f = slot >> 6, lane = slot & 63, n = lane & 31, hh = lane >> 5;
+  const int kind = f >> 5, blk = (f >> 3) & 3, s = f & 7;
+  const int row = blk * 32 + perm32(n);
+  const int c0 = kind == 0 ? 16 * s + 8 * hh : 32 * (s >> 1) + 16 * hh + 8 * (s & 1);
+  const bf16* src = kind == 2 ? w_o + (size_t)row * C : w_proj + (size_t)((kind == 0 ? kRowQ : kRowG) + row) * C;
+  const bf16x8 w = load8(src + c0);
+  bf16x8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = kind == 2 ? w[e] : f2bf(bf2f(w[e]) * gamma[c0 + e]);
+  store8(wt + (size_t)slot * 8, o);
+}
+
+// ---------------------------------------------------------------------------
 // Projection kernel.  Tile = (b, frame row i, 32 frame columns).
 // ---------------------------------------------------------------------------
 template <bool kStarting>
 __global__ __launch_bounds__(kProjThreads) void triatt_proj_kernel(
-    const bf16* __restrict__ z, const uint8_t* __restrict__ mask, const bf16* __restrict__ wf,
-    const bf16* __restrict__ cf, TriAttBuffers buf, int B, int N, int Np) {
+    const bf16* __restrict__ z, const uint8_t* __restrict__ mask, const bf16* __restrict__ w_proj,
+    const float* __restrict__ gamma, const float* __restrict__ beta, const bf16* __restrict__ w_o,
+    bf16* __restrict__ wt, bf16* __restrict__ cf, TriAttBuffers buf, int B, int N, int Np) {
   // LDS rows: k (0 .. C-1), v (C .. 2C-1), bias (2C .. 2C+H-1, zero-padded to 32 rows).
   extern __shared__ __attribute__((aligned(16))) char smem[];
   bf16* wl = reinterpret_cast<bf16*>(smem);
   bf16* cl = wl + kProjRowsLds * kLdw;
-  stage_weights(wl, wf + (size_t)kRowK * C, 2 * C, 2 * C);
-  stage_weights(wl + 2 * C * kLdw, wf + (size_t)kRowB * C, H, 32);
-  stage_bias(cl, cf + 2 * kRowK, 2 * C, 2 * C);
-  stage_bias(cl + 2 * 2 * C, cf + 2 * kRowB, H, 32);
+  if (blockIdx.x < kPrepBlocks) {   // uniform over the workgroup
+    triatt_prep(blockIdx.x, w_proj, gamma, beta, w_o, wt, cf);
+    return;
+  }
+  stage_rows_ln<kProjThreads, kProjRowsLds, C, kLdw>(
+      wl, gamma, beta,
+      [&](int r) { return r >= 2 * C + H ? nullptr : w_proj + (size_t)(r < 2 * C ? kRowK + r : kRowB + r - 2 * C) * C; },
+      [&](int r, float c) { put_bias(cl, r, c); });
   __syncthreads();
 
   const int lane = threadIdx.x & 63, wave = wave_id();
@@ -102,7 +156,7 @@ __global__ __launch_bounds__(kProjThreads) void triatt_proj_kernel(
   // normalised after them.  Vector-memory counters retire in issue order, so
   // waiting for those loads then does not wait for the stores to be written,
   // and, being in straight-line code, the wait the compiler places is exact.
-  const unsigned stride = gridDim.x * waves;
+  const unsigned stride = (gridDim.x - kPrepBlocks) * waves;
   bf16x8 raw[8];
   uint8_t mraw = 0;
   bool mok = false;
@@ -138,7 +192,7 @@ __global__ __launch_bounds__(kProjThreads) void triatt_proj_kernel(
     mv = mok && mraw != 0;
   };
 
-  unsigned t = blockIdx.x * waves + wave;
+  unsigned t = (blockIdx.x - kPrepBlocks) * waves + wave;
   if (t < ntiles) {
     fetch(t);
     prepare(t);
@@ -197,37 +251,6 @@ __global__ __launch_bounds__(kProjThreads) void triatt_proj_kernel(
     if (h == 0) buf.mask[frow + k0 + rho] = mv;
     if (tn < ntiles) prepare(tn);
   }
-}
-
-// ---------------------------------------------------------------------------
-// Weights of the attention kernel's own projections in MFMA A-operand
-// fragment order: fragment f of 32 weight rows x 16 inputs is 1 KB contiguous
-// (lane l at bytes 16 l), so each fragment load reads whole cache lines.
-//   f = 0 .. 31   q rows, LayerNorm gamma folded in: block hd = f / 8, k-step
-//                 s = f % 8, lane (n, hh) holds W'q[hd*32 + perm32(n)][16 s + 8 hh + 0..7]
-//   f = 32 .. 63  g rows, folded: W'g[hd*32 + perm32(n)][32 (s >> 1) + 16 hh + 8 (s & 1) + 0..7]
-//   f = 64 .. 95  Wo: Wo[cb*32 + perm32(n)][32 (s >> 1) + 16 hh + 8 (s & 1) + 0..7]
-// The folded values are W * gamma rounded to bf16, bit for bit the fold of the
-// projection rows.
-// ---------------------------------------------------------------------------
-constexpr int kFragCount = 96;
-constexpr int kFragElems = kFragCount * 64 * 8;
-
-__global__ __launch_bounds__(256) void triatt_frag_kernel(const bf16* __restrict__ w_proj,
-                                                          const float* __restrict__ gamma,
-                                                          const bf16* __restrict__ w_o, bf16* __restrict__ wt) {
-  const int slot = blockIdx.x * 256 + threadIdx.x;   // 16-byte slot
-  if (slot >= kFragCount * 64) return;
-  const int f = slot >> 6, lane = slot & 63, n = lane & 31, hh = lane >> 5;
-  const int kind = f >> 5, blk = (f >> 3) & 3, s = f & 7;
-  const int row = blk * 32 + perm32(n);
-  const int c0 = kind == 0 ? 16 * s + 8 * hh : 32 * (s >> 1) + 16 * hh + 8 * (s & 1);
-  const bf16* src = kind == 2 ? w_o + (size_t)row * C : w_proj + (size_t)((kind == 0 ? kRowQ : kRowG) + row) * C;
-  const bf16x8 w = load8(src + c0);
-  bf16x8 o;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = kind == 2 ? w[e] : f2bf(bf2f(w[e]) * gamma[c0 + e]);
-  store8(wt + (size_t)slot * 8, o);
 }
 
 // ---------------------------------------------------------------------------
@@ -293,9 +316,9 @@ __device__ __forceinline__ int t_off(int r, int chunk) { return r * TLD + ((chun
 // With kTail the residual stream z carries an int8 tail plane (common.h),
 // read with z and rewritten with out (in place).
 // wt: the q and g rows of the packed projection (LayerNorm folded in) and Wo
-// in fragment order (triatt_frag_kernel); cf: the folded projection's bias
-// pairs (fold.hip), of which this kernel uses the q and g rows; z is read for the query side, the gate and the residual (z = zres;
-// out may alias it: every workgroup reads and writes only its own pairs).
+// in fragment order, cf: the bias pairs of the q and g rows (triatt_prep); z is
+// read for the query side, the gate and the residual (z = zres; out may alias it:
+// every workgroup reads and writes only its own pairs).
 template <bool kStarting, bool kTail>
 __global__ __launch_bounds__(kFlashThreads) __attribute__((amdgpu_waves_per_eu(kFlashWavesPerEu, kFlashWavesPerEu)))
 void triatt_flash_kernel(
@@ -936,9 +959,9 @@ extern "C" size_t bioemu_triatt_workspace_bytes(int64_t B, int64_t N, int64_t Dc
   if (B <= 0 || N <= 0 || Dc != C || Hc != H) return 0;
   const size_t Np = triatt_np(N);
   const size_t pairs = (size_t)B * Np * Np;
-  // k, v^T (bf16 x C each) + bias (bf16 x H) + mask (u8), each 256-byte aligned
+  // k, v^T (bf16 x C each) + bias (bf16 x H) + mask (u8) + triatt_prep's bias pairs, each 256-byte aligned, and fragments
   return round_up(pairs * C * 2, 256) * 2 + round_up(pairs * H * 2, 256) + round_up(pairs, 256) +
-         fold_bytes(kProjRows) + (size_t)kFragElems * 2;
+         round_up((size_t)kProjRows * 4, 256) + (size_t)kFragElems * 2;
 }
 
 extern "C" int bioemu_triatt_fwd(const void* z, const uint8_t* mask, const float* norm_w,
@@ -975,19 +998,9 @@ extern "C" int bioemu_triatt_fwd(const void* z, const uint8_t* mask, const float
   p += round_up(pairs * H * 2, 256);
   buf.mask = reinterpret_cast<uint8_t*>(p);
   p += round_up(pairs, 256);
-  bf16* wf = reinterpret_cast<bf16*>(p);
-  bf16* cf = reinterpret_cast<bf16*>(p + round_up((size_t)kProjRows * C * 2, 256));
-  bf16* wt = reinterpret_cast<bf16*>(p + fold_bytes(kProjRows));
+  bf16* cf = reinterpret_cast<bf16*>(p);
+  bf16* wt = reinterpret_cast<bf16*>(p + round_up((size_t)kProjRows * 4, 256));
   if (B * Np * (Np / 32) >= kMaxTiles) return set_error(BIOEMU_ERR_INVALID_ARG, "triatt: too many pair tiles");
-  int rc = launch_fold_ln(w_proj, norm_w, norm_b, wf, cf, kProjRows, stream);
-  if (rc) return rc;
-  {
-    KernelTimerScope timed("triatt_frag", stream);
-    hipLaunchKernelGGL(triatt_frag_kernel, dim3(kFragCount * 64 / 256), dim3(256), 0, stream,
-                       static_cast<const bf16*>(w_proj), norm_w, static_cast<const bf16*>(w_o), wt);
-  }
-  if ((rc = check_launch("triatt_frag"))) return rc;
-
   int dev = 0, cus = 0;
   (void)hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
@@ -997,17 +1010,19 @@ extern "C" int bioemu_triatt_fwd(const void* z, const uint8_t* mask, const float
     return set_error(BIOEMU_ERR_LAUNCH, "triatt_proj: cannot set dynamic LDS size");
   const long long ntiles = (long long)B * Np * (Np / 32);
   const long long per_wg = kProjThreads / 64;
-  const unsigned grid1 = (unsigned)std::min<long long>(cus, (ntiles + per_wg - 1) / per_wg);
+  const unsigned grid1 = kPrepBlocks + (unsigned)std::min<long long>(cus, (ntiles + per_wg - 1) / per_wg);
   {
     KernelTimerScope timed("triatt_proj", stream);
     if (starting)
       hipLaunchKernelGGL(triatt_proj_kernel<true>, dim3(grid1), dim3(kProjThreads), kProjSmem, stream,
-                         static_cast<const bf16*>(z), mask, wf, cf, buf, (int)B, (int)N, (int)Np);
+                         static_cast<const bf16*>(z), mask, static_cast<const bf16*>(w_proj), norm_w, norm_b,
+                         static_cast<const bf16*>(w_o), wt, cf, buf, (int)B, (int)N, (int)Np);
     else
       hipLaunchKernelGGL(triatt_proj_kernel<false>, dim3(grid1), dim3(kProjThreads), kProjSmem, stream,
-                         static_cast<const bf16*>(z), mask, wf, cf, buf, (int)B, (int)N, (int)Np);
+                         static_cast<const bf16*>(z), mask, static_cast<const bf16*>(w_proj), norm_w, norm_b,
+                         static_cast<const bf16*>(w_o), wt, cf, buf, (int)B, (int)N, (int)Np);
   }
-  rc = check_launch("triatt_proj");
+  const int rc = check_launch("triatt_proj");
   if (rc) return rc;
 
   const long long nitems = (long long)B * N * ((Np + kFlashQueries - 1) / kFlashQueries);

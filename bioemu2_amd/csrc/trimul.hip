@@ -52,19 +52,62 @@ inline int in_waves_per_wg(long long tiles, int cus) {
   return pick_waves_per_wg(tiles, cus, waves, gain, 2);
 }
 
+// ---------------------------------------------------------------------------
+// The two LayerNorm affines of stage 3 folded into its projections:
+//   p_out(LN_out(o)) = xhat_o (Wp diag(g_out))^T + Wp b_out
+//   g_out(LN_in(x))  = xhat_x (Wg diag(g_in))^T  + Wg b_in
+// with xhat the normalised (affine-free) rows.  wfold: [Wp' | Wg'] bf16 (D x D each),
+// cfold: [Wp b_out | Wg b_in] fp32.  16 lanes per weight row.  The last workgroups of
+// the projection kernel do this beside the others (a launch of its own: 4.1 us).
+// ---------------------------------------------------------------------------
+struct OutFold {
+  const bf16 *p_w, *g_w;
+  const float *ln_out_w, *ln_out_b, *ln_in_w, *ln_in_b;
+  bf16* wfold;
+  float* cfold;
+};
+template <int kThreads>
+constexpr int kFoldBlocks = (2 * D * (D / 8) + kThreads - 1) / kThreads;
+
+template <int kThreads>
+__device__ __forceinline__ void trimul_fold(int block, const OutFold& f) {
+  const int q = block * kThreads + threadIdx.x, r = q >> 4, c0 = (q & 15) * 8;
+  if (r >= 2 * D) return;   // whole rows: 16 lanes
+  const bool gate = r >= D;
+  const bf16x8 w = load8((gate ? f.g_w + (size_t)(r - D) * D : f.p_w + (size_t)r * D) + c0);
+  const float* gamma = gate ? f.ln_in_w : f.ln_out_w;
+  const float* beta = gate ? f.ln_in_b : f.ln_out_b;
+  bf16x8 o;
+  float dot = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    o[e] = f2bf(bf2f(w[e]) * gamma[c0 + e]);
+    dot += bf2f(w[e]) * beta[c0 + e];
+  }
+#pragma unroll
+  for (int off = 8; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
+  store8(f.wfold + (size_t)r * D + c0, o);
+  if (c0 == 0) f.cfold[r] = dot;
+}
+
 template <bool kOutgoing, int kWaves>
 __global__ __launch_bounds__(64 * kWaves) void trimul_proj_in_kernel(
     const bf16* __restrict__ x, const uint8_t* __restrict__ mask, const float* __restrict__ ln_w,
     const float* __restrict__ ln_b, const bf16* __restrict__ p_w, const bf16* __restrict__ g_w,
-    bf16* __restrict__ ab, int B, int N, int Np) {
+    bf16* __restrict__ ab, OutFold fold, int B, int N, int Np) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int wgs = gridDim.x - kFoldBlocks<64 * kWaves>;
+  if ((int)blockIdx.x >= wgs) {   // uniform over the workgroup
+    trimul_fold<64 * kWaves>(blockIdx.x - wgs, fold);
+    return;
+  }
   bf16* wl = reinterpret_cast<bf16*>(smem);
   // gamma and beta live in LDS: read from global memory inside the tile loop
   // they would be vector-memory loads issued after the previous tile's
   // stores, and waiting for them would wait for those stores.
   float* lnl = reinterpret_cast<float*>(smem + kInRows * kLdw * 2);
-  stage_weights(wl, p_w, 2 * D, 2 * D);
-  stage_weights(wl + 2 * D * kLdw, g_w, 2 * D, 2 * D);
+  stage_rows<64 * kWaves, kInRows, D, kLdw>(
+      wl, [&](int r) { return r < 2 * D ? p_w + (size_t)r * D : g_w + (size_t)(r - 2 * D) * D; });
   for (int q = threadIdx.x; q < D; q += blockDim.x) {
     lnl[q] = ln_w[q];
     lnl[D + q] = ln_b[q];
@@ -86,7 +129,7 @@ __global__ __launch_bounds__(64 * kWaves) void trimul_proj_in_kernel(
   // (pair 0 for slots outside the sequence; such slots are zeroed through
   // `keep`) so that nothing touches their destination registers, or reads the
   // mask byte, before the wait.
-  const unsigned stride = gridDim.x * waves;
+  const unsigned stride = wgs * waves;
   bf16x8 raw[8];
   uint8_t mraw = 0;
   bool inb_next = false;
@@ -150,40 +193,6 @@ __global__ __launch_bounds__(64 * kWaves) void trimul_proj_in_kernel(
       store8(low ? partner : own, low ? recv : first);
     }
     if (tn < ntiles) prepare();
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Stage 3 prep: fold the two LayerNorm affines into the output projections.
-//   p_out(LN_out(o)) = xhat_o (Wp diag(g_out))^T + Wp b_out
-//   g_out(LN_in(x))  = xhat_x (Wg diag(g_in))^T  + Wg b_in
-// with xhat the normalised (affine-free) rows.  One workgroup per output row.
-// fold layout: [Wp' (D x D) | Wg' (D x D)] bf16, then [cp (D) | cg (D)] fp32.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(D) void trimul_fold_kernel(const bf16* __restrict__ p_w, const bf16* __restrict__ g_w,
-                                                      const float* __restrict__ ln_out_w,
-                                                      const float* __restrict__ ln_out_b,
-                                                      const float* __restrict__ ln_in_w,
-                                                      const float* __restrict__ ln_in_b, bf16* __restrict__ wfold,
-                                                      float* __restrict__ cfold) {
-  __shared__ float red[2][D];
-  const int e = blockIdx.x, c = threadIdx.x;
-  const float wp = bf2f(p_w[e * D + c]), wg = bf2f(g_w[e * D + c]);
-  wfold[e * D + c] = f2bf(wp * ln_out_w[c]);
-  wfold[D * D + e * D + c] = f2bf(wg * ln_in_w[c]);
-  red[0][c] = wp * ln_out_b[c];
-  red[1][c] = wg * ln_in_b[c];
-  __syncthreads();
-  for (int st = D / 2; st > 0; st >>= 1) {
-    if (c < st) {
-      red[0][c] += red[0][c + st];
-      red[1][c] += red[1][c + st];
-    }
-    __syncthreads();
-  }
-  if (c == 0) {
-    cfold[e] = red[0][0];
-    cfold[D + e] = red[1][0];
   }
 }
 
@@ -263,12 +272,10 @@ __global__ __launch_bounds__(kOutThreads) void trimul_out_kernel(
   bf16* wl = reinterpret_cast<bf16*>(smem);
   float* cl = reinterpret_cast<float*>(smem + 2 * D * kLdw * 2);
   bf16* obuf = reinterpret_cast<bf16*>(smem + 2 * D * kLdw * 2 + 2 * D * 4);
-  for (int q = threadIdx.x; q < 2 * D * (D / 8); q += blockDim.x) {
-    const int r = q >> 4, part = q & 15;
-    const int half = r / D, cb = (r % D) >> 5, m = r & 31;
-    const int src = half * D + 32 * cb + 16 * ((m & 15) >> 3) + 8 * (m >> 4) + (m & 7);
-    store8(wl + r * kLdw + part * 8, load8(wfold + (size_t)src * D + part * 8));
-  }
+  stage_rows<kOutThreads, 2 * D, D, kLdw>(wl, [&](int r) {
+    const int m = r & 31;
+    return wfold + (size_t)((r & ~31) + 16 * ((m & 15) >> 3) + 8 * (m >> 4) + (m & 7)) * D;
+  });
   // cl[half D + 64 h + 16 cb + u]: bias of the channel lane h holds in register u of block cb
   for (int t = threadIdx.x; t < 2 * D; t += blockDim.x) {
     const int e = t % D, h = e >> 6, cb = (e >> 4) & 3, u = e & 15;
@@ -421,7 +428,7 @@ using namespace bioemu;
 // Launches trimul_proj_in_kernel<outgoing, waves> (waves 8 or 12).
 static int launch_proj_in(bool outgoing, int waves, unsigned grid, const bf16* x, const uint8_t* mask,
                           const float* ln_w, const float* ln_b, const bf16* p_w, const bf16* g_w, bf16* ab,
-                          int64_t B, int64_t N, int64_t Np, hipStream_t stream) {
+                          OutFold fold, int64_t B, int64_t N, int64_t Np, hipStream_t stream) {
   const void* k = nullptr;
   if (waves == 8)
     k = outgoing ? reinterpret_cast<const void*>(trimul_proj_in_kernel<true, 8>)
@@ -435,11 +442,12 @@ static int launch_proj_in(bool outgoing, int waves, unsigned grid, const bf16* x
     return set_error(BIOEMU_ERR_LAUNCH, "trimul: cannot set dynamic LDS size");
   KernelTimerScope timed("trimul_proj_in", stream);
   void* args[] = {(void*)&x, (void*)&mask, (void*)&ln_w, (void*)&ln_b, (void*)&p_w, (void*)&g_w, (void*)&ab,
-                  nullptr, nullptr, nullptr};
+                  (void*)&fold, nullptr, nullptr, nullptr};
   int b32 = (int)B, n32 = (int)N, np32 = (int)Np;
-  args[7] = &b32;
-  args[8] = &n32;
-  args[9] = &np32;
+  args[8] = &b32;
+  args[9] = &n32;
+  args[10] = &np32;
+  grid += waves == 8 ? kFoldBlocks<512> : kFoldBlocks<768>;
   if (hipLaunchKernel(k, dim3(grid), dim3(64 * waves), args, kInSmem, stream) != hipSuccess)
     return set_error(BIOEMU_ERR_LAUNCH, "trimul_proj_in: launch failed");
   return 0;
@@ -499,21 +507,16 @@ extern "C" int bioemu_trimul_fwd(const void* x, const uint8_t* mask, const float
   if (waves_in >= kMaxTiles) return set_error(BIOEMU_ERR_INVALID_ARG, "trimul: too many pair tiles");
   const int in_waves = in_waves_per_wg(waves_in, cus);
   const unsigned grid1 = (unsigned)std::min<long long>(cus, (waves_in + in_waves - 1) / in_waves);
+  const OutFold fold{static_cast<const bf16*>(p_out_w), static_cast<const bf16*>(g_out_w), norm_out_w, norm_out_b,
+                     norm_in_w, norm_in_b, wfold, cfold};
   int rc = launch_proj_in(outgoing != 0, in_waves, grid1, static_cast<const bf16*>(x), mask, norm_in_w, norm_in_b,
-                          static_cast<const bf16*>(p_in_w), static_cast<const bf16*>(g_in_w), ab, B, N, Np, stream);
+                          static_cast<const bf16*>(p_in_w), static_cast<const bf16*>(g_in_w), ab, fold, B, N, Np,
+                          stream);
   if (rc) return rc;
   rc = check_launch("trimul_proj_in");
   if (rc) return rc;
   rc = launch_bgemm_nt(ab, ab + plane_elems, ob, B * D, N, stream);
   if (rc) return rc;
-  {
-    KernelTimerScope timed("trimul_fold", stream);
-    hipLaunchKernelGGL(trimul_fold_kernel, dim3(D), dim3(D), 0, stream, static_cast<const bf16*>(p_out_w),
-                       static_cast<const bf16*>(g_out_w), norm_out_w, norm_out_b, norm_in_w, norm_in_b, wfold, cfold);
-  }
-  rc = check_launch("trimul_fold");
-  if (rc) return rc;
-
   const long long waves_out = (long long)B * N * ((N + 31) / 32);
   const unsigned grid3 = (unsigned)std::min<long long>(cus, (waves_out + kOutWaves - 1) / kOutWaves);
   KernelTimerScope timed("trimul_out", stream);

@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kThreads) void pair_ln_linear_kernel(const bf16* x,
   extern __shared__ __attribute__((aligned(16))) char smem[];
   bf16* wl = reinterpret_cast<bf16*>(smem);
   bf16* cl = wl + C * kLdw;
-  stage_weights(wl, wf, C, C);
+  stage_rows<kThreads, C, C, kLdw>(wl, [&](int r) { return wf + (size_t)r * C; });
   stage_bias(cl, cf, C, C);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = wave_id();

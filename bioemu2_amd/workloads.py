@@ -79,9 +79,6 @@ def trimul_kernel_work(name: str, B: int, N: int, c: int = 128) -> tuple[str, fl
     if name == "trimul_out":
         # LN_out(o) -> p_out, LN_in(x) -> g_out ; reads o and x, writes out
         return ("hbm", float(3 * P * c * 2))
-    if name == "trimul_fold":
-        # folds the LayerNorm affines into the output weights: reads 2 c x c bf16, writes them back
-        return ("hbm", float(4 * c * c * 2))
     return None
 
 
@@ -105,9 +102,6 @@ def triatt_kernel_work(name: str, B: int, N: int, c: int = 128, H: int = 4,
     if name == "triatt_proj":
         # LN + the key side, k, v (c -> 2c) + bias (c -> H): reads z, writes k, v, the bias and the frame mask
         return ("hbm", float(P * (c * 2 + 2 * c * 2 + H * 2 + 1)))
-    if name == "triatt_frag":
-        # the q and g rows of the projection and Wo ([c][c] each) read and written in fragment order
-        return ("hbm", float(2 * 3 * c * c * 2))
     if name == "triatt_flash":
         # q (c -> c) for the queries of rows with a valid key; QK^T and PV over the valid keys for every
         # (valid row, query, head); the gate g (c -> c) and the output projection for every pair
@@ -285,8 +279,8 @@ class BlockWorkload(Workload):
         w = trimul_kernel_work(kernel, 1, n) or triatt_kernel_work(kernel, 1, n, n_valid=n - self.n_pad)
         if w is not None:
             return w
-        if kernel == "fold_ln":  # triatt (516 rows) x2, APB bias (16 rows), transition fc1 + fc2 (1024 rows, one launch)
-            return fold_kernel_work(kernel, 4, 2 * 516 + 16 + 1024)
+        if kernel == "fold_ln":  # transition fc1 + fc2 (1024 rows, one launch)
+            return fold_kernel_work(kernel, 1, 1024)
         if kernel == "transition_pair":
             return ("mfma", 2.0 * n * n * c * 12 * c)
         if kernel == "apb_pair_bias":
@@ -918,8 +912,6 @@ class ApbWorkload(Workload):
             return ("mfma", 4 * 2.0 * B * M * np_ * 384 * 384)
         if kernel in ("apb_proj_o", "token_layernorm"):
             return ("hbm", float(2 * tok + 384 * 384 * 2))
-        if kernel == "fold_ln":
-            return fold_kernel_work(kernel, 1, 16)
         raise KeyError(kernel)
 
 
