@@ -15,7 +15,7 @@
 //                  the 8 logit rows in LDS, masked, softmax over j -> W bf16.
 //   pwa_proj     : LN_m folded into Wm | Wg; per 32 tokens of one MSA row the
 //                  v block comes out channel-major (V^T, j contiguous: the
-//                  GEMM's B operand) and g pair-major.
+//                  GEMM's B operand) and g in the order pwa_fused reads it.
 //   pwa_fused    : per head the averaging GEMM on MFMA, then the gate and
 //                  the output projection from the accumulator registers;
 //                  writes (g * o) Wo^T (+ m) once, after the last head.
@@ -114,6 +114,17 @@ constexpr int kPThreads = 512;
 constexpr int kPRows = 2 * HC;
 constexpr int kPSmem = kPRows * kLdw64 * 2 + kPRows * 2 * 2;
 
+// Offset of lane's gate values of 32 tokens, tile `it` of MSA row s, for head h: [head pair][half j][lane / 4][head of the
+// pair][lane % 4][8] holds channels 16 hh + 8 j + 0..7 of token n of lane (n, hh), as pwa_fused multiplies them (half j:
+// kGateHalf further).  Against token-major rows, of which a load or store touched 32 (S = 511): pwa_proj at N = 333 44.5
+// -> 41.4 us, at N = 512 61.9 -> 55.7; pwa_fused at N = 100 37.8 -> 33.0, at N = 512 133 -> 129.  A line serves two
+// heads, so that only every second head of pwa_fused waits for memory (one head a line: 32 instead of 24 us at N = 40).
+constexpr int kGateHalf = 64 * 2 * 8;
+__device__ __forceinline__ size_t gate_off(int b, int s, int it, int h, int lane, int S8, int Np) {
+  return ((((size_t)b * S8 + s) * (Np / 32) + it) * (NH / 2) + h / 2) * (2 * kGateHalf) + (lane >> 2) * 64 +
+         (h & 1) * 32 + (lane & 3) * 8;
+}
+
 __device__ __forceinline__ f32x16 proj64_cm(const bf16x8 x[4], bf16x8 xb, const bf16* wl, const bf16* cl, int row0,
                                             int n, int h) {
   f32x16 acc = zero16();
@@ -204,7 +215,6 @@ __global__ __launch_bounds__(kPThreads) void pwa_proj_kernel(const bf16* __restr
     const TileIdx ti = split_tile(t, tpr, S8);
     const int it = ti.col, s = ti.row, b = ti.b;
     const int i0 = it * 32;
-    const int ii = i0 + perm32(rho);
     // v^T: D lane (n = channel within head cb, h) holds tokens i0 + 16h + u.
     // (Both output loops are unrolled, one block per scheduling region, so
     // that the compiler sees every store when it places the wait for the
@@ -225,7 +235,15 @@ __global__ __launch_bounds__(kPThreads) void pwa_proj_kernel(const bf16* __restr
       float r[16];
 #pragma unroll
       for (int u = 0; u < 16; ++u) r[u] = sigmoidf_fast(a[u]);
-      store16(g + (((size_t)b * S8 + s) * Np + ii) * HC + cb * 32 + 16 * h, r);
+      bf16x8 lo, hi;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        lo[u] = f2bf(r[u]);
+        hi[u] = f2bf(r[8 + u]);
+      }
+      bf16* dst = g + gate_off(b, s, it, cb, perm32(rho) + 32 * h, S8, Np);
+      store8(dst, lo);
+      store8(dst + kGateHalf, hi);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (tn < ntiles) prepare(tn);
@@ -376,9 +394,8 @@ __global__ __launch_bounds__(kFuThreads) void pwa_fused_kernel(const bf16* __res
       const int s = s0 + 2 * ws + si;
 #pragma unroll
       for (int ib = 0; ib < 2; ++ib) {
-        const int i = min(i0 + offi[ib], N - 1);   // rows past N are not stored
-        const bf16* gp = g + (((size_t)b * S8 + s) * Np + i) * HC + h * CH + 16 * lh;
-        const bf16x8 g0 = load8(gp), g1 = load8(gp + 8);
+        const bf16* gp = g + gate_off(b, s, (i0 + wi * 64) / 32 + ib, h, lane, S8, Np);   // live: the tile is below Np
+        const bf16x8 g0 = load8(gp), g1 = load8(gp + kGateHalf);
         bf16x8 go0, go1;
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
