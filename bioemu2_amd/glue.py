@@ -14,7 +14,7 @@
   concatenated copy); each transition is the fused row kernel with its residual
   add fused, in place.  fp32 inputs with autocast off (the reference runs its
   denoiser so, score_model.py:355) take the fp32 path: fp32 LN over the
-  concatenation read in place, fp32 MFMA projection, fp32 transitions with the
+  concatenation read in place, fp32 projection (split f16 operands), fp32 transitions with the
   residual fused; any token_z + c_rel multiple of 8 and a_z multiple of 32.
 """
 

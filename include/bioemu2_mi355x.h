@@ -344,7 +344,8 @@ int bioemu_msa_embed_fwd(const float* msa, const float* has_deletion, const floa
                          int64_t F0, int64_t E, int64_t msa_s, hipStream_t stream);
 
 /*
- * fp32 arithmetic (fp32 operands, fp32 MFMA accumulation, fp32 softmax) for the
+ * fp32 arithmetic (fp32 operands, products as split f16 or fp32 MFMAs with fp32
+ * accumulation, fp32 softmax) for the
  * ops the reference's denoiser runs with autocast off (src/bioemu2/biomoa/
  * models/score_model.py:355, model.py:387).  Same arguments and semantics as the
  * bf16 entry points above, with every activation, weight and output fp32:
