@@ -167,6 +167,25 @@ def test_trimul_split_edges(gpu_device, mode, n, b):
     assert rel_l2(got, want) <= TOL
 
 
+def test_trimul_split_gate_limits(gpu_device):
+    """Gates whose argument overflows are 0 or 1, and a gate that is no number makes its channel none."""
+    torch.manual_seed(7)
+    m = randomize_params(TriangleMultiplicationHip(128, "outgoing"), 6)
+    x, mask = torch.randn(1, 35, 35, 128).to(gpu_device), torch.ones(1, 35, 35, dtype=torch.bool, device=gpu_device)
+    m = m.to(gpu_device)
+    with torch.no_grad():
+        m.g_out.weight.mul_(2.0**100)   # every argument past the exponential's range, all finite
+        want = m(x, mask)
+        m.g_out.weight.mul_(2.0**27)    # the same signs (powers of two scale exactly), some infinite
+        assert torch.isfinite(want).all() and torch.equal(m(x, mask), want)
+        m = randomize_params(m.cpu(), 6).to(gpu_device)
+        plain = m(x, mask)
+        m.g_out.weight[3] = float("nan")
+        got = m(x, mask)
+    assert got[..., 3].isnan().all()
+    assert torch.equal(got[..., 32:], plain[..., 32:]) and torch.isfinite(got[..., 4:32]).all()
+
+
 @pytest.mark.parametrize("n,pad", [(1, 0), (31, 3), (33, 0), (97, 96), (129, 40)])
 def test_attention_split_edges(gpu_device, n, pad):
     """Key counts around a 32-key block and a 128-query workgroup; whole blocks masked; values of masked tokens,
