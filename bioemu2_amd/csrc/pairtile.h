@@ -242,6 +242,29 @@ __device__ __forceinline__ void stage_rows(bf16* wl, Src src) {
   }
 }
 
+// W[r] . beta of a 128-channel row held by 16 consecutive lanes, 8 channels each (lane part = 0 .. 15: channels
+// 8 part ..); every one of them gets it.  The order of the sum is fold_ln_kernel's, whose lane l adds channels 2 l and
+// 2 l + 1 before a butterfly over 64 lanes (32, 16, .., 1): the bias keeps its last bit wherever it is folded.  Lane
+// distances 32 .. 4 of that butterfly are 8 .. 1 here, on four partial sums; from the second distance on a lane
+// carries the half (then the one) of them that its upper part bits name.
+__device__ __forceinline__ float fold_dot128(bf16x8 w, const float (&be)[8], int part) {
+  float d[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    d[k] = bf2f(w[2 * k]) * be[2 * k];
+    d[k] = __builtin_fmaf(bf2f(w[2 * k + 1]), be[2 * k + 1], d[k]);
+  }
+  const bool b8 = part & 8, b4 = part & 4;
+  float e[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) e[k] = (b8 ? d[k + 2] : d[k]) + __shfl_xor(b8 ? d[k] : d[k + 2], 8);
+  float f = (b4 ? e[1] : e[0]) + __shfl_xor(b4 ? e[0] : e[1], 4);
+  f += __shfl_xor(f, 2);
+  f += __shfl_xor(f, 1);
+  f += __shfl_xor(f, 8);
+  return f + __shfl_xor(f, 4);
+}
+
 // The same with the LayerNorm affine that precedes the product folded in: LDS row r
 // = W[r] * gamma rounded to bf16, and put(r, W[r] . beta) once per row (beta null:
 // zero).  A fold in a launch of its own takes 4.3 us and the gap before the next one;
@@ -252,7 +275,7 @@ template <int kThreads, int kRows, int kC, int kLd, typename Src, typename Put>
 __device__ __forceinline__ void stage_rows_ln(bf16* wl, const float* __restrict__ gamma,
                                               const float* __restrict__ beta, Src src, Put put) {
   constexpr int kParts = kC / 8, kChunks = kRows * kParts, kPer = (kChunks + kThreads - 1) / kThreads;
-  static_assert(kThreads % kParts == 0 && 64 % kParts == 0, "a thread keeps its channels, a row one wave");
+  static_assert(kC == 128 && kThreads % kParts == 0, "16 lanes of one wave hold a row; a thread keeps its channels");
   const int part = threadIdx.x % kParts;
   bf16x8 v[kPer];
 #pragma unroll
@@ -271,16 +294,10 @@ __device__ __forceinline__ void stage_rows_ln(bf16* wl, const float* __restrict_
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int q = threadIdx.x + i * kThreads;
-    float dot = 0.f;
     bf16x8 o;
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const float w = bf2f(v[i][t]);
-      o[t] = f2bf(w * ga[t]);
-      dot += w * be[t];
-    }
-#pragma unroll
-    for (int off = kParts / 2; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
+    for (int t = 0; t < 8; ++t) o[t] = f2bf(bf2f(v[i][t]) * ga[t]);
+    const float dot = fold_dot128(v[i], be, part);
     if (q < kChunks) {
       store8(wl + q / kParts * kLd + part * 8, o);
       if (part == 0) put(q / kParts, dot);

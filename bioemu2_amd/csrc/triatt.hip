@@ -100,11 +100,10 @@ __device__ __forceinline__ void triatt_prep(int block, const bf16* __restrict__ 
     const int q = (block - kPrepFragBlocks) * kProjThreads + threadIdx.x, part = q & 15, r = q >> 4;
     const int row = r < C ? kRowQ + r : kRowG + r - C;
     const bf16x8 w = load8(w_proj + (size_t)row * C + part * 8);
-    float dot = 0.f;
+    float be[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) dot += bf2f(w[e]) * beta[part * 8 + e];
-#pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
+    for (int e = 0; e < 8; ++e) be[e] = beta[part * 8 + e];
+    const float dot = fold_dot128(w, be, part);
     if (part == 0) put_bias(cf, row, dot);
     return;
   }

@@ -71,6 +71,7 @@ constexpr int kFoldBlocks = (2 * D * (D / 8) + kThreads - 1) / kThreads;
 
 template <int kThreads>
 __device__ __forceinline__ void trimul_fold(int block, const OutFold& f) {
+#pragma clang fp contract(off)
   const int q = block * kThreads + threadIdx.x, r = q >> 4, c0 = (q & 15) * 8;
   if (r >= 2 * D) return;   // whole rows: 16 lanes
   const bool gate = r >= D;
@@ -78,16 +79,24 @@ __device__ __forceinline__ void trimul_fold(int block, const OutFold& f) {
   const float* gamma = gate ? f.ln_in_w : f.ln_out_w;
   const float* beta = gate ? f.ln_in_b : f.ln_out_b;
   bf16x8 o;
-  float dot = 0.f;
+  float d[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     o[e] = f2bf(bf2f(w[e]) * gamma[c0 + e]);
-    dot += bf2f(w[e]) * beta[c0 + e];
+    d[e] = bf2f(w[e]) * beta[c0 + e];
   }
-#pragma unroll
-  for (int off = 8; off >= 1; off >>= 1) dot += __shfl_xor(dot, off);
   store8(f.wfold + (size_t)r * D + c0, o);
-  if (c0 == 0) f.cfold[r] = dot;
+  // Products rounded one by one, then a tree over the channels (c and c + 64, c and c + 32, ..): the pairs of terms
+  // that meet first decide the last bit of the bias.  16 lanes hold 8 channels each.
+#pragma unroll
+  for (int off = 8; off >= 1; off >>= 1)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) d[e] += __shfl_xor(d[e], off);
+#pragma unroll
+  for (int off = 4; off >= 1; off >>= 1)
+#pragma unroll
+    for (int e = 0; e < off; ++e) d[e] += d[e + off];
+  if (c0 == 0) f.cfold[r] = d[0];
 }
 
 template <bool kOutgoing, int kWaves>
