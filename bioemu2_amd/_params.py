@@ -16,7 +16,7 @@ def _find(module: nn.Module, path: tuple[str, ...]) -> nn.Parameter:
             break
     else:
         p = owner._parameters.get(path[-1])
-        if p is not None:
+        if isinstance(p, nn.Parameter):
             return p
     return module.get_parameter(".".join(path))   # anything unusual: its answer, or its error
 
