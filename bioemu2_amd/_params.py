@@ -24,23 +24,26 @@ def _find(module: nn.Module, path: tuple[str, ...]) -> nn.Parameter:
 class PreparedParams:
     """Caches ``(param.detach().to(dtype).contiguous(), ...)`` for a module.
 
-    The cache key is (data_ptr, version counter, device, dtype) of every
-    source parameter, so in-place updates (optimizer steps, ``load_state_dict``)
-    and ``.to()`` moves invalidate it.
+    The cache key is the identity and (data_ptr, version counter, device,
+    dtype) of every source parameter, so in-place updates (optimizer steps,
+    ``load_state_dict``), ``.to()`` moves and replaced parameters invalidate it.
+    The sources stay referenced: a new parameter cannot take the identity of
+    one that was freed, as it can take its address.
     """
 
     def __init__(self, spec: list[tuple[str, torch.dtype]]):
         self.spec = spec
         self._paths = [tuple(name.split(".")) for name, _ in spec]
         self._key: tuple | None = None
+        self._src: list[nn.Parameter] | None = None
         self._val: tuple[Tensor, ...] | None = None
 
     def get(self, module: nn.Module) -> tuple[Tensor, ...]:
         params = [_find(module, path) for path in self._paths]
-        key = tuple((p.data_ptr(), p._version, p.device, p.dtype) for p in params)
+        key = tuple((id(p), p.data_ptr(), p._version, p.device, p.dtype) for p in params)
         if key != self._key or self._val is None:
             self._val = tuple(
                 p.detach().to(dtype=dt).contiguous() for p, (_, dt) in zip(params, self.spec)
             )
-            self._key = key
+            self._key, self._src = key, params
         return self._val

@@ -2,6 +2,7 @@
 
 import copy
 
+import numpy as np
 import pytest
 import torch
 from torch.func import functional_call
@@ -24,6 +25,23 @@ def test_plain_tensors_in_a_parameters_place_are_refused(grad):
     m()
     with torch.set_grad_enabled(grad), pytest.raises(AttributeError):
         functional_call(m, _weights(m, 1.0, lambda t: t), ())
+
+
+def test_replaced_and_freed_parameters_are_seen():
+    """A new parameter at a freed one's address (here for certain: both over one array) has the same address, version,
+    device and dtype."""
+    m = _Prepared(128, 256)
+    memory = {name: np.zeros(p.shape, dtype=np.float32) for name, p in m.named_parameters()}
+    for value in range(1, 5):
+        params = {}
+        for name, a in memory.items():
+            a.fill(value)
+            params[name] = torch.nn.Parameter(torch.from_numpy(a))
+        assert all(bool((t == value).all()) for t in functional_call(m, params, ()))
+    for value in range(1, 5):
+        memory["fc2.weight"].fill(value)
+        m.fc2.weight = torch.nn.Parameter(torch.from_numpy(memory["fc2.weight"]))
+        assert bool((m()[3] == value).all())
 
 
 def test_copies_and_updates_are_seen():
