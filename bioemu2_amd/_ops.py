@@ -64,8 +64,8 @@ def mask_u8(mask: Tensor) -> Tensor:
 
 def _plain_call(args: tuple) -> bool:
     """True where the dispatcher has nothing to do for an op but to run its body: no gradients, no compiler, tracer,
-    functorch transform, forward-mode level or mode looking on, and plain tensors only."""
-    if torch.compiler.is_compiling() or torch.is_grad_enabled():
+    functorch transform, forward-mode level, mode or profiler looking on, and plain tensors only."""
+    if torch.compiler.is_compiling() or torch.is_grad_enabled() or torch.autograd._profiler_enabled():
         return False
     for a in args:
         if isinstance(a, Tensor) and (type(a) is not Tensor or not a.is_cuda):
@@ -77,15 +77,23 @@ def _plain_call(args: tuple) -> bool:
 
 class _Op:
     """A ``torch.library`` custom op (``torch.ops.bioemu_mi355x.<name>``, HIP only) whose body an inference program's
-    calls reach directly: the dispatcher's Python layers cost as much host time as the op's own launches."""
+    calls reach directly: the dispatcher's Python layers cost as much host time as the op's own launches.  Not where a
+    program has put a kernel or an autocast rule of its own over the op (``torch.library.register_kernel``,
+    ``register_autocast``) or disabled this one; what it puts there below that level (``Library.impl``) is reached
+    through ``torch.ops``."""
 
     def __init__(self, name: str, body):
         self.body = body
         self.op = torch.library.custom_op(f"bioemu_mi355x::{name}", body, mutates_args=(), device_types="cuda")
         self.register_fake = self.op.register_fake
+        self._def, self._kernel = self.op, self.op._backend_fns["cuda"]
+
+    def _own(self) -> bool:
+        d = self._def
+        return d._backend_fns["cuda"] is self._kernel and not d._disabled_kernel and d._autocast_cuda_dtype is None
 
     def __call__(self, *args):
-        return self.body(*args) if _plain_call(args) else self.op(*args)
+        return self.body(*args) if _plain_call(args) and self._own() else self.op(*args)
 
 
 def _op(name: str):

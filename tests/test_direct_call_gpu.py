@@ -67,6 +67,30 @@ def test_onlookers_see_the_op(gpu_device, counted):
     assert len(counted) == 3
 
 
+def test_profilers_see_the_op(gpu_device, counted):
+    m, x, mask = _case(gpu_device)
+    with torch.no_grad(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        m(x, mask)
+    assert len(counted) == 1
+    assert any("bioemu_mi355x::trimul" in e.key for e in prof.key_averages())
+
+
+def test_kernels_put_over_the_op_are_called(gpu_device):
+    def body(x: torch.Tensor) -> torch.Tensor:
+        return x + 1
+
+    op = _ops._Op("test_direct_call_override", body)
+    x = torch.zeros(3, device=gpu_device)
+    with torch.no_grad():
+        assert op(x)[0] == 1
+        torch.library.register_kernel("bioemu_mi355x::test_direct_call_override", "cuda", lambda x: x + 2)
+        assert op(x)[0] == 2
+        op = _ops._Op("test_direct_call_autocast", body)
+        torch.library.register_autocast("bioemu_mi355x::test_direct_call_autocast", "cuda", torch.float16)
+        with torch.autocast("cuda"):
+            assert op(x).dtype == torch.float16
+
+
 def test_uint8_masks_mean_nonzero(gpu_device):
     m, x, mask = _case(gpu_device)
     with torch.no_grad():
