@@ -750,15 +750,24 @@ static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, Trans
   return c.off;
 }
 
+// Rows of 64 or 128 channels in one kernel, from the row count on at which its workgroups (256 rows, every hidden chunk
+// in order) are many enough.  Below it the three separate products deal columns and k-steps to workgroups too.  Both
+// times in us, one kernel / separate: 128 -> 256 channels, 200 rows 34 / 14, 4096 rows 36 / 21, 16000 rows 39 / 35,
+// 64000 rows 55 / 83; 128 -> 512, 1600 rows 58 / 24, 16000 rows 61 / 49; 64 -> 256, 8000 rows 24 / 19, 12000 rows
+// 25 / 24, 16000 rows 25 / 28.  (590k rows 128 -> 256: 0.44 ms in one kernel.)  The two differ in the order of their
+// sums, so a row's last bits depend on the number of rows of its call; they never depend on the other rows' values.
+static bool transition_f32_fused(int64_t M, int64_t Dc, int64_t hidden, int64_t out_dim) {
+  return out_dim == Dc && hidden <= kTransitionMaxHidden &&
+         ((Dc == 128 && M >= kTransitionFusedRows128) || (Dc == 64 && M >= kTransitionFusedRows64));
+}
+
 static int transition_f32_res(const float* x, const float* res, const float* norm_w, const float* norm_b,
                               const float* fc1_w, const float* fc2_w, const float* fc3_w, float* out, void* workspace,
                               int64_t M, int64_t Dc, int64_t hidden, int64_t out_dim, int use_norm, int residual,
                               hipStream_t stream) {
   TransitionF32Buffers buf;
   transition_f32_layout(M, Dc, hidden, &buf, static_cast<char*>(workspace));
-  // Rows of 64 or 128 channels: one kernel at every row count (590k rows 128 -> 256: 0.46 ms against 2.1 ms for the
-  // three fp32-MFMA kernels it replaced; 200 rows: one launch and 8 chunks of weights instead of three products).
-  if ((Dc == 128 || Dc == 64) && out_dim == Dc && hidden <= kTransitionMaxHidden)
+  if (transition_f32_fused(M, Dc, hidden, out_dim))
     return split_transition_rows(x, residual ? res : nullptr, use_norm ? norm_w : nullptr, norm_b, fc1_w, fc2_w, fc3_w,
                                  buf.w12, buf.scales, out, M, (int)Dc, (int)hidden, stream, "f32_transition_rows");
   const int64_t out0 = out_dim < kTransitionOutRows ? out_dim : kTransitionOutRows;

@@ -118,6 +118,7 @@ __device__ __forceinline__ void stage_floats(float* dst, const float* __restrict
 // Fused transition over rows of C = 64 or 128 channels (split_transition.hip): hidden % 32 == 0, at most
 // kTransitionMaxHidden.  `W` holds split_transition_weight_elems f16, `scales` split_transition_scales floats.
 constexpr int kTransitionMaxHidden = 2048;
+constexpr int64_t kTransitionFusedRows128 = 18432, kTransitionFusedRows64 = 12288;   // fewest rows worth it
 inline size_t split_transition_scales(int64_t C, int64_t hidden) { return (size_t)(hidden / 8 + C / 32 + 2 * hidden); }
 size_t split_transition_weight_elems(int64_t C, int64_t hidden);
 int split_transition_rows(const float* x, const float* res, const float* norm_w, const float* norm_b,

@@ -13,6 +13,8 @@
 // |silu(a) b| <= |a| |b| (SplitMat::norm).  A LayerNorm's affine is folded into fc1
 // and fc2, so the rows are only centred and divided by their deviation.
 //
+// Few rows take the separate products of split_gemm.hip instead (the rule and both times: fp32.hip).
+//
 // Bound by the matrix cores and the gating VALU work of the same waves (two waves per
 // SIMD): 590k rows, 128 -> 256, 0.44 ms (262 TFLOP/s of fp32 products, 787 of f16)
 // against 2.1 ms for LayerNorm, SwiGLU and output products on fp32 MFMA through

@@ -1,0 +1,64 @@
+"""fp32 row kernels on few rows and on many: which form runs, both sides of each rule's line, and what both give.
+
+Bound: TOL of test_split_gpu.py (float64 reference).
+"""
+
+import pytest
+import torch
+
+from bioemu2_amd.timing import KernelTimer
+from bioemu2_amd.transition import Transition
+from tests._helpers import randomize_params, rel_l2
+from tests.test_split_gpu import TOL, _params, _transition
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(module, *args, **kwargs):
+    """The module's output and the names of the kernels that made it."""
+    with torch.no_grad(), KernelTimer() as t:
+        out = module(*args, **kwargs)
+    return out, set(t.results())
+
+
+@pytest.mark.parametrize(
+    "dim,hidden,use_norm,rows",
+    [
+        (128, 256, True, 200),
+        (128, 256, True, 18431),      # the last row count of the separate products
+        (128, 256, True, 18432),      # one kernel: 72 whole workgroups
+        (128, 32, True, 18433),       # ... one row more, one hidden chunk
+        (128, 512, False, 18687),     # ... a workgroup less one row
+        (128, 2048, True, 18500),     # ... its widest hidden dimension
+        (64, 128, False, 12287),
+        (64, 128, False, 12289),
+        (64, 256, True, 12543),
+    ],
+)
+def test_transition_forms(gpu_device, dim, hidden, use_norm, rows):
+    torch.manual_seed(0)
+    m = randomize_params(Transition(dim, hidden, use_norm=use_norm), 3)
+    x = torch.randn(rows, dim)
+    want = _transition(x.double(), _params(m), use_norm)
+    got, names = _run(m.to(gpu_device), x.to(gpu_device))
+    assert rel_l2(got.cpu(), want) <= TOL
+    assert ("f32_transition_rows" in names) == (rows >= (18432 if dim == 128 else 12288))
+
+
+def test_fused_transition_ranges(gpu_device):
+    """Row magnitudes from 1e-12 to 1e12 in one call, checked row by row; other rows' values leave a row's bits alone."""
+    torch.manual_seed(1)
+    rows = 18500
+    m = randomize_params(Transition(128, 256, use_norm=False), 3)
+    x = torch.randn(rows, 128) * torch.logspace(-12, 12, rows)[:, None]
+    x[5] = 0.0
+    want = _transition(x.double(), _params(m), False)
+    got, names = _run(m.to(gpu_device), x.to(gpu_device))
+    assert "f32_transition_rows" in names and torch.equal(got[5].cpu(), torch.zeros(128))
+    err = (got.cpu().double() - want).norm(dim=1) / want.norm(dim=1).clamp_min(1e-300)
+    err[5] = 0.0
+    assert float(err.max()) <= TOL
+    y = x.clone()
+    y[9000:] = torch.randn(rows - 9000, 128)
+    with torch.no_grad():
+        assert torch.equal(m(y.to(gpu_device))[:9000], got[:9000])
