@@ -612,8 +612,8 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
 
 // Rows of 128 channels, held as operand fragments by the wave that reads them (kLn: normalised, the affine folded
 // into W and wbias): 4 waves x 32 rows, the weights walked in blocks of 32 output channels (16 KB of fragments)
-// through double-buffered LDS.  For K = 128 this replaces the separate fragment pass and the short k-loop of the
-// tiled kernel.
+// through double-buffered LDS, `per` of them by a workgroup.  For K = 128 this replaces the separate fragment pass
+// and the short k-loop of the tiled kernel.
 constexpr int kR128Block = 8 * kFrag;   // f16 elements of one 32-channel block
 constexpr int kR128MaxN = 512;          // output channels with a bias
 
@@ -621,7 +621,7 @@ template <int kEpi, bool kLn>
 __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __restrict__ x, const f16* __restrict__ W,
                                                                  const float* __restrict__ winv,
                                                                  const float* __restrict__ wbias, SplitGemmEpi e,
-                                                                 long long M, int nblocks) {
+                                                                 long long M, int nblocks, int per) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][kR128Block];
   __shared__ __attribute__((aligned(16))) float sbias[kLn ? kR128MaxN : 4];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
@@ -633,7 +633,8 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
       copy1k_to_lds(rw, &smem[cb & 1][c * kFragHalf], lane * 16, (unsigned)(cb * kR128Block * 2 + c * 1024));
     }
   };
-  stage(0);
+  const int first = blockIdx.y * per, last = min(first + per, nblocks);   // first < nblocks
+  stage(first);
   if (kLn) stage_floats(sbias, wbias, nblocks * 32, nblocks * 32);
   const long long m = ((long long)blockIdx.x * 4 + wave) * 32 + n;
   const bool valid = m < M;
@@ -645,10 +646,10 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
     xinv = kLn ? normalized_row_half<128>(v, xf) : split_row_half<128>(v, xf);
   }
 #pragma unroll 1
-  for (int cb = 0; cb < nblocks; ++cb) {
+  for (int cb = first; cb < last; ++cb) {
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies of block cb landed
     __syncthreads();                       // ... and everyone's; the other stage is free again
-    if (cb + 1 < nblocks) stage(cb + 1);
+    if (cb + 1 < last) stage(cb + 1);
     f32x16 acc = zero16();
     mfma_block<8>(smem[cb & 1], xf, lane, acc);
     const float sc = xinv * winv[cb];
@@ -672,11 +673,16 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
 
 int split_gemm_r128(int epi, const float* x, const f16* W, const float* winv, const float* wbias,
                     const SplitGemmEpi& e, long long M, int N, hipStream_t stream, const char* name) {
-  const dim3 grid((unsigned)((M + 127) / 128));
+  // As many parts of the columns as fill three workgroups per CU (its resident number): the parts read the same rows,
+  // from L2, and compute the same bits.  Atom attention (us, with one part / this many): 384 rows 62 / 32, 6144 rows
+  // 69 / 46, 12288 rows 86 / 67, 28800 rows 96 / 85, 49152 rows 145 / 138; one workgroup per CU: 32, 47, 71, 96, 145.
+  const long long wgs = (M + 127) / 128, nblocks = N / 32, resident = 3LL * compute_units();
+  const long long parts = std::min(nblocks, std::max(1LL, resident / wgs)), per = (nblocks + parts - 1) / parts;
+  const dim3 grid((unsigned)wgs, (unsigned)((nblocks + per - 1) / per));
   if (wbias && N > kR128MaxN) return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: %d output channels", name, N);
   KernelTimerScope timed(name, stream);
 #define BIOEMU_R128(E, L) \
-  hipLaunchKernelGGL((split_gemm_r128_kernel<E, L>), grid, dim3(256), 0, stream, x, W, winv, wbias, e, M, N / 32)
+  hipLaunchKernelGGL((split_gemm_r128_kernel<E, L>), grid, dim3(256), 0, stream, x, W, winv, wbias, e, M, N / 32, (int)per)
   if (epi == kSplitStore && !wbias)
     BIOEMU_R128(kSplitStore, false);
   else if (epi == kSplitQkvg && !wbias)
