@@ -854,8 +854,10 @@ extern "C" int bioemu_pair_cond_proj_fwd_f32(const float* z_trunk, const float* 
     return set_error(BIOEMU_ERR_INVALID_ARG, "pair_cond_f32: tensors must be 16-byte aligned");
   if (workspace_bytes < bioemu_pair_cond_f32_workspace_bytes(P, token_z, c_rel))
     return set_error(BIOEMU_ERR_WORKSPACE, "pair_cond_f32: workspace too small");
-  if (token_z == 128 && c_rel == 128 && a_z == 128 && aligned16(z_trunk) && aligned16(rel)) {
-    // the denoiser's widths: one pass over both inputs
+  const size_t row_bytes = (size_t)P * 128 * sizeof(float);
+  if (token_z == 128 && c_rel == 128 && a_z == 128 && aligned16(z_trunk) && aligned16(rel) &&
+      !overlap(out, row_bytes, z_trunk, row_bytes) && !overlap(out, row_bytes, rel, row_bytes)) {
+    // the denoiser's widths: one pass over both inputs (which several workgroups read while others write out)
     Carve c{static_cast<char*>(workspace)};
     f16* wf = c.frags(128, 256);
     float *winv = c.floats(4), *wbias = c.floats(128);

@@ -66,6 +66,12 @@ inline int compute_units() {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Whether [a, a + na) and [b, b + nb) share a byte.
+inline bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return x < y + nb && y < x + na;
+}
+
 // Batched bf16 "NT" GEMM: C[z][i][j] = sum_k A[z][i][k] * B[z][j][k] for
 // z < batch over planes of n rows with stride bgemm_ld(n) (zero-filled past n), bf16 output.
 constexpr int kGemmTile = 256;

@@ -15,23 +15,25 @@
 namespace bioemu {
 namespace {
 
-constexpr int kCatWaves = 8;
+constexpr int kCatWaves = 8;   // with all four column blocks in LDS
 constexpr int kCatWeights = 4 * 16 * kFrag;               // f16: [4 column blocks][16 k-steps]
 constexpr int kCatSmem = kCatWeights * (int)sizeof(f16) + 128 * 4;  // 128 KB and the biases
 
 __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
     const float* __restrict__ x1, const float* __restrict__ x2, const f16* __restrict__ W,
-    const float* __restrict__ winv, const float* __restrict__ wbias, float* __restrict__ out, long long P, int tiles) {
+    const float* __restrict__ winv, const float* __restrict__ wbias, float* __restrict__ out, long long P, int tiles,
+    int per) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f16* smem = reinterpret_cast<f16*>(smem_raw);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
-  float* sbias = reinterpret_cast<float*>(smem + kCatWeights);
-  stage_floats(sbias, wbias, 128, 128);
-  stage_fragments(W, smem, kCatWeights / kFragHalf, kCatWaves, wave, lane);
+  const int waves = blockDim.x / 64, cb0 = blockIdx.y * per;   // column blocks cb0 .. cb0 + per - 1
+  float* sbias = reinterpret_cast<float*>(smem + per * 16 * kFrag);
+  stage_floats(sbias, wbias + cb0 * 32, per * 32, per * 32);
+  stage_fragments(W + cb0 * 16 * kFrag, smem, per * 32, waves, wave, lane);
   // half of the next tile's rows is requested as soon as this tile's are fragments, ahead of its products and stores
   float a[64];
   auto row_of = [&](int tile) { return (size_t)std::min((long long)tile * 32 + n, P - 1) * 128; };
-  const int first = blockIdx.x * kCatWaves + wave, step = gridDim.x * kCatWaves;
+  const int first = blockIdx.x * waves + wave, step = gridDim.x * waves;
   if (first < tiles) load_row_half<128>(x1 + row_of(first), h, a);
 #pragma unroll 1
   for (int tile = first; tile < tiles; tile += step) {
@@ -61,14 +63,14 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
     if (tile + step < tiles) load_row_half<128>(x1 + row_of(tile + step), h, a);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
-    for (int cb = 0; cb < 4; ++cb) {
+    for (int cb = 0; cb < per; ++cb) {
       const f16* w = smem + cb * 16 * kFrag;
       f32x16 acc = zero16();
       mfma_block<16>(w, xf, lane, acc);
-      const float sc = winv[cb] * (1.0f / kNormScale);
+      const float sc = winv[cb0 + cb] * (1.0f / kNormScale);
       if (valid) {
         const int c0 = cb * 32 + 16 * h;
-        float* d = out + (size_t)m * 128 + c0;
+        float* d = out + (size_t)m * 128 + cb0 * 32 + c0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           f32x4 v = *reinterpret_cast<const f32x4*>(sbias + c0 + 4 * q);
@@ -134,10 +136,16 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
                                             hipFuncAttributeMaxDynamicSharedMemorySize, kCatSmem);
   if (rc != hipSuccess) return set_error(BIOEMU_ERR_LAUNCH, "%s: %s", name, hipGetErrorString(rc));
   const int tiles = (int)((P + 31) / 32);
-  const int grid = std::min((tiles + kCatWaves - 1) / kCatWaves, 256);
+  // Few tiles: a column block (and 32 KB of weights) a workgroup, four waves of which two workgroups share a CU, as
+  // long as that is one round of workgroups.  us of the projection and two transitions, all columns / this: 1600 rows
+  // 53 / 46, 8100 rows 78 / 72, 16384 rows 95 / 95; past one round, 32400 rows 113 / 124.  The same bits.
+  const int cus = compute_units();
+  const bool few = tiles <= 2 * cus;
+  const int waves = few ? 4 : kCatWaves, per = few ? 1 : 4;
+  const int grid = std::min((tiles + waves - 1) / waves, cus);
   KernelTimerScope timed(name, stream);
-  hipLaunchKernelGGL(cat_proj_f32_kernel, dim3((unsigned)grid), dim3(64 * kCatWaves), kCatSmem, stream, x1, x2, W, winv,
-                     wbias, out, P, tiles);
+  hipLaunchKernelGGL(cat_proj_f32_kernel, dim3((unsigned)grid, 4 / per), dim3(64 * waves),
+                     per * (16 * kFrag * (int)sizeof(f16) + 32 * 4), stream, x1, x2, W, winv, wbias, out, P, tiles, per);
   return check_launch(name);
 }
 

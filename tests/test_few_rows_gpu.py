@@ -5,8 +5,11 @@ Bound: TOL of test_split_gpu.py (float64 reference).
 
 import pytest
 import torch
+import torch.nn.functional as F
 
+from bioemu2_amd import _ops
 from bioemu2_amd.attention_pair_bias import AttentionPairBiasSlidingWindow
+from bioemu2_amd.glue import PairwiseConditioning
 from bioemu2_amd.timing import KernelTimer
 from bioemu2_amd.transition import Transition
 from tests._helpers import randomize_params, rel_l2
@@ -79,3 +82,37 @@ def test_sliding_window_copies_do_not_depend_on_their_number(gpu_device, norm):
         for copies in (2, 17, 37, 260):
             got = m(s.repeat(copies, 1, 1), z, mask, multiplicity=copies).view(copies, nw, 32, 128)
             assert torch.equal(got, alone.expand_as(got))
+
+
+def test_pair_conditioning_rows_do_not_depend_on_their_number(gpu_device):
+    """A column block a workgroup up to 512 tiles of 32 rows, all four beyond; ragged last tiles of both."""
+    torch.manual_seed(3)
+    m = randomize_params(PairwiseConditioning(128, 128), 5).to(gpu_device).eval()
+    p = m.prepared_params_f32()
+    z, rel = torch.randn(16385, 128, device=gpu_device), torch.randn(16385, 128, device=gpu_device)
+
+    def proj(rows):
+        out = torch.empty(rows, 128, device=gpu_device)
+        return _ops.launch_pair_cond_proj_f32(z[:rows], rel[:rows], *p, out)
+
+    want = proj(16385)
+    x = F.layer_norm(torch.cat([z, rel], -1).double(), (256,), p[0].double(), p[1].double(), 1e-5) @ p[2].double().T
+    assert rel_l2(want.cpu(), x.cpu()) <= TOL
+    for rows in (1, 31, 33, 129, 16384):
+        assert torch.equal(proj(rows), want[:rows])
+
+
+@pytest.mark.parametrize("rows", [70, 17000])
+@pytest.mark.parametrize("which", [0, 1])
+def test_pair_conditioning_in_place(gpu_device, which, rows):
+    """The output over one of the inputs, and over rows shifted by one."""
+    torch.manual_seed(4)
+    m = randomize_params(PairwiseConditioning(128, 128), 6).to(gpu_device).eval()
+    p = m.prepared_params_f32()
+    base = [torch.randn(rows + 1, 128, device=gpu_device) for _ in range(2)]
+    want = _ops.launch_pair_cond_proj_f32(base[0][:rows], base[1][:rows], *p, torch.empty(rows, 128, device=gpu_device))
+    for shift in (0, 1):
+        x = [t.clone() for t in base]
+        out = x[which][shift : shift + rows]
+        _ops.launch_pair_cond_proj_f32(x[0][:rows], x[1][:rows], *p, out)
+        assert rel_l2(out.cpu(), want.cpu()) <= TOL
