@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
                                                                const float* __restrict__ wnorm,
                                                                const float* __restrict__ wbias, f16* __restrict__ hi,
                                                                f16* __restrict__ lo, int N, int outgoing,
-                                                               unsigned tiles) {
+                                                               unsigned tiles, int per) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][2 * kWBlock];   // p | g block, double-buffered: 64 KB
   __shared__ float sbias[4 * D];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
@@ -50,7 +50,8 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
       copy1k_to_lds(rw, &smem[cb & 1][c * kFragHalf], lane * 16, (unsigned)(cb * 2 * kWBlock * 2 + c * 1024));
     }
   };
-  stage(0);
+  const int first = blockIdx.y * per, last = first + per;   // this workgroup's column blocks
+  stage(first);
   stage_floats(sbias, wbias, 4 * D, 4 * D);
   // tile (b, i, kb): 32 pairs k = 32 kb .. of line i; a wave past the last tile works on tile 0 and stores nothing
   const unsigned tile = blockIdx.x * 4 + wave;
@@ -70,10 +71,10 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
   const unsigned keep = (unsigned)kept >> (16 * h);   // bit u: pair 16 h + u
   const size_t plane = (size_t)N * ld;
 #pragma unroll 1
-  for (int cb = 0; cb < 8; ++cb) {
+  for (int cb = first; cb < last; ++cb) {
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies of block cb landed
     __syncthreads();                       // ... and everyone's; the other stage is free again
-    if (cb + 1 < 8) stage(cb + 1);
+    if (cb + 1 < last) stage(cb + 1);
     // pair slots are the MFMA rows (in perm32 order), channels its columns: lane (n, h) ends with the 16
     // consecutive pairs 16 h + u of channel perm32(n)
     const f16* st = smem[cb & 1];
@@ -199,7 +200,8 @@ __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const f16* __re
 }
 
 // ---------------------------------------------------------------------------
-// Output: a wave per 32 pairs (i, j0 .. j0 + 31) of a line.
+// Output: a wave per 32 pairs (i, j0 .. j0 + 31) of a line, or (kFew) a workgroup of four waves, each of which
+// normalises the pairs and takes one of the four column blocks.
 // ---------------------------------------------------------------------------
 constexpr int kOutWaves = 8;
 
@@ -211,21 +213,30 @@ __device__ __forceinline__ float gated(float p, float g) {
 constexpr int kOutWeights = 2 * 4 * kWBlock;                                  // f16: p_out | g_out
 constexpr int kOutSmem = kOutWeights * (int)sizeof(f16) + 2 * D * 4;          // 128 KB and the biases
 
-__global__ __launch_bounds__(64 * kOutWaves, 2) void trimul_out_kernel(const float* x, const float* __restrict__ o,
-                                                                       const f16* __restrict__ W,
-                                                                       const float* __restrict__ winv,
-                                                                       const float* __restrict__ wbias, float* out,
-                                                                       int N, int residual, unsigned tiles) {
+template <bool kFew>
+__global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void trimul_out_kernel(
+    const float* x, const float* __restrict__ o, const f16* __restrict__ W, const float* __restrict__ winv,
+    const float* __restrict__ wbias, float* out, int N, int residual, unsigned tiles) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f16* smem = reinterpret_cast<f16*>(smem_raw);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   float* sbias = reinterpret_cast<float*>(smem + kOutWeights);
   stage_floats(sbias, wbias, 2 * D, 2 * D);
-  stage_fragments(W, smem, kOutWeights / kFragHalf, kOutWaves, wave, lane);
+  if (kFew) {   // this wave's two weight blocks; waited for below the rows' loads
+    const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, kOutWeights * 2);
+#pragma unroll
+    for (int c = 0; c < 32; ++c) {
+      const int at = (c < 16 ? wave : 4 + wave) * 16 + c % 16;
+      copy1k_to_lds(rw, smem + at * kFragHalf, lane * 16, (unsigned)at * 1024);
+    }
+  } else {
+    stage_fragments(W, smem, kOutWeights / kFragHalf, kOutWaves, wave, lane);
+  }
   const int ld = plane_ld(N);
   const size_t plane = (size_t)N * ld;
 #pragma unroll 1
-  for (unsigned tile = blockIdx.x * kOutWaves + wave; tile < tiles; tile += gridDim.x * kOutWaves) {
+  for (unsigned tile = kFew ? blockIdx.x : blockIdx.x * kOutWaves + wave; tile < tiles;
+       tile += gridDim.x * (kFew ? 1 : kOutWaves)) {
     const TileIdx t = split_tile(tile, (unsigned)(ld / 32), (unsigned)N);
     const int j = t.col * 32 + n;
     const bool valid = j < N;
@@ -245,8 +256,12 @@ __global__ __launch_bounds__(64 * kOutWaves, 2) void trimul_out_kernel(const flo
       load_row_half<D>(x + m * D, h, v);
       normalized_row_half<D>(v, xf);
     }
+    if (kFew) {   // every wave holds the rows before one overwrites them
+      __builtin_amdgcn_s_waitcnt(0x0f70);
+      __syncthreads();
+    }
 #pragma unroll 1
-    for (int cb = 0; cb < 4; ++cb) {
+    for (int cb = kFew ? wave : 0; cb < (kFew ? wave + 1 : 4); ++cb) {
       const f16* w = smem + cb * kWBlock;
       f32x16 p = zero16(), g = zero16();
       mfma_block2<8>(w, w + 4 * kWBlock, of, xf, lane, p, g);
@@ -325,9 +340,14 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
   if (rc) return rc;
   const unsigned tiles = (unsigned)(B * N * (plane_ld((int)N) / 32));
   {
+    // As many parts of the eight column blocks as make one round of two workgroups per CU.  The call, all blocks / these
+    // parts (us): N = 40 46 / 29, N = 64 50 / 32, N = 100 66 / 52, N = 160 70 / 64; two rounds: 29, 32, 55, 68.
+    const unsigned wgs = (tiles + 3) / 4, resident = 2u * compute_units();
+    unsigned parts = 1;
+    while (parts < 8 && 2 * parts * wgs <= resident) parts *= 2;
     KernelTimerScope timed("f32_trimul_proj", stream);
-    hipLaunchKernelGGL(trimul_planes_kernel, dim3((tiles + 3) / 4), dim3(256), 0, stream, x, mask, win, inv_in,
-                       norm_in, bias_in, hi, lo, (int)N, outgoing, tiles);
+    hipLaunchKernelGGL(trimul_planes_kernel, dim3(wgs, parts), dim3(256), 0, stream, x, mask, win, inv_in, norm_in,
+                       bias_in, hi, lo, (int)N, outgoing, tiles, 8 / (int)parts);
   }
   if ((rc = check_launch("f32_trimul_proj"))) return rc;
   {
@@ -341,12 +361,17 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
   }
   if ((rc = check_launch("f32_trimul_contract"))) return rc;
   {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(trimul_out_kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, kOutSmem);
+    const unsigned cus = compute_units();
+    // Up to two rounds of a tile a workgroup (the call, us, a tile a wave / a workgroup: N = 40 39 / 29, N = 64 43 / 32,
+    // N = 80 48 / 38, N = 128, 512 tiles, 55 / 54, N = 160, 800 tiles, 64 / 81).
+    const bool few = tiles <= 2 * cus;
+    const auto kernel = few ? trimul_out_kernel<true> : trimul_out_kernel<false>;
+    const hipError_t e =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kOutSmem);
     if (e != hipSuccess) return set_error(BIOEMU_ERR_LAUNCH, "f32_trimul_out: %s", hipGetErrorString(e));
-    const unsigned grid = std::min((tiles + kOutWaves - 1) / kOutWaves, 256u);
+    const unsigned grid = few ? tiles : std::min((tiles + kOutWaves - 1) / kOutWaves, cus);
     KernelTimerScope timed("f32_trimul_out", stream);
-    hipLaunchKernelGGL(trimul_out_kernel, dim3(grid), dim3(64 * kOutWaves), kOutSmem, stream, x, o, wout, inv_out,
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * (few ? 4 : kOutWaves)), kOutSmem, stream, x, o, wout, inv_out,
                        bias_out, out, (int)N, residual, tiles);
   }
   return check_launch("f32_trimul_out");

@@ -12,6 +12,7 @@ from bioemu2_amd.attention_pair_bias import AttentionPairBiasSlidingWindow
 from bioemu2_amd.glue import PairwiseConditioning
 from bioemu2_amd.timing import KernelTimer
 from bioemu2_amd.transition import Transition
+from bioemu2_amd.triangle_multiplication import TriangleMultiplicationHip
 from tests._helpers import randomize_params, rel_l2
 from tests.test_split_gpu import TOL, _params, _transition
 
@@ -116,3 +117,25 @@ def test_pair_conditioning_in_place(gpu_device, which, rows):
         out = x[which][shift : shift + rows]
         _ops.launch_pair_cond_proj_f32(x[0][:rows], x[1][:rows], *p, out)
         assert rel_l2(out.cpu(), want.cpu()) <= TOL
+
+
+@pytest.mark.parametrize("mode", ["outgoing", "incoming"])
+@pytest.mark.parametrize("n,few,many", [(2, 1, 257), (33, 7, 8), (40, 1, 13)])
+def test_triangle_multiplication_forms(gpu_device, mode, n, few, many):
+    """Line tiles (32 pairs) on both sides of the 512 up to which a workgroup takes one: the same bits, out of place and
+    over the input."""
+    torch.manual_seed(5)
+    m = randomize_params(TriangleMultiplicationHip(128, mode), 7).to(gpu_device).eval()
+    p = m.prepared_params_f32()
+    x = torch.randn(many, n, n, 128, device=gpu_device)
+    mask = (torch.rand(many, n, n, device=gpu_device) < 0.8).to(torch.uint8)
+
+    def run(b, out, residual):
+        return _ops.launch_trimul_f32(x[:b] if out is None else out, mask[:b], *p,
+                                      torch.empty_like(x[:b]) if out is None else out, mode == "outgoing",
+                                      residual=residual)
+
+    for residual in (False, True):
+        assert torch.equal(run(few, None, residual), run(many, None, residual)[:few])
+    for b in (few, many):
+        assert torch.equal(run(b, x[:b].clone(), True), run(b, None, True))
