@@ -527,7 +527,7 @@ size_t attn_f32_layout(long long rows, int c_s, int heads, int64_t seq_len, long
   b->sp.a = c.frags(rows, c_s);
   b->sp.ainv = c.floats((size_t)rows);
   b->sp.w = c.frags(5 * (int64_t)c_s, c_s);
-  b->sp.winv = c.floats((size_t)5 * c_s / 32 + 1);
+  b->sp.winv = c.floats((size_t)5 * c_s);
   b->q = c.floats((size_t)rows * c_s);
   b->k = c.floats((size_t)rows * c_s);
   b->v = c.floats((size_t)rows * c_s);
@@ -542,7 +542,7 @@ size_t attn_f32_layout(long long rows, int c_s, int heads, int64_t seq_len, long
     b->words = c.bytes<uint32_t>(blocks * 4);
   }
   b->wz = c.frags(heads, 128);
-  b->wzinv = c.floats((size_t)heads / 32 + 1);
+  b->wzinv = c.floats((size_t)round_up(heads, 32));
   b->wzbias = c.floats((size_t)heads);
   b->wbias = c.floats((size_t)4 * c_s);
   return c.off;
@@ -568,8 +568,8 @@ int attn_f32_projections(const float* s, const float* norm_s_w, const float* nor
   const bool bias_split = pb.c_z == 128 && pb.H <= 64 && pb.P < (1LL << 31) && aligned16(pb.w);
   SplitMats mats{};
   mats.m[0] = split_gemm_weight(w_qkv, buf.sp.w, buf.sp.winv, nullptr, 3 * (int64_t)c_s, c_s);
-  mats.m[1] = split_gemm_weight(w_g, buf.sp.w + 3 * per, buf.sp.winv + 3 * nb, nullptr, c_s, c_s);
-  mats.m[2] = split_gemm_weight(w_o, buf.sp.w + 4 * per, buf.sp.winv + 4 * nb, nullptr, c_s, c_s);
+  mats.m[1] = split_gemm_weight(w_g, buf.sp.w + 3 * per, buf.sp.winv + 3 * c_s, nullptr, c_s, c_s);
+  mats.m[2] = split_gemm_weight(w_o, buf.sp.w + 4 * per, buf.sp.winv + 4 * c_s, nullptr, c_s, c_s);
   if (bias_split)
     mats.m[3] = with_fold(split_gemm_weight(pb.w, buf.wz, buf.wzinv, nullptr, pb.H, 128), pb.g, pb.b, buf.wzbias);
   const bool r128 = c_s == 128;
@@ -607,7 +607,7 @@ int attn_f32_out(const float* go, const float* res, float* out, AttnF32Buffers& 
                  hipStream_t stream, const char* name) {
   const int nb = c_s / 32;
   const f16* w = buf.sp.w + (size_t)4 * nb * split_ksteps(c_s) * kFrag;
-  const float* winv = buf.sp.winv + 4 * nb;
+  const float* winv = buf.sp.winv + 4 * c_s;
   SplitGemmEpi e;
   e.out = out;
   e.res = res;
@@ -740,12 +740,12 @@ static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, Trans
   b->xinv = c.floats((size_t)M);
   b->xnorm = c.floats((size_t)M);
   b->w12 = c.frags(3 * hidden, Dc);   // fc1 and fc2; with fc3 in the fused kernel's chunks
-  b->w12inv = c.floats((size_t)hidden / 16);
-  b->w12norm = c.floats((size_t)hidden / 16);
+  b->w12inv = c.floats((size_t)2 * hidden);
+  b->w12norm = c.floats((size_t)2 * hidden);
   b->h = c.frags(M, hidden);
   b->hinv = c.floats((size_t)M);
   b->w3 = c.frags(kTransitionOutRows, hidden);
-  b->w3inv = c.floats((size_t)kTransitionOutRows / 32);
+  b->w3inv = c.floats((size_t)kTransitionOutRows);
   b->scales = c.floats(split_transition_scales(Dc, hidden));
   return c.off;
 }
@@ -860,7 +860,7 @@ extern "C" int bioemu_pair_cond_proj_fwd_f32(const float* z_trunk, const float* 
     // the denoiser's widths: one pass over both inputs (which several workgroups read while others write out)
     Carve c{static_cast<char*>(workspace)};
     f16* wf = c.frags(128, 256);
-    float *winv = c.floats(4), *wbias = c.floats(128);
+    float *winv = c.floats(128), *wbias = c.floats(128);
     SplitMats mats{};
     mats.m[0] = with_fold(split_gemm_weight(w, wf, winv, nullptr, 128, 256), ln_w, ln_b, wbias);
     const int rs = split_weights(mats, 1, stream);

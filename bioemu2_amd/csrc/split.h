@@ -13,12 +13,12 @@
 // 3.5e-7, K = 1024 3.8e-7 vs 5.8e-7; K = 32 is a tie, so shorter products stay
 // off this path).
 //
-// Range: the scale brings the largest magnitude of a scaling group (one
-// activation row, one block of 32 weight rows) into [2^14, 2^15).  hi + lo is
-// then exact to 2^-23 relative for elements down to 2^-16 of that maximum and
-// to 2^-39 of the maximum below it (the f16 MFMA multiplies subnormals).  A
-// scale depends on its own row (or on the weights) alone, so a row's result
-// never depends on another row.
+// Range: the scale brings the largest magnitude of a row (of activations or of
+// weights) into [2^14, 2^15).  hi + lo is then exact to 2^-23 relative for
+// elements down to 2^-16 of that maximum and to 2^-39 of the maximum below it
+// (the f16 MFMA multiplies subnormals).  A scale depends on its own row (or on
+// the weights) alone, so a row's result never depends on another row, nor an
+// output channel's error on another channel's weights.
 //
 // Operand fragments: 32 rows x 16 k are 1 KB of hi followed by 1 KB of lo,
 // lane (n, h) = 8 consecutive values, row n, k = 8 h .. 8 h + 7.  Weight rows
@@ -145,8 +145,8 @@ __device__ __forceinline__ void copy1k_to_lds(__amdgpu_buffer_rsrc_t r, const f1
 // One weight matrix [rows][K] fp32 (K % 8 == 0; rows past the last are zeros) to fragments.  The block of
 // rows 32 rb .. and the k-step ks (16 columns, zero past K) go to
 //   dst + rb * rb_stride + (ks / kgrp) * kgrp_stride + (ks % kgrp) * kFrag
-// for ks < ksteps; inv[rb * inv_stride] = 1 / scale of the block and, unless null,
-// norm[rb * inv_stride] bounds |row . x| / |x| of its rows (their largest 2-norm).
+// for ks < ksteps; inv[32 rb * inv_stride + i] = 1 / scale of row 32 rb + i (rows past the
+// last too) and, unless null, norm[32 rb * inv_stride + i] bounds |row . x| / |x| (its 2-norm).
 //
 // With gamma, a preceding LayerNorm's affine is folded in, so that rows are only
 // centred and divided by their deviation: the fragments hold W diag(gamma),
@@ -193,8 +193,8 @@ inline size_t split_frag_bytes(int64_t rows, int64_t K) {
 inline SplitMat split_gemm_weight(const float* w, f16* dst, float* inv, float* norm, int64_t rows, int64_t K,
                                   int interleave = 1, int first = 0) {
   const int ks = split_ksteps(K);
-  return SplitMat{w, dst + (size_t)first * ks * kFrag, inv + first, norm ? norm + first : nullptr, (int)rows, (int)K,
-                  ks, ks, (long long)interleave * ks * kFrag, 0, interleave, nullptr, nullptr, nullptr};
+  return SplitMat{w, dst + (size_t)first * ks * kFrag, inv + 32 * first, norm ? norm + 32 * first : nullptr, (int)rows,
+                  (int)K, ks, ks, (long long)interleave * ks * kFrag, 0, interleave, nullptr, nullptr, nullptr};
 }
 // With a LayerNorm's affine folded in.
 inline SplitMat with_fold(SplitMat m, const float* gamma, const float* beta, float* bias) {

@@ -58,8 +58,7 @@ __device__ __forceinline__ void weight_chunk(const SplitMat& m, const float* row
 
 template <int kWaves, int kSteps>
 __device__ __forceinline__ void split_weight_block(const SplitMat& m, int rb) {
-  __shared__ float red[kWaves];
-  __shared__ float rown[kWaves][32], rowd[kWaves][32];
+  __shared__ float rowm[kWaves][32], rown[kWaves][32], rowd[kWaves][32];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const int r = rb * 32 + perm32(n), K = r < m.rows ? m.K : 0;   // rows past the matrix read as zeros
   const float* row = m.w + (size_t)r * m.K;
@@ -81,20 +80,20 @@ __device__ __forceinline__ void split_weight_block(const SplitMat& m, int rb) {
     weight_chunk(m, row, ks * 16 + 8 * h, K, c, dot);
     scan(c);
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+  amax = fmaxf(amax, __shfl_xor(amax, 32));
   ss += __shfl_xor(ss, 32);
   dot += __shfl_xor(dot, 32);
-  if (lane == 0) red[wave] = amax;
   if (lane < 32) {
+    rowm[wave][lane] = amax;
     rown[wave][lane] = ss;
     rowd[wave][lane] = dot;
   }
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) amax = fmaxf(amax, red[w]);
+  for (int w = 0; w < kWaves; ++w) amax = fmaxf(amax, rowm[w][n]);
   const float s = split_scale(amax);
-  if (threadIdx.x == 0) m.inv[(size_t)rb * m.inv_stride] = split_inv(s);
+  const size_t at = (size_t)rb * 32 * m.inv_stride + perm32(n);
+  if (threadIdx.x < 32) m.inv[at] = split_inv(s);
   if (wave == 0 && (m.norm || m.bias)) {
     float q = 0.f, d = 0.f;
 #pragma unroll
@@ -105,9 +104,7 @@ __device__ __forceinline__ void split_weight_block(const SplitMat& m, int rb) {
     if (m.bias && lane < 32 && r < m.rows) m.bias[r] = d;
     // |x| <= sqrt(K) for a normalised row
     q = m.gamma ? sqrtf(q * (float)m.K) + fabsf(d) : sqrtf(q);
-#pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) q = fmaxf(q, __shfl_xor(q, off));
-    if (m.norm && lane == 0) m.norm[(size_t)rb * m.inv_stride] = q;
+    if (m.norm && lane < 32) m.norm[at] = q;
   }
   auto put = [&](int ks, const float (&c)[8]) {
     f16x8 hi, lo;
@@ -393,12 +390,13 @@ __device__ __forceinline__ void epi_swiglu_quad(const SplitGemmEpi& e, long long
 }
 
 // |silu(a) b| <= |a| |b| <= (|x| |w1|) (|x| |w2|): the scale of a hidden row from
-// the row's norm and the largest weight-row norms (even entries fc1, odd fc2).
+// the row's norm and the largest weight-row norms (even blocks of 32 fc1, odd fc2).
 __device__ __forceinline__ float hidden_norm_product(const float* wn, int nblocks, int lane) {
   float q1 = 0.f, q2 = 0.f;
-  for (int i = lane; 2 * i < nblocks; i += 64) {
-    q1 = fmaxf(q1, wn[2 * i]);
-    q2 = fmaxf(q2, wn[2 * i + 1]);
+  for (int i = lane; i < nblocks * 16; i += 64) {
+    const float* p = wn + (i >> 5) * 64 + (i & 31);
+    q1 = fmaxf(q1, p[0]);
+    q2 = fmaxf(q2, p[32]);
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
@@ -477,7 +475,13 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
   }
   const int cb0 = nt * 4 + wn * 2;
   if (cb0 >= nblocks) return;
-  const float w0 = winv[cb0], w1 = cb0 + 1 < nblocks ? winv[cb0 + 1] : 0.f;
+  // the weight rows' scales, read before the first store
+  f32x4 w[2][4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      w[j][q] = *reinterpret_cast<const f32x4*>(winv + min(cb0 + j, nblocks - 1) * 32 + 16 * h + 4 * q);
   float wprod = 0.f;
   if (kEpi == kSplitSwiGLU) wprod = hidden_norm_product(e.wnorm, nblocks, lane);
 #pragma unroll
@@ -493,8 +497,8 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
         f32x4 a, b;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-          a[t] = acc[0][i][4 * q + t] * s * w0;
-          b[t] = acc[1][i][4 * q + t] * s * w1;
+          a[t] = acc[0][i][4 * q + t] * s * w[0][q][t];
+          b[t] = acc[1][i][4 * q + t] * s * w[1][q][t];
         }
         epi_swiglu_quad(e, m, cb0 * 16 + 16 * h + 4 * q, a, b, hs);
       }
@@ -509,7 +513,7 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
         for (int q = 0; q < 4; ++q) {
           f32x4 v;
 #pragma unroll
-          for (int t = 0; t < 4; ++t) v[t] = acc[j][i][4 * q + t] * s * (j ? w1 : w0);
+          for (int t = 0; t < 4; ++t) v[t] = acc[j][i][4 * q + t] * s * w[j][q][t];
           epi_quad<kEpi>(e, m, c0 + 4 * q, v, res[q]);
         }
       }
@@ -579,13 +583,15 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
   float wprod = 0.f;
   if (kEpi == kSplitSwiGLU) wprod = hidden_norm_product(e.wnorm, nblocks, lane);
   if (m >= M) return;
-  const float s = ainv[m], w0 = winv[cb0], w1 = two ? winv[cb0 + 1] : 0.f;
+  const int c = 16 * h + 4 * wave;
+  const float s = ainv[m];
+  const f32x4 w0 = *reinterpret_cast<const f32x4*>(winv + cb0 * 32 + c);
+  const f32x4 w1 = *reinterpret_cast<const f32x4*>(winv + (cb0 + two) * 32 + c);
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    sum[0][t] *= s * w0;
-    sum[1][t] *= s * w1;
+    sum[0][t] *= s * w0[t];
+    sum[1][t] *= s * w1[t];
   }
-  const int c = 16 * h + 4 * wave;
   if (kEpi == kSplitSwiGLU) {
     const float hs = hidden_scale(e.rnorm[m], wprod);
     if (cb0 == 0 && h == 0 && wave == 0) e.hinv[m] = split_inv(hs);
@@ -615,7 +621,7 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
 // through double-buffered LDS, `per` of them by a workgroup.  For K = 128 this replaces the separate fragment pass
 // and the short k-loop of the tiled kernel.
 constexpr int kR128Block = 8 * kFrag;   // f16 elements of one 32-channel block
-constexpr int kR128MaxN = 512;          // output channels with a bias
+constexpr int kR128MaxN = 512;          // output channels
 
 template <int kEpi, bool kLn>
 __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __restrict__ x, const f16* __restrict__ W,
@@ -623,7 +629,7 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
                                                                  const float* __restrict__ wbias, SplitGemmEpi e,
                                                                  long long M, int nblocks, int per) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][kR128Block];
-  __shared__ __attribute__((aligned(16))) float sbias[kLn ? kR128MaxN : 4];
+  __shared__ __attribute__((aligned(16))) float swinv[kR128MaxN], sbias[kLn ? kR128MaxN : 4];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, (unsigned)nblocks * kR128Block * 2);
   auto stage = [&](int cb) {
@@ -635,15 +641,19 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
   };
   const int first = blockIdx.y * per, last = min(first + per, nblocks);   // first < nblocks
   stage(first);
+  stage_floats(swinv, winv, nblocks * 32, nblocks * 32, kLn ? 1.0f / kNormScale : 1.0f);
   if (kLn) stage_floats(sbias, wbias, nblocks * 32, nblocks * 32);
   const long long m = ((long long)blockIdx.x * 4 + wave) * 32 + n;
   const bool valid = m < M;
   SplitFrag xf[8];
-  float xinv;
+  float xinv = 1.0f;   // kLn: kNormScale, in swinv
   {
     float v[64];
     load_row_half<128>(x + (size_t)(valid ? m : 0) * 128, h, v);
-    xinv = kLn ? normalized_row_half<128>(v, xf) : split_row_half<128>(v, xf);
+    if (kLn)
+      normalized_row_half<128>(v, xf);
+    else
+      xinv = split_row_half<128>(v, xf);
   }
 #pragma unroll 1
   for (int cb = first; cb < last; ++cb) {
@@ -652,7 +662,6 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
     if (cb + 1 < last) stage(cb + 1);
     f32x16 acc = zero16();
     mfma_block<8>(smem[cb & 1], xf, lane, acc);
-    const float sc = xinv * winv[cb];
     if (valid) {
       const int c0 = cb * 32 + 16 * h;
       f32x4 res[4];
@@ -661,8 +670,9 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
       for (int q = 0; q < 4; ++q) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         if (kLn) v = *reinterpret_cast<const f32x4*>(&sbias[c0 + 4 * q]);
+        const f32x4 w = *reinterpret_cast<const f32x4*>(&swinv[c0 + 4 * q]);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] += acc[4 * q + t] * sc;
+        for (int t = 0; t < 4; ++t) v[t] += (kLn ? acc[4 * q + t] : acc[4 * q + t] * xinv) * w[t];
         epi_quad<kEpi>(e, m, c0 + 4 * q, v, res[q]);
       }
     }
@@ -679,7 +689,7 @@ int split_gemm_r128(int epi, const float* x, const f16* W, const float* winv, co
   const long long wgs = (M + 127) / 128, nblocks = N / 32, resident = 3LL * compute_units();
   const long long parts = std::min(nblocks, std::max(1LL, resident / wgs)), per = (nblocks + parts - 1) / parts;
   const dim3 grid((unsigned)wgs, (unsigned)((nblocks + per - 1) / per));
-  if (wbias && N > kR128MaxN) return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: %d output channels", name, N);
+  if (N > kR128MaxN) return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: %d output channels", name, N);
   KernelTimerScope timed(name, stream);
 #define BIOEMU_R128(E, L) \
   hipLaunchKernelGGL((split_gemm_r128_kernel<E, L>), grid, dim3(256), 0, stream, x, W, winv, wbias, e, M, N / 32, (int)per)

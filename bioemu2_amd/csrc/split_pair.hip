@@ -17,18 +17,20 @@ namespace {
 
 constexpr int kCatWaves = 8;   // with all four column blocks in LDS
 constexpr int kCatWeights = 4 * 16 * kFrag;               // f16: [4 column blocks][16 k-steps]
-constexpr int kCatSmem = kCatWeights * (int)sizeof(f16) + 128 * 4;  // 128 KB and the biases
+constexpr int kCatScales = 2 * 128 * 4;                   // bytes: the biases and the weights' scales
+constexpr int kCatSmem = kCatScales + kCatWeights * (int)sizeof(f16);
 
 __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
     const float* __restrict__ x1, const float* __restrict__ x2, const f16* __restrict__ W,
     const float* __restrict__ winv, const float* __restrict__ wbias, float* __restrict__ out, long long P, int tiles,
     int per) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  f16* smem = reinterpret_cast<f16*>(smem_raw);
+  float *sbias = reinterpret_cast<float*>(smem_raw), *swinv = sbias + 128;
+  f16* smem = reinterpret_cast<f16*>(swinv + 128);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const int waves = blockDim.x / 64, cb0 = blockIdx.y * per;   // column blocks cb0 .. cb0 + per - 1
-  float* sbias = reinterpret_cast<float*>(smem + per * 16 * kFrag);
   stage_floats(sbias, wbias + cb0 * 32, per * 32, per * 32);
+  stage_floats(swinv, winv + cb0 * 32, per * 32, per * 32, 1.0f / kNormScale);
   stage_fragments(W + cb0 * 16 * kFrag, smem, per * 32, waves, wave, lane);
   // half of the next tile's rows is requested as soon as this tile's are fragments, ahead of its products and stores
   float a[64];
@@ -67,15 +69,15 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
       const f16* w = smem + cb * 16 * kFrag;
       f32x16 acc = zero16();
       mfma_block<16>(w, xf, lane, acc);
-      const float sc = winv[cb0 + cb] * (1.0f / kNormScale);
       if (valid) {
         const int c0 = cb * 32 + 16 * h;
         float* d = out + (size_t)m * 128 + cb0 * 32 + c0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           f32x4 v = *reinterpret_cast<const f32x4*>(sbias + c0 + 4 * q);
+          const f32x4 wi = *reinterpret_cast<const f32x4*>(swinv + c0 + 4 * q);
 #pragma unroll
-          for (int t = 0; t < 4; ++t) v[t] += acc[4 * q + t] * sc;
+          for (int t = 0; t < 4; ++t) v[t] += acc[4 * q + t] * wi[t];
           *reinterpret_cast<f32x4*>(d + 4 * q) = v;
         }
       }
@@ -95,7 +97,9 @@ __global__ __launch_bounds__(256, 2) void pair_bias_split_kernel(const float* __
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const int nhb = (H + 31) / 32;
   float* sbias = reinterpret_cast<float*>(smem + nhb * 8 * kFrag);
+  float* swinv = sbias + nhb * 32;
   stage_floats(sbias, wbias, H, nhb * 32);
+  stage_floats(swinv, winv, nhb * 32, nhb * 32, 1.0f / kNormScale);
   stage_fragments(W, smem, nhb * 16, 4, wave, lane);
   float v[64];
   auto load_rows = [&](int tile) { load_row_half<128>(z + (size_t)min((unsigned)tile * 32 + n, P - 1) * 128, h, v); };
@@ -114,13 +118,12 @@ __global__ __launch_bounds__(256, 2) void pair_bias_split_kernel(const float* __
     for (int hb = 0; hb < nhb; ++hb) {
       f32x16 acc = zero16();
       mfma_block<8>(smem + hb * 8 * kFrag, xf, lane, acc);
-      const float sc = winv[hb] * (1.0f / kNormScale);
       const int h0 = hb * 32 + 16 * h;
       if (valid) {
         float* d = out + (((size_t)outer * H + h0) * nrows + r) * ld + col;
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
-          if (h0 + u < H) *d = (acc[u] * sc + sbias[h0 + u]) * scale;
+          if (h0 + u < H) *d = (acc[u] * swinv[h0 + u] + sbias[h0 + u]) * scale;
           d += (size_t)nrows * ld;
         }
       }
@@ -145,13 +148,13 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
   const int grid = std::min((tiles + waves - 1) / waves, cus);
   KernelTimerScope timed(name, stream);
   hipLaunchKernelGGL(cat_proj_f32_kernel, dim3((unsigned)grid, 4 / per), dim3(64 * waves),
-                     per * (16 * kFrag * (int)sizeof(f16) + 32 * 4), stream, x1, x2, W, winv, wbias, out, P, tiles, per);
+                     kCatScales + per * 16 * kFrag * (int)sizeof(f16), stream, x1, x2, W, winv, wbias, out, P, tiles, per);
   return check_launch(name);
 }
 
 int split_pair_bias(const float* z, const f16* W, const float* winv, const float* wbias, float* out, long long P,
                     int nrows, int ncols, int ld, int H, float scale, hipStream_t stream, const char* name) {
-  const int tiles = (int)((P + 31) / 32), smem = (H + 31) / 32 * (8 * kFrag * (int)sizeof(f16) + 32 * 4);
+  const int tiles = (int)((P + 31) / 32), smem = (H + 31) / 32 * (8 * kFrag * (int)sizeof(f16) + 2 * 32 * 4);
   const int grid = std::min((tiles + 3) / 4, 1024);   // four workgroups per CU
   KernelTimerScope timed(name, stream);
   hipLaunchKernelGGL(pair_bias_split_kernel, dim3((unsigned)grid), dim3(256), (unsigned)smem, stream, z, W, winv, wbias,

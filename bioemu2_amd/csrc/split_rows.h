@@ -91,11 +91,10 @@ __device__ __forceinline__ void split_normalized(float (&v)[C / 2], float rstd, 
   split_half<C>(v, kNormScale, f);
 }
 
-// Fragments of the normalised row; returns 1 / scale.
+// Fragments of the normalised row, times kNormScale.
 template <int C>
-__device__ __forceinline__ float normalized_row_half(float (&v)[C / 2], SplitFrag (&f)[C / 16]) {
+__device__ __forceinline__ void normalized_row_half(float (&v)[C / 2], SplitFrag (&f)[C / 16]) {
   split_normalized<C>(v, center_row_half<C>(v), f);
-  return 1.0f / kNormScale;
 }
 
 // Copies `kb` KB of fragments into LDS, split over the workgroup's waves.
@@ -106,10 +105,11 @@ __device__ __forceinline__ void stage_fragments(const f16* W, f16* smem, int kb,
   __syncthreads();
 }
 
-// Copies `count` floats into LDS (whole workgroup; no barrier).  Epilogues read their biases from LDS: a global load
-// there would wait for every store before it (vmcnt counts both, in order).
-__device__ __forceinline__ void stage_floats(float* dst, const float* __restrict__ src, int count, int padded) {
-  for (int i = threadIdx.x; i < padded; i += blockDim.x) dst[i] = i < count ? src[i] : 0.f;
+// Copies `count` floats times `scale` into LDS (whole workgroup; no barrier).  Epilogues read their biases and scales
+// from LDS: a global load there would wait for every store before it (vmcnt counts both, in order).
+__device__ __forceinline__ void stage_floats(float* dst, const float* __restrict__ src, int count, int padded,
+                                             float scale = 1.0f) {
+  for (int i = threadIdx.x; i < padded; i += blockDim.x) dst[i] = i < count ? src[i] * scale : 0.f;
 }
 
 // ---------------------------------------------------------------------------
@@ -119,7 +119,7 @@ __device__ __forceinline__ void stage_floats(float* dst, const float* __restrict
 // kTransitionMaxHidden.  `W` holds split_transition_weight_elems f16, `scales` split_transition_scales floats.
 constexpr int kTransitionMaxHidden = 2048;
 constexpr int64_t kTransitionFusedRows128 = 18432, kTransitionFusedRows64 = 12288;   // fewest rows worth it
-inline size_t split_transition_scales(int64_t C, int64_t hidden) { return (size_t)(hidden / 8 + C / 32 + 2 * hidden); }
+inline size_t split_transition_scales(int64_t C, int64_t hidden) { return (size_t)(6 * hidden + C); }
 size_t split_transition_weight_elems(int64_t C, int64_t hidden);
 int split_transition_rows(const float* x, const float* res, const float* norm_w, const float* norm_b,
                           const float* fc1, const float* fc2, const float* fc3, f16* W, float* scales, float* out,

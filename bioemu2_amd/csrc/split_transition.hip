@@ -56,29 +56,34 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
     }
   };
   stage(0);
-  // fc1 and fc2 biases (W beta) of every chunk: [chunk][fc1 | fc2][32]
-  float* sbias = reinterpret_cast<float*>(smem_raw + 2 * G::Chunk * 2);
+  // 1 / scale of the fc1 and fc2 rows of every chunk, [chunk][fc1 | fc2][32], and of the fc3 rows; the biases (W beta)
+  // of fc1 and fc2
+  float* sinv = reinterpret_cast<float*>(smem_raw + 2 * G::Chunk * 2);
+  float *sinv3 = sinv + chunks * 64, *sbias = sinv3 + C;
+  stage_floats(sinv, inv12, chunks * 64, chunks * 64, kLn ? 1.0f / kNormScale : 1.0f);
+  stage_floats(sinv3, inv3, C, C);
   if (kLn)
     for (int i = threadIdx.x; i < chunks * 64; i += 64 * kWaves)
       sbias[i] = bias12[(i & 32 ? chunks * 32 : 0) + (i >> 6) * 32 + (i & 31)];
   const long long m = ((long long)blockIdx.x * kWaves + wave) * 32 + n;
   const bool valid = m < M;
   SplitFrag xf[G::KS];
-  float xinv, bound = 1.01f;   // bound: of |a| |b|, with room for rounding
+  float xinv = 1.0f, bound = 1.01f;   // kLn: kNormScale, in sinv.  bound: of |a| |b|, with room for rounding
   {
     float v[C / 2];
     load_row_half<C>(x + (size_t)(valid ? m : 0) * C, h, v);
     if (kLn) {
-      xinv = normalized_row_half<C>(v, xf);
+      normalized_row_half<C>(v, xf);
     } else {
       bound *= row_norm2<C>(v);
       xinv = split_row_half<C>(v, xf);
     }
   }
   float q1 = 0.f, q2 = 0.f;
-  for (int i = lane; i < chunks; i += 64) {
-    q1 = fmaxf(q1, norm12[2 * i]);
-    q2 = fmaxf(q2, norm12[2 * i + 1]);
+  for (int i = lane; i < chunks * 32; i += 64) {
+    const float* p = norm12 + (i >> 5) * 64 + (i & 31);
+    q1 = fmaxf(q1, p[0]);
+    q2 = fmaxf(q2, p[32]);
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
@@ -95,14 +100,14 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
     __syncthreads();                       // ... and everyone's; the other stage is free again
     if (hc + 1 < chunks) stage(hc + 1);
     const f16* st = smem + (hc & 1) * G::Chunk;
-    const float s1 = xinv * inv12[2 * hc], s2 = xinv * inv12[2 * hc + 1];
     f32x16 a = zero16(), gt = zero16();
     mfma_block2<G::KS>(st, st + G::KS * kFrag, xf, xf, lane, a, gt);
     SplitFrag hf[2];
-    const float* sb = sbias + hc * 64 + 16 * h;
+    const float *sb = sbias + hc * 64 + 16 * h, *si = sinv + hc * 64 + 16 * h;
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-      const float p = kLn ? a[u] * s1 + sb[u] : a[u] * s1, q = kLn ? gt[u] * s2 + sb[32 + u] : gt[u] * s2;
+      const float p = kLn ? a[u] * si[u] + sb[u] : a[u] * xinv * si[u];
+      const float q = kLn ? gt[u] * si[32 + u] + sb[32 + u] : gt[u] * xinv * si[32 + u];
       f16 hi, lo;
       split_value(p * sigmoidf_fast(p) * q, hs, hi, lo);
       hf[u >> 3].hi[u & 7] = hi;
@@ -119,13 +124,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
   const float hinv = split_inv(hs);
 #pragma unroll
   for (int cb = 0; cb < C / 32; ++cb) {
-    const float s = hinv * inv3[cb];
     const size_t off = (size_t)m * C + cb * 32 + 16 * h;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       f32x4 o;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) o[t] = acc[cb][4 * q + t] * s;
+      for (int t = 0; t < 4; ++t) o[t] = acc[cb][4 * q + t] * hinv * sinv3[cb * 32 + 16 * h + 4 * q + t];
       if (res) {
         const f32x4 r = *reinterpret_cast<const f32x4*>(res + off + 4 * q);
 #pragma unroll
@@ -140,10 +144,10 @@ template <int C, bool kLn>
 int launch(const float* x, const float* res, const f16* W, const float* inv12, const float* norm12,
            const float* bias12, const float* inv3, float* out, long long M, int hidden, hipStream_t stream,
            const char* name) {
-  const int smem = TGeo<C>::Smem + hidden * 8;
+  const int smem = TGeo<C>::Smem + (4 * hidden + C) * 4;
   const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void*>(transition_rows_f32_kernel<C, kLn>),
                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            TGeo<C>::Smem + kTransitionMaxHidden * 8);
+                                            TGeo<C>::Smem + (4 * kTransitionMaxHidden + C) * 4);
   if (rc != hipSuccess) return set_error(BIOEMU_ERR_LAUNCH, "%s: %s", name, hipGetErrorString(rc));
   KernelTimerScope timed(name, stream);
   const unsigned grid = (unsigned)((M + 32 * kWaves - 1) / (32 * kWaves));
@@ -161,13 +165,13 @@ size_t split_transition_weight_elems(int64_t C, int64_t hidden) {
 int split_transition_rows(const float* x, const float* res, const float* norm_w, const float* norm_b,
                           const float* fc1, const float* fc2, const float* fc3, f16* W, float* scales, float* out,
                           long long M, int C, int hidden, hipStream_t stream, const char* name) {
-  const int KS = C / 16, nb = hidden / 32;
+  const int KS = C / 16;
   const long long chunk = C == 128 ? TGeo<128>::Chunk : TGeo<64>::Chunk;
-  float *inv12 = scales, *norm12 = inv12 + 2 * nb, *inv3 = norm12 + 2 * nb, *bias12 = inv3 + C / 32;
+  float *inv12 = scales, *norm12 = inv12 + 2 * hidden, *inv3 = norm12 + 2 * hidden, *bias12 = inv3 + C;
   SplitMats mats{};
   mats.m[0] = with_fold(SplitMat{fc1, W, inv12, norm12, hidden, C, KS, KS, chunk, 0, 2, nullptr, nullptr, nullptr},
                         norm_w, norm_b, norm_w ? bias12 : nullptr);
-  mats.m[1] = with_fold(SplitMat{fc2, W + (size_t)KS * kFrag, inv12 + 1, norm12 + 1, hidden, C, KS, KS, chunk, 0, 2,
+  mats.m[1] = with_fold(SplitMat{fc2, W + (size_t)KS * kFrag, inv12 + 32, norm12 + 32, hidden, C, KS, KS, chunk, 0, 2,
                                  nullptr, nullptr, nullptr},
                         norm_w, norm_b, norm_w ? bias12 + hidden : nullptr);
   mats.m[2] = SplitMat{fc3, W + (size_t)2 * KS * kFrag, inv3, nullptr, C, hidden, hidden / 16, 2, 2 * kFrag, chunk, 1,

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
                                                                f16* __restrict__ lo, int N, int outgoing,
                                                                unsigned tiles, int per) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][2 * kWBlock];   // p | g block, double-buffered: 64 KB
-  __shared__ float sbias[4 * D];
+  __shared__ float sbias[4 * D], swinv[4 * D];   // swinv: [column block][p | g][32], as the weights
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, 8 * 2 * kWBlock * 2);
   auto stage = [&](int cb) {
@@ -53,6 +53,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
   const int first = blockIdx.y * per, last = first + per;   // this workgroup's column blocks
   stage(first);
   stage_floats(sbias, wbias, 4 * D, 4 * D);
+  stage_floats(swinv, winv, 4 * D, 4 * D, 1.0f / kNormScale);
   // tile (b, i, kb): 32 pairs k = 32 kb .. of line i; a wave past the last tile works on tile 0 and stores nothing
   const unsigned tile = blockIdx.x * 4 + wave;
   const bool live = tile < tiles;
@@ -81,8 +82,9 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
     f32x16 p = zero16(), g = zero16();
     mfma_block2<8, false>(st, st + kWBlock, xf, xf, lane, p, g);
     const int c = cb * 32 + perm32(n);
-    const float sp = winv[2 * cb] * (1.0f / kNormScale), sg = winv[2 * cb + 1] * (1.0f / kNormScale);
-    const float bp = sbias[c], bg = sbias[2 * D + c], s = split_scale(wnorm[2 * cb] * 1.01f);
+    const int cw = cb * 64 + perm32(n);
+    const float sp = swinv[cw], sg = swinv[cw + 32];
+    const float bp = sbias[c], bg = sbias[2 * D + c], s = split_scale(wnorm[cw] * 1.01f);
     f16x8 vh[2], vl[2];
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
@@ -182,8 +184,8 @@ __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const f16* __re
         for (int y = 0; y < 2; ++y) mfma_split(fa[ks][x], fb[ks][y], acc[x][y]);
   }
   // lane n: column j, register u: row 8 (u / 4) + 4 h + u % 4; a store covers 128 bytes of two rows
-  const float s = split_inv(split_scale(wnorm[2 * (d / 32)] * 1.01f)) *
-                  split_inv(split_scale(wnorm[2 * (4 + d / 32)] * 1.01f));
+  const int dw = d / 32 * 64 + d % 32;   // channel d's place among the p rows' norms
+  const float s = split_inv(split_scale(wnorm[dw] * 1.01f)) * split_inv(split_scale(wnorm[dw + 2 * D] * 1.01f));
   float* po = o + ((size_t)b * D + d) * plane;
 #pragma unroll
   for (int x = 0; x < 2; ++x)
@@ -211,7 +213,7 @@ __device__ __forceinline__ float gated(float p, float g) {
   return p * sigmoid_ulp(g);
 }
 constexpr int kOutWeights = 2 * 4 * kWBlock;                                  // f16: p_out | g_out
-constexpr int kOutSmem = kOutWeights * (int)sizeof(f16) + 2 * D * 4;          // 128 KB and the biases
+constexpr int kOutSmem = kOutWeights * (int)sizeof(f16) + 4 * D * 4;   // 128 KB, the biases and the weights' scales
 
 template <bool kFew>
 __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void trimul_out_kernel(
@@ -221,7 +223,9 @@ __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void tri
   f16* smem = reinterpret_cast<f16*>(smem_raw);
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   float* sbias = reinterpret_cast<float*>(smem + kOutWeights);
+  float* swinv = sbias + 2 * D;
   stage_floats(sbias, wbias, 2 * D, 2 * D);
+  stage_floats(swinv, winv, 2 * D, 2 * D, 1.0f / kNormScale);
   if (kFew) {   // this wave's two weight blocks; waited for below the rows' loads
     const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(W, kOutWeights * 2);
 #pragma unroll
@@ -265,7 +269,6 @@ __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void tri
       const f16* w = smem + cb * kWBlock;
       f32x16 p = zero16(), g = zero16();
       mfma_block2<8>(w, w + 4 * kWBlock, of, xf, lane, p, g);
-      const float sp = winv[cb] * (1.0f / kNormScale), sg = winv[4 + cb] * (1.0f / kNormScale);
       const int c = cb * 32 + 16 * h;
       if (valid) {
         f32x4 xr[4];   // read ahead of the stores (out may be x)
@@ -276,10 +279,12 @@ __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void tri
         for (int q = 0; q < 4; ++q) {
           const f32x4 bp = *reinterpret_cast<const f32x4*>(sbias + c + 4 * q);
           const f32x4 bg = *reinterpret_cast<const f32x4*>(sbias + D + c + 4 * q);
+          const f32x4 wp = *reinterpret_cast<const f32x4*>(swinv + c + 4 * q);
+          const f32x4 wg = *reinterpret_cast<const f32x4*>(swinv + D + c + 4 * q);
           f32x4 r;
 #pragma unroll
           for (int e = 0; e < 4; ++e)
-            r[e] = gated(p[4 * q + e] * sp + bp[e], g[4 * q + e] * sg + bg[e]);
+            r[e] = gated(p[4 * q + e] * wp[e] + bp[e], g[4 * q + e] * wg[e] + bg[e]);
           if (residual) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) r[e] += xr[q][e];
@@ -306,7 +311,7 @@ Layout layout(int64_t B, int64_t N) {
   };
   L.win = take((size_t)16 * kWBlock * 2);
   L.wout = take((size_t)8 * kWBlock * 2);
-  L.scales = take((16 + 16 + 8 + 4 * D + 2 * D) * 4);
+  L.scales = take((4 * D + 4 * D + 2 * D + 4 * D + 2 * D) * 4);
   L.hi = take((size_t)B * 2 * D * plane * 2);
   L.lo = take((size_t)B * 2 * D * plane * 2);
   L.o = take((size_t)B * D * plane * 4);
@@ -327,14 +332,14 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
   f16 *win = reinterpret_cast<f16*>(base + L.win), *wout = reinterpret_cast<f16*>(base + L.wout);
   f16 *hi = reinterpret_cast<f16*>(base + L.hi), *lo = reinterpret_cast<f16*>(base + L.lo);
   float* o = reinterpret_cast<float*>(base + L.o);
-  float *inv_in = reinterpret_cast<float*>(base + L.scales), *norm_in = inv_in + 16, *inv_out = norm_in + 16,
-        *bias_in = inv_out + 8, *bias_out = bias_in + 4 * D;
+  float *inv_in = reinterpret_cast<float*>(base + L.scales), *norm_in = inv_in + 4 * D,
+        *inv_out = norm_in + 4 * D, *bias_in = inv_out + 2 * D, *bias_out = bias_in + 4 * D;
   SplitMats mats{};
   mats.m[0] = with_fold(split_gemm_weight(p_in_w, win, inv_in, norm_in, 2 * D, D, 2, 0), norm_in_w, norm_in_b, bias_in);
   mats.m[1] =
       with_fold(split_gemm_weight(g_in_w, win, inv_in, norm_in, 2 * D, D, 2, 1), norm_in_w, norm_in_b, bias_in + 2 * D);
   mats.m[2] = with_fold(split_gemm_weight(p_out_w, wout, inv_out, nullptr, D, D), norm_out_w, norm_out_b, bias_out);
-  mats.m[3] = with_fold(split_gemm_weight(g_out_w, wout + 4 * kWBlock, inv_out + 4, nullptr, D, D), norm_in_w,
+  mats.m[3] = with_fold(split_gemm_weight(g_out_w, wout + 4 * kWBlock, inv_out + D, nullptr, D, D), norm_in_w,
                         norm_in_b, bias_out + D);
   int rc = split_weights(mats, 4, stream);
   if (rc) return rc;

@@ -1,0 +1,85 @@
+"""fp32 products on split operands where magnitudes are unlike: weight rows, in float64 terms channel by channel.
+
+Bound: TOL of test_split_gpu.py, which holds for each channel because each weight row has its own scale.
+"""
+
+import pytest
+import torch
+
+from bioemu2_amd import _ops
+from bioemu2_amd.attention_pair_bias import AttentionPairBias
+from bioemu2_amd.glue import PairwiseConditioning
+from bioemu2_amd.transition import Transition
+from bioemu2_amd.triangle_multiplication import TriangleMultiplicationHip
+from tests._helpers import randomize_params
+from tests.test_split_gpu import TOL, _apb64, _ln, _params, _transition
+
+pytestmark = pytest.mark.gpu
+
+
+def _unlike(weight):
+    """Rows of 1, 1e-1 .. 1e-9 of their magnitude, in turn."""
+    with torch.no_grad():
+        weight.mul_(torch.logspace(0, -9, 10).repeat(-(-weight.shape[0] // 10))[: weight.shape[0], None])
+
+
+def _worst_channel(got, want):
+    """The largest relative error (2-norm) of an output channel."""
+    got, want = got.double().cpu().flatten(0, -2), want.flatten(0, -2)
+    return float(((got - want).norm(dim=0) / want.norm(dim=0)).max())
+
+
+@pytest.mark.parametrize("dim,rows", [(128, 200), (128, 18500), (64, 12300), (384, 70), (384, 4300)])
+def test_output_rows_of_a_transition(gpu_device, dim, rows):
+    torch.manual_seed(0)
+    m = randomize_params(Transition(dim, 2 * dim), 3)
+    _unlike(m.fc3.weight)
+    x = torch.randn(rows, dim)
+    want = _transition(x.double(), _params(m))
+    with torch.no_grad():
+        got = m.to(gpu_device)(x.to(gpu_device))
+    assert _worst_channel(got, want) <= TOL
+
+
+@pytest.mark.parametrize("c_s,heads,n", [(128, 4, 40), (384, 16, 40), (384, 16, 1500)])
+def test_output_rows_of_an_attention(gpu_device, c_s, heads, n):
+    torch.manual_seed(1)
+    m = randomize_params(AttentionPairBias(c_s, 16, heads, initial_norm=False), 4)
+    _unlike(m.proj_o.weight)
+    s, z = torch.randn(1, n, c_s), torch.randn(1, n, n, 16)
+    mask = torch.ones(1, n, dtype=torch.bool)
+    want = _apb64(s.double(), z.double(), mask, _params(m), heads, 1, False)
+    with torch.no_grad():
+        got = m.to(gpu_device)(s.to(gpu_device), z.to(gpu_device), mask.to(gpu_device))
+    assert _worst_channel(got, want) <= TOL
+
+
+@pytest.mark.parametrize("rows", [500, 17000])
+def test_output_rows_of_the_conditioning_projection(gpu_device, rows):
+    torch.manual_seed(2)
+    m = randomize_params(PairwiseConditioning(128, 128), 5)
+    _unlike(m.dim_pairwise_init_proj[1].weight)
+    z, rel = torch.randn(rows, 128), torch.randn(rows, 128)
+    p = _params(m)
+    want = _ln(torch.cat([z, rel], -1).double(), p, "dim_pairwise_init_proj.0") @ p["dim_pairwise_init_proj.1.weight"].T
+    m = m.to(gpu_device)
+    got = _ops.launch_pair_cond_proj_f32(z.to(gpu_device), rel.to(gpu_device), *m.prepared_params_f32(),
+                                         torch.empty(rows, 128, device=gpu_device))
+    assert _worst_channel(got, want) <= TOL
+
+
+@pytest.mark.parametrize("n", [33, 130])
+def test_output_rows_of_a_triangle_multiplication(gpu_device, n):
+    torch.manual_seed(3)
+    m = randomize_params(TriangleMultiplicationHip(128, "outgoing"), 6)
+    _unlike(m.p_out.weight)
+    p = _params(m)
+    x = torch.randn(1, n, n, 128)
+    xn = _ln(x.double(), p, "norm_in")
+    a, b = ((xn @ p["p_in.weight"].T) * torch.sigmoid(xn @ p["g_in.weight"].T)).permute(0, 3, 1, 2).chunk(2, 1)
+    o = (a @ b.transpose(2, 3)).permute(0, 2, 3, 1)
+    want = (_ln(o, p, "norm_out") @ p["p_out.weight"].T) * torch.sigmoid(xn @ p["g_out.weight"].T)
+    mask = torch.ones(1, n, n, dtype=torch.bool)
+    with torch.no_grad():
+        got = m.to(gpu_device)(x.to(gpu_device), mask.to(gpu_device))
+    assert _worst_channel(got, want) <= TOL
