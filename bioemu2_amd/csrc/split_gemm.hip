@@ -646,14 +646,11 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
   const long long m = ((long long)blockIdx.x * 4 + wave) * 32 + n;
   const bool valid = m < M;
   SplitFrag xf[8];
-  float xinv = 1.0f;   // kLn: kNormScale, in swinv
+  float xinv;   // kLn: besides 1 / kNormScale, in swinv
   {
     float v[64];
     load_row_half<128>(x + (size_t)(valid ? m : 0) * 128, h, v);
-    if (kLn)
-      normalized_row_half<128>(v, xf);
-    else
-      xinv = split_row_half<128>(v, xf);
+    xinv = kLn ? normalized_row_half<128>(v, xf) : split_row_half<128>(v, xf);
   }
 #pragma unroll 1
   for (int cb = first; cb < last; ++cb) {
@@ -662,6 +659,7 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
     if (cb + 1 < last) stage(cb + 1);
     f32x16 acc = zero16();
     mfma_block<8>(smem[cb & 1], xf, lane, acc);
+    if (kLn) undo_gain(acc, xinv);
     if (valid) {
       const int c0 = cb * 32 + 16 * h;
       f32x4 res[4];

@@ -42,6 +42,7 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
     const long long m = (long long)tile * 32 + n;
     const bool valid = m < P;
     SplitFrag xf[16];
+    float xinv;
     {
       float c[64];
       load_row_half<128>(x2 + row_of(tile), h, c);
@@ -58,9 +59,10 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
         ss += a[i] * a[i] + c[i] * c[i];
       }
       ss += __shfl_xor(ss, 32);
-      const float rstd = 1.0f / sqrtf(ss * (1.0f / 256.0f) + 1e-5f);
-      split_normalized<128>(a, rstd, xf);
-      split_normalized<128>(c, rstd, xf + 8);
+      const float var = ss * (1.0f / 256.0f), rstd = 1.0f / sqrtf(var + 1e-5f), gain = norm_gain(var * rstd * rstd);
+      split_normalized<128>(a, rstd, gain, xf);
+      split_normalized<128>(c, rstd, gain, xf + 8);
+      xinv = split_inv(gain);
     }
     if (tile + step < tiles) load_row_half<128>(x1 + row_of(tile + step), h, a);
     __builtin_amdgcn_sched_barrier(0);
@@ -69,6 +71,7 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
       const f16* w = smem + cb * 16 * kFrag;
       f32x16 acc = zero16();
       mfma_block<16>(w, xf, lane, acc);
+      undo_gain(acc, xinv);
       if (valid) {
         const int c0 = cb * 32 + 16 * h;
         float* d = out + (size_t)m * 128 + cb0 * 32 + c0;
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(256, 2) void pair_bias_split_kernel(const float* __
     const unsigned p = (unsigned)tile * 32 + n;
     const bool valid = p < P;
     SplitFrag xf[8];
-    normalized_row_half<128>(v, xf);
+    const float xinv = normalized_row_half<128>(v, xf);
     if (tile + step < tiles) load_rows(tile + step);
     __builtin_amdgcn_sched_barrier(0);
     const unsigned rr = p / ncols, col = p - rr * ncols, outer = rr / nrows, r = rr - outer * nrows;
@@ -118,6 +121,7 @@ __global__ __launch_bounds__(256, 2) void pair_bias_split_kernel(const float* __
     for (int hb = 0; hb < nhb; ++hb) {
       f32x16 acc = zero16();
       mfma_block<8>(smem + hb * 8 * kFrag, xf, lane, acc);
+      undo_gain(acc, xinv);
       const int h0 = hb * 32 + 16 * h;
       if (valid) {
         float* d = out + (((size_t)outer * H + h0) * nrows + r) * ld + col;

@@ -59,14 +59,22 @@ __device__ __forceinline__ float split_row_half(const float (&v)[C / 2], SplitFr
   return split_inv(s);
 }
 
-// A normalised row of up to 256 channels is below 16 in magnitude: it takes this scale, which brings it below 2^14,
-// whatever its values.
+// A normalised row of up to 256 channels is below 16 in magnitude: it takes this scale, which brings it below 2^14.
+// Rows whose deviation is far below the LayerNorm's epsilon come out small, and take this scale times norm_gain.
 constexpr float kNormScale = 1024.f;
 
-// Centres the row (v -= mean) and returns 1 / sqrt(biased variance + 1e-5): the affine-free LayerNorm in fp32, two
-// passes, over the C channels of lanes l and l ^ 32.
+// 2^k for a normalised row of mean square t (the variance over variance plus epsilon): 1 down to t = 2^-8, below it
+// what brings the root mean square into [0.7, 1.42).  With 22.6 times that (256 channels) the largest magnitude stays
+// below 2^14.6.  Exact split_inv of it.
+__device__ __forceinline__ float norm_gain(float t) {
+  const int e = 127 - (int)((__builtin_bit_cast(uint32_t, t) >> 23) & 0xffu);   // 2^-e <= t
+  return __builtin_bit_cast(float, (uint32_t)(127 + (e > 8 ? e >> 1 : 0)) << 23);
+}
+
+// Centres the row (v -= mean) and returns rstd = 1 / sqrt(biased variance + 1e-5): the affine-free LayerNorm in fp32,
+// two passes, over the C channels of lanes l and l ^ 32; and the row's norm_gain.
 template <int C>
-__device__ __forceinline__ float center_row_half(float (&v)[C / 2]) {
+__device__ __forceinline__ float center_row_half(float (&v)[C / 2], float& gain) {
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < C / 2; ++i) s += v[i];
@@ -79,22 +87,34 @@ __device__ __forceinline__ float center_row_half(float (&v)[C / 2]) {
     ss += v[i] * v[i];
   }
   ss += __shfl_xor(ss, 32);
-  return 1.0f / sqrtf(ss * (1.0f / C) + 1e-5f);
+  const float var = ss * (1.0f / C), rstd = 1.0f / sqrtf(var + 1e-5f);
+  gain = norm_gain(var * rstd * rstd);
+  return rstd;
 }
 
-// Fragments of kNormScale * v * rstd.  v * rstd is rounded to fp32 by itself (see split_value).
+// Fragments of kNormScale * gain * v * rstd.  v * rstd is rounded to fp32 by itself (see split_value).
 template <int C>
-__device__ __forceinline__ void split_normalized(float (&v)[C / 2], float rstd, SplitFrag* f) {
+__device__ __forceinline__ void split_normalized(float (&v)[C / 2], float rstd, float gain, SplitFrag* f) {
 #pragma clang fp contract(off)
 #pragma unroll
   for (int i = 0; i < C / 2; ++i) v[i] = v[i] * rstd;
-  split_half<C>(v, kNormScale, f);
+  split_half<C>(v, kNormScale * gain, f);
 }
 
-// Fragments of the normalised row, times kNormScale.
+// Fragments of the normalised row, times kNormScale * norm_gain; returns 1 / norm_gain.
 template <int C>
-__device__ __forceinline__ void normalized_row_half(float (&v)[C / 2], SplitFrag (&f)[C / 16]) {
-  split_normalized<C>(v, center_row_half<C>(v), f);
+__device__ __forceinline__ float normalized_row_half(float (&v)[C / 2], SplitFrag (&f)[C / 16]) {
+  float gain;
+  const float rstd = center_row_half<C>(v, gain);
+  split_normalized<C>(v, rstd, gain, f);
+  return split_inv(gain);
+}
+
+// acc *= xinv, left out where no row of the wave has a gain.
+__device__ __forceinline__ void undo_gain(f32x16& acc, float xinv) {
+  if (__any(xinv != 1.0f))
+#pragma unroll
+    for (int u = 0; u < 16; ++u) acc[u] *= xinv;
 }
 
 // Copies `kb` KB of fragments into LDS, split over the workgroup's waves.

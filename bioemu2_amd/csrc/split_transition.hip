@@ -68,12 +68,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
   const long long m = ((long long)blockIdx.x * kWaves + wave) * 32 + n;
   const bool valid = m < M;
   SplitFrag xf[G::KS];
-  float xinv = 1.0f, bound = 1.01f;   // kLn: kNormScale, in sinv.  bound: of |a| |b|, with room for rounding
+  float xinv, bound = 1.01f;   // kLn: besides 1 / kNormScale, in sinv.  bound: of |a| |b|, with room for rounding
   {
     float v[C / 2];
     load_row_half<C>(x + (size_t)(valid ? m : 0) * C, h, v);
     if (kLn) {
-      normalized_row_half<C>(v, xf);
+      xinv = normalized_row_half<C>(v, xf);
     } else {
       bound *= row_norm2<C>(v);
       xinv = split_row_half<C>(v, xf);
@@ -102,6 +102,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
     const f16* st = smem + (hc & 1) * G::Chunk;
     f32x16 a = zero16(), gt = zero16();
     mfma_block2<G::KS>(st, st + G::KS * kFrag, xf, xf, lane, a, gt);
+    if (kLn) {
+      undo_gain(a, xinv);
+      undo_gain(gt, xinv);
+    }
     SplitFrag hf[2];
     const float *sb = sbias + hc * 64 + 16 * h, *si = sinv + hc * 64 + 16 * h;
 #pragma unroll

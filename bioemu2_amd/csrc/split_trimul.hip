@@ -64,11 +64,13 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
   auto pair = [&](int k) { return b0 + (outgoing ? (size_t)i * N + k : (size_t)k * N + i); };
   const unsigned long long kept = __ballot(lane < 32 && k0 + lane < N && mask[pair(min(k0 + lane, N - 1))] != 0);
   SplitFrag xf[8];
+  float xinv;   // of pair perm32(n)
   {
     float v[64];
     load_row_half<D>(x + pair(min(k0 + perm32(n), N - 1)) * D, h, v);
-    normalized_row_half<D>(v, xf);
+    xinv = normalized_row_half<D>(v, xf);
   }
+  const bool gains = __any(xinv != 1.0f);
   const unsigned keep = (unsigned)kept >> (16 * h);   // bit u: pair 16 h + u
   const size_t plane = (size_t)N * ld;
 #pragma unroll 1
@@ -81,6 +83,14 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
     const f16* st = smem[cb & 1];
     f32x16 p = zero16(), g = zero16();
     mfma_block2<8, false>(st, st + kWBlock, xf, xf, lane, p, g);
+    if (gains) {   // register u is pair 16 h + u, whose row lane 8 (u / 4) + 4 h + u % 4 holds
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const float xi = __shfl(xinv, 8 * (u >> 2) + 4 * h + (u & 3));
+        p[u] *= xi;
+        g[u] *= xi;
+      }
+    }
     const int c = cb * 32 + perm32(n);
     const int cw = cb * 64 + perm32(n);
     const float sp = swinv[cw], sg = swinv[cw + 32];
@@ -246,6 +256,7 @@ __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void tri
     const bool valid = j < N;
     const size_t m = ((size_t)t.b * N + t.row) * N + min(j, N - 1);
     SplitFrag of[8], xf[8];
+    float oinv, xinv;
     {
       float v[64];
       const float* po = o + ((size_t)t.b * D + 8 * h) * plane + (size_t)t.row * ld + j;
@@ -253,12 +264,12 @@ __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void tri
       for (int s = 0; s < 8; ++s)
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[8 * s + e] = po[(size_t)(16 * s + e) * plane];
-      normalized_row_half<D>(v, of);
+      oinv = normalized_row_half<D>(v, of);
     }
     {
       float v[64];
       load_row_half<D>(x + m * D, h, v);
-      normalized_row_half<D>(v, xf);
+      xinv = normalized_row_half<D>(v, xf);
     }
     if (kFew) {   // every wave holds the rows before one overwrites them
       __builtin_amdgcn_s_waitcnt(0x0f70);
@@ -269,6 +280,8 @@ __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void tri
       const f16* w = smem + cb * kWBlock;
       f32x16 p = zero16(), g = zero16();
       mfma_block2<8>(w, w + 4 * kWBlock, of, xf, lane, p, g);
+      undo_gain(p, oinv);
+      undo_gain(g, xinv);
       const int c = cb * 32 + 16 * h;
       if (valid) {
         f32x4 xr[4];   // read ahead of the stores (out may be x)

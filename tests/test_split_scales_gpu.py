@@ -1,6 +1,7 @@
-"""fp32 products on split operands where magnitudes are unlike: weight rows, in float64 terms channel by channel.
+"""fp32 products on split operands where magnitudes are unlike: weight rows, normalised rows.
 
-Bound: TOL of test_split_gpu.py, which holds for each channel because each weight row has its own scale.
+Bound: TOL of test_split_gpu.py against float64, for each output channel or row by itself, because each weight row and
+each row has its own scale.
 """
 
 import pytest
@@ -83,3 +84,66 @@ def test_output_rows_of_a_triangle_multiplication(gpu_device, n):
     with torch.no_grad():
         got = m.to(gpu_device)(x.to(gpu_device), mask.to(gpu_device))
     assert _worst_channel(got, want) <= TOL
+
+
+def _worst_row(got, want):
+    """The largest relative error (2-norm) of a row."""
+    got, want = got.double().cpu().flatten(0, -2), want.flatten(0, -2)
+    return float(((got - want).norm(dim=1) / want.norm(dim=1)).max())
+
+
+def _zero_biases(module):
+    with torch.no_grad():
+        for name, p in module.named_parameters():
+            if p.ndim == 1 and name.endswith("bias"):
+                p.zero_()
+
+
+@pytest.mark.parametrize("rows", [500, 17000])
+def test_rows_of_little_deviation_in_the_conditioning_projection(gpu_device, rows):
+    """Deviations from 1 to 1e-12 next to each other: normalised rows far below the LayerNorm's epsilon."""
+    torch.manual_seed(4)
+    m = randomize_params(PairwiseConditioning(128, 128), 7)
+    _zero_biases(m)
+    dev = torch.logspace(0, -12, 13).repeat(-(-rows // 13))[:rows, None]
+    z, rel = torch.randn(rows, 128) * dev, torch.randn(rows, 128) * dev
+    p = _params(m)
+    want = _ln(torch.cat([z, rel], -1).double(), p, "dim_pairwise_init_proj.0") @ p["dim_pairwise_init_proj.1.weight"].T
+    m = m.to(gpu_device)
+    got = _ops.launch_pair_cond_proj_f32(z.to(gpu_device), rel.to(gpu_device), *m.prepared_params_f32(),
+                                         torch.empty(rows, 128, device=gpu_device))
+    assert _worst_row(got, want) <= TOL
+
+
+@pytest.mark.parametrize("dev", [1e-3, 1e-5, 1e-7, 1e-9, 1e-12])
+def test_rows_of_little_deviation_in_an_attention(gpu_device, dev):
+    torch.manual_seed(5)
+    m = randomize_params(AttentionPairBias(128, 16, 4), 8)
+    _zero_biases(m)
+    s, z = torch.randn(1, 40, 128) * dev, torch.randn(1, 40, 40, 16)
+    mask = torch.ones(1, 40, dtype=torch.bool)
+    want = _apb64(s.double(), z.double(), mask, _params(m), 4, 1, True)
+    with torch.no_grad():
+        got = m.to(gpu_device)(s.to(gpu_device), z.to(gpu_device), mask.to(gpu_device))
+    assert _worst_row(got, want) <= TOL
+
+
+@pytest.mark.parametrize("n", [33, 130])
+@pytest.mark.parametrize("small", [1e-2, 1e-4, 1e-6])
+def test_rows_of_little_deviation_in_a_triangle_multiplication(gpu_device, n, small):
+    """Input projections so small that the contraction's rows lie far below the output LayerNorm's epsilon."""
+    torch.manual_seed(6)
+    m = randomize_params(TriangleMultiplicationHip(128, "outgoing"), 9)
+    _zero_biases(m)
+    with torch.no_grad():
+        m.p_in.weight.mul_(small)
+    p = _params(m)
+    x = torch.randn(1, n, n, 128)
+    xn = _ln(x.double(), p, "norm_in")
+    a, b = ((xn @ p["p_in.weight"].T) * torch.sigmoid(xn @ p["g_in.weight"].T)).permute(0, 3, 1, 2).chunk(2, 1)
+    o = (a @ b.transpose(2, 3)).permute(0, 2, 3, 1)
+    want = (_ln(o, p, "norm_out") @ p["p_out.weight"].T) * torch.sigmoid(xn @ p["g_out.weight"].T)
+    mask = torch.ones(1, n, n, dtype=torch.bool)
+    with torch.no_grad():
+        got = m.to(gpu_device)(x.to(gpu_device), mask.to(gpu_device))
+    assert _worst_row(got, want) <= TOL
