@@ -70,6 +70,11 @@ __device__ __forceinline__ void split_value(float x, float s, f16& hi, f16& lo) 
   lo = (f16)__builtin_fmaf(x, s, -(float)hi);
 }
 
+// An infinite value as the largest finite one (its lo would be no number); the product overflows again.
+__device__ __forceinline__ float split_finite(float x) {
+  return (__builtin_bit_cast(uint32_t, x) & 0x7fffffffu) == 0x7f800000u ? __builtin_copysignf(3.40282347e38f, x) : x;
+}
+
 // sigmoid(x) to about an ulp: the hardware exp2 on -x log2(e) carried as a rounded product and its error (a plain
 // product would cost |x| 2^-24 relative), and one Newton step on the hardware reciprocal.  Past +-87 the result is 1
 // or 2e-38, where an infinite x would make the product's error and the Newton step NaN; the clamp drops a NaN x, which

@@ -20,15 +20,6 @@ __device__ __forceinline__ void load_row_half(const float* row, int h, float (&v
     }
 }
 
-// Squared 2-norm of the row.
-template <int C>
-__device__ __forceinline__ float row_norm2(const float (&v)[C / 2]) {
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < C / 2; ++i) ss += v[i] * v[i];
-  return ss + __shfl_xor(ss, 32);
-}
-
 // Largest magnitude of the row.
 template <int C>
 __device__ __forceinline__ float row_absmax(const float (&v)[C / 2]) {
@@ -139,7 +130,7 @@ __device__ __forceinline__ void stage_floats(float* dst, const float* __restrict
 // kTransitionMaxHidden.  `W` holds split_transition_weight_elems f16, `scales` split_transition_scales floats.
 constexpr int kTransitionMaxHidden = 2048;
 constexpr int64_t kTransitionFusedRows128 = 18432, kTransitionFusedRows64 = 12288;   // fewest rows worth it
-inline size_t split_transition_scales(int64_t C, int64_t hidden) { return (size_t)(6 * hidden + C); }
+inline size_t split_transition_scales(int64_t C, int64_t hidden) { return (size_t)(4 * hidden + C); }
 size_t split_transition_weight_elems(int64_t C, int64_t hidden);
 int split_transition_rows(const float* x, const float* res, const float* norm_w, const float* norm_b,
                           const float* fc1, const float* fc2, const float* fc3, f16* W, float* scales, float* out,

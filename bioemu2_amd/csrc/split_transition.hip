@@ -9,9 +9,10 @@
 // directly, double-buffered.  A hidden value never leaves registers: silu(a) b
 // comes out of fc1 / fc2 as lane (row n, half h) = hidden 16 h + u, which is the
 // fc3 B operand of k-step j when lane half h supplies hidden 16 h + 8 j + t; the
-// fc3 fragments are read with the same permutation.  Its scale comes from the bound
-// |silu(a) b| <= |a| |b| (SplitMat::norm).  A LayerNorm's affine is folded into fc1
-// and fc2, so the rows are only centred and divided by their deviation.
+// fc3 fragments are read with the same permutation.  A row's hidden scale follows
+// its largest value so far, with three bits to spare before the next step; a step
+// rescales the accumulators (by a power of two).  A LayerNorm's affine is folded into
+// fc1 and fc2, so the rows are only centred and divided by their deviation.
 //
 // Few rows take the separate products of split_gemm.hip instead (the rule and both times: fp32.hip).
 //
@@ -39,8 +40,7 @@ struct TGeo {
 template <int C, bool kLn>
 __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
     const float* x, const float* res, const f16* __restrict__ W, const float* __restrict__ inv12,
-    const float* __restrict__ norm12, const float* __restrict__ bias12, const float* __restrict__ inv3, float* out,
-    long long M, int chunks) {
+    const float* __restrict__ bias12, const float* __restrict__ inv3, float* out, long long M, int chunks) {
   using G = TGeo<C>;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f16* smem = reinterpret_cast<f16*>(smem_raw);
@@ -68,29 +68,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
   const long long m = ((long long)blockIdx.x * kWaves + wave) * 32 + n;
   const bool valid = m < M;
   SplitFrag xf[G::KS];
-  float xinv, bound = 1.01f;   // kLn: besides 1 / kNormScale, in sinv.  bound: of |a| |b|, with room for rounding
+  float xinv;   // kLn: besides 1 / kNormScale, in sinv
   {
     float v[C / 2];
     load_row_half<C>(x + (size_t)(valid ? m : 0) * C, h, v);
-    if (kLn) {
-      xinv = normalized_row_half<C>(v, xf);
-    } else {
-      bound *= row_norm2<C>(v);
-      xinv = split_row_half<C>(v, xf);
-    }
+    xinv = kLn ? normalized_row_half<C>(v, xf) : split_row_half<C>(v, xf);
   }
-  float q1 = 0.f, q2 = 0.f;
-  for (int i = lane; i < chunks * 32; i += 64) {
-    const float* p = norm12 + (i >> 5) * 64 + (i & 31);
-    q1 = fmaxf(q1, p[0]);
-    q2 = fmaxf(q2, p[32]);
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    q1 = fmaxf(q1, __shfl_xor(q1, off));
-    q2 = fmaxf(q2, __shfl_xor(q2, off));
-  }
-  const float hs = split_scale(bound * q1 * q2);
+  float hs = split_scale(0.f);   // the row's hidden scale
   f32x16 acc[C / 32];
 #pragma unroll
   for (int cb = 0; cb < C / 32; ++cb) acc[cb] = zero16();
@@ -108,12 +92,29 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
     }
     SplitFrag hf[2];
     const float *sb = sbias + hc * 64 + 16 * h, *si = sinv + hc * 64 + 16 * h;
+    float hv[16], amax = 0.f;
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
       const float p = kLn ? a[u] * si[u] + sb[u] : a[u] * xinv * si[u];
       const float q = kLn ? gt[u] * si[32 + u] + sb[32 + u] : gt[u] * xinv * si[32 + u];
+      hv[u] = p * sigmoidf_fast(p) * q;
+      amax = fmaxf(amax, fabsf(hv[u]));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    if (__any(amax * hs >= 32768.f)) {   // each row for itself
+      const float ns = amax * hs >= 32768.f ? split_scale(amax) * 0.125f : hs, ratio = ns * split_inv(hs);
+#pragma unroll
+      for (int cb = 0; cb < C / 32; ++cb)
+#pragma unroll
+        for (int u = 0; u < 16; ++u) acc[cb][u] *= ratio;
+#pragma unroll
+      for (int u = 0; u < 16; ++u) hv[u] = split_finite(hv[u]);
+      hs = ns;
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
       f16 hi, lo;
-      split_value(p * sigmoidf_fast(p) * q, hs, hi, lo);
+      split_value(hv[u], hs, hi, lo);
       hf[u >> 3].hi[u & 7] = hi;
       hf[u >> 3].lo[u & 7] = lo;
     }
@@ -145,9 +146,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
 }
 
 template <int C, bool kLn>
-int launch(const float* x, const float* res, const f16* W, const float* inv12, const float* norm12,
-           const float* bias12, const float* inv3, float* out, long long M, int hidden, hipStream_t stream,
-           const char* name) {
+int launch(const float* x, const float* res, const f16* W, const float* inv12, const float* bias12, const float* inv3,
+           float* out, long long M, int hidden, hipStream_t stream, const char* name) {
   const int smem = TGeo<C>::Smem + (4 * hidden + C) * 4;
   const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void*>(transition_rows_f32_kernel<C, kLn>),
                                             hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -156,7 +156,7 @@ int launch(const float* x, const float* res, const f16* W, const float* inv12, c
   KernelTimerScope timed(name, stream);
   const unsigned grid = (unsigned)((M + 32 * kWaves - 1) / (32 * kWaves));
   hipLaunchKernelGGL((transition_rows_f32_kernel<C, kLn>), dim3(grid), dim3(64 * kWaves), (unsigned)smem, stream, x,
-                     res, W, inv12, norm12, bias12, inv3, out, M, hidden / 32);
+                     res, W, inv12, bias12, inv3, out, M, hidden / 32);
   return check_launch(name);
 }
 
@@ -171,11 +171,11 @@ int split_transition_rows(const float* x, const float* res, const float* norm_w,
                           long long M, int C, int hidden, hipStream_t stream, const char* name) {
   const int KS = C / 16;
   const long long chunk = C == 128 ? TGeo<128>::Chunk : TGeo<64>::Chunk;
-  float *inv12 = scales, *norm12 = inv12 + 2 * hidden, *inv3 = norm12 + 2 * hidden, *bias12 = inv3 + C;
+  float *inv12 = scales, *inv3 = inv12 + 2 * hidden, *bias12 = inv3 + C;
   SplitMats mats{};
-  mats.m[0] = with_fold(SplitMat{fc1, W, inv12, norm12, hidden, C, KS, KS, chunk, 0, 2, nullptr, nullptr, nullptr},
+  mats.m[0] = with_fold(SplitMat{fc1, W, inv12, nullptr, hidden, C, KS, KS, chunk, 0, 2, nullptr, nullptr, nullptr},
                         norm_w, norm_b, norm_w ? bias12 : nullptr);
-  mats.m[1] = with_fold(SplitMat{fc2, W + (size_t)KS * kFrag, inv12 + 32, norm12 + 32, hidden, C, KS, KS, chunk, 0, 2,
+  mats.m[1] = with_fold(SplitMat{fc2, W + (size_t)KS * kFrag, inv12 + 32, nullptr, hidden, C, KS, KS, chunk, 0, 2,
                                  nullptr, nullptr, nullptr},
                         norm_w, norm_b, norm_w ? bias12 + hidden : nullptr);
   mats.m[2] = SplitMat{fc3, W + (size_t)2 * KS * kFrag, inv3, nullptr, C, hidden, hidden / 16, 2, 2 * kFrag, chunk, 1,
@@ -183,7 +183,7 @@ int split_transition_rows(const float* x, const float* res, const float* norm_w,
   const int rc = split_weights(mats, 3, stream);
   if (rc) return rc;
 #define BIOEMU_TRANSITION(CC, LN) \
-  return launch<CC, LN>(x, res, W, inv12, norm12, bias12, inv3, out, M, hidden, stream, name)
+  return launch<CC, LN>(x, res, W, inv12, bias12, inv3, out, M, hidden, stream, name)
   if (C == 128) {
     if (norm_w) BIOEMU_TRANSITION(128, true);
     BIOEMU_TRANSITION(128, false);

@@ -147,3 +147,62 @@ def test_rows_of_little_deviation_in_a_triangle_multiplication(gpu_device, n, sm
     with torch.no_grad():
         got = m.to(gpu_device)(x.to(gpu_device), mask.to(gpu_device))
     assert _worst_row(got, want) <= TOL
+
+
+TRANSITIONS = [(128, 18500), (64, 12300)]   # one kernel
+
+
+@pytest.mark.parametrize("dim,rows", TRANSITIONS)
+@pytest.mark.parametrize("factor", [256.0, 4096.0])
+def test_hidden_outliers(gpu_device, dim, rows, factor):
+    """One fc1 row and another fc2 row large, their fc3 columns small in turn: the product of the largest norms says
+    nothing about any hidden value."""
+    torch.manual_seed(7)
+    m = randomize_params(Transition(dim, 2 * dim), 10)
+    with torch.no_grad():
+        for w, unit in ((m.fc1.weight, 3), (m.fc2.weight, 37)):
+            w[unit] *= factor
+            m.fc3.weight[:, unit] /= factor
+    x = torch.randn(rows, dim)
+    want = _transition(x.double(), _params(m))
+    with torch.no_grad():
+        got = m.to(gpu_device)(x.to(gpu_device))
+    assert _worst_row(got, want) <= TOL
+
+
+@pytest.mark.parametrize("dim,rows", TRANSITIONS)
+def test_closed_gates_and_small_rows(gpu_device, dim, rows):
+    """Hidden values far below what the weights' norms allow: gates near -25, and rows of deviation down to 1e-12."""
+    torch.manual_seed(9)
+    m = randomize_params(Transition(dim, 2 * dim), 12)
+    _zero_biases(m)
+    x = torch.randn(rows, dim) * torch.logspace(0, -12, 13).repeat(-(-rows // 13))[:rows, None]
+    want = _transition(x.double(), _params(m))
+    d = m.to(gpu_device)
+    with torch.no_grad():
+        assert _worst_row(d(x.to(gpu_device)), want) <= TOL
+        x = torch.randn(rows, dim)
+        x[:, 0] = 30.0
+        d.fc1.weight.mul_(0.02)
+        d.fc1.weight[:, 0] = -25.0 * (1.0 + 900.0 / dim) ** 0.5 / 30.0   # the channel, normalised, times this: -25
+        want = _transition(x.double(), _params(d))
+        assert float((want.norm(dim=1) / _transition(-x.double(), _params(d)).norm(dim=1)).max()) < 1e-6
+        assert _worst_row(d(x.to(gpu_device)), want) <= 4 * TOL   # the argument is rounded, 25 times: 1.3e-5 with fp32 operands
+
+
+@pytest.mark.parametrize("dim,rows", TRANSITIONS)
+def test_hidden_overflow(gpu_device, dim, rows):
+    """Infinite hidden values give infinite outputs of the weights' signs."""
+    torch.manual_seed(10)
+    m = randomize_params(Transition(dim, 2 * dim, use_norm=False), 13)
+    with torch.no_grad():
+        m.fc1.weight[3] = m.fc2.weight[3] = 0.0
+        m.fc1.weight[3, 0] = m.fc2.weight[3, 0] = 1e20
+    x = torch.randn(rows, dim)
+    x[:, 0] = 1.0
+    x[7, 0] = 0.0
+    with torch.no_grad():
+        got = m.to(gpu_device)(x.to(gpu_device)).cpu()
+    assert torch.isfinite(got[7]).all()
+    got[7] = got[8]
+    assert torch.equal(got, (float("inf") * torch.sign(m.fc3.weight[:, 3].cpu())).expand_as(got))
