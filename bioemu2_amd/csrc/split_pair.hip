@@ -46,20 +46,14 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
     {
       float c[64];
       load_row_half<128>(x2 + row_of(tile), h, c);
-      float s = 0.f;   // LayerNorm statistics over the concatenation
-#pragma unroll
-      for (int i = 0; i < 64; ++i) s += a[i] + c[i];
-      s += __shfl_xor(s, 32);
-      const float mean = s * (1.0f / 256.0f);
-      float ss = 0.f;
+      // LayerNorm statistics over the concatenation
+      const float mean = row_sum<128>([&](int i) { return a[i] + c[i]; }) * (1.0f / 256.0f);
 #pragma unroll
       for (int i = 0; i < 64; ++i) {
         a[i] -= mean;
         c[i] -= mean;
-        ss += a[i] * a[i] + c[i] * c[i];
       }
-      ss += __shfl_xor(ss, 32);
-      const float var = ss * (1.0f / 256.0f), rstd = 1.0f / sqrtf(var + 1e-5f), gain = norm_gain(var * rstd * rstd);
+      const float var = row_sum<128>([&](int i) { return a[i] * a[i] + c[i] * c[i]; }) * (1.0f / 256.0f), rstd = 1.0f / sqrtf(var + 1e-5f), gain = norm_gain(var * rstd * rstd);
       split_normalized<128>(a, rstd, gain, xf);
       split_normalized<128>(c, rstd, gain, xf + 8);
       xinv = split_inv(gain);

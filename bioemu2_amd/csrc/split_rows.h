@@ -62,23 +62,30 @@ __device__ __forceinline__ float norm_gain(float t) {
   return __builtin_bit_cast(float, (uint32_t)(127 + (e > 8 ? e >> 1 : 0)) << 23);
 }
 
+// Sum of the row halves' values f(0) .. f(C / 2 - 1) over lanes l and l ^ 32.  Eight partial sums: a channel close to
+// its row's mean under a large weight shows the mean's rounding, which one chain of C / 2 additions would double.
+template <int C, typename F>
+__device__ __forceinline__ float row_sum(F f) {
+  float p[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) p[i] = f(i);
+#pragma unroll
+  for (int i = 8; i < C / 2; ++i) p[i & 7] += f(i);
+#pragma unroll
+  for (int off = 4; off >= 1; off >>= 1)
+#pragma unroll
+    for (int i = 0; i < off; ++i) p[i] += p[i + off];
+  return p[0] + __shfl_xor(p[0], 32);
+}
+
 // Centres the row (v -= mean) and returns rstd = 1 / sqrt(biased variance + 1e-5): the affine-free LayerNorm in fp32,
 // two passes, over the C channels of lanes l and l ^ 32; and the row's norm_gain.
 template <int C>
 __device__ __forceinline__ float center_row_half(float (&v)[C / 2], float& gain) {
-  float s = 0.f;
+  const float mean = row_sum<C>([&](int i) { return v[i]; }) * (1.0f / C);
 #pragma unroll
-  for (int i = 0; i < C / 2; ++i) s += v[i];
-  s += __shfl_xor(s, 32);
-  const float mean = s * (1.0f / C);
-  float ss = 0.f;
-#pragma unroll
-  for (int i = 0; i < C / 2; ++i) {
-    v[i] -= mean;
-    ss += v[i] * v[i];
-  }
-  ss += __shfl_xor(ss, 32);
-  const float var = ss * (1.0f / C), rstd = 1.0f / sqrtf(var + 1e-5f);
+  for (int i = 0; i < C / 2; ++i) v[i] -= mean;
+  const float var = row_sum<C>([&](int i) { return v[i] * v[i]; }) * (1.0f / C), rstd = 1.0f / sqrtf(var + 1e-5f);
   gain = norm_gain(var * rstd * rstd);
   return rstd;
 }

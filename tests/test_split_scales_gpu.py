@@ -170,6 +170,23 @@ def test_hidden_outliers(gpu_device, dim, rows, factor):
     assert _worst_row(got, want) <= TOL
 
 
+@pytest.mark.parametrize("dim,rows", [(128, 200), (128, 18500), (64, 12300), (384, 70), (384, 4300)])
+def test_gamma_outlier(gpu_device, dim, rows):
+    """A LayerNorm weight of 1024 on a channel that is near its row's mean."""
+    torch.manual_seed(8)
+    m = randomize_params(Transition(dim, 2 * dim), 11)
+    with torch.no_grad():
+        m.norm.weight[5] = 1024.0
+    x = torch.randn(rows, dim)
+    x[:, 5] = 0.0
+    x -= x.mean(1, keepdim=True)
+    x[:, 5] = 0.0
+    want = _transition(x.double(), _params(m))
+    with torch.no_grad():
+        got = m.to(gpu_device)(x.to(gpu_device))
+    assert _worst_row(got, want) <= 2.5 * TOL   # the mean is rounded, 1024 times: 7.4e-6 with fp32 operands
+
+
 @pytest.mark.parametrize("dim,rows", TRANSITIONS)
 def test_closed_gates_and_small_rows(gpu_device, dim, rows):
     """Hidden values far below what the weights' norms allow: gates near -25, and rows of deviation down to 1e-12."""
