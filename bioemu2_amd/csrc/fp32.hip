@@ -577,7 +577,7 @@ int attn_f32_projections(const float* s, const float* norm_s_w, const float* nor
     mats.m[0] = with_fold(mats.m[0], norm_s_w, norm_s_b, buf.wbias);
     mats.m[1] = with_fold(mats.m[1], norm_s_w, norm_s_b, buf.wbias + 3 * c_s);
   }
-  const SplitRows rs{s, norm_s_w, norm_s_b, buf.sp.a, buf.sp.ainv, nullptr, rows, c_s, 0};
+  const SplitRows rs{s, norm_s_w, norm_s_b, buf.sp.a, buf.sp.ainv, rows, c_s, 0};
   int rc = r128 ? split_weights(mats, bias_split ? 4 : 3, stream) : split_prep(mats, bias_split ? 4 : 3, rs, stream);
   if (rc) return rc;
   if (bias_split)
@@ -614,7 +614,7 @@ int attn_f32_out(const float* go, const float* res, float* out, AttnF32Buffers& 
   e.ldo = c_s;
   if (c_s == 128)
     return split_gemm_r128(kSplitStore, go, w, winv, nullptr, e, rows, c_s, stream, name);
-  const SplitRows rs{go, nullptr, nullptr, buf.sp.a, buf.sp.ainv, nullptr, rows, c_s, 0};
+  const SplitRows rs{go, nullptr, nullptr, buf.sp.a, buf.sp.ainv, rows, c_s, 0};
   const int rc = split_prep(SplitMats{}, 0, rs, stream);
   if (rc) return rc;
   return split_gemm(kSplitStore, buf.sp.a, buf.sp.ainv, w, winv, e, rows, c_s, c_s, stream, name);
@@ -724,7 +724,7 @@ extern "C" int bioemu_swa_fwd_f32(const float* s, const float* z, const uint8_t*
 // transition of LN(z_init) to z_init).
 struct TransitionF32Buffers {
   f16 *x, *w12, *h, *w3;
-  float *xinv, *xnorm, *w12inv, *w12norm, *hinv, *w3inv;
+  float *xinv, *w12inv, *hinv, *w3inv;
   float* scales;   // the fused kernel's
 };
 
@@ -738,12 +738,10 @@ static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, Trans
   TransitionF32Buffers* b = buf ? buf : &dummy;
   b->x = c.frags(M, Dc);
   b->xinv = c.floats((size_t)M);
-  b->xnorm = c.floats((size_t)M);
   b->w12 = c.frags(3 * hidden, Dc);   // fc1 and fc2; with fc3 in the fused kernel's chunks
   b->w12inv = c.floats((size_t)2 * hidden);
-  b->w12norm = c.floats((size_t)2 * hidden);
   b->h = c.frags(M, hidden);
-  b->hinv = c.floats((size_t)M);
+  b->hinv = c.floats((size_t)M * ((hidden + 31) / 32));
   b->w3 = c.frags(kTransitionOutRows, hidden);
   b->w3inv = c.floats((size_t)kTransitionOutRows);
   b->scales = c.floats(split_transition_scales(Dc, hidden));
@@ -772,18 +770,16 @@ static int transition_f32_res(const float* x, const float* res, const float* nor
                                  buf.w12, buf.scales, out, M, (int)Dc, (int)hidden, stream, "f32_transition_rows");
   const int64_t out0 = out_dim < kTransitionOutRows ? out_dim : kTransitionOutRows;
   SplitMats mats{};
-  mats.m[0] = split_gemm_weight(fc1_w, buf.w12, buf.w12inv, buf.w12norm, hidden, Dc, 2, 0);
-  mats.m[1] = split_gemm_weight(fc2_w, buf.w12, buf.w12inv, buf.w12norm, hidden, Dc, 2, 1);
+  mats.m[0] = split_gemm_weight(fc1_w, buf.w12, buf.w12inv, nullptr, hidden, Dc, 2, 0);
+  mats.m[1] = split_gemm_weight(fc2_w, buf.w12, buf.w12inv, nullptr, hidden, Dc, 2, 1);
   mats.m[2] = split_gemm_weight(fc3_w, buf.w3, buf.w3inv, nullptr, out0, hidden);
-  const SplitRows rows{x, use_norm ? norm_w : nullptr, norm_b, buf.x, buf.xinv, buf.xnorm, M, (int)Dc, 0};
+  const SplitRows rows{x, use_norm ? norm_w : nullptr, norm_b, buf.x, buf.xinv, M, (int)Dc, 0};
   int rc = split_prep(mats, 3, rows, stream);
   if (rc) return rc;
   SplitGemmEpi e1;
   e1.hfrag = buf.h;
   e1.hinv = buf.hinv;
   e1.hsteps = split_ksteps(hidden);
-  e1.rnorm = buf.xnorm;
-  e1.wnorm = buf.w12norm;
   rc = split_gemm(kSplitSwiGLU, buf.x, buf.xinv, buf.w12, buf.w12inv, e1, M, (int)Dc, (int)(2 * hidden), stream,
                   "f32_transition_swiglu");
   if (rc) return rc;
@@ -797,7 +793,7 @@ static int transition_f32_res(const float* x, const float* res, const float* nor
     e2.out = out + c0;
     e2.res = residual ? res + c0 : nullptr;
     e2.ldo = (int)out_dim;
-    rc = split_gemm(kSplitStore, buf.h, buf.hinv, buf.w3, buf.w3inv, e2, M, (int)hidden, (int)nc, stream,
+    rc = split_gemm(kSplitHidden, buf.h, buf.hinv, buf.w3, buf.w3inv, e2, M, (int)hidden, (int)nc, stream,
                     "f32_transition_out");
     if (rc) return rc;
   }

@@ -173,12 +173,12 @@ struct SplitMats {
   int block_end[kSplitMats];   // set by split_prep
 };
 // M rows x [M][K] fp32 (K % 8 == 0, 16-byte aligned), LayerNormed (biased variance, eps 1e-5) when g, to fragments;
-// inv[row] = 1 / scale, norm[row] (unless null) = the row's 2-norm after the LayerNorm.
+// inv[row] = 1 / scale.
 struct SplitRows {
   const float* x;
   const float *g, *b;
   f16* dst;
-  float *inv, *norm;
+  float* inv;
   long long M;
   int K, ksteps;   // ksteps set by split_prep
 };

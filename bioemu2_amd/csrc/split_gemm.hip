@@ -153,18 +153,17 @@ __device__ __forceinline__ float rows_max(float v, float (&buf)[4][32], int wave
 
 // Rows of K values (a multiple of 8), optionally LayerNormed (biased variance, eps
 // 1e-5, fp32, two passes), to fragments.  A lane holds KPW k-steps x 8 values in
-// registers; wave w takes the k-steps w, w + 4, ...  inv[row] = 1 / scale,
-// norm[row] (unless null) = the row's 2-norm after the LayerNorm.
+// registers; wave w takes the k-steps w, w + 4, ...  inv[row] = 1 / scale.
 template <int KPW, bool kLn>
 __device__ __forceinline__ void split_row_block(const SplitRows& r, long long rb) {
-  __shared__ float buf[4][4][32];
+  __shared__ float buf[3][4][32];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const long long m = rb * 32 + n, M = r.M;
   const bool valid = m < M;
   const int K = r.K, ksteps = r.ksteps;
   const float *g = r.g, *b = r.b;
   f16* dst = r.dst;
-  float *inv = r.inv, *norm = r.norm;
+  float* inv = r.inv;
   float v[KPW][8];
 #pragma unroll
   for (int i = 0; i < KPW; ++i) {
@@ -208,20 +207,13 @@ __device__ __forceinline__ void split_row_block(const SplitRows& r, long long rb
       }
     }
   }
-  float amax = 0.f, ss = 0.f;
+  float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < KPW; ++i)
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      amax = fmaxf(amax, fabsf(v[i][t]));
-      ss += v[i][t] * v[i][t];
-    }
+    for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fabsf(v[i][t]));
   amax = rows_max(amax, buf[2], wave, lane);
   const float s = split_scale(amax);
-  if (norm) {
-    const float q = rows_sum(ss, buf[3], wave, lane);
-    if (wave == 0 && lane < 32 && valid) norm[m] = sqrtf(q);
-  }
   if (wave == 0 && lane < 32 && valid) inv[m] = split_inv(s);
 #pragma unroll
   for (int i = 0; i < KPW; ++i) {
@@ -266,9 +258,8 @@ template <bool kLn>
 __global__ __launch_bounds__(256) void split_long_rows_kernel(const float* __restrict__ x, int K,
                                                               const float* __restrict__ g,
                                                               const float* __restrict__ b, f16* __restrict__ dst,
-                                                              float* __restrict__ inv, float* __restrict__ norm,
-                                                              long long M, int ksteps) {
-  __shared__ float buf[4][4][32];
+                                                              float* __restrict__ inv, long long M, int ksteps) {
+  __shared__ float buf[3][4][32];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const long long rb = blockIdx.x, m = rb * 32 + n;
   const bool valid = m < M;
@@ -295,19 +286,11 @@ __global__ __launch_bounds__(256) void split_long_rows_kernel(const float* __res
     if (k >= K || !valid) return 0.f;
     return kLn ? (row[k] - mean) * rstd * g[k] + (b ? b[k] : 0.f) : row[k];
   };
-  float amax = 0.f, ss = 0.f;
+  float amax = 0.f;
   for (int ks = wave; ks < ksteps; ks += 4)
-    for (int t = 0; t < 8; ++t) {
-      const float v = value(ks * 16 + 8 * h + t);
-      amax = fmaxf(amax, fabsf(v));
-      ss += v * v;
-    }
+    for (int t = 0; t < 8; ++t) amax = fmaxf(amax, fabsf(value(ks * 16 + 8 * h + t)));
   amax = rows_max(amax, buf[2], wave, lane);
   const float s = split_scale(amax);
-  if (norm) {
-    const float q = rows_sum(ss, buf[3], wave, lane);
-    if (wave == 0 && lane < 32 && valid) norm[m] = sqrtf(q);
-  }
   if (wave == 0 && lane < 32 && valid) inv[m] = split_inv(s);
   for (int ks = wave; ks < ksteps; ks += 4) {
     f16x8 hi, lo;
@@ -328,12 +311,14 @@ __global__ __launch_bounds__(256) void split_long_rows_kernel(const float* __res
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float sigmoid_f32(float x) { return 1.0f / (1.0f + __expf(-x)); }
 
-// What is added to channels c0 .. c0 + 15 of row m: the residual (kSplitStore), the q bias (kSplitQkvg).
+constexpr bool stores_rows(int epi) { return epi == kSplitStore || epi == kSplitHidden; }
+
+// What is added to channels c0 .. c0 + 15 of row m: the residual (stores_rows), the q bias (kSplitQkvg).
 template <int kEpi>
 __device__ __forceinline__ void load_addend(const SplitGemmEpi& e, long long m, int c0, f32x4 (&r)[4]) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) r[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-  if (kEpi == kSplitStore && e.res)
+  if (stores_rows(kEpi) && e.res)
 #pragma unroll
     for (int q = 0; q < 4; ++q) r[q] = *reinterpret_cast<const f32x4*>(e.res + (size_t)m * e.ldo + c0 + 4 * q);
   if (kEpi == kSplitQkvg && e.bias && c0 < e.ldo)
@@ -345,7 +330,7 @@ __device__ __forceinline__ void load_addend(const SplitGemmEpi& e, long long m, 
 
 template <int kEpi>
 __device__ __forceinline__ void epi_quad(const SplitGemmEpi& e, long long m, int c, f32x4 v, f32x4 r) {
-  if (kEpi == kSplitStore) {
+  if (stores_rows(kEpi)) {
     float* d = e.out + (size_t)m * e.ldo + c;
 #pragma unroll
     for (int t = 0; t < 4; ++t) v[t] += r[t];
@@ -373,40 +358,30 @@ __device__ __forceinline__ void epi_quad(const SplitGemmEpi& e, long long m, int
   }
 }
 
-// SwiGLU of hidden channels c .. c + 3 of row m, written as the next product's
-// operand fragments with the row's scale s.
-__device__ __forceinline__ void epi_swiglu_quad(const SplitGemmEpi& e, long long m, int c, f32x4 a, f32x4 b, float s) {
+// silu(a) b of four hidden channels; amax: the largest magnitude so far.
+__device__ __forceinline__ f32x4 swiglu_quad(f32x4 a, f32x4 b, float& amax) {
+  f32x4 v;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    v[t] = a[t] * sigmoid_f32(a[t]) * b[t];
+    amax = fmaxf(amax, fabsf(v[t]));
+  }
+  return v;
+}
+
+// Hidden channels c .. c + 3 of row m, written as the next product's operand fragments with scale s.
+__device__ __forceinline__ void epi_hidden_quad(const SplitGemmEpi& e, long long m, int c, f32x4 v, float s) {
   f16x4 hi, lo;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     f16 x, y;
-    split_value(a[t] * sigmoid_f32(a[t]) * b[t], s, x, y);
+    split_value(split_finite(v[t]), s, x, y);
     hi[t] = x;
     lo[t] = y;
   }
   f16* d = e.hfrag + ((size_t)(m >> 5) * e.hsteps + (c >> 4)) * kFrag + (((c >> 3) & 1) * 32 + (int)(m & 31)) * 8 + (c & 4);
   *reinterpret_cast<f16x4*>(d) = hi;
   *reinterpret_cast<f16x4*>(d + kFragHalf) = lo;
-}
-
-// |silu(a) b| <= |a| |b| <= (|x| |w1|) (|x| |w2|): the scale of a hidden row from
-// the row's norm and the largest weight-row norms (even blocks of 32 fc1, odd fc2).
-__device__ __forceinline__ float hidden_norm_product(const float* wn, int nblocks, int lane) {
-  float q1 = 0.f, q2 = 0.f;
-  for (int i = lane; i < nblocks * 16; i += 64) {
-    const float* p = wn + (i >> 5) * 64 + (i & 31);
-    q1 = fmaxf(q1, p[0]);
-    q2 = fmaxf(q2, p[32]);
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    q1 = fmaxf(q1, __shfl_xor(q1, off));
-    q2 = fmaxf(q2, __shfl_xor(q2, off));
-  }
-  return q1 * q2;
-}
-__device__ __forceinline__ float hidden_scale(float row_norm, float wprod) {
-  return split_scale(row_norm * row_norm * wprod * 1.01f);
 }
 
 constexpr int kStageKs = 2;                                   // k-steps per stage
@@ -449,12 +424,29 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < 2; ++i) acc[j][i] = zero16();
+  // kSplitHidden: a stage is the 32 columns of one scale, and its products are added under it.  The next stage's scales
+  // are requested ahead of its copies (loads return in order).
+  static_assert(kStageKs == 2, "a stage is 32 columns");
+  float sc[2], scn[2] = {0.f, 0.f};
+  auto load_scales = [&](int ks0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const long long m = ((long long)mt * 4 + wm * 2 + i) * 32 + n;
+      scn[i] = ainv[(size_t)(ks0 / 2) * M + (m < M ? m : M - 1)];
+    }
+  };
+  if (kEpi == kSplitHidden) load_scales(0);
   stage(0);
 #pragma unroll 1
   for (int ks0 = 0; ks0 < ksteps; ks0 += kStageKs) {
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies of the stage landed
     __syncthreads();                       // ... and everyone's; the other stage is free again
-    if (ks0 + kStageKs < ksteps) stage(ks0 + kStageKs);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) sc[i] = scn[i];
+    if (ks0 + kStageKs < ksteps) {
+      if (kEpi == kSplitHidden) load_scales(ks0 + kStageKs);
+      stage(ks0 + kStageKs);
+    }
     const f16* sa = smem + ((ks0 / kStageKs) & 1) * kTileStage;
     const f16* sw = sa + 4 * kStageKs * kFrag;
     SplitFrag fa[kStageKs][2], fw[kStageKs][2];
@@ -466,12 +458,25 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
         fw[ks][i] = load_frag(sw + ((wn * 2 + i) * kStageKs + ks) * kFrag, lane);
       }
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int ks = 0; ks < kStageKs; ++ks)
+    if (kEpi == kSplitHidden) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) mfma_split(fw[ks][j], fa[ks][i], acc[j][i]);
+        for (int i = 0; i < 2; ++i) {
+          f32x16 part = zero16();
+#pragma unroll
+          for (int ks = 0; ks < kStageKs; ++ks) mfma_split(fw[ks][j], fa[ks][i], part);
+#pragma unroll
+          for (int u = 0; u < 16; ++u) acc[j][i][u] += part[u] * sc[i];
+        }
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < kStageKs; ++ks)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) mfma_split(fw[ks][j], fa[ks][i], acc[j][i]);
+    }
   }
   const int cb0 = nt * 4 + wn * 2;
   if (cb0 >= nblocks) return;
@@ -482,16 +487,14 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       w[j][q] = *reinterpret_cast<const f32x4*>(winv + min(cb0 + j, nblocks - 1) * 32 + 16 * h + 4 * q);
-  float wprod = 0.f;
-  if (kEpi == kSplitSwiGLU) wprod = hidden_norm_product(e.wnorm, nblocks, lane);
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const long long m = ((long long)mt * 4 + wm * 2 + i) * 32 + n;
-    if (m >= M) continue;
-    const float s = ainv[m];
+    if (m >= M) continue;   // both lanes of a row
+    const float s = kEpi == kSplitHidden ? 1.0f : ainv[m];
     if (kEpi == kSplitSwiGLU) {
-      const float hs = hidden_scale(e.rnorm[m], wprod);
-      if (cb0 == 0 && h == 0) e.hinv[m] = split_inv(hs);
+      f32x4 v[4];
+      float amax = 0.f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         f32x4 a, b;
@@ -500,8 +503,12 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
           a[t] = acc[0][i][4 * q + t] * s * w[0][q][t];
           b[t] = acc[1][i][4 * q + t] * s * w[1][q][t];
         }
-        epi_swiglu_quad(e, m, cb0 * 16 + 16 * h + 4 * q, a, b, hs);
+        v[q] = swiglu_quad(a, b, amax);
       }
+      const float hs = split_scale(fmaxf(amax, __shfl_xor(amax, 32)));
+      if (h == 0) e.hinv[(size_t)(cb0 / 2) * M + m] = split_inv(hs);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) epi_hidden_quad(e, m, cb0 * 16 + 16 * h + 4 * q, v[q], hs);
     } else {
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -531,6 +538,7 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
                                                                const float* __restrict__ winv, SplitGemmEpi e,
                                                                long long M, int nblocks, int ksteps) {
   __shared__ __attribute__((aligned(16))) f32x4 part[4][2][4][64];   // [wave][column block][quad][lane]: 32 KB
+  __shared__ float hmax[kEpi == kSplitSwiGLU ? 4 : 1][32];
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   const int ncols = (nblocks + 1) / 2;
   const long long mb = blockIdx.x / ncols;
@@ -540,13 +548,17 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
   const f16* pa = A + (size_t)mb * ksteps * kFrag;
   const f16* pw = W + (size_t)cb0 * ksteps * kFrag;
   const f16* pw1 = two ? pw + (size_t)ksteps * kFrag : pw;
+  const long long m = mb * 32 + n, mc = m < M ? m : M - 1;
   f32x16 acc[2] = {zero16(), zero16()};
   constexpr int kDepth = 4;   // k-steps requested together
   for (int ks = k0; ks < k1; ks += kDepth) {
     SplitFrag fa[kDepth], f0[kDepth], f1[kDepth];
+    float sc[kDepth];
 #pragma unroll
     for (int d = 0; d < kDepth; ++d) {
-      const size_t o = (size_t)min(ks + d, k1 - 1) * kFrag;
+      const int k = min(ks + d, k1 - 1);
+      const size_t o = (size_t)k * kFrag;
+      if (kEpi == kSplitHidden) sc[d] = ainv[(size_t)(k / 2) * M + mc];
       fa[d] = load_frag(pa + o, lane);
       f0[d] = load_frag(pw + o, lane);
       f1[d] = load_frag(pw1 + o, lane);
@@ -554,8 +566,19 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
 #pragma unroll
     for (int d = 0; d < kDepth; ++d)
       if (ks + d < k1) {
-        mfma_split(f0[d], fa[d], acc[0]);
-        mfma_split(f1[d], fa[d], acc[1]);
+        if (kEpi == kSplitHidden) {
+          f32x16 p0 = zero16(), p1 = zero16();
+          mfma_split(f0[d], fa[d], p0);
+          mfma_split(f1[d], fa[d], p1);
+#pragma unroll
+          for (int u = 0; u < 16; ++u) {
+            acc[0][u] += p0[u] * sc[d];
+            acc[1][u] += p1[u] * sc[d];
+          }
+        } else {
+          mfma_split(f0[d], fa[d], acc[0]);
+          mfma_split(f1[d], fa[d], acc[1]);
+        }
       }
   }
 #pragma unroll
@@ -579,12 +602,8 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
       for (int t = 0; t < 4; ++t) sum[j][t] += v[t];
     }
   }
-  const long long m = mb * 32 + n;
-  float wprod = 0.f;
-  if (kEpi == kSplitSwiGLU) wprod = hidden_norm_product(e.wnorm, nblocks, lane);
-  if (m >= M) return;
   const int c = 16 * h + 4 * wave;
-  const float s = ainv[m];
+  const float s = kEpi == kSplitHidden ? 1.0f : ainv[mc];
   const f32x4 w0 = *reinterpret_cast<const f32x4*>(winv + cb0 * 32 + c);
   const f32x4 w1 = *reinterpret_cast<const f32x4*>(winv + (cb0 + two) * 32 + c);
 #pragma unroll
@@ -593,13 +612,20 @@ __global__ __launch_bounds__(256) void split_gemm_small_kernel(const f16* __rest
     sum[1][t] *= s * w1[t];
   }
   if (kEpi == kSplitSwiGLU) {
-    const float hs = hidden_scale(e.rnorm[m], wprod);
-    if (cb0 == 0 && h == 0 && wave == 0) e.hinv[m] = split_inv(hs);
-    epi_swiglu_quad(e, m, cb0 * 16 + c, sum[0], sum[1], hs);
+    float amax = 0.f;
+    const f32x4 v = swiglu_quad(sum[0], sum[1], amax);
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    if (lane < 32) hmax[wave][lane] = amax;
+    __syncthreads();
+    if (m >= M) return;
+    const float hs = split_scale(fmaxf(fmaxf(hmax[0][n], hmax[1][n]), fmaxf(hmax[2][n], hmax[3][n])));
+    if (h == 0 && wave == 0) e.hinv[(size_t)(cb0 / 2) * M + m] = split_inv(hs);
+    epi_hidden_quad(e, m, cb0 * 16 + c, v, hs);
   } else {
+    if (m >= M) return;
     f32x4 r0 = {0.f, 0.f, 0.f, 0.f}, r1 = r0;
     const int c0 = cb0 * 32 + c;
-    if (kEpi == kSplitStore && e.res) {
+    if (stores_rows(kEpi) && e.res) {
       const float* r = e.res + (size_t)m * e.ldo + c0;
       r0 = *reinterpret_cast<const f32x4*>(r);
       if (two) r1 = *reinterpret_cast<const f32x4*>(r + 32);
@@ -731,10 +757,10 @@ int split_prep(SplitMats mats, int count, SplitRows r, hipStream_t stream) {
   if (is_long) {
     if (r.g)
       hipLaunchKernelGGL(split_long_rows_kernel<true>, grid, block, 0, stream, r.x, r.K, r.g, r.b, r.dst, r.inv,
-                         r.norm, r.M, r.ksteps);
+                         r.M, r.ksteps);
     else
       hipLaunchKernelGGL(split_long_rows_kernel<false>, grid, block, 0, stream, r.x, r.K, r.g, r.b, r.dst, r.inv,
-                         r.norm, r.M, r.ksteps);
+                         r.M, r.ksteps);
     return check_launch("f32_split_rows");
   }
 #define BIOEMU_SPLIT_PREP(KPW)                                                                  \
@@ -776,6 +802,7 @@ int split_gemm(int epi, const f16* A, const float* ainv, const f16* W, const flo
   switch (epi) {
     case kSplitStore: BIOEMU_SPLIT_GEMM(kSplitStore); break;
     case kSplitSwiGLU: BIOEMU_SPLIT_GEMM(kSplitSwiGLU); break;
+    case kSplitHidden: BIOEMU_SPLIT_GEMM(kSplitHidden); break;
     default: BIOEMU_SPLIT_GEMM(kSplitQkvg); break;
   }
 #undef BIOEMU_SPLIT_GEMM

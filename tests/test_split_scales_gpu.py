@@ -149,7 +149,8 @@ def test_rows_of_little_deviation_in_a_triangle_multiplication(gpu_device, n, sm
     assert _worst_row(got, want) <= TOL
 
 
-TRANSITIONS = [(128, 18500), (64, 12300)]   # one kernel
+# rows of each form of the transition: separate products (32 x 64 tiles, 128 x 128 tiles), one kernel
+TRANSITIONS = [(128, 200), (128, 18500), (64, 12300), (384, 70), (384, 4300)]
 
 
 @pytest.mark.parametrize("dim,rows", TRANSITIONS)
@@ -170,7 +171,7 @@ def test_hidden_outliers(gpu_device, dim, rows, factor):
     assert _worst_row(got, want) <= TOL
 
 
-@pytest.mark.parametrize("dim,rows", [(128, 200), (128, 18500), (64, 12300), (384, 70), (384, 4300)])
+@pytest.mark.parametrize("dim,rows", TRANSITIONS)
 def test_gamma_outlier(gpu_device, dim, rows):
     """A LayerNorm weight of 1024 on a channel that is near its row's mean."""
     torch.manual_seed(8)
