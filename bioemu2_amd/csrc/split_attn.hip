@@ -15,7 +15,8 @@
 // block's K and V scales are those of its unmasked keys alone (masked keys' logits are replaced and
 // their weight is zero, so their rows are zeroed), and a block's O is added under its V scale.
 // Blocks without an unmasked key are left out unless the sequence has none at all (then every
-// weight is the same, as in softmax over equal logits).
+// weight is the same, as in softmax over equal logits).  Masked keys have a weight all the same where
+// a query's every logit is near -1e6 or below: attend_all_keys computes such queries over all keys.
 //
 // 16 heads of 24, 768 tokens, 8 copies sharing one bias: 0.054 ms and 0.011 ms for the fragments, against 0.129 ms
 // for the same flash form on fp32 MFMAs with per-key mask tests (28 MFMAs of 64 cycles and about 290 VALU
@@ -107,18 +108,55 @@ __global__ __launch_bounds__(256) void kv_fragments_kernel(const float* __restri
   }
 }
 
-// bias [B][H][N][ld] in log2 units.
+// Query qr (one per lane pair) over all N keys in fp32, key by key; masked keys take part with logit -1e6.  Lane half h
+// ends with the average's channels 8 j + 4 h + t in o[4 j + t] and the sum of the weights in l.  Slow, and reached only
+// by queries that a masked key's weight matters to.
+template <int HD>
+__device__ __forceinline__ void attend_all_keys(const float* qr, const float* kb, const float* vb, const uint8_t* mask,
+                                             const float* brow, int N, int c_s, float qscale, int h, float (&o)[16], float& l) {
+  float q[HD];
+#pragma unroll
+  for (int c = 0; c < HD; ++c) q[c] = qr[c];
+#pragma unroll
+  for (int u = 0; u < 16; ++u) o[u] = 0.f;
+  float m = -INFINITY, sum = 0.f;
+  for (int j = 0; j < N; ++j) {
+    float x = kMaskedLogit;
+    if (mask[j]) {
+      const float* kr = kb + (size_t)j * c_s;
+      float dot = 0.f;
+#pragma unroll
+      for (int c = 0; c < HD; ++c) dot += q[c] * kr[c];
+      x = dot * qscale + brow[j];
+    }
+    if (x == -INFINITY) continue;
+    const float mn = fmaxf(m, x), alpha = fast_exp2(m - mn), p = fast_exp2(x - mn);   // alpha 0 at the first key
+    const float* vr = vb + (size_t)j * c_s;
+    sum = sum * alpha + p;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int c = 8 * (u >> 2) + 4 * h + (u & 3);
+      if (8 * (u >> 2) < HD) o[u] = o[u] * alpha + p * vr[c];
+    }
+    m = mn;
+  }
+  l = sum;
+}
+
+// bias [B][H][N][ld] in log2 units; k, v and mask as kv_fragments_kernel's.
 template <int HD>
 __global__ __launch_bounds__(256, 3) void attn_split_kernel(const float* __restrict__ q, const f16* __restrict__ kv,
                                                             const float* __restrict__ kvinv,
                                                             const uint32_t* __restrict__ words,
                                                             const float* __restrict__ g, const float* __restrict__ bias,
+                                                            const float* __restrict__ k, const float* __restrict__ v,
+                                                            const uint8_t* __restrict__ mask,
                                                             float* __restrict__ go, int N, int nkb, int ld, int H,
                                                             int c_s, int mult, float qscale, int mask_per_copy,
                                                             int nqb, int total) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][kKvFrag];
   __shared__ uint16_t active[kMaxBlocks];
-  __shared__ int nactive;
+  __shared__ int nactive, nvalid;   // nvalid: whether a key is valid
   const int lane = threadIdx.x & 63, wave = wave_id(), n = lane & 31, h = lane >> 5;
   // an XCD takes consecutive items, the copies that share a bias block next to each other
   const int per_xcd = (total + 7) / 8, item = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
@@ -136,7 +174,10 @@ __global__ __launch_bounds__(256, 3) void attn_split_kernel(const float* __restr
       if (on) active[count + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)(k0 + lane);
       count += __popcll(m);
     }
-    if (lane == 0) nactive = count;
+    if (lane == 0) {
+      nactive = count;
+      nvalid = some;
+    }
   }
   const int q0 = (qb * 4 + wave) * 32;
   // waves past N run on a clamped row and store nothing: they copy their share of every block and meet every barrier
@@ -267,6 +308,14 @@ __global__ __launch_bounds__(256, 3) void attn_split_kernel(const float* __restr
   }
   l += __shfl_xor(l, 32);
   if (q0 + n >= N) return;
+  if (nvalid && m < kMaskedLogit + 160.f) {   // a masked key's weight is not zero
+    const size_t row0 = (size_t)bm * N * c_s + hd * HD;
+    float oa[16];
+    attend_all_keys<HD>(q + row0 + (size_t)qi * c_s, k + row0, v + row0, mask + (size_t)(mask_per_copy ? bm : b) * N,
+                        brow - 4 * h, N, c_s, qscale, h, oa, l);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) o[u] = oa[u];
+  }
   const float inv = 1.0f / l;
   const size_t off = ((size_t)bm * N + qi) * c_s + hd * HD;
 #pragma unroll
@@ -298,7 +347,7 @@ int launch(const SplitAttn& a, hipStream_t stream, const char* name) {
   KernelTimerScope timed(name, stream);
   const float qscale = kLog2e / sqrtf((float)HD);
   hipLaunchKernelGGL(attn_split_kernel<HD>, dim3((unsigned)((total + 7) / 8 * 8)), dim3(256), 0, stream, a.q, a.kv,
-                     a.kvinv, a.words, a.g, a.bias, a.go, a.N, nkb, a.ld, a.H, a.c_s, a.mult, qscale, a.mask_per_copy,
+                     a.kvinv, a.words, a.g, a.bias, a.k, a.v, a.mask, a.go, a.N, nkb, a.ld, a.H, a.c_s, a.mult, qscale, a.mask_per_copy,
                      nqb, (int)total);
   return check_launch(name);
 }

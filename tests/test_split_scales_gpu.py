@@ -224,3 +224,28 @@ def test_hidden_overflow(gpu_device, dim, rows):
     assert torch.isfinite(got[7]).all()
     got[7] = got[8]
     assert torch.equal(got, (float("inf") * torch.sign(m.fc3.weight[:, 3].cpu())).expand_as(got))
+
+
+@pytest.mark.parametrize("c_s,heads", [(384, 16), (128, 4)])
+@pytest.mark.parametrize("n,masked", [(40, range(5, 9)), (97, range(60, 97)), (200, range(0, 199))])
+def test_valid_keys_below_the_masked_ones(gpu_device, c_s, heads, n, masked):
+    """Queries whose valid keys' logits are near -5e6 attend to the masked keys, whose logit is -1e6; the others next to
+    them do not."""
+    torch.manual_seed(11)
+    m = randomize_params(AttentionPairBias(c_s, 16, heads, initial_norm=False), 14)
+    d = c_s // heads
+    low = 5e6 / (d / d**0.5)
+    with torch.no_grad():
+        m.proj_q_bias.zero_()
+        m.proj_qkv.weight[: 2 * c_s] = 0.0
+        m.proj_qkv.weight[:c_s, 0] = low**0.5
+        m.proj_qkv.weight[c_s : 2 * c_s, 1] = -(low**0.5)
+    s, z = torch.randn(1, n, c_s), torch.randn(1, n, n, 16)
+    s[..., 0] = (torch.arange(n) % 3 == 0).float()
+    s[..., 1] = 1.0
+    mask = torch.ones(1, n, dtype=torch.bool)
+    mask[:, list(masked)] = False
+    want = _apb64(s.double(), z.double(), mask, _params(m), heads, 1, False)
+    with torch.no_grad():
+        got = m.to(gpu_device)(s.to(gpu_device), z.to(gpu_device), mask.to(gpu_device))
+    assert _worst_row(got, want) <= TOL
