@@ -171,6 +171,8 @@ constexpr int kSplitMats = 4;
 struct SplitMats {
   SplitMat m[kSplitMats];
   int block_end[kSplitMats];   // set by split_prep
+  void* zero;                  // split_weights: memory to clear, 16-byte aligned, a multiple of 16 bytes
+  size_t zero_bytes;
 };
 // M rows x [M][K] fp32 (K % 8 == 0, 16-byte aligned), LayerNormed (biased variance, eps 1e-5) when g, to fragments;
 // inv[row] = 1 / scale.

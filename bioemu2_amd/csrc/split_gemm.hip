@@ -129,7 +129,13 @@ __device__ __forceinline__ void split_weight_block(const SplitMat& m, int rb) {
   }
 }
 
-__global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats mats) {
+__global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats mats, int count) {
+  if ((int)blockIdx.y == count) {
+    uint4* p = static_cast<uint4*>(mats.zero);
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < mats.zero_bytes / 16; i += (size_t)gridDim.x * blockDim.x)
+      p[i] = uint4{0, 0, 0, 0};
+    return;
+  }
   const SplitMat& m = mats.m[blockIdx.y];
   if ((int)blockIdx.x * 32 >= m.rows) return;   // uniform over the workgroup
   split_weight_block<kSwWaves, kSwSteps>(m, blockIdx.x);
@@ -732,8 +738,11 @@ int split_gemm_r128(int epi, const float* x, const f16* W, const float* winv, co
 int split_weights(const SplitMats& mats, int count, hipStream_t stream) {
   int blocks = 0;
   for (int i = 0; i < count; ++i) blocks = std::max(blocks, (mats.m[i].rows + 31) / 32);
+  // the memory to clear: 64 KB a workgroup, beside the weights
+  if (mats.zero_bytes) blocks = std::max(blocks, (int)std::min<size_t>((mats.zero_bytes + 65535) / 65536, 2048));
   KernelTimerScope timed("f32_split_weights", stream);
-  hipLaunchKernelGGL(split_weights_kernel, dim3(blocks, count), dim3(64 * kSwWaves), 0, stream, mats);
+  hipLaunchKernelGGL(split_weights_kernel, dim3(blocks, count + (mats.zero_bytes ? 1 : 0)), dim3(64 * kSwWaves), 0, stream,
+                     mats, count);
   return check_launch("f32_split_weights");
 }
 

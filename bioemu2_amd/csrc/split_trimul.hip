@@ -6,7 +6,11 @@
 //                           that both directions contract C = A B^T with k contiguous.  A plane's
 //                           scale is a bound from its weights (|p sigmoid(g)| <= |p|,
 //                           SplitMat::norm), so it is known before the first row is seen.
-//   trimul_contract_kernel  o[d][i][j] = sum_k a[d][i][k] b[d][j][k] on 128 x 128 tiles.
+//                           32 pairs of a line that are all below 2^-12 of that range take
+//                           a power of two more (their gain, one byte); a channel with
+//                           such a line is flagged.
+//   trimul_contract_kernel  o[d][i][j] = sum_k a[d][i][k] b[d][j][k] on 128 x 128 tiles;
+//                           gains of a flagged channel are undone 32 k at a time.
 //   trimul_out_kernel       LN_out(o) Wp * sigmoid(LN_in(x) Wg) (+ x): o read from its planes,
 //                           32 pairs (128 bytes) of a channel per load, both weights resident in LDS.
 //
@@ -31,13 +35,21 @@ constexpr int kWBlock = 8 * kFrag;   // f16 elements: a 32 x 128 weight block
 // Row stride (f16 or fp32 elements) of a plane: N columns, zero-filled to whole 32-wide k-steps.
 __host__ __device__ inline int plane_ld(int N) { return (N + 31) / 32 * 32; }
 
+// Gains: bytes [channel plane][32-k tile][row, plane_ld], 2^gain the factor; row tiles read past the last row.
+__host__ __device__ inline size_t gain_at(size_t plane, int kt, int i, int ld) {
+  return (plane * (ld / 32) + kt) * ld + i;
+}
+constexpr int kGainPad = 128;
+constexpr float kGainBelow = 8.f;   // scaled magnitude
+
 __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __restrict__ x,
                                                                const uint8_t* __restrict__ mask,
                                                                const f16* __restrict__ W,
                                                                const float* __restrict__ winv,
                                                                const float* __restrict__ wnorm,
                                                                const float* __restrict__ wbias, f16* __restrict__ hi,
-                                                               f16* __restrict__ lo, int N, int outgoing,
+                                                               f16* __restrict__ lo, uint8_t* __restrict__ gains,
+                                                               uint32_t* __restrict__ flags, int N, int outgoing,
                                                                unsigned tiles, int per) {
   __shared__ __attribute__((aligned(16))) f16 smem[2][2 * kWBlock];   // p | g block, double-buffered: 64 KB
   __shared__ float sbias[4 * D], swinv[4 * D];   // swinv: [column block][p | g][32], as the weights
@@ -70,7 +82,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
     load_row_half<D>(x + pair(min(k0 + perm32(n), N - 1)) * D, h, v);
     xinv = normalized_row_half<D>(v, xf);
   }
-  const bool gains = __any(xinv != 1.0f);
+  const bool scaled_rows = __any(xinv != 1.0f);
   const unsigned keep = (unsigned)kept >> (16 * h);   // bit u: pair 16 h + u
   const size_t plane = (size_t)N * ld;
 #pragma unroll 1
@@ -83,7 +95,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
     const f16* st = smem[cb & 1];
     f32x16 p = zero16(), g = zero16();
     mfma_block2<8, false>(st, st + kWBlock, xf, xf, lane, p, g);
-    if (gains) {   // register u is pair 16 h + u, whose row lane 8 (u / 4) + 4 h + u % 4 holds
+    if (scaled_rows) {   // register u is pair 16 h + u, whose row lane 8 (u / 4) + 4 h + u % 4 holds
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
         const float xi = __shfl(xinv, 8 * (u >> 2) + 4 * h + (u & 3));
@@ -94,13 +106,30 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
     const int c = cb * 32 + perm32(n);
     const int cw = cb * 64 + perm32(n);
     const float sp = swinv[cw], sg = swinv[cw + 32];
-    const float bp = sbias[c], bg = sbias[2 * D + c], s = split_scale(wnorm[cw] * 1.01f);
+    const float bp = sbias[c], bg = sbias[2 * D + c];
+    float s = split_scale(wnorm[cw] * 1.01f), v[16], amax = 0.f;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      v[u] = (keep >> u) & 1u ? (p[u] * sp + bp) * sigmoid_ulp(g[u] * sg + bg) : 0.f;
+      amax = fmaxf(amax, fabsf(v[u]));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    const bool low = amax * s < kGainBelow && amax > 0.f;
+    if (__any(low)) {
+      const float s2 = low ? split_scale(amax) : s;
+      if (low && live && h == 0) {
+        const size_t ch = (size_t)t.b * 2 * D + c;
+        gains[gain_at(ch, t.col, i, ld)] =
+            (uint8_t)((__builtin_bit_cast(uint32_t, s2) >> 23) - (__builtin_bit_cast(uint32_t, s) >> 23));
+        flags[ch] = 1;
+      }
+      s = s2;
+    }
     f16x8 vh[2], vl[2];
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-      const float v = (keep >> u) & 1u ? (p[u] * sp + bp) * sigmoid_ulp(g[u] * sg + bg) : 0.f;
       f16 a, d;
-      split_value(v, s, a, d);
+      split_value(v[u], s, a, d);
       vh[u >> 3][u & 7] = a;
       vl[u >> 3][u & 7] = d;
     }
@@ -128,6 +157,8 @@ __device__ __forceinline__ int swz(int r) { return (r >> 2) & 3; }
 __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const f16* __restrict__ hi,
                                                                  const f16* __restrict__ lo,
                                                                  const float* __restrict__ wnorm,
+                                                                 const uint8_t* __restrict__ gains,
+                                                                 const uint32_t* __restrict__ flags,
                                                                  float* __restrict__ o, int N, int nt, int total) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   f16* smem = reinterpret_cast<f16*>(smem_raw);
@@ -166,6 +197,8 @@ __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const f16* __re
 #pragma unroll
     for (int y = 0; y < 2; ++y) acc[x][y] = zero16();
   const int nk = ld / 32;
+  const size_t cha = (size_t)b * 2 * D + d, chb = cha + D;
+  const bool flagged = flags[cha] | flags[chb];   // uniform over the workgroup
   stage(0);
 #pragma unroll 1
   for (int kt = 0; kt < nk; ++kt) {
@@ -186,6 +219,31 @@ __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const f16* __re
         fb[ks][x].lo = *reinterpret_cast<const f16x8*>(st + 3 * kPart + ob);
       }
     __builtin_amdgcn_sched_barrier(0);
+    if (flagged) {
+      uint32_t ga[2][4];   // four rows each
+      int gb[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          ga[x][q] = *reinterpret_cast<const uint32_t*>(gains + gain_at(cha, kt, it * 128 + wi * 64 + x * 32 + 8 * q + 4 * h, ld));
+        gb[x] = gains[gain_at(chb, kt, jt * 128 + wj * 64 + x * 32 + n, ld)];
+      }
+      if (__any(ga[0][0] | ga[0][1] | ga[0][2] | ga[0][3] | ga[1][0] | ga[1][1] | ga[1][2] | ga[1][3] | gb[0] | gb[1])) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) {
+            f32x16 part = zero16();
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) mfma_split(fa[ks][x], fb[ks][y], part);
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+              acc[x][y][u] += __builtin_amdgcn_ldexpf(part[u], -((int)(ga[x][u >> 2] >> (8 * (u & 3)) & 0xffu) + gb[y]));
+          }
+        continue;
+      }
+    }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -311,7 +369,7 @@ __global__ __launch_bounds__(64 * (kFew ? 4 : kOutWaves), kFew ? 1 : 2) void tri
 
 // Workspace: weight fragments and their scales, the hi and lo planes, o.
 struct Layout {
-  size_t win, wout, scales, hi, lo, o, total;
+  size_t win, wout, scales, gains, flags, gain_bytes, hi, lo, o, total;
 };
 Layout layout(int64_t B, int64_t N) {
   Layout L;
@@ -325,6 +383,10 @@ Layout layout(int64_t B, int64_t N) {
   L.win = take((size_t)16 * kWBlock * 2);
   L.wout = take((size_t)8 * kWBlock * 2);
   L.scales = take((4 * D + 4 * D + 2 * D + 4 * D + 2 * D) * 4);
+  L.gains = off;   // and the flags, cleared together
+  L.flags = L.gains + (size_t)round_up((int64_t)gain_at((size_t)B * 2 * D, 0, 0, plane_ld((int)N)) + kGainPad, 16);
+  L.gain_bytes = L.flags + (size_t)B * 2 * D * 4 - L.gains;
+  take(L.gain_bytes);
   L.hi = take((size_t)B * 2 * D * plane * 2);
   L.lo = take((size_t)B * 2 * D * plane * 2);
   L.o = take((size_t)B * D * plane * 4);
@@ -354,6 +416,10 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
   mats.m[2] = with_fold(split_gemm_weight(p_out_w, wout, inv_out, nullptr, D, D), norm_out_w, norm_out_b, bias_out);
   mats.m[3] = with_fold(split_gemm_weight(g_out_w, wout + 4 * kWBlock, inv_out + D, nullptr, D, D), norm_in_w,
                         norm_in_b, bias_out + D);
+  uint8_t* gains = reinterpret_cast<uint8_t*>(base + L.gains);
+  uint32_t* flags = reinterpret_cast<uint32_t*>(base + L.flags);
+  mats.zero = gains;
+  mats.zero_bytes = L.gain_bytes;
   int rc = split_weights(mats, 4, stream);
   if (rc) return rc;
   const unsigned tiles = (unsigned)(B * N * (plane_ld((int)N) / 32));
@@ -365,7 +431,7 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
     while (parts < 8 && 2 * parts * wgs <= resident) parts *= 2;
     KernelTimerScope timed("f32_trimul_proj", stream);
     hipLaunchKernelGGL(trimul_planes_kernel, dim3(wgs, parts), dim3(256), 0, stream, x, mask, win, inv_in, norm_in,
-                       bias_in, hi, lo, (int)N, outgoing, tiles, 8 / (int)parts);
+                       bias_in, hi, lo, gains, flags, (int)N, outgoing, tiles, 8 / (int)parts);
   }
   if ((rc = check_launch("f32_trimul_proj"))) return rc;
   {
@@ -375,7 +441,7 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
     const int nt = (int)((N + 127) / 128), total = (int)(B * D) * nt * nt;
     KernelTimerScope timed("f32_trimul_contract", stream);
     hipLaunchKernelGGL(trimul_contract_kernel, dim3((unsigned)((total + 7) / 8 * 8)), dim3(256), kCSmem, stream, hi, lo,
-                       norm_in, o, (int)N, nt, total);
+                       norm_in, gains, flags, o, (int)N, nt, total);
   }
   if ((rc = check_launch("f32_trimul_contract"))) return rc;
   {

@@ -249,3 +249,36 @@ def test_valid_keys_below_the_masked_ones(gpu_device, c_s, heads, n, masked):
     with torch.no_grad():
         got = m.to(gpu_device)(s.to(gpu_device), z.to(gpu_device), mask.to(gpu_device))
     assert _worst_row(got, want) <= TOL
+
+
+def _trimul64(x, p, mode):
+    xn = _ln(x.double(), p, "norm_in")
+    a, b = ((xn @ p["p_in.weight"].T) * torch.sigmoid(xn @ p["g_in.weight"].T)).permute(0, 3, 1, 2).chunk(2, 1)
+    o = (a @ b.transpose(2, 3) if mode == "outgoing" else a.transpose(2, 3) @ b).permute(0, 2, 3, 1)
+    return (_ln(o, p, "norm_out") @ p["p_out.weight"].T) * torch.sigmoid(xn @ p["g_out.weight"].T)
+
+
+@pytest.mark.parametrize("mode", ["outgoing", "incoming"])
+@pytest.mark.parametrize("n", [33, 130])
+def test_triangle_planes_far_below_their_bound(gpu_device, mode, n):
+    """Rows of deviation down to 1e-9, and input gates near -25: the planes' values lie far below what the weights'
+    norms allow, in all lines and in some."""
+    torch.manual_seed(12)
+    m = randomize_params(TriangleMultiplicationHip(128, mode), 15)
+    _zero_biases(m)
+    mask = torch.ones(1, n, n, dtype=torch.bool, device=gpu_device)
+    d = m.to(gpu_device)
+    line = torch.randn(1, n, n, 128)
+    for dev in (1e-5, 1e-7, 1e-9):
+        for x in (line * dev, line * torch.where(torch.arange(n) % 5 == 0, 1.0, dev)[:, None, None],
+                  line * torch.where(torch.arange(n) % 5 == 0, 1.0, dev)[:, None]):
+            with torch.no_grad():
+                assert _worst_row(d(x.to(gpu_device), mask), _trimul64(x, _params(d), mode)) <= TOL
+    x = line.clone()
+    x[..., 0] = 30.0
+    with torch.no_grad():
+        d.g_in.weight.mul_(0.02)
+        d.g_in.weight[:, 0] = -25.0 * (1.0 + 900.0 / 128) ** 0.5 / 30.0
+        assert _worst_row(d(x.to(gpu_device), mask), _trimul64(x, _params(d), mode)) <= 8 * TOL   # two gates' arguments
+        d.g_in.weight[::2, 0] = 0.0   # every other channel open
+        assert _worst_row(d(x.to(gpu_device), mask), _trimul64(x, _params(d), mode)) <= TOL
