@@ -524,8 +524,8 @@ size_t attn_f32_layout(long long rows, int c_s, int heads, int64_t seq_len, long
   Carve c{base};
   AttnF32Buffers dummy;
   AttnF32Buffers* b = buf ? buf : &dummy;
-  b->sp.a = c.frags(rows, c_s);
-  b->sp.ainv = c.floats((size_t)rows);
+  b->sp.a = c.frags(c_s == 128 ? 0 : rows, c_s);   // rows of 128 channels are split in registers
+  b->sp.ainv = c.floats(c_s == 128 ? 0 : (size_t)rows);
   b->sp.w = c.frags(5 * (int64_t)c_s, c_s);
   b->sp.winv = c.floats((size_t)5 * c_s);
   b->q = c.floats((size_t)rows * c_s);
@@ -732,7 +732,18 @@ struct TransitionF32Buffers {
 // not depend on the output width.
 constexpr int64_t kTransitionOutRows = 1024;
 
+// Fewest rows for which split_transition_rows takes the call (none: 0).
+static int64_t transition_f32_fused_rows(int64_t Dc, int64_t hidden) {
+  if (hidden > kTransitionMaxHidden) return 0;
+  return Dc == 128 ? kTransitionFusedRows128 : Dc == 64 ? kTransitionFusedRows64 : 0;
+}
+
+// The separate products hold the row and hidden fragments of up to M rows, or of the row count at which the one-kernel
+// form, which needs neither, takes over: calls of more rows with another output width take the separate products that
+// many rows at a time.
 static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, TransitionF32Buffers* buf, char* base) {
+  const int64_t fused = transition_f32_fused_rows(Dc, hidden);
+  if (fused && M > fused) M = fused;
   Carve c{base};
   TransitionF32Buffers dummy;
   TransitionF32Buffers* b = buf ? buf : &dummy;
@@ -755,8 +766,8 @@ static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, Trans
 // 25 / 24, 16000 rows 25 / 28.  (590k rows 128 -> 256: 0.44 ms in one kernel.)  The two differ in the order of their
 // sums, so a row's last bits depend on the number of rows of its call; they never depend on the other rows' values.
 static bool transition_f32_fused(int64_t M, int64_t Dc, int64_t hidden, int64_t out_dim) {
-  return out_dim == Dc && hidden <= kTransitionMaxHidden &&
-         ((Dc == 128 && M >= kTransitionFusedRows128) || (Dc == 64 && M >= kTransitionFusedRows64));
+  const int64_t fused = transition_f32_fused_rows(Dc, hidden);
+  return out_dim == Dc && fused && M >= fused;
 }
 
 static int transition_f32_res(const float* x, const float* res, const float* norm_w, const float* norm_b,
@@ -768,6 +779,16 @@ static int transition_f32_res(const float* x, const float* res, const float* nor
   if (transition_f32_fused(M, Dc, hidden, out_dim))
     return split_transition_rows(x, residual ? res : nullptr, use_norm ? norm_w : nullptr, norm_b, fc1_w, fc2_w, fc3_w,
                                  buf.w12, buf.scales, out, M, (int)Dc, (int)hidden, stream, "f32_transition_rows");
+  const int64_t most = transition_f32_fused_rows(Dc, hidden);
+  if (most && M > most) {
+    for (int64_t m0 = 0; m0 < M; m0 += most) {
+      const int rc = transition_f32_res(x + m0 * Dc, res ? res + m0 * out_dim : nullptr, norm_w, norm_b, fc1_w, fc2_w,
+                                        fc3_w, out + m0 * out_dim, workspace, M - m0 < most ? M - m0 : most, Dc, hidden,
+                                        out_dim, use_norm, residual, stream);
+      if (rc) return rc;
+    }
+    return 0;
+  }
   const int64_t out0 = out_dim < kTransitionOutRows ? out_dim : kTransitionOutRows;
   SplitMats mats{};
   mats.m[0] = split_gemm_weight(fc1_w, buf.w12, buf.w12inv, nullptr, hidden, Dc, 2, 0);
@@ -830,7 +851,8 @@ extern "C" int bioemu_transition_fwd_f32(const float* x, const float* norm_w, co
 
 extern "C" size_t bioemu_pair_cond_f32_workspace_bytes(int64_t P, int64_t token_z, int64_t c_rel) {
   if (P <= 0 || token_z <= 0 || c_rel < 0) return 0;
-  // the normalised rows, or the projection's weight fragments
+  // the normalised rows of the general kernels (which take a z_trunk, rel or out of any alignment or overlap), or the
+  // weight fragments of the one-pass kernel
   const size_t rows = (size_t)round_up(P * (token_z + c_rel) * 4, 256);
   return rows > (size_t)(192 << 10) ? rows : (size_t)(192 << 10);
 }

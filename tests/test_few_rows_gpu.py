@@ -139,3 +139,17 @@ def test_triangle_multiplication_forms(gpu_device, mode, n, few, many):
         assert torch.equal(run(few, None, residual), run(many, None, residual)[:few])
     for b in (few, many):
         assert torch.equal(run(b, x[:b].clone(), True), run(b, None, True))
+
+
+@pytest.mark.parametrize("dim,rows", [(128, 18432), (128, 40000), (64, 12289)])
+def test_transition_of_another_width_many_rows(gpu_device, dim, rows):
+    """As many rows as the one-kernel form takes, with an output width it does not: the separate products, a part of the
+    rows at a time in a workspace that does not grow with them."""
+    torch.manual_seed(6)
+    m = randomize_params(Transition(dim, 96, out_dim=dim + 32), 8)
+    x = torch.randn(rows, dim)
+    want = _transition(x.double(), _params(m))
+    got, names = _run(m.to(gpu_device), x.to(gpu_device))
+    assert rel_l2(got.cpu(), want) <= TOL and "f32_transition_rows" not in names
+    need = [_ops.transition_f32_workspace_bytes(r, dim, 96) for r in (200, 12287, 12288, 18432, 600000)]
+    assert need == sorted(need) and need[-1] == need[-2]
