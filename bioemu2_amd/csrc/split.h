@@ -75,14 +75,18 @@ __device__ __forceinline__ float split_finite(float x) {
   return (__builtin_bit_cast(uint32_t, x) & 0x7fffffffu) == 0x7f800000u ? __builtin_copysignf(3.40282347e38f, x) : x;
 }
 
-// sigmoid(x) to about an ulp: the hardware exp2 on -x log2(e) carried as a rounded product and its error (a plain
-// product would cost |x| 2^-24 relative), and one Newton step on the hardware reciprocal.  Past +-87 the result is 1
+// log2(e) less its float value: the second part of a two-part constant.
+constexpr float kLog2eLow = (float)(1.4426950408889634074 - (double)kLog2e);
+
+// sigmoid(x) to about an ulp: the hardware exp2 on -x log2(e) carried as a rounded product and its error (the product of
+// the two-part constant by fused multiply-adds; a plain product would cost |x| 2^-24 relative), and one Newton step on
+// the hardware reciprocal.  Past +-87 the result is 1
 // or 2e-38, where an infinite x would make the product's error and the Newton step NaN; the clamp drops a NaN x, which
 // the last select returns (on its bits: the build lets the compiler fold x != x).
 __device__ __forceinline__ float sigmoid_ulp(float x) {
   const float y = -fminf(fmaxf(x, -87.f), 87.f);
   const float t = y * kLog2e;
-  const float r = __builtin_fmaf(y, 1.925963033500e-8f, __builtin_fmaf(y, kLog2e, -t));   // log2(e) - float(log2(e))
+  const float r = __builtin_fmaf(y, kLog2eLow, __builtin_fmaf(y, kLog2e, -t));
   float e = fast_exp2(t);
   e = __builtin_fmaf(e, r * 0.6931471805599453f, e);
   const float d = 1.0f + e, q = fast_rcp(d);
