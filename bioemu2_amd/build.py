@@ -23,9 +23,10 @@ ARCH = os.environ.get("BIOEMU_OFFLOAD_ARCH", "gfx950")
 
 # Packed-fp32 VALU ops are disabled for device code; the host pass warns that
 # it does not know the feature, which is harmless.
-# -fno-honor-nans: no kernel relies on NaN propagation (infinities are still
-# honoured: the softmax masks use -inf), and it lets fmaxf lower to a single
-# v_max_f32 instead of canonicalise + max.
+# -fno-honor-nans: lets fmaxf lower to a single v_max_f32 instead of
+# canonicalise + max.  Infinities are still honoured (the softmax masks use
+# -inf); a kernel that has to tell a NaN apart does so on its bits
+# (sigmoid_ulp), because the compiler may fold comparisons with one.
 # -amdgpu-mfma-vgpr-form: MFMA accumulators live in VGPRs, which removes the
 # AGPR<->VGPR copies around every softmax / epilogue touch of an accumulator.
 HIPCC_FLAGS = [

@@ -4,16 +4,18 @@
 // score_model.py:355, model.py:387), so its attention-with-pair-bias
 // (attention_pair_bias.py:128-225), sliding-window attention (:277-340) and
 // token transitions (transition.py:52-91) compute in fp32 on fp32 inputs.  These
-// entry points do the same: fp32 operands and fp32 accumulation throughout.
+// entry points do the same: fp32 inputs, weights and outputs, fp32 accumulation.
 //
-// The projections of the attentions, the transitions and the pairwise
-// conditioning run on split f16 operands (split.h, split_gemm.hip,
-// split_transition.hip, split_pair.hip): as accurate, and 2 to 5 times as fast.
-// Here:
+// The attentions (but for the sliding window's core), the transitions, the
+// pairwise conditioning and the 128-channel triangle multiplication carry each
+// fp32 operand as two f16 values (split.h, whose head states the errors and what
+// the form does not reach; split_gemm.hip, split_attn.hip, split_transition.hip,
+// split_pair.hip, split_trimul.hip).  Here:
 //
 //   gemm_f32      out = epi(A W^T) on v_mfma_f32_32x32x2_f32, for the products not
 //                 moved to split operands (the distogram, whose raw inputs may be
-//                 infinite, the trunk glue and the MSA-module ops).  A wave owns a
+//                 infinite, the trunk glue, the MSA-module ops, conditioning and
+//                 triangle multiplication of other widths).  A wave owns a
 //                 32 x 32 output block: weight rows (output channels) are the
 //                 MFMA A operand in perm32 order (pairtile.h), token rows the B
 //                 operand, so a lane ends with 16 consecutive channels of one
@@ -22,12 +24,13 @@
 //                 supplies k0 + 4h + e to MFMA e, the same k permutation on both
 //                 operands, so every k is summed once.
 //   rows_ln_f32   LayerNorm per row (biased variance, eps 1e-5), one wave per row.
-//   pair_proj_f32 pair bias of 16- and 32-channel pair rows: LN(z) W^T, one thread
-//                 per row, written head-major ([outer][head][inner]).
-//   attn_f32      softmax(q k^T / sqrt(d) + bias; masked keys -> -1e6) v, gated by
-//                 g: flash attention on the same fp32 MFMA, a wave per 32
-//                 queries, 32-key blocks, online softmax in registers.
-//   swa_attn_f32  the same over the sliding key window of each 32-atom window.
+//   pair_proj_f32 pair bias LN(z) W^T, one thread per row, written head-major
+//                 ([outer][head][inner]): 16- and 32-channel pair rows, PWA's
+//                 logits, more than 64 heads.
+//   swa_attn_f32  softmax(q k^T / sqrt(d) + bias; masked keys -> -1e6) v, gated by
+//                 g, over the sliding key window of each 32-atom window: flash
+//                 attention on the same fp32 MFMA, a wave per 32 queries, 32-key
+//                 blocks, online softmax in registers.
 #include <algorithm>
 #include <cmath>
 
@@ -763,7 +766,7 @@ static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, Trans
 // in order) are many enough.  Below it the three separate products deal columns and k-steps to workgroups too.  Both
 // times in us, one kernel / separate: 128 -> 256 channels, 200 rows 34 / 14, 4096 rows 36 / 21, 16000 rows 39 / 35,
 // 64000 rows 55 / 83; 128 -> 512, 1600 rows 58 / 24, 16000 rows 61 / 49; 64 -> 256, 8000 rows 24 / 19, 12000 rows
-// 25 / 24, 16000 rows 25 / 28.  (590k rows 128 -> 256: 0.44 ms in one kernel.)  The two differ in the order of their
+// 25 / 24, 16000 rows 25 / 28.  (590k rows 128 -> 256: 0.45 ms in one kernel.)  The two differ in the order of their
 // sums, so a row's last bits depend on the number of rows of its call; they never depend on the other rows' values.
 static bool transition_f32_fused(int64_t M, int64_t Dc, int64_t hidden, int64_t out_dim) {
   const int64_t fused = transition_f32_fused_rows(Dc, hidden);

@@ -10,15 +10,21 @@
 // MFMA's for K >= 64, because it rounds its accumulator K / 16 * 3 times
 // instead of K / 2 (relative error of a 32 x 32 block of normal data, measured:
 // K = 64 1.15e-7 vs 1.49e-7, K = 128 1.47e-7 vs 1.89e-7, K = 384 2.3e-7 vs
-// 3.5e-7, K = 1024 3.8e-7 vs 5.8e-7; K = 32 is a tie, so shorter products stay
-// off this path).
+// 3.5e-7, K = 1024 3.8e-7 vs 5.8e-7; K = 32 is a tie: attention's logits, K = 24
+// and 32, and transitions of fewer than 64 channels or hidden units gain time
+// only, and one product alone has up to twice the error of its fp32 form).
 //
 // Range: the scale brings the largest magnitude of a row (of activations or of
 // weights) into [2^14, 2^15).  hi + lo is then exact to 2^-23 relative for
 // elements down to 2^-16 of that maximum and to 2^-39 of the maximum below it
 // (the f16 MFMA multiplies subnormals).  A scale depends on its own row (or on
 // the weights) alone, so a row's result never depends on another row, nor an
-// output channel's error on another channel's weights.
+// output channel's error on another channel's weights.  What a scale does not
+// reach: inside one row, elements below 2^-16 of the row's largest keep fewer
+// bits than fp32, which shows where the others' weights are that much smaller
+// (a channel 1e5, 1e6, 1e7 times the rest under zero weights, through a whole
+// transition: 2e-7, 8e-7, 1.3e-5; fp32 operands: 4e-7); the same holds for the hidden values of a row (per 32 of them, or since the row's
+// largest so far) and for 32 keys' K and V of a head.
 //
 // Operand fragments: 32 rows x 16 k are 1 KB of hi followed by 1 KB of lo,
 // lane (n, h) = 8 consecutive values, row n, k = 8 h .. 8 h + 7.  Weight rows

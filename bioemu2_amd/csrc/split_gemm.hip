@@ -17,9 +17,9 @@
 //
 // Measured on the denoiser's shapes, against the fp32-MFMA kernels (operands from L2,
 // a wave per 32 x 32 block) these replace: q, k, v, g of 6144 rows, K = 384, 0.131 ->
-// 0.039 ms (186 TFLOP/s of fp32 products); of 49152 rows, K = 128, 0.127 -> 0.052 ms
-// (125 MB, bound by its stores); output projections 0.039 -> 0.017 and 0.032 -> 0.018;
-// 200 rows, K = 384 and 768 (small kernel): 0.023 -> 0.007 and 0.028 -> 0.009 ms.  The
+// 0.041 ms (178 TFLOP/s of fp32 products); of 49152 rows, K = 128, 0.127 -> 0.046 ms
+// (125 MB, bound by its stores); output projections 0.039 -> 0.018 and 0.032 -> 0.019;
+// 200 rows, K = 384 and 768 (small kernel): 0.023 -> 0.007 and 0.028 -> 0.008 ms.  The
 // tiled kernel is bound by LDS: 8 fragment reads and 8 staged KB per 12 MFMAs.
 #include <algorithm>
 

@@ -2,9 +2,9 @@
 // the rows each: a wave normalises 32 rows in registers and multiplies them with
 // weights that stay in LDS for the whole launch (grid of resident workgroups,
 // waves walking row tiles).  Both are bound by reading the rows: the conditioning
-// projection (590k rows of 256, 906 MB) takes 0.217 ms, 4.2 TB/s, against 1.17 ms for
+// projection (590k rows of 256, 906 MB) takes 0.214 ms, 4.2 TB/s, against 1.17 ms for
 // a LayerNorm pass and an fp32-MFMA product; the 16-head pair bias (590k rows of 128,
-// 340 MB) 0.076 ms, 4.5 TB/s (a copy on this card: 4.9), against 0.109 ms for one
+// 340 MB) 0.078 ms, 4.4 TB/s (a stream read and written on this card: 6.3), against 0.109 ms for one
 // thread per row on the VALU.  Rows requested a tile ahead and biases read from LDS
 // (a global load in the epilogue waits for the stores before it) took it from 0.097.
 #include <algorithm>

@@ -17,9 +17,9 @@
 // Few rows take the separate products of split_gemm.hip instead (the rule and both times: fp32.hip).
 //
 // Bound by the matrix cores and the gating VALU work of the same waves (two waves per
-// SIMD): 590k rows, 128 -> 256, 0.44 ms (262 TFLOP/s of fp32 products, 787 of f16)
+// SIMD): 590k rows, 128 -> 256, 0.45 ms (259 TFLOP/s of fp32 products, 776 of f16)
 // against 2.1 ms for LayerNorm, SwiGLU and output products on fp32 MFMA through
-// memory; 111k rows, 128 -> 512: 0.143 ms against 0.67.
+// memory; 111k rows, 128 -> 512: 0.151 ms against 0.67.
 #include "split.h"
 #include "split_rows.h"
 

@@ -18,8 +18,8 @@
 //
 // N = 333, against the fp32-MFMA kernels these replace (operands from L2, the contraction stored 4 bytes at a time
 // pair-major, LayerNorms and the gate through memory): projection 0.079 ms (was 0.283, with 0.030 of zero fill and
-// 0.042 of LayerNorm), contraction 0.057 (0.376; 166 TFLOP/s of fp32 products on the padded 384 x 384 x 352, bound by
-// LDS like split_gemm_kernel), output 0.057 (0.226, with 0.042 of LayerNorm and 0.067 of gate).  The sigmoids
+// 0.042 of LayerNorm), contraction 0.054 (0.376; 174 TFLOP/s of fp32 products on the padded 384 x 384 x 352, bound by
+// LDS like split_gemm_kernel), output 0.055 (0.226, with 0.042 of LayerNorm and 0.067 of gate).  The sigmoids
 // keep an ulp's accuracy: with the plain hardware exp2 and reciprocal the result was 1.4 times as far from float64.
 #include <algorithm>
 

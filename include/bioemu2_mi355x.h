@@ -7,12 +7,12 @@
  *
  * Data types:
  *   activations  bf16, channel-last ([B, N, N, C] pair tensors, [B, N, C] singles)
- *   masks        uint8 0/1
+ *   masks        uint8, nonzero = valid
  *   LayerNorm    gamma/beta fp32
  *   Linear       weights bf16, row-major [out, in] (torch nn.Linear layout)
  * Arithmetic: bf16 MFMA operands with fp32 accumulation; LayerNorm statistics,
  * softmax and gates in fp32.  The *_f32 entry points (end of this file) take
- * fp32 activations and weights and compute in fp32 throughout.
+ * fp32 activations and weights and accumulate in fp32.
  *
  * Scratch memory is caller-owned: each op with intermediates has a
  * *_workspace_bytes() query and takes (workspace, workspace_bytes).

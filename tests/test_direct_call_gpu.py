@@ -5,8 +5,11 @@ import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from bioemu2_amd import _ops
-from bioemu2_amd.attention_pair_bias import AttentionPairBiasSlidingWindow
+from bioemu2_amd.attention_pair_bias import AttentionPairBias, AttentionPairBiasSlidingWindow
+from bioemu2_amd.outer_product_mean import OuterProductMeanHip
+from bioemu2_amd.pair_weighted_averaging import PairWeightedAveraging
 from bioemu2_amd.transition import Transition
+from bioemu2_amd.triangle_attention import TriangleAttentionHip
 from bioemu2_amd.triangle_multiplication import TriangleMultiplicationHip
 from tests._helpers import randomize_params
 
@@ -125,3 +128,34 @@ def test_replaced_parameters_are_seen(gpu_device):
         del m.fc3.weight
         with pytest.raises(AttributeError):
             m(x)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["trimul", "triatt", "apb", "swa", "opm", "pwa"])
+def test_any_nonzero_byte_is_valid(gpu_device, kind, dtype):
+    """uint8 masks reach every kernel as they are."""
+    torch.manual_seed(4)
+    n, d = 37, gpu_device
+    z, pair = torch.randn(1, n, n, 128).to(dtype), torch.rand(1, n, n) < 0.7
+    pair[0, 3] = False
+    if kind == "trimul":
+        m, args, mask = TriangleMultiplicationHip(128), (z,), pair
+    elif kind == "triatt":
+        m, args, mask = TriangleAttentionHip(128, 4), (z,), pair
+    elif kind == "apb":
+        m, args, mask = AttentionPairBias(384, 128, 16), (torch.randn(1, n, 384).to(dtype), z), torch.rand(1, n) < 0.7
+    elif kind == "swa":
+        m = AttentionPairBiasSlidingWindow(128, 16, 4)
+        args = (torch.randn(3, 32, 128).to(dtype), torch.randn(1, 3, 32, 128, 16).to(dtype))
+        mask = torch.rand(3, 32) < 0.7
+    elif kind == "opm":
+        m, args, mask = OuterProductMeanHip(64, 32, 128), (torch.randn(1, 9, n, 64).to(dtype),), torch.rand(1, 9, n) < 0.7
+        mask[0, 2] = False
+    else:
+        m, args, mask = PairWeightedAveraging(64, 128, 32, 8), (torch.randn(1, 9, n, 64).to(dtype), z), pair
+    m = randomize_params(m, 5).to(d).eval()
+    args = [a.to(d) for a in args]
+    values = torch.randint(1, 256, mask.shape, dtype=torch.uint8) * mask.to(torch.uint8)
+    with torch.no_grad():
+        want = m(*args, mask.to(d))
+        assert torch.isfinite(want).all() and torch.equal(m(*args, values.to(d)), want)

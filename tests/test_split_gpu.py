@@ -1,9 +1,10 @@
 """fp32 products on split f16 operands (csrc/split.h): tile edges, row counts and value ranges.
 
 The reference is float64 on the CPU.  Bound: an operand is exact to 2^-23 and a sum of K products rounds its fp32
-accumulator 3 K / 16 times, each by at most 2^-24 of a partial sum that is about the result's size, so the relative
-2-norm error stays below (sqrt(3 K / 16) + 2) * 2^-23 per product; two products in a row and the activation between
-them (2^-21) add up to TOL for every width below.
+accumulator 3 K / 16 times, each by at most 2^-24 of a partial sum that is about the result's size.  The roundings are
+independent, so the relative 2-norm error of a product is about (sqrt(3 K / 16) / 2 + 2) * 2^-24: 4e-7 for K = 384, 7e-7
+for the widest below (2080).  Two products in a row, a softmax or the activation between them (2^-21 at most) and a
+LayerNorm stay below 2e-6; TOL is twice that.
 """
 
 import math
@@ -39,11 +40,11 @@ def _transition(x, p, use_norm=True):
 @pytest.mark.parametrize(
     "dim,hidden,out_dim,use_norm,rows",
     [
-        (128, 32, None, True, 1),        # fused kernel: one hidden chunk, one row
-        (128, 256, None, True, 255),     # a workgroup's rows less one
+        (128, 32, None, True, 1),        # one row, one block of hidden channels (the one-kernel form: test_few_rows_gpu.py)
+        (128, 256, None, True, 255),
         (128, 512, None, False, 257),
-        (128, 2048, None, True, 300),    # its widest hidden dimension
-        (128, 2080, None, True, 70),     # one past it: the separate products
+        (128, 2048, None, True, 300),
+        (128, 2080, None, True, 70),
         (64, 256, None, True, 513),
         (64, 128, None, False, 31),
         (384, 768, None, True, 33),      # 32 x 64 tiles, k-steps split over the waves
@@ -64,7 +65,7 @@ def test_transition_split_edges(gpu_device, dim, hidden, out_dim, use_norm, rows
 
 @pytest.mark.parametrize("dim,rows", [(128, 300), (384, 300), (384, 4200)])
 def test_transition_split_ranges(gpu_device, dim, rows):
-    """Row magnitudes from 1e-12 to 1e12 in one call, checked row by row: each row has its own scale."""
+    """Row magnitudes from 1e-12 to 1e12 in one call, checked row by row: each row has its own scales."""
     torch.manual_seed(1)
     m = randomize_params(Transition(dim, 256, use_norm=False), 3)
     x = torch.randn(rows, dim) * torch.logspace(-12, 12, rows)[:, None]
