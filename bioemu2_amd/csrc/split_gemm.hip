@@ -441,6 +441,14 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
       scn[i] = ainv[(size_t)(ks0 / 2) * M + (m < M ? m : M - 1)];
     }
   };
+  f32x16 part[2][2];   // [column block][row block]: a stage's products, not yet added
+  float scp[2] = {0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) part[1][i] = zero16();
+  auto add_part = [&](int j, const float (&s)[2], int q) {   // a quarter of column block j's
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[j][q >> 1][8 * (q & 1) + t] += part[j][q >> 1][8 * (q & 1) + t] * s[q >> 1];
+  };
   if (kEpi == kSplitHidden) load_scales(0);
   stage(0);
 #pragma unroll 1
@@ -465,16 +473,21 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
       }
     __builtin_amdgcn_sched_barrier(0);
     if (kEpi == kSplitHidden) {
+      // a column block's sums (the other's of the stage before, this one's) between the other's products
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j) {
+        f32x16 p0 = zero16(), p1 = zero16();
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          f32x16 part = zero16();
-#pragma unroll
-          for (int ks = 0; ks < kStageKs; ++ks) mfma_split(fw[ks][j], fa[ks][i], part);
-#pragma unroll
-          for (int u = 0; u < 16; ++u) acc[j][i][u] += part[u] * sc[i];
+        for (int q = 0; q < 4; ++q) {
+          mfma_split(fw[q & 1][j], fa[q & 1][q >> 1], q < 2 ? p0 : p1);
+          add_part(1 - j, j ? sc : scp, q);
+          __builtin_amdgcn_sched_barrier(0);
         }
+        part[j][0] = p0;
+        part[j][1] = p1;
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) scp[i] = sc[i];
     } else {
 #pragma unroll
       for (int ks = 0; ks < kStageKs; ++ks)
@@ -484,6 +497,9 @@ __global__ __launch_bounds__(256, 2) void split_gemm_kernel(const f16* __restric
           for (int i = 0; i < 2; ++i) mfma_split(fw[ks][j], fa[ks][i], acc[j][i]);
     }
   }
+  if (kEpi == kSplitHidden)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) add_part(1, scp, q);
   const int cb0 = nt * 4 + wn * 2;
   if (cb0 >= nblocks) return;
   // the weight rows' scales, read before the first store
