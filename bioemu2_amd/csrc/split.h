@@ -21,10 +21,11 @@
 // the weights) alone, so a row's result never depends on another row, nor an
 // output channel's error on another channel's weights.  What a scale does not
 // reach: inside one row, elements below 2^-16 of the row's largest keep fewer
-// bits than fp32, which shows where the others' weights are that much smaller
-// (a channel 1e5, 1e6, 1e7 times the rest under zero weights, through a whole
-// transition: 2e-7, 8e-7, 1.3e-5; fp32 operands: 4e-7); the same holds for the hidden values of a row (per 32 of them, or since the row's
-// largest so far) and for 32 keys' K and V of a head.
+// bits than fp32, which shows where the others' weights are that much smaller (a
+// channel 1e5, 1e6, 1e7 times the rest under zero weights, through a whole
+// transition: 2e-7, 8e-7, 1.3e-5; fp32 operands: 4e-7).  The same holds for a
+// row's hidden values (per 32 of them, or up to the largest so far) and for 32
+// keys' K and V of a head.
 //
 // Operand fragments: 32 rows x 16 k are 1 KB of hi followed by 1 KB of lo,
 // lane (n, h) = 8 consecutive values, row n, k = 8 h .. 8 h + 7.  Weight rows
@@ -67,6 +68,13 @@ __device__ __forceinline__ float split_scale(float amax) {
 // 1 / s of a power of two s from split_scale (exact).
 __device__ __forceinline__ float split_inv(float s) {
   return __builtin_bit_cast(float, (uint32_t)(254 - (int)(__builtin_bit_cast(uint32_t, s) >> 23)) << 23);
+}
+
+// The larger of x in lanes l and l ^ 32: the halves exchanged by one VALU instruction instead of a trip through LDS.
+__device__ __forceinline__ float max_halves(float x) {
+  const unsigned b = __builtin_bit_cast(unsigned, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
 }
 
 // x * s as hi + lo.  s is a power of two: the compiler may round the product to f16 in one step for hi and in two

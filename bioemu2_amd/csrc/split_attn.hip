@@ -113,7 +113,8 @@ __global__ __launch_bounds__(256) void kv_fragments_kernel(const float* __restri
 // by queries that a masked key's weight matters to.
 template <int HD>
 __device__ __forceinline__ void attend_all_keys(const float* qr, const float* kb, const float* vb, const uint8_t* mask,
-                                             const float* brow, int N, int c_s, float qscale, int h, float (&o)[16], float& l) {
+                                                const float* brow, int N, int c_s, float qscale, int h, float (&o)[16],
+                                                float& l) {
   float q[HD];
 #pragma unroll
   for (int c = 0; c < HD; ++c) q[c] = qr[c];
@@ -347,7 +348,8 @@ int launch(const SplitAttn& a, hipStream_t stream, const char* name) {
   KernelTimerScope timed(name, stream);
   const float qscale = kLog2e / sqrtf((float)HD);
   hipLaunchKernelGGL(attn_split_kernel<HD>, dim3((unsigned)((total + 7) / 8 * 8)), dim3(256), 0, stream, a.q, a.kv,
-                     a.kvinv, a.words, a.g, a.bias, a.k, a.v, a.mask, a.go, a.N, nkb, a.ld, a.H, a.c_s, a.mult, qscale, a.mask_per_copy,
+                     a.kvinv, a.words, a.g, a.bias, a.k, a.v, a.mask, a.go, a.N, nkb, a.ld, a.H, a.c_s, a.mult, qscale,
+                     a.mask_per_copy,
                      nqb, (int)total);
   return check_launch(name);
 }

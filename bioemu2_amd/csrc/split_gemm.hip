@@ -132,7 +132,8 @@ __device__ __forceinline__ void split_weight_block(const SplitMat& m, int rb) {
 __global__ __launch_bounds__(64 * kSwWaves) void split_weights_kernel(SplitMats mats, int count) {
   if ((int)blockIdx.y == count) {
     uint4* p = static_cast<uint4*>(mats.zero);
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < mats.zero_bytes / 16; i += (size_t)gridDim.x * blockDim.x)
+    const size_t step = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < mats.zero_bytes / 16; i += step)
       p[i] = uint4{0, 0, 0, 0};
     return;
   }
@@ -385,7 +386,8 @@ __device__ __forceinline__ void epi_hidden_quad(const SplitGemmEpi& e, long long
     hi[t] = x;
     lo[t] = y;
   }
-  f16* d = e.hfrag + ((size_t)(m >> 5) * e.hsteps + (c >> 4)) * kFrag + (((c >> 3) & 1) * 32 + (int)(m & 31)) * 8 + (c & 4);
+  f16* d = e.hfrag + ((size_t)(m >> 5) * e.hsteps + (c >> 4)) * kFrag +
+           (((c >> 3) & 1) * 32 + (int)(m & 31)) * 8 + (c & 4);
   *reinterpret_cast<f16x4*>(d) = hi;
   *reinterpret_cast<f16x4*>(d + kFragHalf) = lo;
 }
@@ -737,8 +739,9 @@ int split_gemm_r128(int epi, const float* x, const f16* W, const float* winv, co
   const dim3 grid((unsigned)wgs, (unsigned)((nblocks + per - 1) / per));
   if (N > kR128MaxN) return set_error(BIOEMU_ERR_UNSUPPORTED, "%s: %d output channels", name, N);
   KernelTimerScope timed(name, stream);
-#define BIOEMU_R128(E, L) \
-  hipLaunchKernelGGL((split_gemm_r128_kernel<E, L>), grid, dim3(256), 0, stream, x, W, winv, wbias, e, M, N / 32, (int)per)
+#define BIOEMU_R128(E, L)                                                                                        \
+  hipLaunchKernelGGL((split_gemm_r128_kernel<E, L>), grid, dim3(256), 0, stream, x, W, winv, wbias, e, M, N / 32, \
+                     (int)per)
   if (epi == kSplitStore && !wbias)
     BIOEMU_R128(kSplitStore, false);
   else if (epi == kSplitQkvg && !wbias)
@@ -757,8 +760,8 @@ int split_weights(const SplitMats& mats, int count, hipStream_t stream) {
   // the memory to clear: 64 KB a workgroup, beside the weights
   if (mats.zero_bytes) blocks = std::max(blocks, (int)std::min<size_t>((mats.zero_bytes + 65535) / 65536, 2048));
   KernelTimerScope timed("f32_split_weights", stream);
-  hipLaunchKernelGGL(split_weights_kernel, dim3(blocks, count + (mats.zero_bytes ? 1 : 0)), dim3(64 * kSwWaves), 0, stream,
-                     mats, count);
+  const dim3 grid(blocks, count + (mats.zero_bytes ? 1 : 0));
+  hipLaunchKernelGGL(split_weights_kernel, grid, dim3(64 * kSwWaves), 0, stream, mats, count);
   return check_launch("f32_split_weights");
 }
 

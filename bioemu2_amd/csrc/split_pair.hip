@@ -4,8 +4,8 @@
 // waves walking row tiles).  Both are bound by reading the rows: the conditioning
 // projection (590k rows of 256, 906 MB) takes 0.214 ms, 4.2 TB/s, against 1.17 ms for
 // a LayerNorm pass and an fp32-MFMA product; the 16-head pair bias (590k rows of 128,
-// 340 MB) 0.078 ms, 4.4 TB/s (a stream read and written on this card: 6.3), against 0.109 ms for one
-// thread per row on the VALU.  Rows requested a tile ahead and biases read from LDS
+// 340 MB) 0.078 ms, 4.4 TB/s (a stream read and written on this card: 6.3), against
+// 0.109 ms for one thread per row on the VALU.  Rows requested a tile ahead and biases read from LDS
 // (a global load in the epilogue waits for the stores before it) took it from 0.097.
 #include <algorithm>
 
@@ -53,7 +53,8 @@ __global__ __launch_bounds__(64 * kCatWaves, 2) void cat_proj_f32_kernel(
         a[i] -= mean;
         c[i] -= mean;
       }
-      const float var = row_sum<128>([&](int i) { return a[i] * a[i] + c[i] * c[i]; }) * (1.0f / 256.0f), rstd = 1.0f / sqrtf(var + 1e-5f), gain = norm_gain(var * rstd * rstd);
+      const float var = row_sum<128>([&](int i) { return a[i] * a[i] + c[i] * c[i]; }) * (1.0f / 256.0f);
+      const float rstd = 1.0f / sqrtf(var + 1e-5f), gain = norm_gain(var * rstd * rstd);
       split_normalized<128>(a, rstd, gain, xf);
       split_normalized<128>(c, rstd, gain, xf + 8);
       xinv = split_inv(gain);
@@ -146,7 +147,8 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
   const int grid = std::min((tiles + waves - 1) / waves, cus);
   KernelTimerScope timed(name, stream);
   hipLaunchKernelGGL(cat_proj_f32_kernel, dim3((unsigned)grid, 4 / per), dim3(64 * waves),
-                     kCatScales + per * 16 * kFrag * (int)sizeof(f16), stream, x1, x2, W, winv, wbias, out, P, tiles, per);
+                     kCatScales + per * 16 * kFrag * (int)sizeof(f16), stream, x1, x2, W, winv, wbias, out, P, tiles,
+                     per);
   return check_launch(name);
 }
 

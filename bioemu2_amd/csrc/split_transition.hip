@@ -100,7 +100,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void transition_rows_f32_kernel(
       hv[u] = p * sigmoidf_fast(p) * q;
       amax = fmaxf(amax, fabsf(hv[u]));
     }
-    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    amax = max_halves(amax);
     if (__any(amax * hs >= 32768.f)) {   // each row for itself
       const float ns = amax * hs >= 32768.f ? split_scale(amax) * 0.125f : hs, ratio = ns * split_inv(hs);
 #pragma unroll

@@ -22,6 +22,7 @@
 // LDS like split_gemm_kernel), output 0.055 (0.226, with 0.042 of LayerNorm and 0.067 of gate).  The sigmoids
 // keep an ulp's accuracy: with the plain hardware exp2 and reciprocal the result was 1.4 times as far from float64.
 #include <algorithm>
+#include <type_traits>
 
 #include "split.h"
 #include "split_rows.h"
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(256, 2) void trimul_planes_kernel(const float* __re
       v[u] = (keep >> u) & 1u ? (p[u] * sp + bp) * sigmoid_ulp(g[u] * sg + bg) : 0.f;
       amax = fmaxf(amax, fabsf(v[u]));
     }
-    amax = fmaxf(amax, __shfl_xor(amax, 32));
+    amax = max_halves(amax);
     const bool low = amax * s < kGainBelow && amax > 0.f;
     if (__any(low)) {
       const float s2 = low ? split_scale(amax) : s;
@@ -200,57 +201,68 @@ __global__ __launch_bounds__(256, 2) void trimul_contract_kernel(const f16* __re
   const size_t cha = (size_t)b * 2 * D + d, chb = cha + D;
   const bool flagged = flags[cha] | flags[chb];   // uniform over the workgroup
   stage(0);
+  auto run = [&](auto gained) {   // two loops: the one without gains is free of their registers and branches
 #pragma unroll 1
-  for (int kt = 0; kt < nk; ++kt) {
-    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies of the stage landed
-    __syncthreads();                       // ... and everyone's; the other stage is free again
-    if (kt + 1 < nk) stage(kt + 1);
-    const f16* st = smem + (kt & 1) * kCStage;
-    SplitFrag fa[2][2], fb[2][2];
+    for (int kt = 0; kt < nk; ++kt) {
+      __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies of the stage landed
+      __syncthreads();                       // ... and everyone's; the other stage is free again
+      if (kt + 1 < nk) stage(kt + 1);
+      const f16* st = smem + (kt & 1) * kCStage;
+      SplitFrag fa[2][2], fb[2][2];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const int ra = wi * 64 + x * 32 + n, rb = wj * 64 + x * 32 + n;
-        const int oa = (ra * 4 + ((2 * ks + h) ^ swz(ra))) * 8, ob = (rb * 4 + ((2 * ks + h) ^ swz(rb))) * 8;
-        fa[ks][x].hi = *reinterpret_cast<const f16x8*>(st + oa);
-        fa[ks][x].lo = *reinterpret_cast<const f16x8*>(st + kPart + oa);
-        fb[ks][x].hi = *reinterpret_cast<const f16x8*>(st + 2 * kPart + ob);
-        fb[ks][x].lo = *reinterpret_cast<const f16x8*>(st + 3 * kPart + ob);
+        for (int x = 0; x < 2; ++x) {
+          const int ra = wi * 64 + x * 32 + n, rb = wj * 64 + x * 32 + n;
+          const int oa = (ra * 4 + ((2 * ks + h) ^ swz(ra))) * 8, ob = (rb * 4 + ((2 * ks + h) ^ swz(rb))) * 8;
+          fa[ks][x].hi = *reinterpret_cast<const f16x8*>(st + oa);
+          fa[ks][x].lo = *reinterpret_cast<const f16x8*>(st + kPart + oa);
+          fb[ks][x].hi = *reinterpret_cast<const f16x8*>(st + 2 * kPart + ob);
+          fb[ks][x].lo = *reinterpret_cast<const f16x8*>(st + 3 * kPart + ob);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+      if (gained.value) {
+        uint32_t ga[2][4], some = 0;   // ga: four rows each
+        int gb[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int row = it * 128 + wi * 64 + x * 32 + 8 * q + 4 * h;
+            ga[x][q] = *reinterpret_cast<const uint32_t*>(gains + gain_at(cha, kt, row, ld));
+            some |= ga[x][q];
+          }
+          gb[x] = gains[gain_at(chb, kt, jt * 128 + wj * 64 + x * 32 + n, ld)];
+          some |= gb[x];
+        }
+        if (__any(some != 0)) {
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) {
+              f32x16 part = zero16();
+#pragma unroll
+              for (int ks = 0; ks < 2; ++ks) mfma_split(fa[ks][x], fb[ks][y], part);
+#pragma unroll
+              for (int u = 0; u < 16; ++u)
+                acc[x][y][u] +=
+                    __builtin_amdgcn_ldexpf(part[u], -((int)(ga[x][u >> 2] >> (8 * (u & 3)) & 0xffu) + gb[y]));
+            }
+          continue;
+        }
       }
-    __builtin_amdgcn_sched_barrier(0);
-    if (flagged) {
-      uint32_t ga[2][4];   // four rows each
-      int gb[2];
 #pragma unroll
-      for (int x = 0; x < 2; ++x) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          ga[x][q] = *reinterpret_cast<const uint32_t*>(gains + gain_at(cha, kt, it * 128 + wi * 64 + x * 32 + 8 * q + 4 * h, ld));
-        gb[x] = gains[gain_at(chb, kt, jt * 128 + wj * 64 + x * 32 + n, ld)];
-      }
-      if (__any(ga[0][0] | ga[0][1] | ga[0][2] | ga[0][3] | ga[1][0] | ga[1][1] | ga[1][2] | ga[1][3] | gb[0] | gb[1])) {
+      for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
         for (int x = 0; x < 2; ++x)
 #pragma unroll
-          for (int y = 0; y < 2; ++y) {
-            f32x16 part = zero16();
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) mfma_split(fa[ks][x], fb[ks][y], part);
-#pragma unroll
-            for (int u = 0; u < 16; ++u)
-              acc[x][y][u] += __builtin_amdgcn_ldexpf(part[u], -((int)(ga[x][u >> 2] >> (8 * (u & 3)) & 0xffu) + gb[y]));
-          }
-        continue;
-      }
+          for (int y = 0; y < 2; ++y) mfma_split(fa[ks][x], fb[ks][y], acc[x][y]);
     }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y) mfma_split(fa[ks][x], fb[ks][y], acc[x][y]);
-  }
+  };
+  if (flagged)
+    run(std::true_type{});
+  else
+    run(std::false_type{});
   // lane n: column j, register u: row 8 (u / 4) + 4 h + u % 4; a store covers 128 bytes of two rows
   const int dw = d / 32 * 64 + d % 32;   // channel d's place among the p rows' norms
   const float s = split_inv(split_scale(wnorm[dw] * 1.01f)) * split_inv(split_scale(wnorm[dw + 2 * D] * 1.01f));
