@@ -25,7 +25,8 @@
 // channel 1e5, 1e6, 1e7 times the rest under zero weights, through a whole
 // transition: 2e-7, 8e-7, 1.3e-5; fp32 operands: 4e-7).  The same holds for a
 // row's hidden values (per 32 of them, or up to the largest so far) and for 32
-// keys' K and V of a head.
+// keys' K and V of a head.  An infinite operand has no second part: its products
+// are no numbers, where fp32 gives infinities (hidden values excepted).
 //
 // Operand fragments: 32 rows x 16 k are 1 KB of hi followed by 1 KB of lo,
 // lane (n, h) = 8 consecutive values, row n, k = 8 h .. 8 h + 7.  Weight rows
