@@ -741,12 +741,13 @@ static int64_t transition_f32_fused_rows(int64_t Dc, int64_t hidden) {
   return Dc == 128 ? kTransitionFusedRows128 : Dc == 64 ? kTransitionFusedRows64 : 0;
 }
 
-// The separate products hold the row and hidden fragments of up to M rows, or of the row count at which the one-kernel
-// form, which needs neither, takes over: calls of more rows with another output width take the separate products that
-// many rows at a time.
+// Most rows the separate products hold fragments of: four times the row count at which the one-kernel form, which needs
+// none, takes over.  Calls of more rows with another output width take the separate products that many at a time.
+static int64_t transition_f32_most_rows(int64_t Dc, int64_t hidden) { return 4 * transition_f32_fused_rows(Dc, hidden); }
+
 static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, TransitionF32Buffers* buf, char* base) {
-  const int64_t fused = transition_f32_fused_rows(Dc, hidden);
-  if (fused && M > fused) M = fused;
+  const int64_t most = transition_f32_most_rows(Dc, hidden);
+  if (most && M > most) M = most;
   Carve c{base};
   TransitionF32Buffers dummy;
   TransitionF32Buffers* b = buf ? buf : &dummy;
@@ -764,9 +765,9 @@ static size_t transition_f32_layout(int64_t M, int64_t Dc, int64_t hidden, Trans
 
 // Rows of 64 or 128 channels in one kernel, from the row count on at which its workgroups (256 rows, every hidden chunk
 // in order) are many enough.  Below it the three separate products deal columns and k-steps to workgroups too.  Both
-// times in us, one kernel / separate: 128 -> 256 channels, 200 rows 34 / 14, 4096 rows 36 / 21, 16000 rows 39 / 35,
-// 64000 rows 55 / 83; 128 -> 512, 1600 rows 58 / 24, 16000 rows 61 / 49; 64 -> 256, 8000 rows 24 / 19, 12000 rows
-// 25 / 24, 16000 rows 25 / 28.  (590k rows 128 -> 256: 0.45 ms in one kernel.)  The two differ in the order of their
+// times in us, one kernel / separate: 128 -> 256 channels, 200 rows 34 / 13, 4096 rows 36 / 20, 16000 rows 38 / 35,
+// 64000 rows 55 / 83; 128 -> 512, 1600 rows 57 / 23, 16000 rows 61 / 49; 64 -> 256, 8000 rows 25 / 19, 12000 rows
+// 25 / 24, 16000 rows 26 / 28.  (590k rows 128 -> 256: 0.45 ms in one kernel.)  The two differ in the order of their
 // sums, so a row's last bits depend on the number of rows of its call; they never depend on the other rows' values.
 static bool transition_f32_fused(int64_t M, int64_t Dc, int64_t hidden, int64_t out_dim) {
   const int64_t fused = transition_f32_fused_rows(Dc, hidden);
@@ -782,7 +783,7 @@ static int transition_f32_res(const float* x, const float* res, const float* nor
   if (transition_f32_fused(M, Dc, hidden, out_dim))
     return split_transition_rows(x, residual ? res : nullptr, use_norm ? norm_w : nullptr, norm_b, fc1_w, fc2_w, fc3_w,
                                  buf.w12, buf.scales, out, M, (int)Dc, (int)hidden, stream, "f32_transition_rows");
-  const int64_t most = transition_f32_fused_rows(Dc, hidden);
+  const int64_t most = transition_f32_most_rows(Dc, hidden);
   if (most && M > most) {
     for (int64_t m0 = 0; m0 < M; m0 += most) {
       const int rc = transition_f32_res(x + m0 * Dc, res ? res + m0 * out_dim : nullptr, norm_w, norm_b, fc1_w, fc2_w,

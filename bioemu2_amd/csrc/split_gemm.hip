@@ -732,8 +732,8 @@ __global__ __launch_bounds__(256, 3) void split_gemm_r128_kernel(const float* __
 int split_gemm_r128(int epi, const float* x, const f16* W, const float* winv, const float* wbias,
                     const SplitGemmEpi& e, long long M, int N, hipStream_t stream, const char* name) {
   // As many parts of the columns as fill three workgroups per CU (its resident number): the parts read the same rows,
-  // from L2, and compute the same bits.  Atom attention (us, with one part / this many): 384 rows 62 / 32, 6144 rows
-  // 69 / 46, 12288 rows 86 / 67, 28800 rows 96 / 85, 49152 rows 145 / 138; one workgroup per CU: 32, 47, 71, 96, 145.
+  // from L2, and compute the same bits.  Atom attention (us, with one part / this many): 384 rows 66 / 32, 6144 rows
+  // 75 / 47, 12288 rows 91 / 68, 23040 rows 101 / 87, 49152 rows 151 / 140; one workgroup per CU: 32, 49, 74, 101, 151.
   const long long wgs = (M + 127) / 128, nblocks = N / 32, resident = 3LL * compute_units();
   const long long parts = std::min(nblocks, std::max(1LL, resident / wgs)), per = (nblocks + parts - 1) / parts;
   const dim3 grid((unsigned)wgs, (unsigned)((nblocks + per - 1) / per));

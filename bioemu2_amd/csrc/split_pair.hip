@@ -140,7 +140,7 @@ int split_cat_proj(const float* x1, const float* x2, const f16* W, const float* 
   const int tiles = (int)((P + 31) / 32);
   // Few tiles: a column block (and 32 KB of weights) a workgroup, four waves of which two workgroups share a CU, as
   // long as that is one round of workgroups.  us of the projection and two transitions, all columns / this: 1600 rows
-  // 53 / 46, 8100 rows 78 / 72, 16384 rows 95 / 95; past one round, 32400 rows 113 / 124.  The same bits.
+  // 53 / 46, 8100 rows 78 / 71, 16384 rows 91 / 88; past one round, 32400 rows 110 / 123.  The same bits.
   const int cus = compute_units();
   const bool few = tiles <= 2 * cus;
   const int waves = few ? 4 : kCatWaves, per = few ? 1 : 4;

@@ -10,7 +10,9 @@
 //                           a power of two more (their gain, one byte); a channel with
 //                           such a line is flagged.
 //   trimul_contract_kernel  o[d][i][j] = sum_k a[d][i][k] b[d][j][k] on 128 x 128 tiles;
-//                           gains of a flagged channel are undone 32 k at a time.
+//                           gains of a flagged channel are undone 32 k at a time (a wave
+//                           sums 32 k that hold one by themselves: there the last bits of
+//                           its 64 x 64 block depend on its other rows' gains).
 //   trimul_out_kernel       LN_out(o) Wp * sigmoid(LN_in(x) Wg) (+ x): o read from its planes,
 //                           32 pairs (128 bytes) of a channel per load, both weights resident in LDS.
 //
@@ -437,7 +439,7 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
   const unsigned tiles = (unsigned)(B * N * (plane_ld((int)N) / 32));
   {
     // As many parts of the eight column blocks as make one round of two workgroups per CU.  The call, all blocks / these
-    // parts (us): N = 40 46 / 29, N = 64 50 / 32, N = 100 66 / 52, N = 160 70 / 64; two rounds: 29, 32, 55, 68.
+    // parts (us): N = 40 48 / 31, N = 64 52 / 33, N = 100 69 / 56, N = 160 72 / 65; two rounds: 31, 34, 59, 70.
     const unsigned wgs = (tiles + 3) / 4, resident = 2u * compute_units();
     unsigned parts = 1;
     while (parts < 8 && 2 * parts * wgs <= resident) parts *= 2;
@@ -458,9 +460,9 @@ int split_trimul(const float* x, const uint8_t* mask, const float* norm_in_w, co
   if ((rc = check_launch("f32_trimul_contract"))) return rc;
   {
     const unsigned cus = compute_units();
-    // Up to two rounds of a tile a workgroup (the call, us, a tile a wave / a workgroup: N = 40 39 / 29, N = 64 43 / 32,
-    // N = 80 48 / 38, N = 128, 512 tiles, 55 / 54, N = 160, 800 tiles, 64 / 81).
-    const bool few = tiles <= 2 * cus;
+    // One round of a tile a workgroup (the call, us, a tile a wave / a workgroup: N = 40 38 / 31, N = 64 41 / 33, N = 80,
+    // 240 tiles, 48 / 40; N = 100, 400 tiles, 54 / 56, N = 160, 800 tiles, 65 / 88).
+    const bool few = tiles <= cus;
     const auto kernel = few ? trimul_out_kernel<true> : trimul_out_kernel<false>;
     const hipError_t e =
         hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kOutSmem);
