@@ -38,6 +38,12 @@ class PreparedParams:
         self._src: list[nn.Parameter] | None = None
         self._val: tuple[Tensor, ...] | None = None
 
+    def __getstate__(self) -> dict:
+        return {"spec": self.spec}   # a copy or a saved module has parameters of its own, and prepares them itself
+
+    def __setstate__(self, state: dict) -> None:
+        PreparedParams.__init__(self, state["spec"])
+
     def get(self, module: nn.Module) -> tuple[Tensor, ...]:
         params = [_find(module, path) for path in self._paths]
         key = tuple((id(p), p.data_ptr(), p._version, p.device, p.dtype) for p in params)
