@@ -62,10 +62,13 @@ def mask_u8(mask: Tensor) -> Tensor:
     return mask.ne(0).contiguous().view(torch.uint8)
 
 
+_profiler_enabled = torch.autograd._profiler_enabled
+
+
 def _plain_call(args: tuple) -> bool:
     """True where the dispatcher has nothing to do for an op but to run its body: no gradients, no compiler, tracer,
     functorch transform, forward-mode level, mode or profiler looking on, and plain tensors only."""
-    if torch.compiler.is_compiling() or torch.is_grad_enabled() or torch.autograd._profiler_enabled():
+    if torch.compiler.is_compiling() or torch.is_grad_enabled() or _profiler_enabled():
         return False
     for a in args:
         if isinstance(a, Tensor) and (type(a) is not Tensor or not a.is_cuda):

@@ -34,9 +34,8 @@ class PreparedParams:
     def __init__(self, spec: list[tuple[str, torch.dtype]]):
         self.spec = spec
         self._paths = [tuple(name.split(".")) for name, _ in spec]
-        self._key: tuple | None = None
-        self._src: list[nn.Parameter] | None = None
-        self._val: tuple[Tensor, ...] | None = None
+        # (prepared copies, [(parameter, data_ptr, version, device index, dtype)]), replaced as one
+        self._cache: tuple[tuple[Tensor, ...], list[tuple]] | None = None
 
     def __getstate__(self) -> dict:
         return {"spec": self.spec}   # a copy or a saved module has parameters of its own, and prepares them itself
@@ -45,11 +44,20 @@ class PreparedParams:
         PreparedParams.__init__(self, state["spec"])
 
     def get(self, module: nn.Module) -> tuple[Tensor, ...]:
+        cache = self._cache
+        if cache is not None:
+            for path, (src, ptr, version, device, dtype) in zip(self._paths, cache[1]):
+                p = _find(module, path)
+                if (p is not src or p.data_ptr() != ptr or p._version != version or p.dtype != dtype
+                        or p.get_device() != device):
+                    break
+            else:
+                return cache[0]
         params = [_find(module, path) for path in self._paths]
-        key = tuple((id(p), p.data_ptr(), p._version, p.device, p.dtype) for p in params)
-        if key != self._key or self._val is None:
-            self._val = tuple(
-                p.detach().to(dtype=dt).contiguous() for p, (_, dt) in zip(params, self.spec)
-            )
-            self._key, self._src = key, params
-        return self._val
+        val = self._pack(*(p.detach().to(dtype=dt).contiguous() for p, (_, dt) in zip(params, self.spec)))
+        self._cache = val, [(p, p.data_ptr(), p._version, p.get_device(), p.dtype) for p in params]
+        return val
+
+    def _pack(self, *prepared: Tensor) -> tuple[Tensor, ...]:
+        """What is kept of the copies: themselves, or what a subclass lays out from them."""
+        return prepared

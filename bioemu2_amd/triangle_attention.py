@@ -41,13 +41,8 @@ class _PackedTriAttParams(PreparedParams):
             + [(f"proj_{n}.weight", dtype) for n in ("q", "k", "v", "g", "b", "o")]
         )
 
-    def get(self, module: nn.Module) -> tuple[Tensor, ...]:
-        key_before = self._key
-        val = super().get(module)
-        if self._key != key_before or not hasattr(self, "_packed"):
-            nw, nb, wq, wk, wv, wg, wb, wo = val
-            self._packed = (nw, nb, torch.cat([wq, wk, wv, wg, wb], dim=0).contiguous(), wo)
-        return self._packed
+    def _pack(self, nw, nb, wq, wk, wv, wg, wb, wo) -> tuple[Tensor, ...]:
+        return nw, nb, torch.cat([wq, wk, wv, wg, wb], dim=0).contiguous(), wo
 
 
 class TriangleAttentionHip(nn.Module):
